@@ -274,3 +274,41 @@ def test_rabitq_multibit_flat_scan(lib, metric, mname, bits, n, d, nq, k):
     rids, rds = orc.flat_scan_topk(orc.RABITQ, metric, d, codes, qcodes, k, qbits=word)
     assert_topk_close(ids, ds, rids, rds, rtol=1e-4, atol=2e-5, tie_rtol=2e-4, label="rabitq %d-bit %s" % (bits, mname))
     st.destroy()
+
+
+@pytest.mark.parametrize("metric", [orc.L2, orc.IP, orc.COSINE])
+@pytest.mark.parametrize("n", [1, 63, 64, 65, 257])
+@pytest.mark.parametrize("d", [31, 32, 33, 36, 96])
+def test_encoders_at_the_edges_of_a_row_tile(lib, metric, n, d):
+    """64 rows x 32 dimensions are what a wave holds at a time: rows and dimensions around those, and dimensions that are
+    no multiple of the vector loads.  Bytes, so equal."""
+    L = lib.load_library()
+    rng = np.random.default_rng(1000 * n + d)
+    x = (rng.standard_normal((n, d)) * 0.3 + 0.5).astype(np.float32)
+    xb = dev(x)
+    for bits in (4, 8):
+        lb, diff = orc.sq_train(x, bits, metric)
+        ref = orc.sq_encode(x, bits, lb, diff, metric)
+        lbb, dfb, out = dev(lb), dev(diff), capi.DeviceBuffer(ref.nbytes)
+        capi.check(L.vsag_amd_sq_encode(xb.ptr, n, d, bits, metric, lbb.ptr, dfb.ptr, out.ptr, None))
+        assert np.array_equal(out.to_numpy(np.uint8, ref.shape), ref), bits
+        ulb, udiff = orc.sq_train_uniform(x, bits, metric, mode=3 if bits == 4 else 1)
+        ref = orc.squ_encode(x, bits, ulb, udiff, metric)
+        bb, out = dev(np.array([ulb, udiff], np.float32)), capi.DeviceBuffer(ref.nbytes)
+        capi.check(L.vsag_amd_squ_encode(xb.ptr, n, d, bits, metric, bb.ptr, out.ptr, None))
+        assert np.array_equal(out.to_numpy(np.uint8, ref.shape), ref), bits
+
+
+@pytest.mark.parametrize("kind", ["wide", "equal", "two values", "signs", "tail"])
+@pytest.mark.parametrize("n", [2047, 2049, 65537])
+def test_sq_bounds_of_awkward_columns(lib, kind, n):
+    """Columns whose keys crowd into one bin of the histogram, or spread over the whole float range."""
+    rng = np.random.default_rng(n)
+    x = {"wide": rng.standard_normal((n, 5)) * np.exp(rng.uniform(-80, 80, (n, 5))),
+         "equal": np.full((n, 5), 0.25), "two values": rng.integers(0, 2, (n, 5)) * 1e-3 + 1.0,
+         "signs": rng.choice([-1.0, 0.0, -0.0, 1.0], (n, 5)),
+         "tail": np.where(rng.random((n, 5)) < 1e-3, 1e6, rng.random((n, 5)))}[kind].astype(np.float32)
+    for bits in (4, 8):
+        lb, diff = _train(lib, x, bits, orc.L2, capi.SQ_TRAIN_TRUNC_BOUND)
+        rlb, rdiff = orc.sq_train(x, bits, orc.L2, mode=capi.SQ_TRAIN_TRUNC_BOUND)
+        assert np.array_equal(lb, rlb) and np.array_equal(diff, rdiff), (bits, lb, rlb)
