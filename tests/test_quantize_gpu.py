@@ -277,11 +277,12 @@ def test_rabitq_multibit_flat_scan(lib, metric, mname, bits, n, d, nq, k):
 
 
 @pytest.mark.parametrize("metric", [orc.L2, orc.IP, orc.COSINE])
-@pytest.mark.parametrize("n", [1, 63, 64, 65, 257])
-@pytest.mark.parametrize("d", [31, 32, 33, 36, 96])
+@pytest.mark.parametrize("n,d", [(n, d) for n in (1, 63, 65, 257) for d in (1, 31, 32, 33, 36, 96)] +
+                         [(n, d) for n in (32768, 32769, 32831) for d in (7, 33, 36)] + [(3, 4096), (65, 4100)])
 def test_encoders_at_the_edges_of_a_row_tile(lib, metric, n, d):
-    """64 rows x 32 dimensions are what a wave holds at a time: rows and dimensions around those, and dimensions that are
-    no multiple of the vector loads.  Bytes, so equal."""
+    """64 rows x 32 dimensions are what a wave holds at a time of many rows, a whole row of few: rows and dimensions around
+    those and around where one changes to the other, and dimensions that are no multiple of the vector loads.  Bytes, so
+    equal."""
     L = lib.load_library()
     rng = np.random.default_rng(1000 * n + d)
     x = (rng.standard_normal((n, d)) * 0.3 + 0.5).astype(np.float32)

@@ -315,6 +315,110 @@ squ_encode_kernel(const float* x, uint64_t n, uint32_t dim, int metric, const fl
     }
 }
 
+// The same for few rows (the queries of a search): a wave per row, which it keeps in LDS, and the norm of a cosine row with
+// it.  64 rows per wave would leave most of the machine idle and wait for memory once per chunk (987 queries x 128: 21 us
+// against 4 us).  The sums in element order are one lane's chain of adds over LDS; the sum of the codes is a sum of small
+// integers, exact in any order.  dim <= kRowEncodeMaxDim.
+constexpr uint32_t kRowEncodeMaxDim = 4096;
+constexpr uint64_t kRowEncodeMaxRows = 32768;  // 64 rows per wave: one wave per SIMD from twice that on
+
+template <int BITS>
+__global__ void __launch_bounds__(256)
+squ_encode_row_kernel(const float* x, uint64_t n, uint32_t dim, uint32_t dim_pad, int metric, const float* bounds,
+                      uint32_t code_size, uint32_t payload, uint32_t off_norm, uint32_t off_sum, uint32_t off_codes_sum,
+                      uint8_t* codes) {
+    extern __shared__ __align__(16) float row_lds[];
+    constexpr uint32_t kDims = 32 / BITS;  // per code word
+    const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const uint64_t row = static_cast<uint64_t>(blockIdx.x) * 4 + wave;
+    if (row >= n) {
+        return;
+    }
+    float* v = row_lds + wave * dim_pad;  // dim_pad: a multiple of 32
+    for (uint32_t d = lane; d < dim_pad; d += kWave) {
+        v[d] = d < dim ? x[row * dim + d] : 0.0F;
+    }
+    wave_lds_fence();
+    float nrm = 1.0F;
+    if (metric == VSAG_AMD_METRIC_COSINE) {
+        float s = 0.0F;  // every lane the same chain (row_norm_kernel's; the zeros behind the row add nothing)
+        for (uint32_t d = 0; d < dim_pad; d += 32) {
+#pragma unroll
+            for (uint32_t u = 0; u < 32; u += 4) {
+                const float4 f = *reinterpret_cast<const float4*>(v + d + u);
+                s = f.x * f.x + s;
+                s = f.y * f.y + s;
+                s = f.z * f.z + s;
+                s = f.w * f.w + s;
+            }
+        }
+        nrm = sqrtf(s);
+        nrm = nrm == 0.0F ? 1.0F : nrm;
+        wave_lds_fence();
+    }
+    const float lb = bounds[0], diff = bounds[1];
+    const float inv_diff = diff == 0.0F ? 0.0F : 1.0F / diff;
+    const float levels = BITS == 4 ? 15.0F : 255.0F;
+    uint8_t* c = codes + row * code_size;
+    const bool aligned = (reinterpret_cast<uintptr_t>(codes) & 3U) == 0;
+    auto put = [&](uint32_t at, uint32_t word) {
+        if (aligned) {
+            *reinterpret_cast<uint32_t*>(c + at) = word;
+        } else {
+            for (uint32_t k = 0; k < 4; ++k) {
+                c[at + k] = static_cast<uint8_t>(word >> (8 * k));
+            }
+        }
+    };
+    const uint32_t payload_words = (payload + 3) / 4;
+    uint32_t norm_part = 0, codes_sum = 0;
+    for (uint32_t w = lane; w < payload_words; w += kWave) {
+        uint32_t word = 0;
+#pragma unroll
+        for (uint32_t e = 0; e < kDims; ++e) {
+            const uint32_t d = w * kDims + e;
+            if (d < dim) {
+                const float value = metric == VSAG_AMD_METRIC_COSINE ? v[d] / nrm : v[d];
+                v[d] = value;
+                const uint32_t scaled = static_cast<uint8_t>(levels * clamp_delta((value - lb) * inv_diff));
+                word |= scaled << (e * BITS);
+                norm_part += scaled * scaled;
+                codes_sum += scaled;
+            }
+        }
+        put(4 * w, word);
+    }
+    for (int off = 32; off > 0; off >>= 1) {
+        norm_part += __shfl_xor(norm_part, off);
+        codes_sum += __shfl_xor(codes_sum, off);
+    }
+    float sum = 0.0F;
+    if (metric != VSAG_AMD_METRIC_L2) {
+        wave_lds_fence();
+        for (uint32_t d = 0; d < dim_pad; d += 32) {
+#pragma unroll
+            for (uint32_t u = 0; u < 32; u += 4) {
+                const float4 f = *reinterpret_cast<const float4*>(v + d + u);
+                sum += f.x;
+                sum += f.y;
+                sum += f.z;
+                sum += f.w;
+            }
+        }
+    }
+    for (uint32_t b = 4 * (payload_words + lane); b < code_size; b += 4 * kWave) {
+        uint32_t word = 0;
+        if (metric == VSAG_AMD_METRIC_L2) {
+            word = b == off_norm ? norm_part : 0U;  // a u64 whose upper half is zero
+        } else if (b == off_sum) {
+            word = __float_as_uint(sum);
+        } else if (BITS == 4 && b == off_codes_sum) {
+            word = __float_as_uint(static_cast<float>(codes_sum));
+        }
+        put(b, word);
+    }
+}
+
 // ------------------------------------------------------------------ C = A * B^T, k in element order
 // C[i][j] = sum_k A[i][k] * B[j][k], one unfused multiply and add per k in increasing k, so every output
 // equals a scalar running-sum dot product (the RowMajor sgemv of random_orthogonal_transformer.cpp:58-77
@@ -1169,6 +1273,15 @@ squ_encode_launch(const float* x, uint64_t n, uint32_t dim, int bits, int metric
     uint32_t off_norm = off;
     uint32_t off_sum = off + (norm ? 8 : 0);
     uint32_t off_codes_sum = off_sum + align;
+    if (n <= kRowEncodeMaxRows && dim <= kRowEncodeMaxDim) {
+        const uint32_t dim_pad = static_cast<uint32_t>(round_up(dim, 32));
+        const dim3 grid(static_cast<uint32_t>(div_up(n, 4)));
+        auto kernel = bits == 4 ? squ_encode_row_kernel<4> : squ_encode_row_kernel<8>;
+        hipLaunchKernelGGL(kernel, grid, dim3(256), 4ull * dim_pad * 4, st, x, n, dim, dim_pad, metric, bounds, code_size,
+                           payload, off_norm, off_sum, off_codes_sum, codes);
+        VA_HIP(hipGetLastError());
+        return 0;
+    }
     // Cosine needs a float per row; a caller that must not allocate brings them (norm_scratch, n floats).
     float* norms = nullptr;
     if (metric == VSAG_AMD_METRIC_COSINE) {
