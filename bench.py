@@ -569,12 +569,13 @@ def run_c3(env):
             b.free()
     flops = 2.0 * n * k * d
     tf = flops / (kms * 1e-3) / 1e12
-    roof = {"bound": "mfma", "achieved": tf, "peak": MFMA_F32_PEAK_TFLOPS, "unit": "TFLOP/s",
-            "frac": tf / MFMA_F32_PEAK_TFLOPS,
-            # rocprofv3 --pmc FETCH_SIZE (x 2.00) + WRITE_SIZE of one launch: profiles/kmeans_assign_c3.md.  Above the
-            # 3.9 GB of inputs: an XCD's L2 holds the k-slices of one macro tile (1024 rows x 2048 centroids) at a time.
-            "traffic": 11786276.4 * 2.00 * 1024 + 2125360.1 * 1024 if (n, d, k) == (1000000, 960, 4096) else None,
-            "kernel": "kmeans_assign_tile_kernel<4>" if d % 4 == 0 and k > 384 else
+    # The contraction pre-selects on the fp16 matrix cores (kmeans_h16.hip) where there is enough of it: kernel_ms then
+    # spans that pass and the fp32 rescoring of what it leaves, the flops are the contraction's.
+    h16 = 32 <= d <= 8192 and k >= 256 and k * d >= 49152 and n * k * d >= 4e9
+    peak = MFMA_F16_PEAK_TFLOPS if h16 else MFMA_F32_PEAK_TFLOPS
+    roof = {"bound": "mfma", "achieved": tf, "peak": peak, "unit": "TFLOP/s", "frac": tf / peak, "traffic": None,
+            "kernel": "kmeans_h16_kernel + kmeans_round_rows_kernel + kmeans_h16_rescore_kernel" if h16 else
+                      "kmeans_assign_tile_kernel<4>" if d % 4 == 0 and k > 384 else
                       "kmeans_assign_tile_kernel<2>" if d % 4 == 0 else "kmeans_assign_kernel", "kernel_ms": kms,
             "flops_per_launch": flops}
     return env.base_line("k-means assign rows/s", "rows/s", n / sec, sec, "f32",

@@ -155,3 +155,93 @@ def test_plus_plus_seeding_on_coincident_rows(lib):
     assert np.array_equal(picks, rpicks) and list(picks[3:]) == [0, 75, 149]
     L = capi.load_library()
     assert L.vsag_amd_kmeans_init_plus_plus(1, 10, 4, 3, 10, draws.ctypes.data, 1, None, None, 0, None) == capi.INVALID_ARGUMENT
+
+
+def _routed_data(kind, n, d, k):
+    rng = np.random.default_rng(n + 3 * d + k)
+    x = rng.standard_normal((n, d)).astype(np.float32)
+    cent = x[rng.choice(n, k, replace=False)].copy()
+    if kind == "offset":  # far from the origin: the centre takes the common part away
+        x += 30.0
+        cent += 30.0
+    elif kind == "scaled":  # lengths over twelve octaves
+        x *= np.exp2(rng.integers(-6, 7, (n, 1))).astype(np.float32)
+    elif kind == "copies":  # every centroid five times: whole groups stay possible, and most rows go to the fp32 kernels
+        cent = np.tile(cent[: k // 5], (5, 1))[rng.permutation(k // 5 * 5)]
+        cent = np.concatenate([cent, cent[: k - len(cent)]])
+    elif kind == "same":  # one point: every distance ties
+        x[:] = x[0]
+        cent[:] = x[0]
+    return x, cent
+
+
+# At the edges of the pre-selection's tiles (256 x 256 x 64), with 4e9 products and more each.
+@pytest.mark.parametrize("kind,n,d,k", [("plain", 20011, 130, 1601), ("plain", 65537, 64, 1024), ("plain", 4096, 1030, 1025),
+                                        ("plain", 62001, 257, 257), ("offset", 20011, 101, 2049), ("scaled", 16385, 128, 2048),
+                                        ("copies", 16385, 128, 2050), ("same", 16384, 128, 2048), ("plain", 33000, 64, 2111)])
+def test_assign_after_the_fp16_preselection(lib, kind, n, d, k):
+    x, cent = _routed_data(kind, n, d, k)
+    labels, mind, loss = gpu_assign(x, cent)
+    assert labels.min() >= 0 and labels.max() < k
+    check_assignment(x, cent, labels, mind)
+    # bit for bit what the fp32 kernels return: pieces too small for the pre-selection take those
+    rows = min(n, int(3.9e9 / (k * d)))
+    for r0 in range(0, n, rows):
+        few, few_mind, _ = gpu_assign(x[r0:r0 + rows], cent)
+        assert np.array_equal(labels[r0:r0 + rows], few)
+        assert np.array_equal(mind[r0:r0 + rows].view(np.int32), few_mind.view(np.int32))
+    x64, c64 = x.astype(np.float64), cent.astype(np.float64)
+    assert abs(loss - (mind.astype(np.float64) + (x64 ** 2).sum(1)).mean()) <= 1e-5 * (x64 ** 2).sum(1).mean()
+    if kind in ("copies", "same"):  # of equal centroids the first
+        first = {}
+        for j in range(k):
+            first.setdefault(c64[j].tobytes(), j)
+        assert all(first[c64[j].tobytes()] == j for j in np.unique(labels))
+
+
+def test_assign_after_the_fp16_preselection_with_values_out_of_range(lib):
+    # rows that fp16 or the error bound cannot cover go to the fp32 kernels; what they return is what those return alone
+    n, d, k = 16500, 128, 2048
+    x, cent = _routed_data("plain", n, d, k)
+    odd = [3, 64, 700, 4097, n - 1]
+    x[3, 5] = np.nan
+    x[64] *= np.float32(1e18)
+    x[700] = 0.0
+    x[4097, 0] = np.inf
+    x[n - 1] *= np.float32(1e-25)
+    labels, mind, _ = gpu_assign(x, cent)
+    few, few_mind, _ = gpu_assign(x[odd].copy(), cent)  # too few rows for the pre-selection
+    assert np.array_equal(labels[odd], few)
+    assert np.array_equal(mind[odd].view(np.int32), few_mind.view(np.int32))
+    keep = np.setdiff1d(np.arange(n), odd)
+    check_assignment(x[keep], cent, labels[keep], mind[keep])
+    cent[7, 3] = np.inf  # one centroid out of range: every row takes the fp32 kernels, and nobody chooses it
+    labels2, _, _ = gpu_assign(x[keep], cent)
+    assert not (labels2 == 7).any() and (labels2 == labels[keep]).mean() > 0.999
+
+
+def test_run_with_the_fp16_preselection_keeps_its_rows(lib):
+    # the rows are rounded once per run; the centre is that of the first iteration
+    L = lib.load_library()
+    n, d, k, iters = 16400, 128, 2048, 4
+    rng = np.random.default_rng(5)
+    x, _ = gaussian_mixture(rng, n, d, 300, 0.2, uniform_means=False)
+    cent0 = x[rng.choice(n, k, replace=False)].copy()
+    xb, cb = dev(x), dev(cent0)
+    labels = capi.DeviceBuffer(n * 4)
+    loss = C.c_double()
+    wsb = L.vsag_amd_kmeans_run_workspace_bytes(n, d, k)
+    ws = capi.DeviceBuffer(wsb)
+    capi.check(L.vsag_amd_kmeans_run(xb.ptr, n, d, cb.ptr, k, iters, 7, labels.ptr, C.byref(loss), ws.ptr, wsb, None))
+    lab = labels.to_numpy(np.int32, (n,))
+    # the same steps one by one
+    cc, last = dev(cent0), None
+    counts = capi.DeviceBuffer(k * 4)
+    for _ in range(iters):
+        last = gpu_assign(x, cc.to_numpy(np.float32, (k, d)))
+        lb = dev(last[0])
+        wsu = capi.DeviceBuffer(L.vsag_amd_kmeans_update_workspace_bytes(n, d, k))
+        capi.check(L.vsag_amd_kmeans_update(xb.ptr, lb.ptr, n, d, k, cc.ptr, counts.ptr, wsu.ptr,
+                                            L.vsag_amd_kmeans_update_workspace_bytes(n, d, k), None))
+        assert (counts.to_numpy(np.int32, (k,)) > 0).all()
+    assert np.array_equal(lab, last[0]) and loss.value == last[2]

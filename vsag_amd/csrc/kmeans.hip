@@ -19,6 +19,7 @@
 #include <vector>
 
 #include "common.h"
+#include "kmeans_h16.h"
 
 namespace vsag_amd {
 
@@ -72,10 +73,47 @@ stage_store(float4* plane, uint32_t row, uint32_t g, float4 v) {
     *reinterpret_cast<float2*>(odd) = make_float2(v.y, v.w);
 }
 
+// Which rows an assignment kernel works on: all (null pointers) or those that the fp16 pre-selection left open
+// (kmeans_h16.hip): a flag per row, a word per 64 rows that says whether one of them is set, and one for all rows.  Such a
+// launch has a workgroup per compute unit that walks the tiles, so that it costs little when nothing is open (a workgroup
+// per tile, each of which found its rows done, took 178 us at 1M rows x 4096 centroids).
+struct OpenRows {
+    const uint8_t* row;
+    const uint32_t* per64;
+    const uint32_t* all;
+    __device__ bool
+    none() const {
+        return all != nullptr && *all == 0;
+    }
+    OpenRows
+    from(uint64_t r0) const {  // r0: a multiple of 64
+        return row == nullptr ? *this : OpenRows{row + r0, per64 + r0 / 64, all};
+    }
+    __device__ bool
+    any(uint64_t row0, uint32_t count, uint64_t n) const {
+        if (per64 == nullptr) {
+            return true;
+        }
+        uint32_t found = 0;
+        for (uint64_t r = row0; r < row0 + count && r < n; r += 64) {
+            found |= per64[r / 64];
+        }
+        return found != 0;
+    }
+    __device__ bool
+    has(uint64_t r) const {
+        return row == nullptr || row[r] != 0;
+    }
+};
+
 __global__ void __launch_bounds__(256, 2)
 kmeans_assign_kernel(const float* __restrict__ X, uint64_t n, const float* __restrict__ C, uint32_t k, uint32_t dim,
-                     const float* __restrict__ ynorm, unsigned long long* __restrict__ best, uint32_t groups) {
+                     const float* __restrict__ ynorm, unsigned long long* __restrict__ best, uint32_t groups,
+                     OpenRows open) {
     __shared__ Stage stage[2];  // 64 KiB: two workgroups fit the 160 KiB of a gfx950 CU
+    if (open.none()) {
+        return;
+    }
 
     const uint32_t tid = threadIdx.x;
     const uint32_t lane = tid & 63;
@@ -84,7 +122,6 @@ kmeans_assign_kernel(const float* __restrict__ X, uint64_t n, const float* __res
     const uint32_t wn = wave >> 1;  // which 64 data rows of the tile
     const uint32_t half = lane >> 5;
     const uint32_t l32 = lane & 31;
-    const uint64_t row0 = static_cast<uint64_t>(blockIdx.y) * BN;
     const bool aligned = (dim & 3) == 0;
     const uint32_t ktiles = (dim + BK - 1) / BK;
     const uint32_t ctiles = (k + BM - 1) / BM;
@@ -98,6 +135,10 @@ kmeans_assign_kernel(const float* __restrict__ X, uint64_t n, const float* __res
         ld_g[r] = idx & 7;
     }
 
+    for (uint64_t row0 = static_cast<uint64_t>(blockIdx.y) * BN; row0 < n; row0 += static_cast<uint64_t>(gridDim.y) * BN) {
+    if (!open.any(row0, BN, n)) {
+        continue;
+    }
     unsigned long long my_best[2] = {~0ull, ~0ull};  // per n-block of this wave, for row l32
 
     for (uint32_t ct = blockIdx.x; ct < ctiles; ct += groups) {
@@ -199,9 +240,10 @@ kmeans_assign_kernel(const float* __restrict__ X, uint64_t n, const float* __res
         unsigned long long other = __shfl_xor(my_best[j], 32);
         unsigned long long key = other < my_best[j] ? other : my_best[j];
         uint64_t row = row0 + wn * 64 + j * 32 + l32;
-        if (half == 0 && row < n && key != ~0ull) {
+        if (half == 0 && row < n && key != ~0ull && open.has(row)) {
             atomicMin(&best[row], key);
         }
+    }
     }
 }
 
@@ -245,6 +287,7 @@ struct TilePlan {
     uint64_t ld;       // STORE: floats per row of the output
     float alpha;       // STORE: factor of the product
     uint32_t macros;
+    OpenRows open;
 };
 
 constexpr int kTileRows = 256;  // data rows per workgroup tile
@@ -260,17 +303,17 @@ tile_lds_bytes(int mi) {
 // STORE: instead of the argmin, every product goes out as out[m * plan.ld + n] = (ynorm ? ynorm[n] : 0) + plan.alpha *
 // <c_m, x_n> (m a row of C, n a row of X; `best` is that float matrix, ynorm is indexed by rows of X): the table of
 // approximate distances a routing call selects from (scan.hip, route_select_kernel).
-template <int MI, bool STORE = false>
-__global__ void __launch_bounds__(kTileThreads, 1)
-kmeans_assign_tile_kernel(const float* __restrict__ X, uint64_t n, const float* __restrict__ C, uint32_t k, uint32_t dim,
-                          const float* __restrict__ ynorm, unsigned long long* __restrict__ best, TilePlan plan) {
+template <int MI, bool STORE, bool OPEN>
+__device__ __forceinline__ void
+assign_tile(const float* __restrict__ X, uint64_t n, const float* __restrict__ C, uint32_t k, uint32_t dim,
+            const float* __restrict__ ynorm, unsigned long long* __restrict__ best, const TilePlan& plan, uint32_t id) {
     constexpr uint32_t TM = 64 * MI;                   // centroids per tile
     constexpr uint32_t kSlot = 4 * (TM + kTileRows);   // float4 per ring slot: A planes, then B planes
     constexpr int RA = MI / 2;                         // float4 of A a thread loads per stage
     extern __shared__ float4 lds[];
 
-    const uint32_t xcd = blockIdx.x & 7;
-    const uint32_t local = blockIdx.x >> 3;
+    const uint32_t xcd = id & 7;
+    const uint32_t local = id >> 3;
     const uint32_t macro = (local >> 5) * 8 + xcd;
     if (macro >= plan.macros) {
         return;
@@ -279,6 +322,9 @@ kmeans_assign_tile_kernel(const float* __restrict__ X, uint64_t n, const float* 
     const uint32_t rt = (macro / plan.mcols) * (32U >> plan.mc_log2) + (within >> plan.mc_log2);
     const uint32_t ct = ((macro % plan.mcols) << plan.mc_log2) + (within & ((1U << plan.mc_log2) - 1));
     if (rt >= plan.rtiles || ct >= plan.ctiles) {
+        return;
+    }
+    if (OPEN && !plan.open.any(static_cast<uint64_t>(rt) * kTileRows, kTileRows, n)) {
         return;
     }
 
@@ -481,9 +527,31 @@ kmeans_assign_tile_kernel(const float* __restrict__ X, uint64_t n, const float* 
         const unsigned long long other = __shfl_xor(key, 32);
         key = other < key ? other : key;
         const uint64_t row = row0 + wn * 64 + j * 32 + l32;
-        if (half == 0 && row < n && key != ~0ull) {
+        if (half == 0 && row < n && key != ~0ull && (!OPEN || plan.open.has(row))) {
             atomicMin(&best[row], key);
         }
+    }
+}
+
+template <int MI, bool STORE = false>
+__global__ void __launch_bounds__(kTileThreads, 1)
+kmeans_assign_tile_kernel(const float* __restrict__ X, uint64_t n, const float* __restrict__ C, uint32_t k, uint32_t dim,
+                          const float* __restrict__ ynorm, unsigned long long* __restrict__ best, TilePlan plan) {
+    assign_tile<MI, STORE, false>(X, n, C, k, dim, ynorm, best, plan, blockIdx.x);
+}
+
+// The tiles that hold an open row; gridDim.x is a multiple of 8, so a workgroup's tiles stay on its XCD.
+template <int MI>
+__global__ void __launch_bounds__(kTileThreads, 1)
+kmeans_assign_open_kernel(const float* __restrict__ X, uint64_t n, const float* __restrict__ C, uint32_t k, uint32_t dim,
+                          const float* __restrict__ ynorm, unsigned long long* __restrict__ best, TilePlan plan,
+                          uint32_t tiles) {
+    if (plan.open.none()) {
+        return;
+    }
+    for (uint32_t id = blockIdx.x; id < tiles; id += gridDim.x) {
+        assign_tile<MI, false, true>(X, n, C, k, dim, ynorm, best, plan, id);
+        __syncthreads();  // the next tile's first stages overwrite LDS
     }
 }
 
@@ -546,14 +614,25 @@ kmeans_finalize_kernel(const unsigned long long* best, const float* xnorm, uint6
     }
 }
 
-__global__ void
+// The block sums in a fixed order: a thread its run of them, then a tree over the threads (one thread took 197 us for the
+// 3907 sums of 1M rows).
+__global__ void __launch_bounds__(1024)
 loss_reduce_kernel(const double* partial, uint64_t count, uint64_t n, double* loss) {
-    if (threadIdx.x == 0 && blockIdx.x == 0) {
-        double s = 0.0;
-        for (uint64_t i = 0; i < count; ++i) {
-            s += partial[i];
+    __shared__ double sums[1024];
+    double s = 0.0;
+    for (uint64_t i = threadIdx.x; i < count; i += blockDim.x) {
+        s += partial[i];
+    }
+    sums[threadIdx.x] = s;
+    __syncthreads();
+    for (uint32_t w = 512; w > 0; w >>= 1) {
+        if (threadIdx.x < w) {
+            sums[threadIdx.x] += sums[threadIdx.x + w];
         }
-        *loss = s / static_cast<float>(n);
+        __syncthreads();
+    }
+    if (threadIdx.x == 0) {
+        *loss = sums[0] / static_cast<float>(n);
     }
 }
 
@@ -689,6 +768,7 @@ launch_row_products(const float* x, uint64_t nx, const float* c, uint32_t nc, ui
     plan.macros = mrows * plan.mcols;
     plan.ld = ld;
     plan.alpha = alpha;
+    plan.open = {nullptr, nullptr, nullptr};
     const uint32_t per_xcd = (plan.macros + 7) / 8;
     const dim3 grid(per_xcd * 32 * 8);
     hipLaunchKernelGGL((kmeans_assign_tile_kernel<4, true>), grid, dim3(kTileThreads), tile_lds_bytes(4), st, x, nx, c, nc,
@@ -737,15 +817,21 @@ struct AssignBuffers {
     unsigned long long* best;
     double* partial;
     double* loss_tmp;
+    bool h16;  // the fp16 pre-selection comes first (kmeans_h16.hip)
+    KmeansH16Buffers pre;
 };
 
 static size_t
-carve_assign(Carver& c, uint64_t n, uint32_t k, AssignBuffers* b) {
+carve_assign(Carver& c, uint64_t n, uint32_t dim, uint32_t k, AssignBuffers* b) {
     b->ynorm = c.take<float>(k);
     b->xnorm = c.take<float>(n);
     b->best = c.take<unsigned long long>(n);
     b->partial = c.take<double>(div_up(n, 256));
     b->loss_tmp = c.take<double>(1);
+    b->h16 = kmeans_h16_takes(n, dim, k);
+    if (b->h16) {
+        carve_kmeans_h16(c, n, dim, k, &b->pre);
+    }
     return c.used;
 }
 
@@ -754,14 +840,22 @@ assign_launch(const float* x, uint64_t n, uint32_t dim, const float* cent, uint3
               float* min_dist, double* loss_dev, const AssignBuffers& b, bool have_xnorm, hipStream_t st) {
     hipLaunchKernelGGL(row_sqnorm_kernel, dim3(static_cast<uint32_t>(div_up(k, 4))), dim3(256), 0, st, cent,
                        static_cast<uint64_t>(k), dim, b.ynorm);
-    if (!have_xnorm) {
+    if (!have_xnorm && !b.h16) {
         hipLaunchKernelGGL(row_sqnorm_kernel, dim3(static_cast<uint32_t>(div_up(n, 4))), dim3(256), 0, st, x, n, dim,
                            b.xnorm);
     }
-    hipLaunchKernelGGL(fill_u64_kernel, dim3(static_cast<uint32_t>(div_up(n, 256))), dim3(256), 0, st, b.best, ~0ull,
-                       n);
+    if (!b.h16) {
+        hipLaunchKernelGGL(fill_u64_kernel, dim3(static_cast<uint32_t>(div_up(n, 256))), dim3(256), 0, st, b.best, ~0ull,
+                           n);
+    }
     uint32_t ctiles = (k + BM - 1) / BM;
     timing_begin(st);
+    OpenRows open = {nullptr, nullptr, nullptr};
+    if (b.h16) {
+        VA_TRY(launch_kmeans_h16(x, n, dim, cent, k, b.ynorm, b.xnorm, have_xnorm, b.best, b.pre, st));
+        // what follows does the rows that were left open: usually none, and its workgroups return at once
+        open = {b.pre.row_open, b.pre.open64, b.pre.maxima + 3};
+    }
     if ((dim & 3) == 0) {
         // 256 centroids per tile when there are enough of them to fill it, else 128
         const int mi = k > 384 ? 4 : 2;
@@ -769,13 +863,16 @@ assign_launch(const float* x, uint64_t n, uint32_t dim, const float* cent, uint3
         static std::once_flag lds_once;
         static hipError_t lds_rc = hipSuccess;
         std::call_once(lds_once, []() {
-            lds_rc = hipFuncSetAttribute(reinterpret_cast<const void*>(kmeans_assign_tile_kernel<2>),
-                                         hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(tile_lds_bytes(2)));
-            if (lds_rc == hipSuccess) {
-                lds_rc = hipFuncSetAttribute(reinterpret_cast<const void*>(kmeans_assign_tile_kernel<4>),
-                                             hipFuncAttributeMaxDynamicSharedMemorySize,
-                                             static_cast<int>(tile_lds_bytes(4)));
-            }
+            auto allow = [](const void* kernel, int mi_of) {
+                if (lds_rc == hipSuccess) {
+                    lds_rc = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                                 static_cast<int>(tile_lds_bytes(mi_of)));
+                }
+            };
+            allow(reinterpret_cast<const void*>(kmeans_assign_tile_kernel<2>), 2);
+            allow(reinterpret_cast<const void*>(kmeans_assign_tile_kernel<4>), 4);
+            allow(reinterpret_cast<const void*>(kmeans_assign_open_kernel<2>), 2);
+            allow(reinterpret_cast<const void*>(kmeans_assign_open_kernel<4>), 4);
         });
         VA_HIP(lds_rc);
         // rows go slab by slab so that the tile count stays far inside the grid limit
@@ -791,9 +888,21 @@ assign_launch(const float* x, uint64_t n, uint32_t dim, const float* cent, uint3
             plan.macros = mrows * plan.mcols;
             plan.ld = 0;
             plan.alpha = 0.0F;
+            plan.open = open.from(r0);
             const uint32_t per_xcd = (plan.macros + 7) / 8;
-            const dim3 grid(per_xcd * 32 * 8);
-            if (mi == 4) {
+            const uint32_t tiles = per_xcd * 32 * 8;
+            const dim3 grid(tiles);
+            if (b.h16) {
+                const uint32_t cus = static_cast<uint32_t>(device_cu_count()) / 8 * 8;
+                const dim3 few(tiles < cus || cus == 0 ? tiles : cus);
+                if (mi == 4) {
+                    hipLaunchKernelGGL(kmeans_assign_open_kernel<4>, few, dim3(kTileThreads), tile_lds_bytes(4), st,
+                                       x + r0 * dim, rows, cent, k, dim, b.ynorm, b.best + r0, plan, tiles);
+                } else {
+                    hipLaunchKernelGGL(kmeans_assign_open_kernel<2>, few, dim3(kTileThreads), tile_lds_bytes(2), st,
+                                       x + r0 * dim, rows, cent, k, dim, b.ynorm, b.best + r0, plan, tiles);
+                }
+            } else if (mi == 4) {
                 hipLaunchKernelGGL(kmeans_assign_tile_kernel<4>, grid, dim3(kTileThreads), tile_lds_bytes(4), st,
                                    x + r0 * dim, rows, cent, k, dim, b.ynorm, b.best + r0, plan);
             } else {
@@ -807,15 +916,16 @@ assign_launch(const float* x, uint64_t n, uint32_t dim, const float* cent, uint3
         const uint64_t slab_rows = 65535ull * BN;
         for (uint64_t r0 = 0; r0 < n; r0 += slab_rows) {
             uint64_t rows = n - r0 < slab_rows ? n - r0 : slab_rows;
-            dim3 grid(groups, static_cast<uint32_t>(div_up(rows, BN)));
+            const uint32_t rtiles = static_cast<uint32_t>(div_up(rows, BN));
+            dim3 grid(groups, b.h16 && rtiles > 128 ? 128 : rtiles);
             hipLaunchKernelGGL(kmeans_assign_kernel, grid, dim3(256), 0, st, x + r0 * dim, rows, cent, k, dim, b.ynorm,
-                               b.best + r0, groups);
+                               b.best + r0, groups, open.from(r0));
         }
     }
     timing_end(st);
     hipLaunchKernelGGL(kmeans_finalize_kernel, dim3(static_cast<uint32_t>(div_up(n, 256))), dim3(256), 0, st, b.best,
                        b.xnorm, n, labels, min_dist, b.partial);
-    hipLaunchKernelGGL(loss_reduce_kernel, dim3(1), dim3(64), 0, st, b.partial, div_up(n, 256), n,
+    hipLaunchKernelGGL(loss_reduce_kernel, dim3(1), dim3(1024), 0, st, b.partial, div_up(n, 256), n,
                        loss_dev ? loss_dev : b.loss_tmp);
     VA_HIP(hipGetLastError());
     return 0;
@@ -1192,10 +1302,9 @@ vsag_amd_kmeans_init_plus_plus(const float* x_dev, uint64_t n, uint32_t dim, uin
 
 extern "C" size_t
 vsag_amd_kmeans_assign_workspace_bytes(uint64_t n, uint32_t dim, uint32_t k) {
-    (void)dim;
     Carver c(nullptr, 0);
     AssignBuffers b;
-    return carve_assign(c, n, k, &b) + 256;
+    return carve_assign(c, n, dim, k, &b) + 256;
 }
 
 extern "C" int
@@ -1207,7 +1316,7 @@ vsag_amd_kmeans_assign(const float* x_dev, uint64_t n, uint32_t dim, const float
     VA_CHECK_ARG(labels_dev != nullptr, "labels_dev is null");
     Carver c(workspace_dev, workspace_bytes);
     AssignBuffers b;
-    carve_assign(c, n, k, &b);
+    carve_assign(c, n, dim, k, &b);
     VA_CHECK_ARG(c.ok(), "workspace too small: need %zu bytes, got %zu", c.used, workspace_bytes);
     return assign_launch(x_dev, n, dim, centroids_dev, k, labels_dev, min_dist_dev, loss_dev, b, false,
                          static_cast<hipStream_t>(stream));
@@ -1240,14 +1349,13 @@ vsag_amd_kmeans_update(const float* x_dev, const int32_t* labels_dev, uint64_t n
 
 extern "C" size_t
 vsag_amd_kmeans_run_workspace_bytes(uint64_t n, uint32_t dim, uint32_t k) {
-    (void)dim;
     if (ensure_init() != 0) {
         return 0;
     }
     Carver c(nullptr, 0);
     AssignBuffers a;
     UpdateBuffers u;
-    carve_assign(c, n, k, &a);
+    carve_assign(c, n, dim, k, &a);
     carve_update(c, n, k, &u);
     c.take<int32_t>(k);
     return c.used + 256;
@@ -1266,7 +1374,7 @@ vsag_amd_kmeans_run(const float* x_dev, uint64_t n, uint32_t dim, float* centroi
     Carver c(workspace_dev, workspace_bytes);
     AssignBuffers a;
     UpdateBuffers u;
-    carve_assign(c, n, k, &a);
+    carve_assign(c, n, dim, k, &a);
     carve_update(c, n, k, &u);
     int32_t* counts_dev = c.take<int32_t>(k);
     VA_CHECK_ARG(c.ok(), "workspace too small: need %zu bytes, got %zu", c.used, workspace_bytes);

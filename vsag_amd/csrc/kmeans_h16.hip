@@ -1,0 +1,773 @@
+// Pre-selection of the k-means assignment on the fp16 matrix cores.
+//
+// The fp32 contraction of kmeans.hip is bound by the fp32 matrix rate (1M rows x 960 x 4096 centroids: 62 ms at 127
+// TFLOP/s, 80 % of that peak).  The fp16 instruction is sixteen times as fast, and almost every centroid of a row can be
+// ruled out with far less than fp32 accuracy, so the contraction runs on rows and centroids rounded to fp16 and only
+// decides which centroids are still possible; those get their distance from the fp32 values by the chain of fma that the
+// fp32 kernels run, and the smallest (distance, index) wins: the result is theirs bit for bit.
+//
+// What the test rests on.  With a centre m (any point; the mean of some centroids keeps the lengths small), x' = x - m,
+// c' = c - m and their fp16 forms X, C:  |x - c|^2 - |x'|^2 = |c'|^2 - 2 <x', c'>, and
+//     |<x', c'> - <X, C>| <= |x' - X| |c'| + |X| |c' - C|
+// with the lengths of the actual remainders, summed per row and centroid when they are rounded.  Together with the
+// roundings of the accumulation, of |c'|^2, of the stored value and of the final fp32 distances that is the row's error
+// bound E (largest |c'| and |c' - C| taken): a centroid is possible only if its approximate distance is within 2 E of the
+// row's least one.
+//
+// The contraction leaves, per row and group of 64 centroids, the three least approximate distances, the low six mantissa
+// bits of each saying which centroid: 12 bytes where the products would be 256.  A group brings those of the first two
+// that are possible, or all its 64 centroids where the third is possible too (with two values per group, and a group
+// open once its second was possible, a first form of the rescoring took 4.2 ms and not 1.9: every group of 64 is 64
+// distances).  Rows with more than kMaxWork distances to form, and rows or centroids that are not finite or too large, are marked and left to the fp32 kernels.
+//
+// 1M x 960 rows, 4096 centroids (one assignment): 63.3 -> 13.2 ms.  Of that the contraction takes 9.0 (7.9e12 flop: 870
+// TFLOP/s, 35 % of the fp16 peak; a workgroup waits at each of its fifteen stages for all eight waves), the rounding of
+// the rows 1.25 (5.8 GB at 4.6 TB/s) and the rescoring 2.8 (3.8 GB of rows, 0.8 GB of table, one to three centroids a
+// row).
+#include "kmeans_h16.h"
+
+#include <mutex>
+
+namespace vsag_amd {
+
+typedef _Float16 halfx8 __attribute__((ext_vector_type(8)));
+typedef _Float16 halfx4 __attribute__((ext_vector_type(4)));
+typedef float floatx16 __attribute__((ext_vector_type(16)));
+
+constexpr uint32_t kTile = 256;        // centroids x rows of a workgroup's tile
+constexpr uint32_t kThreads = 512;
+constexpr uint32_t kStage = 64;        // dimensions per stage: a row's part is one 128-byte line
+constexpr uint32_t kSlots = kStage / 8;
+constexpr uint32_t kGroup = 64;        // centroids per entry of the table
+constexpr uint32_t kRowsPerBlock = 64; // rescoring: rows of a workgroup
+constexpr uint32_t kParts = 4;         // rescoring: waves of a workgroup
+constexpr uint32_t kPairs = 128;       // rescoring: (row, centroid) pairs at a time
+constexpr uint32_t kPiece = 32;        // rescoring: dimensions at a time
+constexpr uint32_t kPitch = kPiece + 4;
+constexpr uint32_t kMaxList = 24;      // rescoring: entries (a centroid, or a whole group) per row
+constexpr uint32_t kMaxWork = 160;     // rescoring: distances per row
+constexpr uint64_t kSlabHalves = 64ull << 20;  // fp16 values per slab: 128 MB stay in the 256 MB memory-side cache
+constexpr uint32_t kMaxDim = 8192;
+
+static uint32_t
+padded_dim(uint32_t dim) {
+    return static_cast<uint32_t>(round_up(dim, kStage));
+}
+static uint64_t
+slab_rows(uint64_t n, uint32_t dim) {
+    uint64_t rows = kSlabHalves / padded_dim(dim) / kTile * kTile;
+    const uint64_t most = 1ull << 18;
+    rows = rows > most ? most : rows;
+    return n < rows ? round_up(n, kTile) : rows;
+}
+static uint32_t
+tile_count(uint32_t k) {
+    return (k + kTile - 1) / kTile;
+}
+
+// Where it pays: rounding and rescoring cost a row about 0.7 ns up to 128 dimensions (one read of it each), which the
+// fp32 kernels need for 40 000 products at 110 TFLOP/s; the six launches before and after the contraction take 40 us, and
+// a tile holds 256 centroids.  Measured, fp32 -> this, ms: 131072 x 128, k 256 0.148 -> 0.156 (not taken); 65536 x 128,
+// k 512 0.128 -> 0.112; 300000 x 101, k 512 0.65 -> 0.43; 22000 x 960, k 200 0.165 -> 0.175 (not taken); 1M x 960, k 256
+// 5.28 -> 3.65; 1M x 32, k 256 0.62 -> 0.85 (not taken); 1M x 37, k 4096 7.4 -> 2.5.
+bool
+kmeans_h16_takes(uint64_t n, uint32_t dim, uint32_t k) {
+    const double products = static_cast<double>(k) * dim;
+    return dim >= 32 && dim <= kMaxDim && k >= 256 && products >= 49152.0 && static_cast<double>(n) * products >= 4.0e9;
+}
+
+void
+carve_kmeans_h16(Carver& c, uint64_t n, uint32_t dim, uint32_t k, KmeansH16Buffers* b) {
+    const uint64_t rows = slab_rows(n, dim);
+    const uint32_t dpad = padded_dim(dim);
+    b->x16 = c.take<uint16_t>(rows * dpad);
+    b->c16 = c.take<uint16_t>(static_cast<uint64_t>(k) * dpad);
+    b->xinfo = c.take<float2>(rows);
+    b->xscale = c.take<float>(rows);
+    b->group_min = c.take<float>(static_cast<uint64_t>(tile_count(k)) * (kTile / kGroup) * 3 * rows);
+    b->centre = c.take<float>(dim);
+    b->cnorm = c.take<float>(k);
+    b->maxima = c.take<uint32_t>(4);
+    b->row_open = c.take<uint8_t>(n);
+    b->open64 = c.take<uint32_t>(div_up(n, kRowsPerBlock));
+}
+
+// The mean of up to 256 of the centroids, 64 dimensions per workgroup; finite whatever they hold.
+__global__ void __launch_bounds__(1024)
+kmeans_centre_kernel(const float* cent, uint32_t k, uint32_t dim, float* centre, uint32_t* maxima) {
+    __shared__ float part[16][64];
+    if (blockIdx.x == 0 && threadIdx.x < 4) {
+        maxima[threadIdx.x] = 0;
+    }
+    const uint32_t lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const uint32_t d = blockIdx.x * 64 + lane;
+    const uint32_t take = k < 256 ? k : 256;
+    const uint32_t step = k / take;
+    float s = 0.0F;
+    if (d < dim) {
+        for (uint32_t i = w; i < take; i += 16) {
+            s += cent[static_cast<uint64_t>(i) * step * dim + d];
+        }
+    }
+    part[w][lane] = s;
+    __syncthreads();
+    if (w == 0 && d < dim) {
+        float t = 0.0F;
+        for (uint32_t i = 0; i < 16; ++i) {
+            t += part[i][lane];
+        }
+        t *= 1.0F / static_cast<float>(take);
+        centre[d] = t - t == 0.0F ? t : 0.0F;
+    }
+}
+
+__global__ void
+kmeans_clear_maxima_kernel(uint32_t* maxima) {
+    if (threadIdx.x < 4) {
+        maxima[threadIdx.x] = 0;
+    }
+}
+
+__device__ inline float4
+load4(const float* row, uint32_t d, uint32_t dim, bool wide) {
+    if (wide) {
+        return *reinterpret_cast<const float4*>(row + d);
+    }
+    float4 v;
+    v.x = row[d];
+    v.y = d + 1 < dim ? row[d + 1] : 0.0F;
+    v.z = d + 2 < dim ? row[d + 2] : 0.0F;
+    v.w = d + 3 < dim ? row[d + 3] : 0.0F;
+    return v;
+}
+
+// Not negative: orders like the value, NaN above infinity.
+__device__ inline uint32_t
+magnitude_bits(float v) {
+    return __float_as_uint(v) & 0x7FFFFFFFU;
+}
+
+__device__ inline float
+wave_sum(float v) {
+    for (int off = 32; off > 0; off >>= 1) {
+        v += __shfl_xor(v, off);
+    }
+    return v;
+}
+
+// |c'|^2 per centroid and the largest |c'|^2 and |c|^2 (positive floats order like their bits; NaN above infinity).
+// A workgroup of sixteen waves takes 64 centroids: one atomic per maximum and workgroup.
+__global__ void __launch_bounds__(1024)
+kmeans_cnorm_kernel(const float* cent, uint32_t k, uint32_t dim, const float* centre, const float* cnorm_raw, float* cnorm,
+                    uint32_t* maxima) {
+    __shared__ uint32_t most[2];
+    const uint32_t lane = threadIdx.x & 63;
+    if (threadIdx.x < 2) {
+        most[threadIdx.x] = 0;
+    }
+    __syncthreads();
+    for (uint32_t c = blockIdx.x * kGroup + (threadIdx.x >> 6); c < (blockIdx.x + 1) * kGroup && c < k; c += 16) {
+        const float* row = cent + static_cast<uint64_t>(c) * dim;
+        float s = 0.0F;
+        for (uint32_t d = lane; d < dim; d += 64) {
+            const float v = row[d] - centre[d];
+            s = fmaf(v, v, s);
+        }
+        s = wave_sum(s);
+        if (lane == 0) {
+            cnorm[c] = s;
+            atomicMax(&most[0], magnitude_bits(s));
+            atomicMax(&most[1], magnitude_bits(cnorm_raw[c]));
+        }
+    }
+    __syncthreads();
+    if (threadIdx.x < 2) {
+        atomicMax(&maxima[threadIdx.x], most[threadIdx.x]);
+    }
+}
+
+// 2^e with 2^e sqrt(sq) in [2^13, 2^14): no entry exceeds the length, so none leaves the fp16 range.  The exponent is
+// kept within bounds that leave products of two scales normal; below them fp16 holds fewer bits, which the remainders say.
+__device__ inline int
+scale_exponent(float sq) {
+    int e = 0;
+    (void)frexpf(sqrtf(sq), &e);
+    e = 14 - e;
+    return e > 50 ? 50 : e < -49 ? -49 : e;
+}
+
+// Rounds a row (less the centre, times 2^e) to fp16, zeros up to dpad; what is left out (|x' - X|^2) and kept (|X|^2),
+// in the scale of the row.  x - m is taken in fp32 and its own rounding (2^-24 of it) added to the remainder.
+__device__ inline void
+round_row(const float* row, uint32_t dim, uint32_t dpad, const float* centre, bool wide, float up, uint16_t* out,
+          float* missed, float* kept) {
+    const uint32_t lane = threadIdx.x & 63;
+    float ms = 0.0F, ks = 0.0F;
+    for (uint32_t d = 4 * lane; d < dpad; d += 256) {
+        float v[4] = {0.0F, 0.0F, 0.0F, 0.0F};
+        if (d < dim) {
+            const float4 a = load4(row, d, dim, wide);
+            const float4 m = load4(centre, d, dim, wide);
+            v[0] = (a.x - m.x) * up;
+            v[1] = (a.y - m.y) * up;
+            v[2] = (a.z - m.z) * up;
+            v[3] = (a.w - m.w) * up;
+        }
+        halfx4 h;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            h[i] = static_cast<_Float16>(v[i]);
+            const float back = static_cast<float>(h[i]);
+            const float left = fabsf(v[i] - back) + 6.0e-8F * fabsf(v[i]);
+            ms = fmaf(left, left, ms);
+            ks = fmaf(back, back, ks);
+        }
+        *reinterpret_cast<halfx4*>(out + d) = h;
+    }
+    *missed = wave_sum(ms);
+    *kept = wave_sum(ks);
+}
+
+__global__ void __launch_bounds__(1024)
+kmeans_round_centroids_kernel(const float* cent, uint32_t k, uint32_t dim, uint32_t dpad, const float* centre, int wide,
+                              uint16_t* c16, uint32_t* maxima) {
+    __shared__ uint32_t most;
+    if (threadIdx.x == 0) {
+        most = 0;
+    }
+    __syncthreads();
+    const int e = scale_exponent(__uint_as_float(maxima[0]));
+    for (uint32_t c = blockIdx.x * kGroup + (threadIdx.x >> 6); c < (blockIdx.x + 1) * kGroup && c < k; c += 16) {
+        float missed, kept;
+        round_row(cent + static_cast<uint64_t>(c) * dim, dim, dpad, centre, wide != 0, ldexpf(1.0F, e),
+                  c16 + static_cast<uint64_t>(c) * dpad, &missed, &kept);
+        if ((threadIdx.x & 63) == 0) {
+            atomicMax(&most, magnitude_bits(ldexpf(sqrtf(missed), -e)));
+        }
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        atomicMax(&maxima[2], most);
+    }
+}
+
+// A wave per row: |x|^2 (unless it is known), the row in fp16 and its lengths.  The row is read twice, the second time
+// from the caches.
+__global__ void __launch_bounds__(256)
+kmeans_round_rows_kernel(const float* x, uint64_t rows, uint32_t dim, uint32_t dpad, const float* centre, int wide,
+                         uint16_t* x16, float2* xinfo, float* xscale, float* xnorm) {
+    const uint64_t r = static_cast<uint64_t>(blockIdx.x) * 4 + (threadIdx.x >> 6);
+    if (r >= rows) {
+        return;
+    }
+    const uint32_t lane = threadIdx.x & 63;
+    const float* row = x + r * dim;
+    float sq = 0.0F, raw = 0.0F;
+    for (uint32_t d = 4 * lane; d < dim; d += 256) {
+        const float4 a = load4(row, d, dim, wide != 0);
+        const float4 m = load4(centre, d, dim, wide != 0);
+        raw = fmaf(a.x, a.x, fmaf(a.y, a.y, fmaf(a.z, a.z, fmaf(a.w, a.w, raw))));
+        // entries past the dimension are zero on both sides
+        const float vx = a.x - m.x, vy = a.y - m.y, vz = a.z - m.z, vw = a.w - m.w;
+        sq = fmaf(vx, vx, fmaf(vy, vy, fmaf(vz, vz, fmaf(vw, vw, sq))));
+    }
+    sq = wave_sum(sq);
+    if (xnorm != nullptr) {
+        raw = wave_sum(raw);
+        if (lane == 0) {
+            xnorm[r] = raw;
+        }
+    }
+    const bool usable = sq < 1.0e30F;  // false for NaN as well
+    const int e = usable ? scale_exponent(sq) : 0;
+    float missed, kept;
+    round_row(row, usable ? dim : 0, dpad, centre, wide != 0, ldexpf(1.0F, e), x16 + r * dpad, &missed, &kept);
+    if (lane == 0) {
+        const float down = ldexpf(1.0F, -e);
+        xinfo[r] = make_float2(usable ? sqrtf(missed) * down : __builtin_inff(), sqrtf(kept) * down);
+        xscale[r] = down;
+    }
+}
+
+struct KmeansH16Args {
+    const uint4* x16;  // [rows][dpad / 8]
+    const uint4* c16;  // [k][dpad / 8]
+    uint64_t rows;
+    uint32_t k;
+    uint32_t slots;    // dpad / 8
+    const float* xscale;
+    const float* cnorm;
+    const uint32_t* maxima;
+    float* group_min;
+    uint64_t ld;       // the table: [group][3][ld]
+    uint32_t rtiles, ctiles, mc_log2, mcols, macros;
+};
+
+// 256 centroids (the M side, so that a lane's sixteen results belong to one row) x 256 rows, eight waves of 128 x 64.  A
+// stage of 64 dimensions is 64 KB; two are in LDS, the next one's loads are in flight through registers while a stage is
+// multiplied, and there is one barrier per stage.
+//
+// LDS: 16-byte slots [row][8], slot s of row r at position s ^ ((r >> 1) & 7): the 16 consecutive rows that a
+// ds_read_b128 serves at a time fall on the sixteen 16-byte columns of the 64 banks, and a global line of a row stays one
+// 128-byte run on the way in.
+//
+// Grid: as kmeans_assign_tile_kernel, id % 8 is the XCD, and the 32 workgroups that run on an XCD at the same time form a
+// macro tile whose rows and centroids they share through that XCD's L2.
+__global__ void __launch_bounds__(kThreads, 2)
+kmeans_h16_kernel(KmeansH16Args p) {
+    extern __shared__ uint4 lds[];  // [2][A: kTile x kSlots, B: kTile x kSlots], then |c'|^2 of the tile
+    const uint32_t xcd = blockIdx.x & 7;
+    const uint32_t local = blockIdx.x >> 3;
+    const uint32_t macro = (local >> 5) * 8 + xcd;
+    if (macro >= p.macros) {
+        return;
+    }
+    const uint32_t within = local & 31;
+    const uint32_t rt = (macro / p.mcols) * (32U >> p.mc_log2) + (within >> p.mc_log2);
+    const uint32_t ct = ((macro % p.mcols) << p.mc_log2) + (within & ((1U << p.mc_log2) - 1));
+    if (rt >= p.rtiles || ct >= p.ctiles) {
+        return;
+    }
+    constexpr uint32_t kSide = kTile * kSlots;
+    float* cn = reinterpret_cast<float*>(lds + 4 * kSide);
+    const uint32_t tid = threadIdx.x;
+    const uint32_t lane = tid & 63;
+    const uint32_t wave = tid >> 6;
+    const uint32_t wm = wave & 1;   // which 128 centroids
+    const uint32_t wn = wave >> 1;  // which 64 rows
+    const uint32_t half = lane >> 5;
+    const uint32_t l32 = lane & 31;
+    const uint64_t row0 = static_cast<uint64_t>(rt) * kTile;
+    const uint32_t c0 = ct * kTile;
+    const uint32_t stages = p.slots / kSlots;
+
+    // Loader: thread t moves slot t % 8 of rows t / 8 + 64 i of both sides; rows past the end repeat the last one.
+    const uint32_t lr = tid >> 3, ls = tid & 7;
+    const uint4* side_a = p.c16 + static_cast<uint64_t>(c0) * p.slots;
+    const uint4* side_b = p.x16 + row0 * p.slots;
+    const uint32_t a_last = p.k - 1 - c0;
+    const uint32_t b_last = static_cast<uint32_t>(p.rows - 1 - row0 < kTile ? p.rows - 1 - row0 : kTile);
+    auto offset = [&](uint32_t r, uint32_t last) __attribute__((always_inline)) { return (r < last ? r : last) * p.slots + ls; };
+    const uint32_t oa0 = offset(lr, a_last), oa1 = offset(lr + 64, a_last), oa2 = offset(lr + 128, a_last),
+                   oa3 = offset(lr + 192, a_last);
+    const uint32_t ob0 = offset(lr, b_last), ob1 = offset(lr + 64, b_last), ob2 = offset(lr + 128, b_last),
+                   ob3 = offset(lr + 192, b_last);
+    const uint32_t put = lr * kSlots + (ls ^ ((lr >> 1) & 7));  // + 64 i rows
+    if (tid < kTile) {
+        cn[tid] = c0 + tid < p.k ? p.cnorm[c0 + tid] : 3.0e38F;
+    }
+
+    uint4 ga0, ga1, ga2, ga3, gb0, gb1, gb2, gb3;  // (separate variables: an array went to scratch memory)
+    auto fetch = [&](uint32_t st) __attribute__((always_inline)) {
+        const uint4* a = side_a + st * kSlots;
+        const uint4* b = side_b + st * kSlots;
+        ga0 = a[oa0];
+        ga1 = a[oa1];
+        ga2 = a[oa2];
+        ga3 = a[oa3];
+        gb0 = b[ob0];
+        gb1 = b[ob1];
+        gb2 = b[ob2];
+        gb3 = b[ob3];
+    };
+    auto park = [&](uint4* buf) __attribute__((always_inline)) {
+        buf[put] = ga0;
+        buf[put + 64 * kSlots] = ga1;
+        buf[put + 128 * kSlots] = ga2;
+        buf[put + 192 * kSlots] = ga3;
+        buf[kSide + put] = gb0;
+        buf[kSide + put + 64 * kSlots] = gb1;
+        buf[kSide + put + 128 * kSlots] = gb2;
+        buf[kSide + put + 192 * kSlots] = gb3;
+    };
+    const uint32_t swap = (l32 >> 1) & 7;
+    const uint32_t a_row = (wm * 128 + l32) * kSlots;
+    const uint32_t b_row = kSide + (wn * 64 + l32) * kSlots;
+
+    floatx16 acc[4][2];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+#pragma unroll
+            for (int e = 0; e < 16; ++e) {
+                acc[i][j][e] = 0.0F;
+            }
+        }
+    }
+    // One step of sixteen dimensions; its six operands are in registers a step ahead.
+    halfx8 fa[2][4], fb[2][2];
+    auto operands = [&](const uint4* buf, uint32_t step, int u) __attribute__((always_inline)) {
+        const uint32_t at = (2 * step + half) ^ swap;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            fa[u][i] = __builtin_bit_cast(halfx8, buf[a_row + 32 * i * kSlots + at]);
+        }
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            fb[u][j] = __builtin_bit_cast(halfx8, buf[b_row + 32 * j * kSlots + at]);
+        }
+    };
+    auto multiply = [&](int u) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+#pragma unroll
+            for (int j = 0; j < 2; ++j) {
+                acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(fa[u][i], fb[u][j], acc[i][j], 0, 0, 0);
+            }
+        }
+    };
+
+    fetch(0);
+    park(lds);
+    __syncthreads();
+    for (uint32_t st = 0; st + 1 < stages; ++st) {
+        const uint4* cur = lds + (st & 1) * 2 * kSide;
+        fetch(st + 1);
+        operands(cur, 0, 0);
+        operands(cur, 1, 1);
+        multiply(0);
+        operands(cur, 2, 0);
+        multiply(1);
+        operands(cur, 3, 1);
+        multiply(0);
+        park(lds + ((st + 1) & 1) * 2 * kSide);  // its last readers passed the barrier that ended stage st - 1
+        multiply(1);
+        __syncthreads();
+    }
+    {
+        const uint4* cur = lds + ((stages - 1) & 1) * 2 * kSide;
+        operands(cur, 0, 0);
+        operands(cur, 1, 1);
+        multiply(0);
+        operands(cur, 2, 0);
+        multiply(1);
+        operands(cur, 3, 1);
+        multiply(0);
+        multiply(1);
+    }
+
+    // acc[i][j][e] = <C, X> (scaled) of centroid c0 + wm 128 + 32 i + 8 (e / 4) + 4 half + e % 4 and row wn 64 + 32 j + l32:
+    // the 64 of a lane are one group of the table, 16 i + e the place in it.
+    const float cdown = ldexpf(-2.0F, -scale_exponent(__uint_as_float(p.maxima[0])));
+    const uint32_t group = (ct * 2 + wm) * 2 + half;
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+        const uint64_t row = row0 + wn * 64 + 32 * j + l32;
+        const float factor = (row < p.rows ? p.xscale[row] : 0.0F) * cdown;
+        float least = __builtin_inff(), second = __builtin_inff(), third = __builtin_inff();
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+#pragma unroll
+            for (int e4 = 0; e4 < 4; ++e4) {
+                const float4 n4 = *reinterpret_cast<const float4*>(cn + wm * 128 + 32 * i + 8 * e4 + 4 * half);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const float base = e == 0 ? n4.x : e == 1 ? n4.y : e == 2 ? n4.z : n4.w;
+                    const float d = fmaf(factor, acc[i][j][4 * e4 + e], base);
+                    const float v = __uint_as_float((__float_as_uint(d) & ~63U) | (16U * i + 4U * e4 + e));
+                    third = __builtin_amdgcn_fmed3f(second, third, v);
+                    second = __builtin_amdgcn_fmed3f(least, second, v);
+                    least = fminf(least, v);
+                }
+            }
+            __builtin_amdgcn_sched_barrier(0);  // keeps the reads of cn from piling up in registers
+        }
+        if (row < p.rows) {
+            float* entry = p.group_min + static_cast<uint64_t>(group) * 3 * p.ld + row;
+            entry[0] = least;
+            entry[p.ld] = second;
+            entry[2 * p.ld] = third;
+        }
+    }
+}
+
+struct KmeansRescoreArgs {
+    const float* x;  // the slab's rows
+    uint64_t rows;
+    uint32_t dim;
+    const float* cent;
+    uint32_t k;
+    uint32_t groups;
+    const float* group_min;
+    uint64_t ld;
+    const float2* xinfo;
+    const float* xnorm;
+    const float* cnorm_raw;
+    const uint32_t* maxima;
+    int wide;
+    int natural;  // order of the products, see the kernel
+    unsigned long long* best;
+    uint8_t* row_open;
+    uint32_t* open64;
+    uint32_t* any_open;
+};
+
+// 64 rows per workgroup.  First four threads a row look through the table (coalesced along the rows); then a lane per
+// (row, centroid) that is still possible forms the distance exactly as the fp32 kernels do, one fma after the other in the
+// order of their matrix instructions (natural: k = 0, 1, 2, ...; else, for dimensions that are a multiple of 4, k = 0, 4,
+// 1, 5, 2, 6, 3, 7 of every eight), so labels and distances are those of the fp32 kernels bit for bit.  128 pairs at a
+// time; their rows come through LDS in pieces of 32 dimensions (whole 128-byte lines in, a pitch of 36 floats so that
+// the lanes' reads fall on all banks), the next piece in flight while one is summed.
+__global__ void __launch_bounds__(256)
+kmeans_h16_rescore_kernel(KmeansRescoreArgs p) {
+    __shared__ __align__(16) float seg_x[kPairs][kPitch], seg_c[kPairs][kPitch];
+    __shared__ uint32_t least_bits[kRowsPerBlock], count[kRowsPerBlock], cost[kRowsPerBlock], offset[kRowsPerBlock + 1];
+    __shared__ uint32_t list[kRowsPerBlock][kMaxList];
+    __shared__ uint32_t pair_row[kPairs], pair_c[kPairs];
+    __shared__ unsigned long long best[kRowsPerBlock];
+    __shared__ uint32_t any;
+    const uint32_t tid = threadIdx.x;
+    const uint32_t rl = tid & 63, part = tid >> 6;
+    const uint64_t block_row = static_cast<uint64_t>(blockIdx.x) * kRowsPerBlock;
+    const uint64_t row = block_row + rl;
+    if (tid < kRowsPerBlock) {
+        count[tid] = 0;
+        cost[tid] = 0;
+        least_bits[tid] = 0xFFFFFFFFU;
+        best[tid] = ~0ull;
+    }
+    if (tid == 0) {
+        any = 0;
+    }
+    __syncthreads();
+    float least = __builtin_inff();
+    if (row < p.rows) {
+#pragma unroll 8
+        for (uint32_t g = part; g < p.groups; g += kParts) {
+            least = fminf(least, p.group_min[static_cast<uint64_t>(g) * 3 * p.ld + row]);
+        }
+        atomicMin(&least_bits[rl], float_to_ordered(least));
+    }
+    __syncthreads();
+    if (row < p.rows) {
+        least = ordered_to_float(least_bits[rl]);
+        constexpr float kU = 5.9604645e-8F;  // 2^-24
+        const float2 info = p.xinfo[row];
+        const float cmax = sqrtf(__uint_as_float(p.maxima[0])) * 1.00001F;
+        const float craw = sqrtf(__uint_as_float(p.maxima[1])) * 1.00001F;
+        const float cmiss = __uint_as_float(p.maxima[2]) * 1.00001F;
+        const float missed = info.x * 1.00001F, kept = info.y * 1.00001F;
+        const float steps = static_cast<float>(p.dim);
+        // 2 |<x', c'> - <X, C>|
+        float err = 2.0F * (missed * cmax + kept * cmiss);
+        // four roundings of the absolute sum per matrix instruction of sixteen dimensions; |c'|^2 summed by a wave, the
+        // fma that adds it, and six mantissa bits of the stored value
+        const float big = cmax * cmax + 2.0F * (kept + missed) * (cmax + cmiss);
+        err += 2.0F * 4.0F * (steps / 16.0F + 5.0F) * kU * kept * (cmax + cmiss);
+        err += (steps / 64.0F + 12.0F) * 2.0F * kU * cmax * cmax + 66.0F * 2.0F * kU * big;
+        // the distances formed below: |c|^2 by a wave, <x, c> by a chain of dim roundings, the sum of the two
+        err += (steps / 64.0F + 12.0F) * 2.0F * kU * craw * craw;
+        err += 2.0F * (steps + 4.0F) * kU * sqrtf(p.xnorm[row]) * 1.00001F * craw;
+        const float limit = least + 2.0F * err;
+        if (!(err < 1.0e30F) || !(fabsf(limit) < 1.0e30F)) {
+            cost[rl] = kMaxWork + 1;  // (its threads write the same)
+        } else {
+#pragma unroll 4
+            for (uint32_t g = part; g < p.groups; g += kParts) {
+                const float* entry = p.group_min + static_cast<uint64_t>(g) * 3 * p.ld + row;
+                const float v1 = entry[0];
+                if (v1 <= limit) {
+                    const float v2 = entry[p.ld], v3 = entry[2 * p.ld];
+                    const uint32_t more = v3 <= limit ? 0 : v2 <= limit ? 2 : 1;  // 0: the whole group
+                    const uint32_t at = atomicAdd(&count[rl], more == 2 ? 2U : 1U);
+                    atomicAdd(&cost[rl], more == 0 ? kGroup : more);
+                    if (at < kMaxList) {
+                        list[rl][at] = (g << 7) | (more == 0 ? 64U : (__float_as_uint(v1) & 63U));
+                    }
+                    if (more == 2 && at + 1 < kMaxList) {
+                        list[rl][at + 1] = (g << 7) | (__float_as_uint(v2) & 63U);
+                    }
+                }
+            }
+        }
+    }
+    __syncthreads();
+    if (part == 0) {
+        const bool real = row < p.rows;
+        const bool open = real && (count[rl] == 0 || count[rl] > kMaxList || cost[rl] > kMaxWork);
+        if (real) {
+            p.row_open[row] = open ? 1 : 0;
+        }
+        if (open) {
+            any = 1;
+        }
+        // where the pairs of each row begin
+        const uint32_t mine = real && !open ? cost[rl] : 0;
+        uint32_t sum = mine;
+        for (int off = 1; off < 64; off <<= 1) {
+            const uint32_t up = __shfl_up(sum, off);
+            sum += rl >= static_cast<uint32_t>(off) ? up : 0;
+        }
+        offset[rl] = sum - mine;
+        if (rl == 63) {
+            offset[64] = sum;
+        }
+    }
+    __syncthreads();
+    if (tid == 0) {
+        p.open64[blockIdx.x] = any;
+        if (any != 0) {
+            *p.any_open = 1;
+        }
+    }
+
+    const uint32_t total = offset[kRowsPerBlock];
+    const uint32_t pieces = (p.dim + kPiece - 1) / kPiece;
+    const uint32_t quad = 4 * (tid & 7);
+    for (uint32_t base = 0; base < total; base += kPairs) {
+        if (tid < kPairs) {
+            uint32_t r = 0, c = 0xFFFFFFFFU;
+            const uint32_t t = base + tid;
+            if (t < total) {
+                for (uint32_t step = 32; step > 0; step >>= 1) {
+                    r += offset[r + step] <= t ? step : 0;  // the last row whose pairs begin at or before t
+                }
+                uint32_t at = t - offset[r], i = 0;
+                while ((list[r][i] & 64U) != 0 ? at >= kGroup : at >= 1) {
+                    at -= (list[r][i] & 64U) != 0 ? kGroup : 1;
+                    ++i;
+                }
+                // group g = (tile, half of the tile, lane half); place 16 i + j of it is centroid
+                // 32 i + 8 (j / 4) + 4 half + j % 4
+                const uint32_t e = list[r][i], g = e >> 7, j = (e & 64U) != 0 ? at : e & 63U;
+                c = (g >> 1) * 128 + 4 * (g & 1) + 32 * (j >> 4) + 8 * ((j >> 2) & 3) + (j & 3);
+                c = c < p.k ? c : p.k - 1;  // past the end: once more the last centroid, a true distance all the same
+            }
+            pair_row[tid] = r;
+            pair_c[tid] = c;
+        }
+        __syncthreads();
+        float4 gx[4], gc[4];
+        auto fetch = [&](uint32_t d) __attribute__((always_inline)) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const uint32_t pr = (tid >> 3) + 32 * i;
+                const uint32_t c = pair_c[pr];
+                const bool in = c != 0xFFFFFFFFU && d < p.dim;
+                gx[i] = in ? load4(p.x + (block_row + pair_row[pr]) * p.dim, d, p.dim, p.wide != 0)
+                           : make_float4(0.0F, 0.0F, 0.0F, 0.0F);
+                gc[i] = in ? load4(p.cent + static_cast<uint64_t>(c) * p.dim, d, p.dim, p.wide != 0)
+                           : make_float4(0.0F, 0.0F, 0.0F, 0.0F);
+            }
+        };
+        float acc = 0.0F;
+        fetch(quad);
+        for (uint32_t piece = 0; piece < pieces; ++piece) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const uint32_t pr = (tid >> 3) + 32 * i;
+                *reinterpret_cast<float4*>(&seg_x[pr][quad]) = gx[i];
+                *reinterpret_cast<float4*>(&seg_c[pr][quad]) = gc[i];
+            }
+            __syncthreads();
+            if (piece + 1 < pieces) {
+                fetch((piece + 1) * kPiece + quad);
+            }
+            if (tid < kPairs) {
+#pragma unroll
+                for (uint32_t d = 0; d < kPiece; d += 8) {
+                    const float4 xa = *reinterpret_cast<const float4*>(&seg_x[tid][d]);
+                    const float4 xb = *reinterpret_cast<const float4*>(&seg_x[tid][d + 4]);
+                    const float4 ca = *reinterpret_cast<const float4*>(&seg_c[tid][d]);
+                    const float4 cb = *reinterpret_cast<const float4*>(&seg_c[tid][d + 4]);
+                    if (p.natural != 0) {
+                        acc = fmaf(xa.w, ca.w, fmaf(xa.z, ca.z, fmaf(xa.y, ca.y, fmaf(xa.x, ca.x, acc))));
+                        acc = fmaf(xb.w, cb.w, fmaf(xb.z, cb.z, fmaf(xb.y, cb.y, fmaf(xb.x, cb.x, acc))));
+                    } else {
+                        acc = fmaf(xb.y, cb.y, fmaf(xa.y, ca.y, fmaf(xb.x, cb.x, fmaf(xa.x, ca.x, acc))));
+                        acc = fmaf(xb.w, cb.w, fmaf(xa.w, ca.w, fmaf(xb.z, cb.z, fmaf(xa.z, ca.z, acc))));
+                    }
+                }
+            }
+            __syncthreads();
+        }
+        if (base + tid < total && tid < kPairs) {
+            const uint32_t c = pair_c[tid];
+            atomicMin(&best[pair_row[tid]], static_cast<unsigned long long>(make_key(p.cnorm_raw[c] + (-2.0F * acc), c)));
+        }
+        __syncthreads();  // pair_row / pair_c are written again
+    }
+    if (tid < kRowsPerBlock && row < p.rows) {
+        p.best[row] = best[tid];
+    }
+}
+
+int
+launch_kmeans_h16(const float* x, uint64_t n, uint32_t dim, const float* cent, uint32_t k, const float* cnorm_raw,
+                  float* xnorm, bool have_xnorm, unsigned long long* best, const KmeansH16Buffers& b, hipStream_t st) {
+    constexpr size_t lds_bytes = 4 * static_cast<size_t>(kTile) * kSlots * sizeof(uint4) + kTile * sizeof(float);
+    static std::once_flag lds_once;
+    static hipError_t lds_rc = hipSuccess;
+    std::call_once(lds_once, []() {
+        lds_rc = hipFuncSetAttribute(reinterpret_cast<const void*>(kmeans_h16_kernel),
+                                     hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds_bytes));
+    });
+    VA_HIP(lds_rc);
+    const uint32_t dpad = padded_dim(dim);
+    const uint64_t slab = slab_rows(n, dim);
+    const int wide = (dim & 3) == 0 && ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(cent)) & 15) == 0;
+    const bool kept = have_xnorm && n <= slab;  // the rows' fp16 form of the call before, and the centre it was formed with
+    const uint32_t cblocks = (k + kGroup - 1) / kGroup;
+    if (!kept) {
+        hipLaunchKernelGGL(kmeans_centre_kernel, dim3((dim + 63) / 64), dim3(1024), 0, st, cent, k, dim, b.centre, b.maxima);
+    } else {
+        hipLaunchKernelGGL(kmeans_clear_maxima_kernel, dim3(1), dim3(64), 0, st, b.maxima);
+    }
+    hipLaunchKernelGGL(kmeans_cnorm_kernel, dim3(cblocks), dim3(1024), 0, st, cent, k, dim, b.centre, cnorm_raw, b.cnorm,
+                       b.maxima);
+    hipLaunchKernelGGL(kmeans_round_centroids_kernel, dim3(cblocks), dim3(1024), 0, st, cent, k, dim, dpad, b.centre, wide,
+                       b.c16, b.maxima);
+    for (uint64_t r0 = 0; r0 < n; r0 += slab) {
+        const uint64_t rows = n - r0 < slab ? n - r0 : slab;
+        if (!kept) {
+            hipLaunchKernelGGL(kmeans_round_rows_kernel, dim3(static_cast<uint32_t>(div_up(rows, 4))), dim3(256), 0, st,
+                               x + r0 * dim, rows, dim, dpad, b.centre, wide, b.x16, b.xinfo, b.xscale,
+                               have_xnorm ? nullptr : xnorm + r0);
+        }
+        KmeansH16Args a;
+        a.x16 = reinterpret_cast<const uint4*>(b.x16);
+        a.c16 = reinterpret_cast<const uint4*>(b.c16);
+        a.rows = rows;
+        a.k = k;
+        a.slots = dpad / 8;
+        a.xscale = b.xscale;
+        a.cnorm = b.cnorm;
+        a.maxima = b.maxima;
+        a.group_min = b.group_min;
+        a.ld = slab;
+        a.rtiles = static_cast<uint32_t>(div_up(rows, kTile));
+        a.ctiles = tile_count(k);
+        a.mc_log2 = a.ctiles >= 8 ? 3 : a.ctiles >= 4 ? 2 : a.ctiles >= 2 ? 1 : 0;
+        a.mcols = (a.ctiles + (1U << a.mc_log2) - 1) >> a.mc_log2;
+        const uint32_t mrows = (a.rtiles + (32U >> a.mc_log2) - 1) / (32U >> a.mc_log2);
+        a.macros = mrows * a.mcols;
+        hipLaunchKernelGGL(kmeans_h16_kernel, dim3((a.macros + 7) / 8 * 32 * 8), dim3(kThreads), lds_bytes, st, a);
+
+        KmeansRescoreArgs s;
+        s.x = x + r0 * dim;
+        s.rows = rows;
+        s.dim = dim;
+        s.cent = cent;
+        s.k = k;
+        s.groups = a.ctiles * (kTile / kGroup);
+        s.group_min = b.group_min;
+        s.ld = slab;
+        s.xinfo = b.xinfo;
+        s.xnorm = xnorm + r0;
+        s.cnorm_raw = cnorm_raw;
+        s.maxima = b.maxima;
+        s.wide = wide;
+        s.natural = (dim & 3) != 0;
+        s.best = best + r0;
+        s.row_open = b.row_open + r0;
+        s.open64 = b.open64 + r0 / kRowsPerBlock;
+        s.any_open = b.maxima + 3;
+        const dim3 grid(static_cast<uint32_t>(div_up(rows, kRowsPerBlock)));
+        hipLaunchKernelGGL(kmeans_h16_rescore_kernel, grid, dim3(256), 0, st, s);
+    }
+    VA_HIP(hipGetLastError());
+    return 0;
+}
+
+}  // namespace vsag_amd
