@@ -84,6 +84,30 @@ def test_update_matches_oracle(lib, n, d, k):
     assert np.allclose(cent, rcent, rtol=1e-5, atol=1e-6)
 
 
+@pytest.mark.parametrize("d", [1, 3, 5, 20, 64, 65, 68, 128, 131])
+def test_update_sums_in_row_order(lib, d):
+    """Clusters around the kernel's stages of 64 rows (and empty ones): the means are the sequential fp32 sums, bit for bit."""
+    L = lib.load_library()
+    rng = np.random.default_rng(d)
+    sizes = np.concatenate([[0, 1, 2, 15, 17, 63, 64, 65, 127, 128, 129, 191, 192, 193, 1000, 0, 16],
+                            rng.integers(1, 40, 600)])
+    k, n = len(sizes), int(sizes.sum())
+    labels = rng.permutation(np.repeat(np.arange(k), sizes)).astype(np.int32)
+    x = rng.standard_normal((n, d)).astype(np.float32)
+    cent0 = rng.standard_normal((k, d)).astype(np.float32)
+    xb, lb, cb, counts = dev(x), dev(labels), dev(cent0), capi.DeviceBuffer(k * 4)
+    wsb = L.vsag_amd_kmeans_update_workspace_bytes(n, d, k)
+    ws = capi.DeviceBuffer(wsb)
+    capi.check(L.vsag_amd_kmeans_update(xb.ptr, lb.ptr, n, d, k, cb.ptr, counts.ptr, ws.ptr, wsb, None))
+    want = cent0.copy()
+    for j in range(k):
+        if sizes[j]:
+            sums = np.cumsum(x[labels == j], axis=0, dtype=np.float32)[-1]
+            want[j] = sums * (np.float32(1) / np.float32(sizes[j]))
+    assert np.array_equal(counts.to_numpy(np.int32, (k,)), sizes)
+    assert np.array_equal(cb.to_numpy(np.float32, (k, d)), want)
+
+
 def test_run_matches_oracle_and_reduces_loss(lib):
     L = lib.load_library()
     rng = np.random.default_rng(11)
