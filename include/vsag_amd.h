@@ -325,7 +325,7 @@ VSAG_AMD_API int vsag_amd_flat_scan_topk_noalloc(const vsag_amd_store_t* store, 
  * int8 matrix cores when a batch has at least 8192 (query, list) groups (same results; off with mode -1).
  * sq8 stores of at most 128 dimensions pre-select on the int8 matrix cores (queries split into two int8 planes
  * with a rigorous bound on the remainder), the others on the fp32 matrix cores.
- * mode: 0 = when it pays (default: >= 512 queries, k <= 128, >= 65536 codes), 1 = whenever the store and k
+ * mode: 0 = when it pays (default: >= 512 queries, or fewer against enough codes, k <= 128, >= 65536 codes), 1 = whenever the store and k
  * allow it, 2 = like 1 but always on the fp32 matrix cores, -1 = never.  Process-wide; affects
  * vsag_amd_flat_scan_workspace_bytes as well.  No counterpart in the reference (it scans one query at a time). */
 VSAG_AMD_API int vsag_amd_set_scan_contraction(int mode);

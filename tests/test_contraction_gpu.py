@@ -5,7 +5,7 @@ import numpy as np
 import pytest
 
 import oracle as orc
-from gpu_helpers import Store, assert_topk_close, gaussian_mixture
+from gpu_helpers import Store, assert_topk_close, dev, gaussian_mixture
 from vsag_amd import capi
 
 pytestmark = pytest.mark.gpu
@@ -51,6 +51,40 @@ def test_sq8_contraction_equals_streaming(lib, modes, metric, n, d, nq, k):
         assert same(plain, fast)
     ri, rd = orc.flat_scan_topk(orc.SQ8, metric, d, codes, q[:16], k, lb=lb, diff=diff)
     assert_topk_close(fast[0][:16], fast[1][:16], ri, rd, label="sq8 contraction")
+    st.destroy()
+
+
+@pytest.mark.parametrize("kind,d,nq,k,pre", [("fp32", 100, 16, 10, False), ("fp32", 100, 64, 10, False),
+                                             ("fp32", 100, 127, 10, True), ("fp32", 131, 511, 1, True),
+                                             ("sq8", 100, 33, 10, False), ("sq8", 100, 450, 10, True),
+                                             ("sq8", 260, 17, 10, False), ("sq8", 260, 190, 10, True),
+                                             ("sq8", 260, 511, 100, False)])
+def test_small_batches_equal_streaming(lib, modes, kind, d, nq, k, pre):
+    """Batches on both sides of the line from which fewer than 512 queries are pre-selected; a workspace without room for
+    the candidate lists serves them by streaming."""
+    rng = np.random.default_rng(d + nq)
+    n = 70001
+    x, means = gaussian_mixture(rng, n, d, 30, 0.05)
+    q, _ = gaussian_mixture(rng, nq, d, 30, 0.05, means=means)
+    if kind == "fp32":
+        st = Store(capi.KIND_FP32, orc.L2, d)
+        st.append(x.view(np.uint8).reshape(n, -1))
+    else:
+        lb, diff = orc.sq_train(x, 8, orc.L2)
+        st = Store(capi.KIND_SQ8, orc.L2, d, lb=lb, diff=diff)
+        st.append(orc.sq_encode(x, 8, lb, diff, orc.L2))
+    L, ws = st.lib, st.lib.vsag_amd_flat_scan_workspace_bytes
+    need = ws(st.handle, nq, k)
+    plain, auto, tile = modes(st, q, k, 0)
+    assert same(plain, auto) and (tile >= 128) == pre
+    capi.check(L.vsag_amd_store_set_scan_contraction(st.handle, -1))
+    streaming = ws(st.handle, nq, k)
+    capi.check(L.vsag_amd_store_set_scan_contraction(st.handle, -2))
+    assert (need > streaming) == pre
+    qb, ids, ds, room = dev(q), capi.DeviceBuffer(nq * k * 4), capi.DeviceBuffer(nq * k * 4), capi.DeviceBuffer(streaming)
+    capi.check(L.vsag_amd_flat_scan_topk(st.handle, qb.ptr, nq, k, ids.ptr, ds.ptr, room.ptr, streaming, None))
+    assert np.array_equal(ids.to_numpy(np.uint32, (nq, k)), plain[0].view(np.uint32))
+    assert np.array_equal(ds.to_numpy(np.uint32, (nq, k)), plain[1].view(np.uint32))
     st.destroy()
 
 

@@ -1166,6 +1166,48 @@ prefilter_supports(const vsag_amd_store* s) {
     return s->nlist == 0 && (s->kind == VSAG_AMD_KIND_FP32 || s->kind == VSAG_AMD_KIND_SQ8) && s->pf_term != nullptr;
 }
 
+// Whether a batch of nq queries is pre-selected (stores of at least 1024 tiles).  From 512 queries on always; below, the
+// dozen launches, the exact prefix and the rescoring (which grows with k) have to be less than the streaming kernel's time,
+// which grows with queries x codes x dimensions.  Measured under L2, us per call, streaming -> pre-selected, beside the line:
+//   fp32 (fp32 matrix cores): 100k x 128, k 10, 64 queries 271 -> 261, 128 338 -> 273 (32: 214 -> 242, not taken); 1M x 128,
+//     k 100, 64 queries 1160 -> 1057; 100k x 768, k 100, 128 queries 1377 -> 1801 (not taken); 600k x 960, k 10, 256 queries
+//     11896 -> 3866.  Their time hardly depends on the dimension's share of the work from 128 on: both sides grow with it.
+//   sq8 / sq4 on the int8 matrix cores: 1M x 128, k 10, 32 queries 497 -> 343, 16 274 -> 340 (not taken); k 100, 64 queries
+//     791 -> 630; 100k x 128, k 10, 256 queries 303 -> 273, 128 208 -> 264 (not taken).
+//   sq8 / sq4 on the fp16 matrix cores: 200k x 768, k 10, 32 queries 842 -> 474, 16 440 -> 469 (not taken); k 100, 128
+//     queries 1411 -> 1147, 64 870 -> 1119 (not taken); 600k x 960, k 10, 256 queries 8015 -> 1028.
+//   sq8_uniform / sq4_uniform (dot products of bytes, cheap to stream): 500k x 128, k 10, 256 queries 391 -> 352, 128
+//     317 -> 335 (not taken); 1M x 96, k 100, 256 queries 713 -> 622.
+//   RaBitQ, k 200: 1M x 768, 256 queries 2518 -> 1679, 128 1517 -> 1690 (not taken); 3M x 128, 256 queries 2248 -> 1470.
+// The other metrics stream up to 1.4 times as fast: their line lies half as far again out.  Below 64 dimensions the
+// streaming kernel's own overhead per code decides, and 512 stays the line.
+bool
+prefilter_pays(const vsag_amd_store* s, uint64_t nq, uint32_t k) {
+    if (nq >= 512) {
+        return true;
+    }
+    if (s->dim < 64) {
+        return false;
+    }
+    const double kk = k < 10 ? 10.0 : static_cast<double>(k);
+    const double pairs = static_cast<double>(nq) * static_cast<double>(s->n);
+    const double work = pairs * s->dim;
+    const double far = s->metric == VSAG_AMD_METRIC_L2 ? 1.0 : 1.5;
+    if (prefilter_rb_supports(s)) {
+        return nq >= 128 && pairs * (140.0 + s->dim) >= far * 1.9e11;  // streaming: a fixed part per code, worth 140 bits
+    }
+    switch (s->kind) {
+        case VSAG_AMD_KIND_FP32:
+            return nq >= 64 && pairs * (s->dim < 128 ? s->dim / 128.0 : 1.0) >= far * (4.0e5 + 6.0e5 * kk);
+        case VSAG_AMD_KIND_SQ8_UNIFORM:
+        case VSAG_AMD_KIND_SQ4_UNIFORM:
+            return nq >= 64 && work >= far * (1.1e10 + 8.0e7 * kk);
+        default:
+            return s->dim <= 128 ? nq >= 32 && work >= far * (2.7e9 + 2.0e7 * kk)
+                                 : nq >= 16 && work >= far * (2.0e9 + 1.25e8 * kk);
+    }
+}
+
 // sq8_uniform: the per-code term of the int8 test, from the code's stored scalar (prefilter_i8.hip).
 __global__ void __launch_bounds__(256)
 uniform_term_kernel(const uint32_t* meta, uint64_t first, uint64_t count, int is_l2, float lb, float* term) {

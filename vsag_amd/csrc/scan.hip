@@ -836,6 +836,7 @@ uint32_t one_query_run_tiles(const vsag_amd_store* s);
 int launch_one_query(const vsag_amd_store* s, const ScanArgs& a, uint32_t k, const vsag_amd_search_options_t* options,
                      uint32_t* dist, uint64_t* mins, uint32_t* ids_dev, float* dists_dev, hipStream_t st);
 bool prefilter_supports(const vsag_amd_store* s);
+bool prefilter_pays(const vsag_amd_store* s, uint64_t nq, uint32_t k);
 int launch_prefilter(const vsag_amd_store* s, const ScanArgs& a, uint64_t nq, uint32_t k, uint32_t S, uint64_t tile_begin,
                      uint64_t tile_end, uint32_t* bound, float* tau, uint32_t* cand, uint32_t* cand_cnt, uint32_t cap,
                      uint64_t* partial, uint32_t* partial_cnt, uint32_t nslots, uint32_t first_slot, uint32_t out_slot,
@@ -880,7 +881,7 @@ make_call_plan(const vsag_amd_store* s, uint64_t nq, uint32_t k, CallPlan* c) {
     }
     const bool forced = prefilter_mode(s) > 0;
     const bool rb = prefilter_rb_supports(s);
-    if (!forced && (nq < 512 || k > (rb ? 256U : 128U) || s->ntiles < 1024)) {
+    if (!forced && (k > (rb ? 256U : 128U) || s->ntiles < 1024 || !prefilter_pays(s, nq, k))) {
         return;
     }
     // Candidate buffers: at most 2 GiB in all, 1024 to 4096 candidates per query (RaBitQ stores are searched with
@@ -974,6 +975,20 @@ make_call_plan(const vsag_amd_store* s, uint64_t nq, uint32_t k, CallPlan* c) {
     uint32_t pf_slots = static_cast<uint32_t>(c->prefix.chunks * c->prefix.waves + c->levels + c->rest.chunks * c->rest.waves);
     c->nslots = std::max(c->nslots, pf_slots);
     c->any_seeded = c->any_seeded || c->prefix.seeded || c->rest.seeded;
+}
+
+// A batch below this many queries is served without the pre-selection where the workspace has no room for its lists.
+constexpr uint64_t kListsOptionalBelow = 512;
+static bool
+drop_candidate_lists(const vsag_amd_store* s, uint64_t nq, CallPlan* c) {
+    if (!c->contraction || nq >= kListsOptionalBelow || prefilter_mode(s) != 0) {
+        return false;
+    }
+    c->contraction = c->int8 = c->rb = false;
+    c->h16_scratch = 0;
+    c->nslots = static_cast<uint32_t>(c->all.chunks * c->all.waves);
+    c->any_seeded = c->all.seeded;
+    return true;
 }
 
 struct ScanBuffers {
@@ -1479,6 +1494,11 @@ flat_scan_call(const vsag_amd_store_t* s, const float* queries_dev, uint64_t nq,
         c = Carver(workspace_dev, workspace_bytes);
         carve_scan(c, cp, nq, k, &b);
     }
+    if (!c.ok() && drop_candidate_lists(s, nq, &cp)) {
+        // Nor does a workspace without the candidate lists keep a small batch from being served.
+        c = Carver(workspace_dev, workspace_bytes);
+        carve_scan(c, cp, nq, k, &b);
+    }
     VA_CHECK_ARG(c.ok(), "workspace too small: need %zu bytes, got %zu", c.used, workspace_bytes);
     // A pre-filter or a radius goes the streaming way (the prefilter knows neither).
     const bool plain = options == nullptr || (options->deny_bits_dev == nullptr && options->use_radius == 0);
@@ -1634,7 +1654,16 @@ vsag_amd_flat_scan_topk_noalloc(const vsag_amd_store_t* s, const float* queries_
         VA_TRY(static_scratch_setup(device));
     }
     void* const scratch_dev = g_scratch_ptr[device].load(std::memory_order_acquire);
-    const size_t need = vsag_amd_flat_scan_workspace_bytes(s, nq, k);
+    size_t need = vsag_amd_flat_scan_workspace_bytes(s, nq, k);
+    if (need > kStaticScratchBytes) {
+        CallPlan cp;
+        make_call_plan(s, nq, k, &cp);
+        if (drop_candidate_lists(s, nq, &cp)) {
+            Carver c(nullptr, 0);
+            ScanBuffers b;
+            need = carve_scan(c, cp, nq, k, &b) + 256;
+        }
+    }
     VA_CHECK_ARG(need != 0 && need <= kStaticScratchBytes,
                  "this scan needs %zu bytes of scratch memory, the library's own array holds %zu: send fewer queries "
                  "per call or use vsag_amd_flat_scan_topk_ex with a workspace",
