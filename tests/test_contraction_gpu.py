@@ -1,6 +1,8 @@
 """Large batches on flat fp32 / sq8 stores: the matrix-core contraction pre-selects, the streaming arithmetic
 decides.  Its results must equal the streaming scan's bit for bit (and therefore the checker's within the usual
 tolerance), including when candidates overflow and the streaming kernel takes over."""
+import time
+
 import numpy as np
 import pytest
 
@@ -85,6 +87,36 @@ def test_small_batches_equal_streaming(lib, modes, kind, d, nq, k, pre):
     capi.check(L.vsag_amd_flat_scan_topk(st.handle, qb.ptr, nq, k, ids.ptr, ds.ptr, room.ptr, streaming, None))
     assert np.array_equal(ids.to_numpy(np.uint32, (nq, k)), plain[0].view(np.uint32))
     assert np.array_equal(ds.to_numpy(np.uint32, (nq, k)), plain[1].view(np.uint32))
+    st.destroy()
+
+
+@pytest.mark.parametrize("kind,bits", [("sq8", 8), ("sq4", 4)])
+def test_fp16_preselection_keeps_few_candidates_under_cosine(lib, modes, kind, bits):
+    """The thresholds of a cosine batch are as narrow as its distances: no query overflows its candidates (every query did,
+    and the batch then took twenty times as long as streaming it; three times is the line here)."""
+    rng = np.random.default_rng(12)
+    n, d, nq, k = 70001, 200, 512, 10
+    x, means = gaussian_mixture(rng, n, d, 70, 0.05)
+    q, _ = gaussian_mixture(rng, nq, d, 70, 0.05, means=means)
+    lb, diff = orc.sq_train(x, bits, orc.COSINE)
+    st = Store(capi.KIND_SQ8 if bits == 8 else capi.KIND_SQ4, orc.COSINE, d, lb=lb, diff=diff)
+    st.append(orc.sq_encode(x, bits, lb, diff, orc.COSINE))
+    plain, auto, tile = modes(st, q, k, 0)
+    assert same(plain, auto) and tile == 128
+    qb, ids, ds = dev(q), capi.DeviceBuffer(nq * k * 4), capi.DeviceBuffer(nq * k * 4)
+    best = {-1: 1e9, 0: 1e9}
+    for _ in range(8):
+        for mode in best:
+            capi.check(st.lib.vsag_amd_store_set_scan_contraction(st.handle, mode))
+            wsb = st.lib.vsag_amd_flat_scan_workspace_bytes(st.handle, nq, k)
+            ws = capi.DeviceBuffer(wsb)
+            capi.synchronize()
+            t0 = time.perf_counter()
+            capi.check(st.lib.vsag_amd_flat_scan_topk(st.handle, qb.ptr, nq, k, ids.ptr, ds.ptr, ws.ptr, wsb, None))
+            capi.synchronize()
+            best[mode] = min(best[mode], time.perf_counter() - t0)
+            ws.free()
+    assert best[0] < 3.0 * best[-1], best
     st.destroy()
 
 

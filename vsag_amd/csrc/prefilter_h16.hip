@@ -180,8 +180,9 @@ h16_split_kernel(H16SplitArgs p) {
     // sum per matrix instruction (sixteen dimensions each) plus four for the closing operations
     const double roundings = 2.0 * (p.kdim / 16.0 + 4.0) * kU;
     const double extra = fabs(static_cast<double>(p.dot_factor)) * static_cast<double>(p.cmax) * (miss + roundings * sum_abs);
-    // the test itself: fl(term + fl(factor acc)) against the threshold rounded to fp32
-    const double e_test = 4.0 * kU * (ymax * ymax + 2.0 * dots + fabs(t) + extra);
+    // the test itself: fl(term + fl(factor acc)) against the threshold rounded to fp32 (no term under ip: there
+    // |y|^2 would be that of raw code bytes, thousands of times the spread of cosine distances, and every code passed)
+    const double e_test = 4.0 * kU * ((p.is_l2 ? ymax * ymax : 0.0) + 2.0 * dots + fabs(t) + extra);
     t += extra + e_test;
     const float tf = static_cast<float>(t);
     const float up1 = tf + fabsf(tf) * 1.2e-7F + 1.0e-37F;  // not below t after the rounding to fp32
