@@ -120,6 +120,26 @@ def test_fp16_preselection_keeps_few_candidates_under_cosine(lib, modes, kind, b
     st.destroy()
 
 
+@pytest.mark.parametrize("tile,chunks", [(2, -1), (8, 0), (-1, 7), (0, 7)])
+def test_tuning_knobs_ask_for_the_streaming_kernel(lib, modes, tile, chunks):
+    """A query tile or a number of chunks set by hand: a batch of fewer than 512 queries that would be pre-selected streams
+    with them; from 512 on they do not change the route."""
+    rng = np.random.default_rng(5)
+    n, d, k = 70001, 100, 10
+    x, means = gaussian_mixture(rng, n, d, 30, 0.05)
+    q, _ = gaussian_mixture(rng, 512, d, 30, 0.05, means=means)
+    lb, diff = orc.sq_train(x, 8, orc.L2)
+    st = Store(capi.KIND_SQ8, orc.L2, d, lb=lb, diff=diff)
+    st.append(orc.sq_encode(x, 8, lb, diff, orc.L2))
+    plain, auto, route = modes(st, q[:450], k, 0)
+    assert same(plain, auto) and route == 256
+    capi.check(st.lib.vsag_amd_store_set_scan_tuning(st.handle, tile, chunks))
+    plain2, tuned, route = modes(st, q[:450], k, 0)
+    assert same(plain, plain2) and same(plain, tuned) and route == (tile if tile > 0 else 4)
+    assert modes(st, q, k, 0)[2] == 256
+    st.destroy()
+
+
 @pytest.mark.parametrize("metric", [orc.L2, orc.IP, orc.COSINE])
 @pytest.mark.parametrize("n,d,nq,k", [(30000, 129, 600, 10), (20000, 200, 520, 100), (12000, 960, 512, 10),
                                       (9000, 1000, 130, 7)])

@@ -861,6 +861,10 @@ small_store_table(const vsag_amd_store* s, uint64_t nq, uint32_t k) {
            s->n >= kTableMinCodes && s->ntiles * kWave <= kTableMaxCodes && nq * (s->ntiles * kWave) * 4 <= (2ull << 30);
 }
 
+// Below this many queries the streaming kernel serves a batch wherever the pre-selection is not asked for or its lists find
+// no room in the workspace.
+constexpr uint64_t kListsOptionalBelow = 512;
+
 static void
 make_call_plan(const vsag_amd_store* s, uint64_t nq, uint32_t k, CallPlan* c) {
     make_plan(s, nq, k, s->ntiles, &c->all);
@@ -881,7 +885,9 @@ make_call_plan(const vsag_amd_store* s, uint64_t nq, uint32_t k, CallPlan* c) {
     }
     const bool forced = prefilter_mode(s) > 0;
     const bool rb = prefilter_rb_supports(s);
-    if (!forced && (k > (rb ? 256U : 128U) || s->ntiles < 1024 || !prefilter_pays(s, nq, k))) {
+    // (The tuning knobs are the streaming kernel's: a batch that either route could serve streams where one is set.)
+    const bool tuned = nq < kListsOptionalBelow && (tile_override(s) > 0 || chunk_override(s) > 0);
+    if (!forced && (tuned || k > (rb ? 256U : 128U) || s->ntiles < 1024 || !prefilter_pays(s, nq, k))) {
         return;
     }
     // Candidate buffers: at most 2 GiB in all, 1024 to 4096 candidates per query (RaBitQ stores are searched with
@@ -977,8 +983,6 @@ make_call_plan(const vsag_amd_store* s, uint64_t nq, uint32_t k, CallPlan* c) {
     c->any_seeded = c->any_seeded || c->prefix.seeded || c->rest.seeded;
 }
 
-// A batch below this many queries is served without the pre-selection where the workspace has no room for its lists.
-constexpr uint64_t kListsOptionalBelow = 512;
 static bool
 drop_candidate_lists(const vsag_amd_store* s, uint64_t nq, CallPlan* c) {
     if (!c->contraction || nq >= kListsOptionalBelow || prefilter_mode(s) != 0) {
