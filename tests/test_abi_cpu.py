@@ -96,3 +96,12 @@ def test_fht_rotator_matrix_is_the_rotator(d):
     # the images of the basis vectors, entry for entry
     cols = orc.fht_kac_transform(flip, np.eye(d, dtype=np.float32))
     np.testing.assert_allclose(rot.T, cols, rtol=0, atol=1e-6)
+
+
+@pytest.mark.parametrize("n,d,k", [(1000000, 960, 4096), (10000000, 128, 65536), (2000000, 128, 262144),
+                                   (2000000, 32, 1000000), (131072, 8192, 349525), (30000, 64, 10000000)])
+def test_kmeans_workspace_is_bounded(n, d, k):
+    """Beside 13 bytes a row and half the size of the centroids: at most 128 MB of rounded rows and 256 MB of approximate
+    distances with what belongs to them, whatever the number of centroids."""
+    need = capi.load_library().vsag_amd_kmeans_assign_workspace_bytes(n, d, k)
+    assert 12 * n <= need <= 14 * n + 8 * k + 2 * k * ((d + 63) // 64 * 64) + (390 << 20)

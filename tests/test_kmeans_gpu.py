@@ -223,6 +223,38 @@ def test_assign_after_the_fp16_preselection(lib, kind, n, d, k):
         assert all(first[c64[j].tobytes()] == j for j in np.unique(labels))
 
 
+def _fp32_assign_bytes(n, k):
+    """What the fp32 kernels need: |c|^2, |x|^2, a key a row, the partial sums of the loss."""
+    return sum((b + 255) // 256 * 256 for b in (4 * k, 4 * n, 8 * n, 8 * ((n + 255) // 256), 8))
+
+
+def test_a_workspace_without_room_for_the_preselection_is_served_by_the_fp32_kernels(lib):
+    L = lib.load_library()
+    n, d, k = 20011, 128, 2048
+    x, cent = _routed_data("plain", n, d, k)
+    labels, mind, _ = gpu_assign(x, cent)
+    xb, cb, lab, dist = dev(x), dev(cent), capi.DeviceBuffer(n * 4), capi.DeviceBuffer(n * 4)
+    room = _fp32_assign_bytes(n, k)
+    assert room < L.vsag_amd_kmeans_assign_workspace_bytes(n, d, k)
+    ws = capi.DeviceBuffer(room)
+    args = (xb.ptr, n, d, cb.ptr, k, lab.ptr, dist.ptr, None, ws.ptr)
+    capi.check(L.vsag_amd_kmeans_assign(*args, room, None))
+    assert np.array_equal(lab.to_numpy(np.int32, (n,)), labels)
+    assert np.array_equal(dist.to_numpy(np.int32, (n,)), mind.view(np.int32))
+    assert L.vsag_amd_kmeans_assign(*args, room - 256, None) == capi.INVALID_ARGUMENT
+    assert b"workspace too small" in L.vsag_amd_last_error()
+    # Lloyd iterations: the same centroids with either workspace
+    out = []
+    rest = L.vsag_amd_kmeans_run_workspace_bytes(n, d, k) - L.vsag_amd_kmeans_assign_workspace_bytes(n, d, k)
+    for wsb in (L.vsag_amd_kmeans_run_workspace_bytes(n, d, k), room + rest):
+        cc, ws, loss = dev(cent), capi.DeviceBuffer(wsb), C.c_double()
+        capi.check(L.vsag_amd_kmeans_run(xb.ptr, n, d, cc.ptr, k, 3, 7, lab.ptr, C.byref(loss), ws.ptr, wsb, None))
+        out.append((cc.to_numpy(np.int32, (k, d)), lab.to_numpy(np.int32, (n,)), loss.value))
+    assert np.array_equal(out[0][0], out[1][0]) and np.array_equal(out[0][1], out[1][1])
+    # (the two routes add |x|^2 up in different orders, each a wave's sum of d / 64 terms a lane)
+    assert abs(out[0][2] - out[1][2]) <= 2 * (d / 64 + 12) * 2.0 ** -24 * (x.astype(np.float64) ** 2).sum(1).mean()
+
+
 def test_assign_after_the_fp16_preselection_with_values_out_of_range(lib):
     # rows that fp16 or the error bound cannot cover go to the fp32 kernels; what they return is what those return alone
     n, d, k = 16500, 128, 2048

@@ -873,14 +873,16 @@ struct AssignBuffers {
     KmeansH16Buffers pre;
 };
 
+// The pre-selection's buffers are up to 400 MB beside what the fp32 kernels need (12 bytes a row); a workspace without room
+// for them is served by those (`preselect` false).
 static size_t
-carve_assign(Carver& c, uint64_t n, uint32_t dim, uint32_t k, AssignBuffers* b) {
+carve_assign(Carver& c, uint64_t n, uint32_t dim, uint32_t k, bool preselect, AssignBuffers* b) {
     b->ynorm = c.take<float>(k);
     b->xnorm = c.take<float>(n);
     b->best = c.take<unsigned long long>(n);
     b->partial = c.take<double>(div_up(n, 256));
     b->loss_tmp = c.take<double>(1);
-    b->h16 = kmeans_h16_takes(n, dim, k);
+    b->h16 = preselect && kmeans_h16_takes(n, dim, k);
     if (b->h16) {
         carve_kmeans_h16(c, n, dim, k, &b->pre);
     }
@@ -1363,7 +1365,7 @@ extern "C" size_t
 vsag_amd_kmeans_assign_workspace_bytes(uint64_t n, uint32_t dim, uint32_t k) {
     Carver c(nullptr, 0);
     AssignBuffers b;
-    return carve_assign(c, n, dim, k, &b) + 256;
+    return carve_assign(c, n, dim, k, true, &b) + 256;
 }
 
 extern "C" int
@@ -1375,7 +1377,11 @@ vsag_amd_kmeans_assign(const float* x_dev, uint64_t n, uint32_t dim, const float
     VA_CHECK_ARG(labels_dev != nullptr, "labels_dev is null");
     Carver c(workspace_dev, workspace_bytes);
     AssignBuffers b;
-    carve_assign(c, n, dim, k, &b);
+    carve_assign(c, n, dim, k, true, &b);
+    if (!c.ok() && b.h16) {
+        c = Carver(workspace_dev, workspace_bytes);
+        carve_assign(c, n, dim, k, false, &b);
+    }
     VA_CHECK_ARG(c.ok(), "workspace too small: need %zu bytes, got %zu", c.used, workspace_bytes);
     return assign_launch(x_dev, n, dim, centroids_dev, k, labels_dev, min_dist_dev, loss_dev, b, false,
                          static_cast<hipStream_t>(stream));
@@ -1406,18 +1412,30 @@ vsag_amd_kmeans_update(const float* x_dev, const int32_t* labels_dev, uint64_t n
     return update_launch(x_dev, labels_dev, n, dim, k, centroids_dev, counts_dev, b, static_cast<hipStream_t>(stream));
 }
 
+namespace vsag_amd {
+struct RunBuffers {
+    AssignBuffers assign;
+    UpdateBuffers update;
+    int32_t* counts;
+};
+
+static size_t
+carve_run(Carver& c, uint64_t n, uint32_t dim, uint32_t k, bool preselect, RunBuffers* b) {
+    carve_assign(c, n, dim, k, preselect, &b->assign);
+    carve_update(c, n, k, &b->update);
+    b->counts = c.take<int32_t>(k);
+    return c.used;
+}
+}  // namespace vsag_amd
+
 extern "C" size_t
 vsag_amd_kmeans_run_workspace_bytes(uint64_t n, uint32_t dim, uint32_t k) {
     if (ensure_init() != 0) {
         return 0;
     }
     Carver c(nullptr, 0);
-    AssignBuffers a;
-    UpdateBuffers u;
-    carve_assign(c, n, dim, k, &a);
-    carve_update(c, n, k, &u);
-    c.take<int32_t>(k);
-    return c.used + 256;
+    RunBuffers b;
+    return carve_run(c, n, dim, k, true, &b) + 256;
 }
 
 extern "C" int
@@ -1431,11 +1449,15 @@ vsag_amd_kmeans_run(const float* x_dev, uint64_t n, uint32_t dim, float* centroi
     VA_CHECK_ARG(iters >= 0, "iters must not be negative");
     hipStream_t st = static_cast<hipStream_t>(stream);
     Carver c(workspace_dev, workspace_bytes);
-    AssignBuffers a;
-    UpdateBuffers u;
-    carve_assign(c, n, dim, k, &a);
-    carve_update(c, n, k, &u);
-    int32_t* counts_dev = c.take<int32_t>(k);
+    RunBuffers b;
+    carve_run(c, n, dim, k, true, &b);
+    if (!c.ok() && b.assign.h16) {
+        c = Carver(workspace_dev, workspace_bytes);
+        carve_run(c, n, dim, k, false, &b);
+    }
+    const AssignBuffers& a = b.assign;
+    const UpdateBuffers& u = b.update;
+    int32_t* const counts_dev = b.counts;
     VA_CHECK_ARG(c.ok(), "workspace too small: need %zu bytes, got %zu", c.used, workspace_bytes);
 
     std::mt19937 gen(static_cast<uint32_t>(seed));

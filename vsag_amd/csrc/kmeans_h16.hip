@@ -26,6 +26,7 @@
 // row).
 #include "kmeans_h16.h"
 
+#include <algorithm>
 #include <mutex>
 
 namespace vsag_amd {
@@ -47,6 +48,8 @@ constexpr uint32_t kPitch = kPiece + 4;
 constexpr uint32_t kMaxList = 24;      // rescoring: entries (a centroid, or a whole group) per row
 constexpr uint32_t kMaxWork = 160;     // rescoring: distances per row
 constexpr uint64_t kSlabHalves = 64ull << 20;  // fp16 values per slab: 128 MB stay in the 256 MB memory-side cache
+constexpr uint64_t kTableBytes = 256ull << 20;  // the table of a slab: the rows get fewer as the centroids get more ...
+constexpr uint64_t kMinSlabRows = 4096;         // ... down to this
 constexpr uint32_t kMaxDim = 8192;
 
 static uint32_t
@@ -54,15 +57,18 @@ padded_dim(uint32_t dim) {
     return static_cast<uint32_t>(round_up(dim, kStage));
 }
 static uint64_t
-slab_rows(uint64_t n, uint32_t dim) {
-    uint64_t rows = kSlabHalves / padded_dim(dim) / kTile * kTile;
-    const uint64_t most = 1ull << 18;
-    rows = rows > most ? most : rows;
-    return n < rows ? round_up(n, kTile) : rows;
-}
-static uint32_t
 tile_count(uint32_t k) {
-    return (k + kTile - 1) / kTile;
+    return div_up(k, kTile);
+}
+static uint64_t
+table_row_bytes(uint32_t k) {
+    return tile_count(k) * (kTile / kGroup) * 3 * sizeof(float);
+}
+static uint64_t
+slab_rows(uint64_t n, uint32_t dim, uint32_t k) {
+    const uint64_t rows = std::min({kSlabHalves / padded_dim(dim), kTableBytes / table_row_bytes(k), uint64_t{1} << 18}) /
+                          kTile * kTile;
+    return n < rows ? round_up(n, kTile) : rows;
 }
 
 // Where it pays: rounding and rescoring cost a row about 0.7 ns up to 128 dimensions (one read of it each), which the
@@ -73,18 +79,19 @@ tile_count(uint32_t k) {
 bool
 kmeans_h16_takes(uint64_t n, uint32_t dim, uint32_t k) {
     const double products = static_cast<double>(k) * dim;
-    return dim >= 32 && dim <= kMaxDim && k >= 256 && products >= 49152.0 && static_cast<double>(n) * products >= 4.0e9;
+    return dim >= 32 && dim <= kMaxDim && k >= 256 && products >= 49152.0 && static_cast<double>(n) * products >= 4.0e9 &&
+           slab_rows(n, dim, k) >= std::min(n, kMinSlabRows);
 }
 
 void
 carve_kmeans_h16(Carver& c, uint64_t n, uint32_t dim, uint32_t k, KmeansH16Buffers* b) {
-    const uint64_t rows = slab_rows(n, dim);
+    const uint64_t rows = slab_rows(n, dim, k);
     const uint32_t dpad = padded_dim(dim);
     b->x16 = c.take<uint16_t>(rows * dpad);
     b->c16 = c.take<uint16_t>(static_cast<uint64_t>(k) * dpad);
     b->xinfo = c.take<float2>(rows);
     b->xscale = c.take<float>(rows);
-    b->group_min = c.take<float>(static_cast<uint64_t>(tile_count(k)) * (kTile / kGroup) * 3 * rows);
+    b->group_min = c.take<float>(table_row_bytes(k) / sizeof(float) * rows);
     b->centre = c.take<float>(dim);
     b->cnorm = c.take<float>(k);
     b->maxima = c.take<uint32_t>(4);
@@ -705,7 +712,7 @@ launch_kmeans_h16(const float* x, uint64_t n, uint32_t dim, const float* cent, u
     });
     VA_HIP(lds_rc);
     const uint32_t dpad = padded_dim(dim);
-    const uint64_t slab = slab_rows(n, dim);
+    const uint64_t slab = slab_rows(n, dim, k);
     const int wide = (dim & 3) == 0 && ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(cent)) & 15) == 0;
     const bool kept = have_xnorm && n <= slab;  // the rows' fp16 form of the call before, and the centre it was formed with
     const uint32_t cblocks = (k + kGroup - 1) / kGroup;
@@ -737,7 +744,7 @@ launch_kmeans_h16(const float* x, uint64_t n, uint32_t dim, const float* cent, u
         a.group_min = b.group_min;
         a.ld = slab;
         a.rtiles = static_cast<uint32_t>(div_up(rows, kTile));
-        a.ctiles = tile_count(k);
+        a.ctiles = static_cast<uint32_t>(tile_count(k));
         a.mc_log2 = a.ctiles >= 8 ? 3 : a.ctiles >= 4 ? 2 : a.ctiles >= 2 ? 1 : 0;
         a.mcols = (a.ctiles + (1U << a.mc_log2) - 1) >> a.mc_log2;
         const uint32_t mrows = (a.rtiles + (32U >> a.mc_log2) - 1) / (32U >> a.mc_log2);
