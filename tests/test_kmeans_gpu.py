@@ -223,6 +223,20 @@ def test_assign_after_the_fp16_preselection(lib, kind, n, d, k):
         assert all(first[c64[j].tobytes()] == j for j in np.unique(labels))
 
 
+@pytest.mark.parametrize("scale", [1e-16, 1e-19, 1e-21, 1e-23, 1e-30])
+def test_assign_after_the_fp16_preselection_of_tiny_values(lib, scale):
+    """Distances down among the denormal numbers (and below): what the fp32 kernels return, bit for bit."""
+    n, d, k = 16385, 128, 2048
+    x, cent = _routed_data("plain", n, d, k)
+    x *= np.float32(scale)
+    cent *= np.float32(scale)
+    labels, mind, _ = gpu_assign(x, cent)
+    half = n // 2 + 1  # too few rows for the pre-selection
+    few = [gpu_assign(part, cent) for part in (x[:half], x[half:])]
+    assert np.array_equal(labels, np.concatenate([f[0] for f in few]))
+    assert np.array_equal(mind.view(np.int32), np.concatenate([f[1] for f in few]).view(np.int32))
+
+
 def _fp32_assign_bytes(n, k):
     """What the fp32 kernels need: |c|^2, |x|^2, a key a row, the partial sums of the loss."""
     return sum((b + 255) // 256 * 256 for b in (4 * k, 4 * n, 8 * n, 8 * ((n + 255) // 256), 8))

@@ -551,10 +551,15 @@ kmeans_h16_rescore_kernel(KmeansRescoreArgs p) {
         least = ordered_to_float(least_bits[rl]);
         constexpr float kU = 5.9604645e-8F;  // 2^-24
         const float2 info = p.xinfo[row];
-        const float cmax = sqrtf(__uint_as_float(p.maxima[0])) * 1.00001F;
-        const float craw = sqrtf(__uint_as_float(p.maxima[1])) * 1.00001F;
-        const float cmiss = __uint_as_float(p.maxima[2]) * 1.00001F;
-        const float missed = info.x * 1.00001F, kept = info.y * 1.00001F;
+        // Squares and products that underflow lose bits that no relative term covers: kTinyLength^2 is what 8192 squares can
+        // lose, kTinyRest the same for the remainders (in scales of 2^14 and more), kTinySquare what the products can.  Rows and
+        // centroids that small have every centroid possible and go to the fp32 kernels.
+        constexpr float kTinyLength = 2.0e-17F, kTinyRest = 1.0e-20F, kTinySquare = 1.0e-33F;
+        const float cmax = sqrtf(__uint_as_float(p.maxima[0])) * 1.00001F + kTinyLength;
+        const float craw = sqrtf(__uint_as_float(p.maxima[1])) * 1.00001F + kTinyLength;
+        const float cmiss = __uint_as_float(p.maxima[2]) * 1.00001F + kTinyRest;
+        const float missed = info.x * 1.00001F + kTinyRest, kept = info.y * 1.00001F + kTinyRest;
+        const float xraw = sqrtf(p.xnorm[row]) * 1.00001F + kTinyLength;
         const float steps = static_cast<float>(p.dim);
         // 2 |<x', c'> - <X, C>|
         float err = 2.0F * (missed * cmax + kept * cmiss);
@@ -565,7 +570,7 @@ kmeans_h16_rescore_kernel(KmeansRescoreArgs p) {
         err += (steps / 64.0F + 12.0F) * 2.0F * kU * cmax * cmax + 66.0F * 2.0F * kU * big;
         // the distances formed below: |c|^2 by a wave, <x, c> by a chain of dim roundings, the sum of the two
         err += (steps / 64.0F + 12.0F) * 2.0F * kU * craw * craw;
-        err += 2.0F * (steps + 4.0F) * kU * sqrtf(p.xnorm[row]) * 1.00001F * craw;
+        err += 2.0F * (steps + 4.0F) * kU * xraw * craw + kTinySquare;
         const float limit = least + 2.0F * err;
         if (!(err < 1.0e30F) || !(fabsf(limit) < 1.0e30F)) {
             cost[rl] = kMaxWork + 1;  // (its threads write the same)
