@@ -1,5 +1,6 @@
 """k-means on the device against the CPU checker and against an fp64 brute force."""
 import ctypes as C
+import time
 
 import numpy as np
 import pytest
@@ -196,18 +197,29 @@ def _routed_data(kind, n, d, k):
     elif kind == "same":  # one point: every distance ties
         x[:] = x[0]
         cent[:] = x[0]
+    elif kind == "outliers":  # centroids far out, one of them with rows next to it, and centroids that are not finite
+        cent[3] *= np.float32(100.0)
+        cent[k - 1] *= np.float32(1e12)
+        cent[64] *= np.float32(1e20)
+        cent[70, 1] = np.nan
+        cent[130, 0] = np.inf
+        x[5], x[n - 1] = cent[3], cent[k - 1]
+        x[700] = cent[3] * np.float32(0.5)  # halfway
     return x, cent
 
 
 # At the edges of the pre-selection's tiles (256 x 256 x 64), with 4e9 products and more each.
 @pytest.mark.parametrize("kind,n,d,k", [("plain", 20011, 130, 1601), ("plain", 65537, 64, 1024), ("plain", 4096, 1030, 1025),
                                         ("plain", 62001, 257, 257), ("offset", 20011, 101, 2049), ("scaled", 16385, 128, 2048),
-                                        ("copies", 16385, 128, 2050), ("same", 16384, 128, 2048), ("plain", 33000, 64, 2111)])
+                                        ("copies", 16385, 128, 2050), ("same", 16384, 128, 2048), ("plain", 33000, 64, 2111),
+                                        ("outliers", 16385, 128, 2048), ("outliers", 20011, 101, 2049),
+                                        ("outliers", 62001, 260, 256)])
 def test_assign_after_the_fp16_preselection(lib, kind, n, d, k):
     x, cent = _routed_data(kind, n, d, k)
     labels, mind, loss = gpu_assign(x, cent)
     assert labels.min() >= 0 and labels.max() < k
-    check_assignment(x, cent, labels, mind)
+    if kind != "outliers":
+        check_assignment(x, cent, labels, mind)
     # bit for bit what the fp32 kernels return: pieces too small for the pre-selection take those
     rows = min(n, int(3.9e9 / (k * d)))
     for r0 in range(0, n, rows):
@@ -221,6 +233,29 @@ def test_assign_after_the_fp16_preselection(lib, kind, n, d, k):
         for j in range(k):
             first.setdefault(c64[j].tobytes(), j)
         assert all(first[c64[j].tobytes()] == j for j in np.unique(labels))
+
+
+def test_centroids_far_out_do_not_open_every_row(lib):
+    """The rows that are not near them stay with the pre-selection: all of them went to the fp32 kernels behind it, which took
+    four times as long; twice is the line here."""
+    L = lib.load_library()
+    n, d, k = 200000, 256, 2048
+    x, cent = _routed_data("plain", n, d, k)
+    bad = cent.copy()
+    bad[77] *= np.float32(1000.0)
+    bad[1500, 3] = np.nan
+    xb, lab = dev(x), capi.DeviceBuffer(n * 4)
+    wsb = L.vsag_amd_kmeans_assign_workspace_bytes(n, d, k)
+    ws = capi.DeviceBuffer(wsb)
+    cents, best = (dev(cent), dev(bad)), [1e9, 1e9]
+    for _ in range(8):
+        for i in range(2):
+            capi.synchronize()
+            t0 = time.perf_counter()
+            capi.check(L.vsag_amd_kmeans_assign(xb.ptr, n, d, cents[i].ptr, k, lab.ptr, None, None, ws.ptr, wsb, None))
+            capi.synchronize()
+            best[i] = min(best[i], time.perf_counter() - t0)
+    assert best[1] < 2.0 * best[0], best
 
 
 @pytest.mark.parametrize("scale", [1e-16, 1e-19, 1e-21, 1e-23, 1e-30])

@@ -908,7 +908,7 @@ assign_launch(const float* x, uint64_t n, uint32_t dim, const float* cent, uint3
     if (b.h16) {
         VA_TRY(launch_kmeans_h16(x, n, dim, cent, k, b.ynorm, b.xnorm, have_xnorm, b.best, b.pre, st));
         // what follows does the rows that were left open: usually none, and its workgroups return at once
-        open = {b.pre.row_open, b.pre.open64, b.pre.maxima + 3};
+        open = {b.pre.row_open, b.pre.open64, &b.pre.state->any_open};
     }
     if ((dim & 3) == 0) {
         // 256 centroids per tile when there are enough of them to fill it, else 128

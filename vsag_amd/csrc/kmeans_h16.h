@@ -5,16 +5,25 @@
 
 namespace vsag_amd {
 
+// What the kernels of a call tell each other.  Lengths are squared and as float bits, but `missed`.
+struct KmeansH16State {
+    uint32_t centred;      // largest |c - centre|^2 of the centroids that are not far
+    uint32_t raw;          // largest |c|^2 of them
+    uint32_t missed;       // largest length that fp16 misses of one of them
+    uint32_t any_open;     // whether any row is left open
+    uint32_t far_from;     // centroids with |c - centre|^2 above this are far: only their distance from the centre is used
+    uint32_t nearest_far;  // least |c - centre|^2 of the far ones (infinity: none that any row could choose)
+};
+
 struct KmeansH16Buffers {
     uint16_t* x16;      // [slab rows][dpad] rows of the slab, less the centre, in fp16
     uint16_t* c16;      // [k][dpad] centroids, less the centre, in fp16
     float2* xinfo;      // per row of the slab: length of what fp16 misses, length of what it holds
-    float* xscale;      // per row of the slab: -2 / (scale of the row x scale of the centroids); 0: not usable
+    float* xscale;      // per row of the slab: 1 / scale of the row
     float* group_min;   // [group of 64 centroids][3][slab rows]: the three least approximate distances
     float* centre;      // [dim]
     float* cnorm;       // [k] |c - centre|^2
-    uint32_t* maxima;   // float bits: largest |c - centre|^2, largest |c|^2, largest length fp16 misses of a centroid;
-                        // [3]: whether any row is left open
+    KmeansH16State* state;
     uint8_t* row_open;  // [n] rows the fp32 matrix cores still have to do
     uint32_t* open64;   // [n / 64] whether there is one among 64
 };

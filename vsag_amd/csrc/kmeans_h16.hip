@@ -18,10 +18,15 @@
 // bits of each saying which centroid: 12 bytes where the products would be 256.  A group brings those of the first two
 // that are possible, or all its 64 centroids where the third is possible too (with two values per group, and a group
 // open once its second was possible, a first form of the rescoring took 4.2 ms and not 1.9: every group of 64 is 64
-// distances).  Rows with more than kMaxWork distances to form, and rows or centroids that are not finite or too large, are marked and left to the fp32 kernels.
+// distances).  Rows with more than kMaxWork distances to form, and rows that are not finite or too large, are
+// marked and left to the fp32 kernels.  What those cost does not depend on how many rows of a
+// tile of 256 are open, so a few in a hundred, scattered, cost what all do: where a common offset of rows and centroids is
+// many times their spread (the fp32 distances themselves are rounded to that), or centroids are missing from whole clusters,
+// a call can pay for both (1M x 960, k 4096, clusters of width 0.05 and ten times the centres' range from the origin: 76.8 ms
+// against 63.4 of the fp32 kernels; 65536 x 128, k 512: 0.26 against 0.13).
 //
-// 1M x 960 rows, 4096 centroids (one assignment): 63.3 -> 13.2 ms.  Of that the contraction takes 9.0 (7.9e12 flop: 870
-// TFLOP/s, 35 % of the fp16 peak; a workgroup waits at each of its fifteen stages for all eight waves), the rounding of
+// 1M x 960 rows, 4096 centroids (one assignment): 63.3 -> 13.0 ms.  Of that the contraction takes 9.3 (7.9e12 flop: 847
+// TFLOP/s, 34 % of the fp16 peak; a workgroup waits at each of its fifteen stages for all eight waves), the rounding of
 // the rows 1.25 (5.8 GB at 4.6 TB/s) and the rescoring 2.8 (3.8 GB of rows, 0.8 GB of table, one to three centroids a
 // row).
 #include "kmeans_h16.h"
@@ -94,44 +99,56 @@ carve_kmeans_h16(Carver& c, uint64_t n, uint32_t dim, uint32_t k, KmeansH16Buffe
     b->group_min = c.take<float>(table_row_bytes(k) / sizeof(float) * rows);
     b->centre = c.take<float>(dim);
     b->cnorm = c.take<float>(k);
-    b->maxima = c.take<uint32_t>(4);
+    b->state = c.take<KmeansH16State>(1);
     b->row_open = c.take<uint8_t>(n);
     b->open64 = c.take<uint32_t>(div_up(n, kRowsPerBlock));
 }
 
-// The mean of up to 256 of the centroids, 64 dimensions per workgroup; finite whatever they hold.
+__device__ inline void
+reset_state(KmeansH16State* state) {
+    *state = {0, 0, 0, 0, 0, __float_as_uint(__builtin_inff())};
+}
+
+// A centre: per dimension, sixteen means of sixteen centroids each, the middle half of them averaged -- a few centroids far
+// out do not move it.  64 dimensions per workgroup; finite whatever the centroids hold.
 __global__ void __launch_bounds__(1024)
-kmeans_centre_kernel(const float* cent, uint32_t k, uint32_t dim, float* centre, uint32_t* maxima) {
+kmeans_centre_kernel(const float* cent, uint32_t k, uint32_t dim, float* centre, KmeansH16State* state) {
     __shared__ float part[16][64];
-    if (blockIdx.x == 0 && threadIdx.x < 4) {
-        maxima[threadIdx.x] = 0;
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        reset_state(state);
     }
     const uint32_t lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     const uint32_t d = blockIdx.x * 64 + lane;
-    const uint32_t take = k < 256 ? k : 256;
-    const uint32_t step = k / take;
+    const uint32_t step = k / 256;  // k >= 256
     float s = 0.0F;
     if (d < dim) {
-        for (uint32_t i = w; i < take; i += 16) {
+        for (uint32_t i = w; i < 256; i += 16) {
             s += cent[static_cast<uint64_t>(i) * step * dim + d];
         }
     }
-    part[w][lane] = s;
+    s *= 1.0F / 16.0F;
+    part[w][lane] = s - s == 0.0F ? s : 3.0e38F;
     __syncthreads();
     if (w == 0 && d < dim) {
         float t = 0.0F;
         for (uint32_t i = 0; i < 16; ++i) {
-            t += part[i][lane];
+            const float v = part[i][lane];
+            uint32_t rank = 0;
+            for (uint32_t j = 0; j < 16; ++j) {
+                const float o = part[j][lane];
+                rank += o < v || (o == v && j < i) ? 1U : 0U;
+            }
+            t += rank >= 4 && rank < 12 ? v : 0.0F;
         }
-        t *= 1.0F / static_cast<float>(take);
+        t *= 1.0F / 8.0F;
         centre[d] = t - t == 0.0F ? t : 0.0F;
     }
 }
 
 __global__ void
-kmeans_clear_maxima_kernel(uint32_t* maxima) {
-    if (threadIdx.x < 4) {
-        maxima[threadIdx.x] = 0;
+kmeans_reset_kernel(KmeansH16State* state) {
+    if (threadIdx.x == 0) {
+        reset_state(state);
     }
 }
 
@@ -162,17 +179,10 @@ wave_sum(float v) {
     return v;
 }
 
-// |c'|^2 per centroid and the largest |c'|^2 and |c|^2 (positive floats order like their bits; NaN above infinity).
-// A workgroup of sixteen waves takes 64 centroids: one atomic per maximum and workgroup.
+// |c'|^2 per centroid, a wave each.
 __global__ void __launch_bounds__(1024)
-kmeans_cnorm_kernel(const float* cent, uint32_t k, uint32_t dim, const float* centre, const float* cnorm_raw, float* cnorm,
-                    uint32_t* maxima) {
-    __shared__ uint32_t most[2];
+kmeans_cnorm_kernel(const float* cent, uint32_t k, uint32_t dim, const float* centre, float* cnorm) {
     const uint32_t lane = threadIdx.x & 63;
-    if (threadIdx.x < 2) {
-        most[threadIdx.x] = 0;
-    }
-    __syncthreads();
     for (uint32_t c = blockIdx.x * kGroup + (threadIdx.x >> 6); c < (blockIdx.x + 1) * kGroup && c < k; c += 16) {
         const float* row = cent + static_cast<uint64_t>(c) * dim;
         float s = 0.0F;
@@ -183,13 +193,7 @@ kmeans_cnorm_kernel(const float* cent, uint32_t k, uint32_t dim, const float* ce
         s = wave_sum(s);
         if (lane == 0) {
             cnorm[c] = s;
-            atomicMax(&most[0], magnitude_bits(s));
-            atomicMax(&most[1], magnitude_bits(cnorm_raw[c]));
         }
-    }
-    __syncthreads();
-    if (threadIdx.x < 2) {
-        atomicMax(&maxima[threadIdx.x], most[threadIdx.x]);
     }
 }
 
@@ -235,26 +239,79 @@ round_row(const float* row, uint32_t dim, uint32_t dpad, const float* centre, bo
     *kept = wave_sum(ks);
 }
 
+// The error bound of every row holds the largest centroid, so one far out would make all centroids of all rows possible.
+// Those are left out instead (zeros, and the contraction takes them for padding), and a row asks whether the nearest of them
+// can be ruled out by the triangle inequality alone.  Far: 32 times as far from the centre as all but one in 64 of (up to
+// 4096 of) the centroids, rounded up to the next power of two, or not finite.  (1M x 960, k 4096 with one centroid a thousand
+// times as long as the rest, or one NaN: 75 -> 13.0 ms, as without it.)
 __global__ void __launch_bounds__(1024)
 kmeans_round_centroids_kernel(const float* cent, uint32_t k, uint32_t dim, uint32_t dpad, const float* centre, int wide,
-                              uint16_t* c16, uint32_t* maxima) {
-    __shared__ uint32_t most;
-    if (threadIdx.x == 0) {
-        most = 0;
+                              const float* cnorm_raw, const float* cnorm, uint16_t* c16, KmeansH16State* state) {
+    __shared__ uint32_t hist[256], most[3], nearest_far;
+    __shared__ float far_from;
+    const uint32_t tid = threadIdx.x, lane = tid & 63;
+    if (tid < 256) {
+        hist[tid] = 0;
+    }
+    if (tid < 3) {
+        most[tid] = 0;
+    }
+    if (tid == 0) {
+        nearest_far = __float_as_uint(__builtin_inff());
     }
     __syncthreads();
-    const int e = scale_exponent(__uint_as_float(maxima[0]));
-    for (uint32_t c = blockIdx.x * kGroup + (threadIdx.x >> 6); c < (blockIdx.x + 1) * kGroup && c < k; c += 16) {
-        float missed, kept;
-        round_row(cent + static_cast<uint64_t>(c) * dim, dim, dpad, centre, wide != 0, ldexpf(1.0F, e),
-                  c16 + static_cast<uint64_t>(c) * dpad, &missed, &kept);
-        if ((threadIdx.x & 63) == 0) {
-            atomicMax(&most, magnitude_bits(ldexpf(sqrtf(missed), -e)));
+    const uint32_t take = k < 4096 ? k : 4096, step = k / take;
+    for (uint32_t i = tid; i < take; i += 1024) {
+        atomicAdd(&hist[magnitude_bits(cnorm[static_cast<uint64_t>(i) * step]) >> 23], 1U);
+    }
+    __syncthreads();
+    if (tid < 64) {
+        uint32_t incl = 0;
+        for (uint32_t i = 0; i < 4; ++i) {
+            incl += hist[4 * lane + i];
+        }
+        const uint32_t sum = incl;
+        for (int off = 1; off < 64; off <<= 1) {
+            const uint32_t up = __shfl_up(incl, off);
+            incl += lane >= static_cast<uint32_t>(off) ? up : 0;
+        }
+        const uint32_t want = take - take / 64;
+        uint32_t before = incl - sum;
+        if (before < want && want <= incl) {
+            uint32_t bin = 4 * lane;  // |c'|^2 in [2^(bin - 127), 2^(bin - 126))
+            while (before + hist[bin] < want) {
+                before += hist[bin];
+                ++bin;
+            }
+            far_from = bin > 215 ? 1.0e30F : ldexpf(1.0F, static_cast<int>(bin) - 126 + 10);
         }
     }
     __syncthreads();
-    if (threadIdx.x == 0) {
-        atomicMax(&maxima[2], most);
+    const float limit = far_from;
+    const int e = scale_exponent(limit);
+    for (uint32_t c = blockIdx.x * kGroup + (tid >> 6); c < (blockIdx.x + 1) * kGroup && c < k; c += 16) {
+        const float sq = cnorm[c], raw = cnorm_raw[c];
+        const bool near = sq <= limit;  // false for NaN as well
+        float missed, kept;
+        round_row(cent + static_cast<uint64_t>(c) * dim, near ? dim : 0, dpad, centre, wide != 0, ldexpf(1.0F, e),
+                  c16 + static_cast<uint64_t>(c) * dpad, &missed, &kept);
+        if (lane == 0) {
+            if (near) {
+                atomicMax(&most[0], magnitude_bits(sq));
+                atomicMax(&most[1], magnitude_bits(raw));
+                atomicMax(&most[2], magnitude_bits(ldexpf(sqrtf(missed), -e)));
+            } else if (raw - raw == 0.0F) {  // (the fp32 kernels choose none whose |c|^2 is not finite)
+                atomicMin(&nearest_far, magnitude_bits(fminf(sq, 3.0e38F)));
+            }
+        }
+    }
+    __syncthreads();
+    if (tid == 0) {
+        atomicMax(&state->centred, most[0]);
+        atomicMax(&state->raw, most[1]);
+        atomicMax(&state->missed, most[2]);
+        atomicMin(&state->nearest_far, nearest_far);
+        state->far_from = __float_as_uint(limit);  // (all workgroups the same)
     }
 }
 
@@ -304,7 +361,7 @@ struct KmeansH16Args {
     uint32_t slots;    // dpad / 8
     const float* xscale;
     const float* cnorm;
-    const uint32_t* maxima;
+    const KmeansH16State* state;
     float* group_min;
     uint64_t ld;       // the table: [group][3][ld]
     uint32_t rtiles, ctiles, mc_log2, mcols, macros;
@@ -361,7 +418,8 @@ kmeans_h16_kernel(KmeansH16Args p) {
                    ob3 = offset(lr + 192, b_last);
     const uint32_t put = lr * kSlots + (ls ^ ((lr >> 1) & 7));  // + 64 i rows
     if (tid < kTile) {
-        cn[tid] = c0 + tid < p.k ? p.cnorm[c0 + tid] : 3.0e38F;
+        const float sq = c0 + tid < p.k ? p.cnorm[c0 + tid] : 3.0e38F;
+        cn[tid] = sq <= __uint_as_float(p.state->far_from) ? sq : 3.0e38F;
     }
 
     uint4 ga0, ga1, ga2, ga3, gb0, gb1, gb2, gb3;  // (separate variables: an array went to scratch memory)
@@ -456,7 +514,7 @@ kmeans_h16_kernel(KmeansH16Args p) {
 
     // acc[i][j][e] = <C, X> (scaled) of centroid c0 + wm 128 + 32 i + 8 (e / 4) + 4 half + e % 4 and row wn 64 + 32 j + l32:
     // the 64 of a lane are one group of the table, 16 i + e the place in it.
-    const float cdown = ldexpf(-2.0F, -scale_exponent(__uint_as_float(p.maxima[0])));
+    const float cdown = ldexpf(-2.0F, -scale_exponent(__uint_as_float(p.state->far_from)));
     const uint32_t group = (ct * 2 + wm) * 2 + half;
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
@@ -501,13 +559,12 @@ struct KmeansRescoreArgs {
     const float2* xinfo;
     const float* xnorm;
     const float* cnorm_raw;
-    const uint32_t* maxima;
+    KmeansH16State* state;
     int wide;
     int natural;  // order of the products, see the kernel
     unsigned long long* best;
     uint8_t* row_open;
     uint32_t* open64;
-    uint32_t* any_open;
 };
 
 // 64 rows per workgroup.  First four threads a row look through the table (coalesced along the rows); then a lane per
@@ -555,9 +612,9 @@ kmeans_h16_rescore_kernel(KmeansRescoreArgs p) {
         // lose, kTinyRest the same for the remainders (in scales of 2^14 and more), kTinySquare what the products can.  Rows and
         // centroids that small have every centroid possible and go to the fp32 kernels.
         constexpr float kTinyLength = 2.0e-17F, kTinyRest = 1.0e-20F, kTinySquare = 1.0e-33F;
-        const float cmax = sqrtf(__uint_as_float(p.maxima[0])) * 1.00001F + kTinyLength;
-        const float craw = sqrtf(__uint_as_float(p.maxima[1])) * 1.00001F + kTinyLength;
-        const float cmiss = __uint_as_float(p.maxima[2]) * 1.00001F + kTinyRest;
+        const float cmax = sqrtf(__uint_as_float(p.state->centred)) * 1.00001F + kTinyLength;
+        const float craw = sqrtf(__uint_as_float(p.state->raw)) * 1.00001F + kTinyLength;
+        const float cmiss = __uint_as_float(p.state->missed) * 1.00001F + kTinyRest;
         const float missed = info.x * 1.00001F + kTinyRest, kept = info.y * 1.00001F + kTinyRest;
         const float xraw = sqrtf(p.xnorm[row]) * 1.00001F + kTinyLength;
         const float steps = static_cast<float>(p.dim);
@@ -572,7 +629,15 @@ kmeans_h16_rescore_kernel(KmeansRescoreArgs p) {
         err += (steps / 64.0F + 12.0F) * 2.0F * kU * craw * craw;
         err += 2.0F * (steps + 4.0F) * kU * xraw * craw + kTinySquare;
         const float limit = least + 2.0F * err;
-        if (!(err < 1.0e30F) || !(fabsf(limit) < 1.0e30F)) {
+        // A far centroid at r from the centre: |c'|^2 - 2 <x', c'> >= r^2 - 2 r |x'|, which as well as its fp32 distance
+        // (roundings: 1e-3 |x| |c| and 2e-5 |c|^2 at most, up to 8192 dimensions; |c| <= r + |x| + |x'|) grows with r from
+        // four times |x| + |x'| on, so that the nearest one speaks for all.
+        const float far = sqrtf(__uint_as_float(p.state->nearest_far)) * 0.9999F;
+        const float len = kept + missed, both = len + xraw;
+        const bool far_out = p.state->nearest_far == __float_as_uint(__builtin_inff()) ||
+                             (far >= 4.0F * both &&
+                              0.99F * far * far - 2.0F * far * len - 2.0e-3F * xraw * (far + both) > limit);
+        if (!(err < 1.0e30F) || !(fabsf(limit) < 1.0e30F) || !far_out) {
             cost[rl] = kMaxWork + 1;  // (its threads write the same)
         } else {
 #pragma unroll 4
@@ -620,7 +685,7 @@ kmeans_h16_rescore_kernel(KmeansRescoreArgs p) {
     if (tid == 0) {
         p.open64[blockIdx.x] = any;
         if (any != 0) {
-            *p.any_open = 1;
+            p.state->any_open = 1;
         }
     }
 
@@ -696,7 +761,10 @@ kmeans_h16_rescore_kernel(KmeansRescoreArgs p) {
         }
         if (base + tid < total && tid < kPairs) {
             const uint32_t c = pair_c[tid];
-            atomicMin(&best[pair_row[tid]], static_cast<unsigned long long>(make_key(p.cnorm_raw[c] + (-2.0F * acc), c)));
+            const float dist = p.cnorm_raw[c] + (-2.0F * acc);
+            if (dist < __builtin_inff()) {  // (a whole group may hold a centroid that is not finite: nobody chooses it)
+                atomicMin(&best[pair_row[tid]], static_cast<unsigned long long>(make_key(dist, c)));
+            }
         }
         __syncthreads();  // pair_row / pair_c are written again
     }
@@ -722,14 +790,13 @@ launch_kmeans_h16(const float* x, uint64_t n, uint32_t dim, const float* cent, u
     const bool kept = have_xnorm && n <= slab;  // the rows' fp16 form of the call before, and the centre it was formed with
     const uint32_t cblocks = (k + kGroup - 1) / kGroup;
     if (!kept) {
-        hipLaunchKernelGGL(kmeans_centre_kernel, dim3((dim + 63) / 64), dim3(1024), 0, st, cent, k, dim, b.centre, b.maxima);
+        hipLaunchKernelGGL(kmeans_centre_kernel, dim3((dim + 63) / 64), dim3(1024), 0, st, cent, k, dim, b.centre, b.state);
     } else {
-        hipLaunchKernelGGL(kmeans_clear_maxima_kernel, dim3(1), dim3(64), 0, st, b.maxima);
+        hipLaunchKernelGGL(kmeans_reset_kernel, dim3(1), dim3(64), 0, st, b.state);
     }
-    hipLaunchKernelGGL(kmeans_cnorm_kernel, dim3(cblocks), dim3(1024), 0, st, cent, k, dim, b.centre, cnorm_raw, b.cnorm,
-                       b.maxima);
+    hipLaunchKernelGGL(kmeans_cnorm_kernel, dim3(cblocks), dim3(1024), 0, st, cent, k, dim, b.centre, b.cnorm);
     hipLaunchKernelGGL(kmeans_round_centroids_kernel, dim3(cblocks), dim3(1024), 0, st, cent, k, dim, dpad, b.centre, wide,
-                       b.c16, b.maxima);
+                       cnorm_raw, b.cnorm, b.c16, b.state);
     for (uint64_t r0 = 0; r0 < n; r0 += slab) {
         const uint64_t rows = n - r0 < slab ? n - r0 : slab;
         if (!kept) {
@@ -745,7 +812,7 @@ launch_kmeans_h16(const float* x, uint64_t n, uint32_t dim, const float* cent, u
         a.slots = dpad / 8;
         a.xscale = b.xscale;
         a.cnorm = b.cnorm;
-        a.maxima = b.maxima;
+        a.state = b.state;
         a.group_min = b.group_min;
         a.ld = slab;
         a.rtiles = static_cast<uint32_t>(div_up(rows, kTile));
@@ -768,13 +835,12 @@ launch_kmeans_h16(const float* x, uint64_t n, uint32_t dim, const float* cent, u
         s.xinfo = b.xinfo;
         s.xnorm = xnorm + r0;
         s.cnorm_raw = cnorm_raw;
-        s.maxima = b.maxima;
+        s.state = b.state;
         s.wide = wide;
         s.natural = (dim & 3) != 0;
         s.best = best + r0;
         s.row_open = b.row_open + r0;
         s.open64 = b.open64 + r0 / kRowsPerBlock;
-        s.any_open = b.maxima + 3;
         const dim3 grid(static_cast<uint32_t>(div_up(rows, kRowsPerBlock)));
         hipLaunchKernelGGL(kmeans_h16_rescore_kernel, grid, dim3(256), 0, st, s);
     }
