@@ -90,6 +90,50 @@ def test_small_batches_equal_streaming(lib, modes, kind, d, nq, k, pre):
     st.destroy()
 
 
+def _store_of(kind, metric, x, rng):
+    """A store of the rows' codes, quantizer trained on the first of them."""
+    d = x.shape[1]
+    if kind == "fp32":
+        st, codes = Store(capi.KIND_FP32, metric, d), x.view(np.uint8).reshape(len(x), -1)
+    elif kind == "rabitq":
+        rot, _ = np.linalg.qr(rng.standard_normal((d, d)))
+        rot = rot.astype(np.float32)
+        cen = orc.rabitq_train(x[:20000], rot)
+        st, codes = Store(capi.KIND_RABITQ, metric, d, rot=rot, centroid=cen), orc.rabitq_encode(x, rot, cen, metric)
+    elif kind.endswith("uniform"):
+        bits = int(kind[2])
+        lb, diff = orc.sq_train_uniform(x[:20000], bits, metric, mode=3 if bits == 4 else 1)
+        st, codes = Store(capi.KINDS[kind], metric, d, bounds=[lb, diff]), orc.squ_encode(x, bits, lb, diff, metric)
+    else:
+        bits = int(kind[2])
+        lb, diff = orc.sq_train(x[:20000], bits, metric)
+        st, codes = Store(capi.KINDS[kind], metric, d, lb=lb, diff=diff), orc.sq_encode(x, bits, lb, diff, metric)
+    st.append(codes)
+    return st
+
+
+@pytest.mark.parametrize("kind,metric,n,d,k,last_streamed", [
+    ("fp32", orc.IP, 70001, 100, 10, 175), ("fp32", orc.COSINE, 70001, 64, 1, 274), ("fp32", orc.L2, 150001, 131, 100, 402),
+    ("sq8", orc.IP, 150001, 100, 10, 289), ("sq8", orc.L2, 1000001, 100, 10, 31), ("sq4", orc.L2, 70001, 128, 10, 323),
+    ("sq4", orc.COSINE, 150001, 128, 7, 226), ("sq4", orc.IP, 150001, 300, 10, 108), ("sq8", orc.COSINE, 100001, 200, 10, 243),
+    ("sq8", orc.IP, 320001, 960, 10, 16), ("sq4", orc.COSINE, 320001, 960, 7, 15),
+    ("sq8_uniform", orc.L2, 300001, 128, 10, 307), ("sq8_uniform", orc.IP, 300001, 128, 10, 460),
+    ("sq4_uniform", orc.COSINE, 500001, 96, 10, 368), ("sq4_uniform", orc.L2, 300001, 128, 10, 307),
+    ("rabitq", orc.L2, 2000001, 96, 200, 402), ("rabitq", orc.IP, 2500001, 96, 10, 483)])
+def test_small_batches_of_every_kind_and_metric(lib, modes, kind, metric, n, d, k, last_streamed):
+    """The largest batch that streams and the smallest that is pre-selected, of every kind and metric: the line lies between
+    them, and both return what streaming returns."""
+    rng = np.random.default_rng(n + d)
+    x, means = gaussian_mixture(rng, n, d, 100, 0.05)
+    q, _ = gaussian_mixture(rng, 511, d, 100, 0.05, means=means)
+    st = _store_of(kind, metric, x, rng)
+    for nq, pre in ((last_streamed, False), (last_streamed + 1, True)):
+        plain, auto, tile = modes(st, q[:nq], k, 0)
+        assert same(plain, auto), nq
+        assert (tile >= 128) == pre, (nq, tile)
+    st.destroy()
+
+
 @pytest.mark.parametrize("kind,bits", [("sq8", 8), ("sq4", 4)])
 def test_fp16_preselection_keeps_few_candidates_under_cosine(lib, modes, kind, bits):
     """The thresholds of a cosine batch are as narrow as its distances: no query overflows its candidates (every query did,

@@ -1168,19 +1168,24 @@ prefilter_supports(const vsag_amd_store* s) {
 
 // Whether a batch of nq queries is pre-selected (stores of at least 1024 tiles).  From 512 queries on always; below, the
 // dozen launches, the exact prefix and the rescoring (which grows with k) have to be less than the streaming kernel's time,
-// which grows with queries x codes x dimensions.  Measured under L2, us per call, streaming -> pre-selected, beside the line:
-//   fp32 (fp32 matrix cores): 100k x 128, k 10, 64 queries 271 -> 261, 128 338 -> 273 (32: 214 -> 242, not taken); 1M x 128,
-//     k 100, 64 queries 1160 -> 1057; 100k x 768, k 100, 128 queries 1377 -> 1801 (not taken); 600k x 960, k 10, 256 queries
-//     11896 -> 3866.  Their time hardly depends on the dimension's share of the work from 128 on: both sides grow with it.
-//   sq8 / sq4 on the int8 matrix cores: 1M x 128, k 10, 32 queries 497 -> 343, 16 274 -> 340 (not taken); k 100, 64 queries
-//     791 -> 630; 100k x 128, k 10, 256 queries 303 -> 273, 128 208 -> 264 (not taken).
-//   sq8 / sq4 on the fp16 matrix cores: 200k x 768, k 10, 32 queries 842 -> 474, 16 440 -> 469 (not taken); k 100, 128
-//     queries 1411 -> 1147, 64 870 -> 1119 (not taken); 600k x 960, k 10, 256 queries 8015 -> 1028.
-//   sq8_uniform / sq4_uniform (dot products of bytes, cheap to stream): 500k x 128, k 10, 256 queries 391 -> 352, 128
-//     317 -> 335 (not taken); 1M x 96, k 100, 256 queries 713 -> 622.
-//   RaBitQ, k 200: 1M x 768, 256 queries 2518 -> 1679, 128 1517 -> 1690 (not taken); 3M x 128, 256 queries 2248 -> 1470.
-// The other metrics stream up to 1.4 times as fast: their line lies half as far again out.  Below 64 dimensions the
-// streaming kernel's own overhead per code decides, and 512 stays the line.
+// which grows with queries x codes x dimensions.  Measured on Gaussian mixtures with the plan that the default mode makes,
+// under L2, us per call, streaming -> pre-selected, beside the line:
+//   fp32 (fp32 matrix cores): 100k x 128, k 10, 64 queries 291 -> 208 (32: 236 -> 182, not taken); 1M x 100, k 100, 128
+//     queries 1759 -> 831; 100k x 768, k 100, 64 queries 955 -> 1075, 128 1406 -> 1154 (not taken); 600k x 960, k 10, 256
+//     queries 12109 -> 3907.  Their time hardly depends on the dimension's share of the work from 128 on: both sides grow
+//     with it.
+//   sq8 / sq4 on the int8 matrix cores: 1M x 100, k 10, 32 queries 474 -> 358, 16 269 -> 333 (not taken); k 100, 64 queries
+//     752 -> 606; 100k x 128, k 10, 256 queries 314 -> 243, 128 224 -> 237 (not taken).
+//   sq8 / sq4 on the fp16 matrix cores: 200k x 768, k 10, 32 queries 849 -> 462, 16 458 -> 450 (not taken); k 100, 128
+//     queries 1358 -> 1018, 64 849 -> 959 (not taken); 600k x 960, k 10, 256 queries 8158 -> 1013.
+//   sq8_uniform / sq4_uniform (dot products of bytes, cheap to stream): 500k x 128, k 10, 256 queries 386 -> 325, 128
+//     321 -> 314 (not taken); 1M x 96, k 100, 256 queries 810 -> 592.
+//   RaBitQ, k 200: 1M x 768, 256 queries 2439 -> 1392, 128 1454 -> 1436 (not taken); 3M x 128, 256 queries 2356 -> 1384.
+// The other metrics stream up to twice as fast (sq8, 600k x 960, 32 queries: 2390 under L2, 1240 under inner product) and
+// are pre-selected no faster: their line lies half as far again out, and the 16 queries that four passes of the streaming
+// kernel serve stay with it from k 8 on (sq4, 600k x 960, cosine: k 10 568 -> 616, k 30 599 -> 854, k 1 640 -> 456; 20
+// queries, k 30: 850 -> 854).  Below 64 dimensions the streaming kernel's own overhead per code decides, and 512 stays the
+// line.
 bool
 prefilter_pays(const vsag_amd_store* s, uint64_t nq, uint32_t k) {
     if (nq >= 512) {
@@ -1204,7 +1209,7 @@ prefilter_pays(const vsag_amd_store* s, uint64_t nq, uint32_t k) {
             return nq >= 64 && work >= far * (1.1e10 + 8.0e7 * kk);
         default:
             return s->dim <= 128 ? nq >= 32 && work >= far * (2.7e9 + 2.0e7 * kk)
-                                 : nq >= 16 && work >= far * (2.0e9 + 1.25e8 * kk);
+                                 : nq >= (far > 1.0 && k >= 8 ? 17U : 16U) && work >= far * (2.0e9 + 1.25e8 * kk);
     }
 }
 
