@@ -191,12 +191,25 @@ def _routed_data(kind, n, d, k):
         cent += 30.0
     elif kind == "scaled":  # lengths over twelve octaves
         x *= np.exp2(rng.integers(-6, 7, (n, 1))).astype(np.float32)
-    elif kind == "copies":  # every centroid five times: whole groups stay possible, and most rows go to the fp32 kernels
+    elif kind == "copies":  # every centroid five times: ties, and here and there a whole group that stays possible
         cent = np.tile(cent[: k // 5], (5, 1))[rng.permutation(k // 5 * 5)]
         cent = np.concatenate([cent, cent[: k - len(cent)]])
     elif kind == "same":  # one point: every distance ties
         x[:] = x[0]
         cent[:] = x[0]
+    elif kind == "crowd":  # every centroid forty times, more than a row's list holds: every row goes to the fp32 kernels
+        cent = cent[np.arange(k) % (k // 40)][rng.permutation(k)]
+    elif kind == "holes":  # a row in 64 too long for fp16: every tile of the fp32 kernels has something to do
+        x[::64] *= np.float32(1e16)
+    elif kind == "exact":  # whole numbers of eleven bits around a centre of zero: fp16 holds them, only sums are rounded
+        x = rng.integers(-2047, 2048, (n, d)).astype(np.float32)
+        cent = rng.integers(-2047, 2048, (k, d)).astype(np.float32)
+        cent[k // 2:k // 2 * 2] = cent[:k // 2]  # near ties: copies with one entry off by one
+        cent[np.arange(k // 2), rng.integers(0, d, k // 2)] += 1.0
+        step = k // 256  # the centre is made of sums of the rows (w + 16 i) * step: opposites in pairs
+        for w in range(16):
+            for i in range(0, 16, 2):
+                cent[(w + 16 * (i + 1)) * step] = -cent[(w + 16 * i) * step]
     elif kind == "outliers":  # centroids far out, one of them with rows next to it, and centroids that are not finite
         cent[3] *= np.float32(100.0)
         cent[k - 1] *= np.float32(1e12)
@@ -213,12 +226,16 @@ def _routed_data(kind, n, d, k):
                                         ("plain", 62001, 257, 257), ("offset", 20011, 101, 2049), ("scaled", 16385, 128, 2048),
                                         ("copies", 16385, 128, 2050), ("same", 16384, 128, 2048), ("plain", 33000, 64, 2111),
                                         ("outliers", 16385, 128, 2048), ("outliers", 20011, 101, 2049),
-                                        ("outliers", 62001, 260, 256)])
+                                        ("outliers", 62001, 260, 256), ("plain", 20011, 100, 2049), ("plain", 20011, 132, 1601),
+                                        ("plain", 62001, 196, 400), ("exact", 20011, 132, 1601), ("crowd", 20011, 101, 2049),
+                                        ("crowd", 70001, 192, 320), ("holes", 20011, 101, 2049), ("holes", 70001, 192, 320),
+                                        # more rows than are rounded at a time (65536)
+                                        ("holes", 70001, 1000, 260), ("outliers", 70001, 1000, 260)])
 def test_assign_after_the_fp16_preselection(lib, kind, n, d, k):
     x, cent = _routed_data(kind, n, d, k)
     labels, mind, loss = gpu_assign(x, cent)
     assert labels.min() >= 0 and labels.max() < k
-    if kind != "outliers":
+    if kind not in ("outliers", "holes"):
         check_assignment(x, cent, labels, mind)
     # bit for bit what the fp32 kernels return: pieces too small for the pre-selection take those
     rows = min(n, int(3.9e9 / (k * d)))
@@ -320,18 +337,20 @@ def test_assign_after_the_fp16_preselection_with_values_out_of_range(lib):
     assert np.array_equal(mind[odd].view(np.int32), few_mind.view(np.int32))
     keep = np.setdiff1d(np.arange(n), odd)
     check_assignment(x[keep], cent, labels[keep], mind[keep])
-    cent[7, 3] = np.inf  # one centroid out of range: every row takes the fp32 kernels, and nobody chooses it
+    cent[7, 3] = np.inf  # one centroid out of range: nobody chooses it
     labels2, _, _ = gpu_assign(x[keep], cent)
     assert not (labels2 == 7).any() and (labels2 == labels[keep]).mean() > 0.999
 
 
-def test_run_with_the_fp16_preselection_keeps_its_rows(lib):
-    # the rows are rounded once per run; the centre is that of the first iteration
+@pytest.mark.parametrize("n,d,k,iters", [(16400, 128, 2048, 4), (70001, 1000, 260, 3)])
+def test_run_with_the_fp16_preselection_keeps_its_rows(lib, n, d, k, iters):
+    # the rows are rounded once per run where one slab holds them, and the centre is that of the first iteration; more rows
+    # are rounded again in every iteration, and only their lengths are kept
     L = lib.load_library()
-    n, d, k, iters = 16400, 128, 2048, 4
     rng = np.random.default_rng(5)
-    x, _ = gaussian_mixture(rng, n, d, 300, 0.2, uniform_means=False)
-    cent0 = x[rng.choice(n, k, replace=False)].copy()
+    x, means = gaussian_mixture(rng, n, d, 300, 0.2, uniform_means=False)
+    # (no cluster may run empty: the steps below do not re-seed)
+    cent0 = np.ascontiguousarray(means[:k]) if k <= len(means) else x[rng.choice(n, k, replace=False)].copy()
     xb, cb = dev(x), dev(cent0)
     labels = capi.DeviceBuffer(n * 4)
     loss = C.c_double()

@@ -109,7 +109,7 @@ def _rotation(rng, d):
 
 
 @pytest.mark.parametrize("metric", [orc.L2, orc.IP])
-@pytest.mark.parametrize("n,d", [(500, 128), (200, 15), (64, 768)])
+@pytest.mark.parametrize("n,d", [(500, 128), (200, 15), (64, 768), (63, 31), (65, 36), (257, 33)])
 def test_rabitq_train_encode_query_bit_exact(lib, metric, n, d):
     """The device keeps every running sum in element order and does not fuse multiply-adds, so the codes,
     the trailing floats and the processed queries equal the checker's bit for bit."""
@@ -313,3 +313,67 @@ def test_sq_bounds_of_awkward_columns(lib, kind, n):
         lb, diff = _train(lib, x, bits, orc.L2, capi.SQ_TRAIN_TRUNC_BOUND)
         rlb, rdiff = orc.sq_train(x, bits, orc.L2, mode=capi.SQ_TRAIN_TRUNC_BOUND)
         assert np.array_equal(lb, rlb) and np.array_equal(diff, rdiff), (bits, lb, rlb)
+
+
+class _Shifted:
+    """Device memory whose data begin `shift` bytes behind an aligned address."""
+
+    def __init__(self, shift, data=None, nbytes=0):
+        self.shift = shift
+        raw = np.zeros(shift + (data.nbytes if data is not None else nbytes), np.uint8)
+        if data is not None:
+            raw[shift:] = np.ascontiguousarray(data).view(np.uint8).reshape(-1)
+        self.buf, self.nbytes = dev(raw), raw.nbytes
+        self.ptr = self.buf.ptr + shift
+
+    def bytes(self, shape):
+        return self.buf.to_numpy(np.uint8, (self.nbytes,))[self.shift:].reshape(shape)
+
+
+@pytest.mark.parametrize("metric", [orc.L2, orc.COSINE])
+@pytest.mark.parametrize("row_shift,code_shift", [(4, 0), (0, 1), (8, 3), (0, 2)])
+@pytest.mark.parametrize("n,d", [(65, 36), (32769, 32), (130, 33)])
+def test_encoders_take_any_alignment(lib, metric, row_shift, code_shift, n, d):
+    """Rows at any float and codes at any byte: the forms without vector loads and word stores, of few and of many rows."""
+    L = lib.load_library()
+    rng = np.random.default_rng(n + d)
+    x = (rng.standard_normal((n, d)) * 0.3 + 0.5).astype(np.float32)
+    xb = _Shifted(row_shift, x)
+    for bits in (4, 8):
+        lb, diff = orc.sq_train(x, bits, metric)
+        ref = orc.sq_encode(x, bits, lb, diff, metric)
+        lbb, dfb, out = _Shifted(row_shift, lb), _Shifted(row_shift, diff), _Shifted(code_shift, nbytes=ref.nbytes)
+        capi.check(L.vsag_amd_sq_encode(xb.ptr, n, d, bits, metric, lbb.ptr, dfb.ptr, out.ptr, None))
+        assert np.array_equal(out.bytes(ref.shape), ref), bits
+        ulb, udiff = orc.sq_train_uniform(x, bits, metric, mode=3 if bits == 4 else 1)
+        ref = orc.squ_encode(x, bits, ulb, udiff, metric)
+        bb, out = dev(np.array([ulb, udiff], np.float32)), _Shifted(code_shift, nbytes=ref.nbytes)
+        capi.check(L.vsag_amd_squ_encode(xb.ptr, n, d, bits, metric, bb.ptr, out.ptr, None))
+        assert np.array_equal(out.bytes(ref.shape), ref), bits
+    if n > 1000 or metric == orc.COSINE:
+        return
+    rot = _rotation(rng, d)
+    cen = orc.rabitq_train(x, rot)
+    ref = orc.rabitq_encode(x, rot, cen, metric)
+    rb, cb, out = dev(rot), dev(cen), _Shifted(code_shift, nbytes=ref.nbytes)
+    capi.check(L.vsag_amd_rabitq_encode(xb.ptr, n, d, rb.ptr, cb.ptr, metric, 4, out.ptr, None))
+    assert np.array_equal(out.bytes(ref.shape), ref)
+
+
+@pytest.mark.parametrize("odd", [[np.inf], [-np.inf], [np.inf, -np.inf], [np.nan], [np.nan, np.inf, -np.inf]])
+@pytest.mark.parametrize("bits,n", [(8, 2049), (4, 2047), (4, 70001)])
+def test_sq_bounds_of_columns_that_are_not_finite(lib, bits, n, odd):
+    """Order statistics where infinities lie at the ends and NaN of positive sign behind infinity; columns with more of them
+    than are ignored, with fewer and with none."""
+    rng = np.random.default_rng(n + len(odd))
+    ignore = max(1, int((n - 1) * float(np.float32(0.05) if bits == 4 else 0.001)))
+    x = rng.standard_normal((n, 4)).astype(np.float32)
+    for c, count in enumerate((1, ignore + 1, 3 * ignore)):  # the last column stays finite
+        at = rng.permutation(n)[:count]
+        x[at, c] = np.resize(np.array(odd, np.float32), count)
+    lb, diff = _train(lib, x, bits, orc.L2, capi.SQ_TRAIN_TRUNC_BOUND)
+    column = np.sort(x, axis=0)  # numpy puts NaN last, too
+    lower, upper = column[ignore - 1], column[n - ignore]
+    assert np.array_equal(lb, lower, equal_nan=True)
+    with np.errstate(invalid="ignore"):
+        assert np.array_equal(diff, upper - lower, equal_nan=True)

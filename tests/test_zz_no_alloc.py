@@ -157,3 +157,27 @@ def test_noalloc_uniform_store_under_cosine(lib, bits):
                                 lb=lb, diff=diff)
     assert_topk_close(a2[0], a2[1], oi, od, label="noalloc uniform cosine")
     store.destroy()
+
+
+def test_noalloc_small_batch_without_room_for_candidate_lists(lib):
+    """Fewer than 512 queries that a caller's workspace lets the matrix cores pre-select: the array has no room for their
+    candidate lists, and the streaming kernel serves them."""
+    l = capi.load_library()
+    rng = np.random.default_rng(31)
+    n, d, nq, k = 2000001, 64, 500, 10
+    x = rng.standard_normal((n, d), dtype=np.float32)
+    rot = _rotation(rng, d)
+    cen = orc.rabitq_train(x[:20000], rot)
+    store = Store(capi.KIND_RABITQ, orc.L2, d, rot=rot, centroid=cen)
+    store.append(orc.rabitq_encode(x, rot, cen, orc.L2))
+    q = rng.standard_normal((nq, d), dtype=np.float32)
+    assert l.vsag_amd_flat_scan_workspace_bytes(store.handle, nq, k) > (32 << 20)
+    noalloc_scan(l, store, q, k, count_memory=False)  # first launches of these kernels in the process: see above
+    a = noalloc_scan(l, store, q, k)
+    tile = C.c_int()
+    l.vsag_amd_last_scan_info(C.byref(tile), None, None)
+    assert tile.value < 128
+    b = store.flat_scan(q, k)
+    l.vsag_amd_last_scan_info(C.byref(tile), None, None)
+    assert tile.value >= 128 and same(a, b)
+    store.destroy()
