@@ -570,8 +570,9 @@ def run_c3(env):
     flops = 2.0 * n * k * d
     tf = flops / (kms * 1e-3) / 1e12
     # The contraction pre-selects on the fp16 matrix cores (kmeans_h16.hip) where there is enough of it: kernel_ms then
-    # spans that pass and the fp32 rescoring of what it leaves, the flops are the contraction's.
-    h16 = 32 <= d <= 8192 and k >= 256 and k * d >= 49152 and n * k * d >= 4e9
+    # spans that pass and the fp32 rescoring of what it leaves, the flops are the contraction's.  The workspace says which
+    # route a call takes: the fp32 kernels need twelve bytes a row and little else.
+    h16 = wsb_a > 12.1 * n + 4 * k + 4096
     peak = MFMA_F16_PEAK_TFLOPS if h16 else MFMA_F32_PEAK_TFLOPS
     roof = {"bound": "mfma", "achieved": tf, "peak": peak, "unit": "TFLOP/s", "frac": tf / peak, "traffic": None,
             "kernel": "kmeans_h16_kernel + kmeans_round_rows_kernel + kmeans_h16_rescore_kernel" if h16 else
