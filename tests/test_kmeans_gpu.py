@@ -201,6 +201,8 @@ def _routed_data(kind, n, d, k):
         cent = cent[np.arange(k) % (k // 40)][rng.permutation(k)]
     elif kind == "holes":  # a row in 64 too long for fp16: every tile of the fp32 kernels has something to do
         x[::64] *= np.float32(1e16)
+    elif kind == "long start":
+        x[:65536] *= np.float32(1e16)
     elif kind == "exact":  # whole numbers of eleven bits around a centre of zero: fp16 holds them, only sums are rounded
         x = rng.integers(-2047, 2048, (n, d)).astype(np.float32)
         cent = rng.integers(-2047, 2048, (k, d)).astype(np.float32)
@@ -230,12 +232,15 @@ def _routed_data(kind, n, d, k):
                                         ("plain", 62001, 196, 400), ("exact", 20011, 132, 1601), ("crowd", 20011, 101, 2049),
                                         ("crowd", 70001, 192, 320), ("holes", 20011, 101, 2049), ("holes", 70001, 192, 320),
                                         # more rows than are rounded at a time (65536)
-                                        ("holes", 70001, 1000, 260), ("outliers", 70001, 1000, 260)])
+                                        ("holes", 70001, 1000, 260), ("outliers", 70001, 1000, 260),
+                                        # the rows behind a slab of open ones are not pre-selected
+                                        ("crowd", 70001, 1000, 260), ("long start", 70001, 1000, 260),
+                                        ("long start", 70001, 1001, 260)])
 def test_assign_after_the_fp16_preselection(lib, kind, n, d, k):
     x, cent = _routed_data(kind, n, d, k)
     labels, mind, loss = gpu_assign(x, cent)
     assert labels.min() >= 0 and labels.max() < k
-    if kind not in ("outliers", "holes"):
+    if kind not in ("outliers", "holes", "long start"):
         check_assignment(x, cent, labels, mind)
     # bit for bit what the fp32 kernels return: pieces too small for the pre-selection take those
     rows = min(n, int(3.9e9 / (k * d)))
@@ -273,6 +278,46 @@ def test_centroids_far_out_do_not_open_every_row(lib):
             capi.synchronize()
             best[i] = min(best[i], time.perf_counter() - t0)
     assert best[1] < 2.0 * best[0], best
+
+
+def test_rows_that_stay_open_are_not_preselected_over_and_over(lib):
+    """Where rows all over the place go to the fp32 kernels (the distances of clusters far from the origin are rounded to a
+    good part of their spread), only every fourth slab is tried first: all were, which took 1.46 times as long as the fp32
+    kernels alone, and 1.11 now; 1.3 is the line here."""
+    L = lib.load_library()
+    n, d, k = 480000, 960, 256
+    rng = np.random.default_rng(3)
+    x = gaussian_mixture(rng, n // 10, d, 1000, 0.05)[0] + np.float32(10.0)
+    cent = x[rng.choice(len(x), k, replace=False)]
+    xb, cb, lab = dev(np.tile(x, (10, 1))), dev(cent), capi.DeviceBuffer(n * 4)
+    sizes = (_fp32_assign_bytes(n, k), L.vsag_amd_kmeans_assign_workspace_bytes(n, d, k))
+    ws, best, out = capi.DeviceBuffer(sizes[1]), [1e9, 1e9], [None, None]
+    for _ in range(8):
+        for i in range(2):
+            capi.synchronize()
+            t0 = time.perf_counter()
+            capi.check(L.vsag_amd_kmeans_assign(xb.ptr, n, d, cb.ptr, k, lab.ptr, None, None, ws.ptr, sizes[i], None))
+            capi.synchronize()
+            best[i] = min(best[i], time.perf_counter() - t0)
+            out[i] = lab.to_numpy(np.int32, (n,))
+    assert np.array_equal(out[0], out[1])
+    assert best[1] < 1.3 * best[0], best
+
+
+@pytest.mark.parametrize("n,d,k,iters", [(16400, 128, 2048, 6), (70001, 1000, 260, 3)])
+def test_run_from_crowded_centroids(lib, n, d, k, iters):
+    """Every row is open in the first iteration, few are in the later ones, some of which are not pre-selected: the centroids
+    are those of the fp32 kernels alone."""
+    L = lib.load_library()
+    x, cent = _routed_data("crowd", n, d, k)
+    xb, lab, out = dev(x), capi.DeviceBuffer(n * 4), []
+    whole = L.vsag_amd_kmeans_run_workspace_bytes(n, d, k)
+    rest = whole - L.vsag_amd_kmeans_assign_workspace_bytes(n, d, k)
+    for wsb in (whole, _fp32_assign_bytes(n, k) + rest):
+        cc, ws = dev(cent), capi.DeviceBuffer(wsb)
+        capi.check(L.vsag_amd_kmeans_run(xb.ptr, n, d, cc.ptr, k, iters, 7, lab.ptr, None, ws.ptr, wsb, None))
+        out.append((cc.to_numpy(np.int32, (k, d)), lab.to_numpy(np.int32, (n,))))
+    assert np.array_equal(out[0][0], out[1][0]) and np.array_equal(out[0][1], out[1][1])
 
 
 @pytest.mark.parametrize("scale", [1e-16, 1e-19, 1e-21, 1e-23, 1e-30])

@@ -891,10 +891,10 @@ carve_assign(Carver& c, uint64_t n, uint32_t dim, uint32_t k, bool preselect, As
 
 static int
 assign_launch(const float* x, uint64_t n, uint32_t dim, const float* cent, uint32_t k, int32_t* labels,
-              float* min_dist, double* loss_dev, const AssignBuffers& b, bool have_xnorm, hipStream_t st) {
+              float* min_dist, double* loss_dev, const AssignBuffers& b, int iteration, hipStream_t st) {
     hipLaunchKernelGGL(row_sqnorm_kernel, dim3(static_cast<uint32_t>(div_up(k, 4))), dim3(256), 0, st, cent,
                        static_cast<uint64_t>(k), dim, b.ynorm);
-    if (!have_xnorm && !b.h16) {
+    if (iteration == 0 && !b.h16) {  // (from the second Lloyd iteration on |x|^2 is there)
         hipLaunchKernelGGL(row_sqnorm_kernel, dim3(static_cast<uint32_t>(div_up(n, 4))), dim3(256), 0, st, x, n, dim,
                            b.xnorm);
     }
@@ -906,7 +906,7 @@ assign_launch(const float* x, uint64_t n, uint32_t dim, const float* cent, uint3
     timing_begin(st);
     OpenRows open = {nullptr, nullptr, nullptr};
     if (b.h16) {
-        VA_TRY(launch_kmeans_h16(x, n, dim, cent, k, b.ynorm, b.xnorm, have_xnorm, b.best, b.pre, st));
+        VA_TRY(launch_kmeans_h16(x, n, dim, cent, k, b.ynorm, b.xnorm, iteration, b.best, b.pre, st));
         // what follows does the rows that were left open: usually none, and its workgroups return at once
         open = {b.pre.row_open, b.pre.open64, &b.pre.state->any_open};
     }
@@ -1383,7 +1383,7 @@ vsag_amd_kmeans_assign(const float* x_dev, uint64_t n, uint32_t dim, const float
         carve_assign(c, n, dim, k, false, &b);
     }
     VA_CHECK_ARG(c.ok(), "workspace too small: need %zu bytes, got %zu", c.used, workspace_bytes);
-    return assign_launch(x_dev, n, dim, centroids_dev, k, labels_dev, min_dist_dev, loss_dev, b, false,
+    return assign_launch(x_dev, n, dim, centroids_dev, k, labels_dev, min_dist_dev, loss_dev, b, 0,
                          static_cast<hipStream_t>(stream));
 }
 
@@ -1464,7 +1464,7 @@ vsag_amd_kmeans_run(const float* x_dev, uint64_t n, uint32_t dim, float* centroi
     std::vector<int32_t> counts(k);
     double last = 0.0;
     for (int it = 0; it < iters; ++it) {
-        VA_TRY(assign_launch(x_dev, n, dim, centroids_dev, k, labels_dev, nullptr, a.loss_tmp, a, it > 0, st));
+        VA_TRY(assign_launch(x_dev, n, dim, centroids_dev, k, labels_dev, nullptr, a.loss_tmp, a, it, st));
         VA_TRY(update_launch(x_dev, labels_dev, n, dim, k, centroids_dev, counts_dev, u, st));
         VA_HIP(hipMemcpyAsync(counts.data(), counts_dev, k * sizeof(int32_t), hipMemcpyDeviceToHost, st));
         VA_HIP(hipMemcpyAsync(&last, a.loss_tmp, sizeof(double), hipMemcpyDeviceToHost, st));

@@ -13,6 +13,7 @@ struct KmeansH16State {
     uint32_t any_open;     // whether any row is left open
     uint32_t far_from;     // centroids with |c - centre|^2 above this are far: only their distance from the centre is used
     uint32_t nearest_far;  // least |c - centre|^2 of the far ones (infinity: none that any row could choose)
+    uint32_t open_groups;  // of every sixteenth group of 64 rows: those in which the last probe left one open
 };
 
 struct KmeansH16Buffers {
@@ -31,9 +32,9 @@ struct KmeansH16Buffers {
 bool kmeans_h16_takes(uint64_t n, uint32_t dim, uint32_t k);
 void carve_kmeans_h16(Carver& c, uint64_t n, uint32_t dim, uint32_t k, KmeansH16Buffers* b);
 // Fills best[] (keys of (|c|^2 - 2 <c, x>, centroid)) of every row but those marked in row_open / open64, whose keys are
-// left at ~0.  cnorm_raw = |c|^2 per centroid; xnorm = |x|^2 per row, written when have_xnorm is false.  With have_xnorm
-// the rows are those of the call before, so where one slab holds all of them their fp16 form is still there.
+// left at ~0.  cnorm_raw = |c|^2 per centroid; xnorm = |x|^2 per row, written in iteration 0.  From iteration 1 on the rows
+// are those of the call before, so where one slab holds all of them their fp16 form is still there.
 int launch_kmeans_h16(const float* x, uint64_t n, uint32_t dim, const float* cent, uint32_t k, const float* cnorm_raw,
-                      float* xnorm, bool have_xnorm, unsigned long long* best, const KmeansH16Buffers& b, hipStream_t st);
+                      float* xnorm, int iteration, unsigned long long* best, const KmeansH16Buffers& b, hipStream_t st);
 
 }  // namespace vsag_amd

@@ -22,8 +22,11 @@
 // marked and left to the fp32 kernels.  What those cost does not depend on how many rows of a
 // tile of 256 are open, so a few in a hundred, scattered, cost what all do: where a common offset of rows and centroids is
 // many times their spread (the fp32 distances themselves are rounded to that), or centroids are missing from whole clusters,
-// a call can pay for both (1M x 960, k 4096, clusters of width 0.05 and ten times the centres' range from the origin: 76.8 ms
-// against 63.4 of the fp32 kernels; 65536 x 128, k 512: 0.26 against 0.13).
+// a call can pay for both.  So every fourth slab (of one slab: every fourth Lloyd iteration) is a probe, and where it left
+// rows open in more than half of its groups of 64, the three behind it go to the fp32 kernels at once.  Clusters of width 0.05
+// ten times the centres' range from the origin, fp32 kernels / every slab tried / this, ms: 1M x 960, k 4096 63.3 / 77.4 /
+// 67.9; 480k x 960, k 256 2.42 / 3.51 / 2.68; of a single slab (65536 x 128, k 512) 0.12 / 0.18 / 0.18.  Where nothing is
+// open, asking costs 0.5 to 1 %.
 //
 // 1M x 960 rows, 4096 centroids (one assignment): 63.3 -> 13.0 ms.  Of that the contraction takes 9.3 (7.9e12 flop: 847
 // TFLOP/s, 34 % of the fp16 peak; a workgroup waits at each of its fifteen stages for all eight waves), the rounding of
@@ -52,6 +55,8 @@ constexpr uint32_t kPiece = 32;        // rescoring: dimensions at a time
 constexpr uint32_t kPitch = kPiece + 4;
 constexpr uint32_t kMaxList = 24;      // rescoring: entries (a centroid, or a whole group) per row
 constexpr uint32_t kMaxWork = 160;     // rescoring: distances per row
+constexpr uint32_t kProbes = 4;        // every fourth slab or iteration is a probe
+constexpr uint32_t kProbeStep = 16;    // of which every 16th workgroup counts (all of them: 60 us of atomics on one word)
 constexpr uint64_t kSlabHalves = 64ull << 20;  // fp16 values per slab: 128 MB stay in the 256 MB memory-side cache
 constexpr uint64_t kTableBytes = 256ull << 20;  // the table of a slab: the rows get fewer as the centroids get more ...
 constexpr uint64_t kMinSlabRows = 4096;         // ... down to this
@@ -105,8 +110,8 @@ carve_kmeans_h16(Carver& c, uint64_t n, uint32_t dim, uint32_t k, KmeansH16Buffe
 }
 
 __device__ inline void
-reset_state(KmeansH16State* state) {
-    *state = {0, 0, 0, 0, 0, __float_as_uint(__builtin_inff())};
+reset_state(KmeansH16State* state, uint32_t open_groups) {
+    *state = {0, 0, 0, 0, 0, __float_as_uint(__builtin_inff()), open_groups};
 }
 
 // A centre: per dimension, sixteen means of sixteen centroids each, the middle half of them averaged -- a few centroids far
@@ -115,7 +120,7 @@ __global__ void __launch_bounds__(1024)
 kmeans_centre_kernel(const float* cent, uint32_t k, uint32_t dim, float* centre, KmeansH16State* state) {
     __shared__ float part[16][64];
     if (blockIdx.x == 0 && threadIdx.x == 0) {
-        reset_state(state);
+        reset_state(state, 0);
     }
     const uint32_t lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     const uint32_t d = blockIdx.x * 64 + lane;
@@ -146,9 +151,9 @@ kmeans_centre_kernel(const float* cent, uint32_t k, uint32_t dim, float* centre,
 }
 
 __global__ void
-kmeans_reset_kernel(KmeansH16State* state) {
+kmeans_reset_kernel(KmeansH16State* state, int probe) {
     if (threadIdx.x == 0) {
-        reset_state(state);
+        reset_state(state, probe != 0 ? 0 : state->open_groups);
     }
 }
 
@@ -315,14 +320,28 @@ kmeans_round_centroids_kernel(const float* cent, uint32_t k, uint32_t dim, uint3
     }
 }
 
+// Whether a slab goes to the fp32 kernels without the pre-selection: the probe before it left rows open in open_groups of the
+// `probed` groups that were looked at (0: this slab is a probe itself, whose count is being formed).  The kernels read the
+// count first and ask late, so that its way from memory is hidden (1M x 128, k 1024: 1.185 ms without, 1.23 ms with waves
+// that wait for it).
+__device__ inline bool
+given_up(uint32_t open_groups, uint32_t probed) {
+    return probed != 0 && open_groups > probed / 2;
+}
+
 // A wave per row: |x|^2 (unless it is known), the row in fp16 and its lengths.  The row is read twice, the second time
 // from the caches.
 __global__ void __launch_bounds__(256)
 kmeans_round_rows_kernel(const float* x, uint64_t rows, uint32_t dim, uint32_t dpad, const float* centre, int wide,
-                         uint16_t* x16, float2* xinfo, float* xscale, float* xnorm) {
+                         KmeansH16State* state, uint32_t probed, uint16_t* x16, float2* xinfo, float* xscale,
+                         float* xnorm) {
     const uint64_t r = static_cast<uint64_t>(blockIdx.x) * 4 + (threadIdx.x >> 6);
     if (r >= rows) {
         return;
+    }
+    const uint32_t open_groups = state->open_groups;
+    if (probed == 0 && r == 0 && threadIdx.x == 0) {
+        state->open_groups = 0;  // the rescoring of this slab counts
     }
     const uint32_t lane = threadIdx.x & 63;
     const float* row = x + r * dim;
@@ -341,6 +360,9 @@ kmeans_round_rows_kernel(const float* x, uint64_t rows, uint32_t dim, uint32_t d
         if (lane == 0) {
             xnorm[r] = raw;
         }
+    }
+    if (given_up(open_groups, probed)) {
+        return;
     }
     const bool usable = sq < 1.0e30F;  // false for NaN as well
     const int e = usable ? scale_exponent(sq) : 0;
@@ -362,6 +384,7 @@ struct KmeansH16Args {
     const float* xscale;
     const float* cnorm;
     const KmeansH16State* state;
+    uint32_t probed;   // see given_up
     float* group_min;
     uint64_t ld;       // the table: [group][3][ld]
     uint32_t rtiles, ctiles, mc_log2, mcols, macros;
@@ -417,6 +440,7 @@ kmeans_h16_kernel(KmeansH16Args p) {
     const uint32_t ob0 = offset(lr, b_last), ob1 = offset(lr + 64, b_last), ob2 = offset(lr + 128, b_last),
                    ob3 = offset(lr + 192, b_last);
     const uint32_t put = lr * kSlots + (ls ^ ((lr >> 1) & 7));  // + 64 i rows
+    const uint32_t open_groups = p.state->open_groups;
     if (tid < kTile) {
         const float sq = c0 + tid < p.k ? p.cnorm[c0 + tid] : 3.0e38F;
         cn[tid] = sq <= __uint_as_float(p.state->far_from) ? sq : 3.0e38F;
@@ -484,6 +508,9 @@ kmeans_h16_kernel(KmeansH16Args p) {
     };
 
     fetch(0);
+    if (given_up(open_groups, p.probed)) {
+        return;
+    }
     park(lds);
     __syncthreads();
     for (uint32_t st = 0; st + 1 < stages; ++st) {
@@ -560,6 +587,7 @@ struct KmeansRescoreArgs {
     const float* xnorm;
     const float* cnorm_raw;
     KmeansH16State* state;
+    uint32_t probed;  // see given_up
     int wide;
     int natural;  // order of the products, see the kernel
     unsigned long long* best;
@@ -585,6 +613,7 @@ kmeans_h16_rescore_kernel(KmeansRescoreArgs p) {
     const uint32_t rl = tid & 63, part = tid >> 6;
     const uint64_t block_row = static_cast<uint64_t>(blockIdx.x) * kRowsPerBlock;
     const uint64_t row = block_row + rl;
+    const uint32_t open_groups = p.state->open_groups;
     if (tid < kRowsPerBlock) {
         count[tid] = 0;
         cost[tid] = 0;
@@ -602,6 +631,17 @@ kmeans_h16_rescore_kernel(KmeansRescoreArgs p) {
             least = fminf(least, p.group_min[static_cast<uint64_t>(g) * 3 * p.ld + row]);
         }
         atomicMin(&least_bits[rl], float_to_ordered(least));
+    }
+    if (given_up(open_groups, p.probed)) {  // (the table is not this slab's: nothing of it was used)
+        if (tid < kRowsPerBlock && row < p.rows) {
+            p.row_open[row] = 1;
+            p.best[row] = ~0ull;
+        }
+        if (tid == 0) {
+            p.open64[blockIdx.x] = 1;
+            p.state->any_open = 1;
+        }
+        return;
     }
     __syncthreads();
     if (row < p.rows) {
@@ -686,6 +726,9 @@ kmeans_h16_rescore_kernel(KmeansRescoreArgs p) {
         p.open64[blockIdx.x] = any;
         if (any != 0) {
             p.state->any_open = 1;
+            if (p.probed == 0 && blockIdx.x % kProbeStep == 0) {
+                atomicAdd(&p.state->open_groups, 1U);
+            }
         }
     }
 
@@ -775,7 +818,7 @@ kmeans_h16_rescore_kernel(KmeansRescoreArgs p) {
 
 int
 launch_kmeans_h16(const float* x, uint64_t n, uint32_t dim, const float* cent, uint32_t k, const float* cnorm_raw,
-                  float* xnorm, bool have_xnorm, unsigned long long* best, const KmeansH16Buffers& b, hipStream_t st) {
+                  float* xnorm, int iteration, unsigned long long* best, const KmeansH16Buffers& b, hipStream_t st) {
     constexpr size_t lds_bytes = 4 * static_cast<size_t>(kTile) * kSlots * sizeof(uint4) + kTile * sizeof(float);
     static std::once_flag lds_once;
     static hipError_t lds_rc = hipSuccess;
@@ -787,21 +830,25 @@ launch_kmeans_h16(const float* x, uint64_t n, uint32_t dim, const float* cent, u
     const uint32_t dpad = padded_dim(dim);
     const uint64_t slab = slab_rows(n, dim, k);
     const int wide = (dim & 3) == 0 && ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(cent)) & 15) == 0;
+    const bool have_xnorm = iteration > 0;
     const bool kept = have_xnorm && n <= slab;  // the rows' fp16 form of the call before, and the centre it was formed with
     const uint32_t cblocks = (k + kGroup - 1) / kGroup;
+    const uint32_t probe_groups = static_cast<uint32_t>(div_up(std::min(n, slab), kRowsPerBlock * kProbeStep));
     if (!kept) {
         hipLaunchKernelGGL(kmeans_centre_kernel, dim3((dim + 63) / 64), dim3(1024), 0, st, cent, k, dim, b.centre, b.state);
     } else {
-        hipLaunchKernelGGL(kmeans_reset_kernel, dim3(1), dim3(64), 0, st, b.state);
+        hipLaunchKernelGGL(kmeans_reset_kernel, dim3(1), dim3(64), 0, st, b.state, iteration % kProbes == 0 ? 1 : 0);
     }
     hipLaunchKernelGGL(kmeans_cnorm_kernel, dim3(cblocks), dim3(1024), 0, st, cent, k, dim, b.centre, b.cnorm);
     hipLaunchKernelGGL(kmeans_round_centroids_kernel, dim3(cblocks), dim3(1024), 0, st, cent, k, dim, dpad, b.centre, wide,
                        cnorm_raw, b.cnorm, b.c16, b.state);
     for (uint64_t r0 = 0; r0 < n; r0 += slab) {
         const uint64_t rows = n - r0 < slab ? n - r0 : slab;
+        const bool probe = (kept ? static_cast<uint64_t>(iteration) : r0 / slab) % kProbes == 0;
+        const uint32_t probed = probe ? 0 : probe_groups;
         if (!kept) {
             hipLaunchKernelGGL(kmeans_round_rows_kernel, dim3(static_cast<uint32_t>(div_up(rows, 4))), dim3(256), 0, st,
-                               x + r0 * dim, rows, dim, dpad, b.centre, wide, b.x16, b.xinfo, b.xscale,
+                               x + r0 * dim, rows, dim, dpad, b.centre, wide, b.state, probed, b.x16, b.xinfo, b.xscale,
                                have_xnorm ? nullptr : xnorm + r0);
         }
         KmeansH16Args a;
@@ -813,6 +860,7 @@ launch_kmeans_h16(const float* x, uint64_t n, uint32_t dim, const float* cent, u
         a.xscale = b.xscale;
         a.cnorm = b.cnorm;
         a.state = b.state;
+        a.probed = probed;
         a.group_min = b.group_min;
         a.ld = slab;
         a.rtiles = static_cast<uint32_t>(div_up(rows, kTile));
@@ -836,6 +884,7 @@ launch_kmeans_h16(const float* x, uint64_t n, uint32_t dim, const float* cent, u
         s.xnorm = xnorm + r0;
         s.cnorm_raw = cnorm_raw;
         s.state = b.state;
+        s.probed = probed;
         s.wide = wide;
         s.natural = (dim & 3) != 0;
         s.best = best + r0;
