@@ -317,15 +317,16 @@ VSAG_AMD_API int vsag_amd_flat_scan_topk_noalloc(const vsag_amd_store_t* store, 
                                     uint32_t k, const vsag_amd_search_options_t* options, uint32_t* ids_dev,
                                     float* dists_dev, void* stream);
 
-/* Large batches on flat fp32 / sq8 / sq8_uniform / sq4_uniform (the uniform kinds: at most 128 dimensions) / rabitq stores are served by a matrix-core contraction that pre-selects
+/* Large batches on flat fp32 / sq8 / sq4 / sq8_uniform / sq4_uniform (the uniform kinds: at most 128 dimensions) / rabitq stores are served by a matrix-core contraction that pre-selects
  * candidates, which are then recomputed and selected exactly as the streaming scan does (same results, bit for bit).
- * rabitq stores with 4-bit queries and at most 1024 dimensions (L2, inner product) expand code bits and query nibbles to
- * bytes for the int8 matrix cores (the integer product is exact; k up to 256 by default).
+ * rabitq stores with 4-bit queries and at most 1024 dimensions (L2, inner product) expand code bits to fp4 and query nibbles
+ * to fp6 for the scaled matrix instruction (the integer product is exact; k up to 256 by default).
  * Posting lists of sq4_uniform codes of at most 128 dimensions (any metric) scan the probe columns behind the first on the
  * int8 matrix cores when a batch has at least 8192 (query, list) groups (same results; off with mode -1).
- * sq8 stores of at most 128 dimensions pre-select on the int8 matrix cores (queries split into two int8 planes
- * with a rigorous bound on the remainder), the others on the fp32 matrix cores.
- * mode: 0 = when it pays (default: >= 512 queries, or fewer against enough codes, k <= 128, >= 65536 codes), 1 = whenever the store and k
+ * sq8 and sq4 stores of at most 128 dimensions pre-select on the int8 matrix cores (queries split into two int8 planes
+ * with a rigorous bound on the remainder), those beyond on the fp16 and fp32 stores on the fp32 matrix cores.
+ * mode: 0 = when it pays (default: >= 512 queries, or 16 and more against enough codes, k <= 128, >= 65536 codes; below 512
+ * not where a query tile or a number of chunks is set, see the tuning knobs), 1 = whenever the store and k
  * allow it, 2 = like 1 but always on the fp32 matrix cores, -1 = never.  Process-wide; affects
  * vsag_amd_flat_scan_workspace_bytes as well.  No counterpart in the reference (it scans one query at a time). */
 VSAG_AMD_API int vsag_amd_set_scan_contraction(int mode);
@@ -355,7 +356,10 @@ VSAG_AMD_API int vsag_amd_last_kernel_ms(float* ms);
 
 /* KMeansCluster::find_nearest_one_with_blas (impl/cluster/kmeans_cluster.cpp:193-305):
  * labels[i] = first argmin_j (||c_j||^2 - 2<c_j, x_i>), min_dist[i] = that minimum (may be NULL),
- * *loss_dev (double, may be NULL) = sum_i (min + ||x_i||^2) / n. */
+ * *loss_dev (double, may be NULL) = sum_i (min + ||x_i||^2) / n.
+ * Large calls pre-select on the fp16 matrix cores (same labels and distances, bit for bit); their workspace holds up to 400 MB
+ * beside 13 bytes a row and the centroids in fp16.  One with room for the fp32 kernels alone (12 bytes a row) is served by
+ * those, here and in vsag_amd_kmeans_run. */
 VSAG_AMD_API size_t vsag_amd_kmeans_assign_workspace_bytes(uint64_t n, uint32_t dim, uint32_t k);
 VSAG_AMD_API int vsag_amd_kmeans_assign(const float* x_dev, uint64_t n, uint32_t dim, const float* centroids_dev,
                            uint32_t k, int32_t* labels_dev, float* min_dist_dev, double* loss_dev,
