@@ -337,6 +337,28 @@ def test_fp32_contraction_equals_streaming(lib, modes, metric, n, d, nq, k):
     st.destroy()
 
 
+@pytest.mark.parametrize("metric", [orc.L2, orc.IP, orc.COSINE])
+@pytest.mark.parametrize("n,d,nq,k", [(1500, 17, 1, 1), (2049, 32, 31, 5), (4097, 36, 33, 10), (5003, 130, 64, 10),
+                                      (3001, 64, 65, 20), (6000, 260, 129, 3)])
+def test_fp32_on_the_bf16_matrix_cores(lib, modes, metric, n, d, nq, k):
+    """Two bf16 values per operand select, the streaming arithmetic decides: 32, 64 and 128 queries per workgroup, code
+    tiles and stages with a remainder, rows of very different lengths and copies of stored rows among the queries."""
+    rng = np.random.default_rng(n + d)
+    x, means = gaussian_mixture(rng, n, d, 20, 0.05)
+    q, _ = gaussian_mixture(rng, nq, d, 20, 0.05, means=means)
+    x[::7] *= np.float32(1e3)
+    x[1::7] *= np.float32(1e-6)
+    x[2::70] = 0
+    q[::3] = x[rng.integers(0, n, len(q[::3]))]
+    for scale in (1.0, 1e-18, 1e12):
+        st = Store(capi.KIND_FP32, metric, d)
+        st.append((x * np.float32(scale)).view(np.uint8).reshape(n, -1))
+        plain, fast, tile = modes(st, q * np.float32(scale), k)
+        assert tile == 128, "the contraction path did not run"
+        assert same(plain, fast)
+        st.destroy()
+
+
 @pytest.mark.parametrize("kind", ["fp32", "sq8"])
 def test_many_short_tiles_per_workgroup(lib, modes, kind):
     """100000 x 128 against 1000 queries: every workgroup walks many code tiles with a short contraction each, so

@@ -45,6 +45,38 @@ def test_flat_scan_with_deny_mask(lib, metric, n, d, nq, k, deny_rate):
     st.destroy()
 
 
+@pytest.mark.parametrize("metric", [orc.L2, orc.IP, orc.COSINE])
+@pytest.mark.parametrize("kind,n,d,nq,k,deny_rate", [("sq8", 30001, 100, 200, 100, 0.7), ("sq8", 9000, 17, 33, 10, 0.99),
+                                                     ("sq8", 20000, 260, 65, 10, 0.3), ("sq4", 12345, 128, 40, 7, 0.5),
+                                                     ("sq4", 7000, 200, 150, 20, 0.95), ("fp32", 15000, 96, 70, 10, 0.6),
+                                                     ("fp32", 4000, 33, 20, 10, 0.9985), ("sq8", 700, 40, 9, 5, 1.0)])
+def test_masked_batches_on_the_bf16_matrix_cores(lib, kind, metric, n, d, nq, k, deny_rate):
+    """A deny mask over a pre-selected batch: ids and distance bits of the streaming kernel, also where fewer than k codes
+    are allowed."""
+    rng = np.random.default_rng(n + d)
+    x, means = gaussian_mixture(rng, n, d, 20, 0.05)
+    q, _ = gaussian_mixture(rng, nq, d, 20, 0.05, means=means)
+    if kind == "fp32":
+        st = Store(capi.KIND_FP32, metric, d)
+        st.append(x.view(np.uint8).reshape(n, -1))
+    else:
+        bits = 8 if kind == "sq8" else 4
+        lb, diff = orc.sq_train(x, bits, metric)
+        st = Store(capi.KIND_SQ8 if bits == 8 else capi.KIND_SQ4, metric, d, lb=lb, diff=diff)
+        st.append(orc.sq_encode(x, bits, lb, diff, metric))
+    deny = rng.random(n) < deny_rate
+    res = []
+    try:
+        for mode in (-1, 1):
+            capi.check(st.lib.vsag_amd_set_scan_contraction(mode))
+            res.append(st.flat_scan(q, k, deny=deny))
+    finally:
+        capi.check(st.lib.vsag_amd_set_scan_contraction(0))
+    assert np.array_equal(res[0][0], res[1][0])
+    assert np.array_equal(res[0][1].view(np.uint32), res[1][1].view(np.uint32))
+    st.destroy()
+
+
 @pytest.mark.parametrize("metric", [orc.L2, orc.IP])
 def test_flat_scan_with_radius(lib, metric):
     rng = np.random.default_rng(91)

@@ -21,7 +21,7 @@ HIP_FLAGS = [
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
     "-Wall", "-Wno-unused-function", "-Wno-unknown-attributes",
 ]
-KERNEL_SOURCES = ["runtime.hip", "store.hip", "quantize.hip", "prepare.hip", "scan.hip", "prefilter.hip", "prefilter_i8.hip", "prefilter_rb.hip", "prefilter_h16.hip", "ivf.hip", "ivf_i8.hip", "ivf_pq.hip",
+KERNEL_SOURCES = ["runtime.hip", "store.hip", "quantize.hip", "prepare.hip", "scan_flat.hip", "ivf_scan.hip", "scan.hip", "prefilter.hip", "prefilter_i8.hip", "prefilter_rb.hip", "prefilter_h16.hip", "prefilter_b16.hip", "ivf.hip", "ivf_i8.hip", "ivf_pq.hip",
                   "kmeans.hip", "kmeans_h16.hip", "lookup.hip", "export.hip", "scan_one.hip", "pq.hip"]
 
 
@@ -44,7 +44,7 @@ def build_kernels(verbose=True):
             print(out)
         return obj
 
-    with ThreadPoolExecutor(max_workers=6) as pool:
+    with ThreadPoolExecutor(max_workers=8) as pool:
         objs = list(pool.map(compile_one, sources))
     lib = os.path.join(LIB, "libvsag_amd.so")
     _run([HIPCC, "-shared", "-fPIC", "--offload-arch=gfx950", "-o", lib] + objs)

@@ -403,6 +403,10 @@ struct RescoreArgs {
     uint32_t sub_lists, sub_cap, gather;
     const uint4* rows;  // the codes a row per code (store.h), or null: read the tiles
     uint32_t row_granules;  // granules of a row: G, or G + 1 with the code's metadata words behind the code
+    // VALUED: records of the approximate distance's ordered bits above the slot, cap a query, and per query twice what the
+    // approximation can be off by.
+    const uint64_t* valued;
+    const float* slack;
 };
 
 // Words of LDS for gathered candidates: small, so that many of these one-wave workgroups share a compute unit (the
@@ -410,7 +414,13 @@ struct RescoreArgs {
 constexpr uint32_t kRescoreGather = 1024;
 
 // One wave per query: exact distances of its candidates by the streaming kernel's arithmetic, best k kept.
-template <int KIND, int METRIC>
+//
+// VALUED: a candidate comes with its approximate distance v.  At least k of them have v at or below a_k, and v is off by
+// at most slack / 2 from the streaming distance less the query's constant, so whoever has v above a_k + slack stands
+// behind k others: of the hundreds of candidates that the bound of the level before let through, the few that are left
+// are rescored.  (fp32 rows are gathered a memory line per granule: 300 queries x 160 candidates x 768 dimensions took
+// 312 us.)
+template <int KIND, int METRIC, bool VALUED>
 __global__ void __launch_bounds__(64)
 rescore_kernel(ScanArgs a, RescoreArgs r) {
     extern __shared__ uint64_t keys[];
@@ -460,7 +470,9 @@ rescore_kernel(ScanArgs a, RescoreArgs r) {
             // A few granules are fetched before the first is used: a candidate's loads wait for memory together.
             // (sq8 l2 holds scale and query of every dimension in flight in scalar registers: two granules' worth; an sq4
             // granule is 32 dimensions.)
-            constexpr uint32_t kAhead = KIND == VSAG_AMD_KIND_SQ4 ? (METRIC == VSAG_AMD_METRIC_L2 ? 1 : 2)
+            // VALUED: a wave or two of candidates per query, so latency is all there is: as many as registers allow.
+            constexpr uint32_t kAhead = VALUED && KIND == VSAG_AMD_KIND_FP32 ? 16
+                                       : KIND == VSAG_AMD_KIND_SQ4 ? (METRIC == VSAG_AMD_METRIC_L2 ? 1 : 2)
                                        : (KIND == VSAG_AMD_KIND_SQ8 && METRIC == VSAG_AMD_METRIC_L2 ? 2 : 4);
             for (uint32_t j0 = 0; j0 < a.G; j0 += kAhead) {
                 uint4 c[kAhead];
@@ -506,7 +518,48 @@ rescore_kernel(ScanArgs a, RescoreArgs r) {
             }
         }
     };
-    if (r.sub_lists == 0) {
+    if constexpr (VALUED) {
+        uint32_t* pick = reinterpret_cast<uint32_t*>(keys + S);  // 128 slots waiting, then 256 bins
+        const uint64_t* valued = r.valued + static_cast<uint64_t>(q) * r.cap;
+        const uint32_t total = as_const(counts)[0];
+        float limit = __builtin_inff();
+        if (total > k) {
+            const float kth = kth_value_or_above(
+                [&](uint32_t i) { return ordered_to_float(static_cast<uint32_t>(valued[i] >> 32)); }, total, k, pick + 128, lane);
+            const float slack = r.slack[q];
+            if (slack < 3.0e38F && kth > -3.0e38F) {
+                limit = kth + slack;
+                limit += fabsf(limit) * 2.4e-7F;  // not below the sum
+            }
+        }
+        uint32_t waiting = 0;
+        for (uint32_t base = 0; base < total; base += kWave) {
+            const uint64_t key = base + lane < total ? valued[base + lane] : kInfKey;
+            const bool take = base + lane < total && ordered_to_float(static_cast<uint32_t>(key >> 32)) <= limit;
+            const uint64_t mask = __ballot(take);
+            if (take) {
+                pick[waiting + mask_rank(mask)] = static_cast<uint32_t>(key);
+            }
+            waiting += static_cast<uint32_t>(__popcll(mask));
+            wave_lds_fence();
+            if (waiting >= kWave || base + kWave >= total) {
+                // (a round of at most 64, what is left over moves to the front)
+                const uint32_t now = waiting < kWave ? waiting : kWave;
+                rescore(pick, now);
+                const uint32_t left = waiting - now;
+                const uint32_t moved = lane < left ? pick[kWave + lane] : 0U;
+                wave_lds_fence();
+                if (lane < left) {
+                    pick[lane] = moved;
+                }
+                waiting = left;
+                wave_lds_fence();
+            }
+        }
+        if (waiting != 0) {
+            rescore(pick, waiting);
+        }
+    } else if (r.sub_lists == 0) {
         rescore(r.cand + static_cast<uint64_t>(q) * r.cap, as_const(counts)[0]);
     } else {
         // Gather the private lists of the query behind the selector -- a lane per list, offsets by a wave scan -- and
@@ -1250,13 +1303,13 @@ launch_code_terms(vsag_amd_store* s, uint64_t first, uint64_t count, hipStream_t
     return 0;
 }
 
-template <int KIND>
+template <int KIND, bool VALUED = false>
 static void
 launch_rescore_m(int metric, dim3 grid, size_t lds, hipStream_t st, const ScanArgs& a, const RescoreArgs& r) {
     if (metric == VSAG_AMD_METRIC_L2) {
-        hipLaunchKernelGGL((rescore_kernel<KIND, VSAG_AMD_METRIC_L2>), grid, dim3(kWave), lds, st, a, r);
+        hipLaunchKernelGGL((rescore_kernel<KIND, VSAG_AMD_METRIC_L2, VALUED>), grid, dim3(kWave), lds, st, a, r);
     } else {
-        hipLaunchKernelGGL((rescore_kernel<KIND, VSAG_AMD_METRIC_IP>), grid, dim3(kWave), lds, st, a, r);
+        hipLaunchKernelGGL((rescore_kernel<KIND, VSAG_AMD_METRIC_IP, VALUED>), grid, dim3(kWave), lds, st, a, r);
     }
 }
 
@@ -1310,6 +1363,40 @@ launch_rescore(const vsag_amd_store* s, const ScanArgs& a, uint64_t nq, uint32_t
     return 0;
 }
 
+// The records of a flat scan on the bf16 matrix cores (prefilter_b16.hip): cap a query, into list out_slot.
+int
+launch_rescore_valued(const vsag_amd_store* s, const ScanArgs& a, uint64_t nq, uint32_t k, uint32_t S, uint32_t* bound,
+                      const uint64_t* valued, const float* slack, const uint32_t* cand_cnt, uint32_t cap, uint64_t* partial,
+                      uint32_t* partial_cnt, uint32_t nslots, uint32_t out_slot, uint32_t* gate, hipStream_t st) {
+    RescoreArgs r{};
+    r.valued = valued;
+    r.slack = slack;
+    r.first_slot = out_slot;
+    r.cand_cnt = cand_cnt;
+    r.cap = cap;
+    r.n = s->n;
+    r.k = k;
+    r.S = S;
+    r.bound = bound;
+    r.partial = partial;
+    r.partial_cnt = partial_cnt;
+    r.nslots = nslots;
+    r.out_slot = out_slot;
+    r.gate = gate;
+    r.rows = s->rows;
+    r.row_granules = s->row_granules;
+    const dim3 grid(static_cast<uint32_t>(nq));
+    const size_t lds = S * 8 + (128 + 256) * 4;
+    if (s->kind == VSAG_AMD_KIND_SQ8) {
+        launch_rescore_m<VSAG_AMD_KIND_SQ8, true>(s->metric, grid, lds, st, a, r);
+    } else if (s->kind == VSAG_AMD_KIND_SQ4) {
+        launch_rescore_m<VSAG_AMD_KIND_SQ4, true>(s->metric, grid, lds, st, a, r);
+    } else {
+        launch_rescore_m<VSAG_AMD_KIND_FP32, true>(s->metric, grid, lds, st, a, r);
+    }
+    VA_HIP(hipGetLastError());
+    return 0;
+}
 
 // Steps 2 and 3 of the header comment for tiles [tile_begin, tile_end); the exact prefix scan has already
 // left its bounds in `bound`.  Writes one partial list per query (out_slot) and raises the overflow flags.

@@ -1,0 +1,949 @@
+// Pre-selection for query batches on the bf16 matrix cores: flat fp32, sq8 and sq4 stores, fp32 posting lists.
+//
+// The inner product <b, c> of a query with a code is formed from two bf16 values per operand, x = h + l + r with h =
+// bf16(x), l = bf16(x - h) and |r| <= 2^-18 |x| (bf16 keeps eight bits, rounded to nearest).  A code byte or nibble is one
+// bf16 value exactly, so
+//   sq8, sq4   <b, c>  ~  <h_b, c> + <l_b, c>                        (b: the query with the scale folded in)
+//   fp32       <a, y>  ~  <h_a, h_y> + <l_a, h_y> + <h_a, l_y>
+// two or three v_mfma_f32_32x32x16_bf16 for sixteen dimensions.  The products are exact in the fp32 accumulator; what is
+// left out is known (the remainders of the query are summed, those of an fp32 code are at most 2^-18 of it), so the value
+//   v = |y|^2 - 2 <b, c>  (inner product: -<b, c>)
+// stands within a bound e of the streaming kernel's distance less the query's constant.  bf16 has the exponent range of
+// fp32: no operand needs a scale, and what is below the normal range may be taken as zero.
+//
+// A flat scan (launch_scan_b16) needs no exact distance before the end:
+//   1. a sample of the code tiles, spread over the store, leaves the least v of every 64 (32) codes; k of those lie at or
+//      below the k-th smallest, m;
+//   2. whoever is among the k best has v <= m + 2 e: the pass over all codes records (v, slot) of those, a few hundred a
+//      query (b16_tau_kernel says how many are expected);
+//   3. of the records only those within 2 e of their own k-th smallest are rescored with the streaming kernel's arithmetic
+//      (rescore_kernel): k and a handful, and the result is the streaming result, bit for bit.
+// A query with more records than there is room for is gated and streams.  A deny mask takes part in 1 and 2 as an infinite
+// |y|^2.  100k x 128 fp32, 1000 queries, k 10 (fp32 matrix cores, an exact prefix and levels before: 460 us): 209 us.
+// 100k x 768 fp32, 32 queries (streamed before: 684 us on the device): MEASURED_B.  500k x 100 sq8 under a deny mask, 200
+// queries, k 100 (streamed before: 664 us): 209 us.
+//
+// What bounds it: with 128 queries per workgroup the matrix cores beside the splitting of the codes and the verdicts; with
+// few queries the bytes of the codes, each read once per 32, 64 or 128 queries.
+//
+// Work split: a workgroup of four waves takes 256 codes (four storage tiles) and 128, 64 or 32 queries (kernel
+// parameters IB, JB, WN: a wave has IB x JB blocks of 32 x 32, WN waves stand side by side along the queries) in
+// stages of 32 dimensions (sq8, sq4: 64).  A stage sits in LDS as 16-byte slots of eight bf16 values [eight
+// dimensions][part][row], the operand order of the instruction (lane % 32 = row, lane / 32 = which eight of sixteen
+// dimensions).  The codes are split while they are parked in LDS (a thread owns a code), the queries once per call into a
+// table in slot order.
+#include "distance.h"
+#include "store.h"
+#include "topk.h"
+
+namespace vsag_amd {
+
+void timing_begin(hipStream_t st);
+void timing_end(hipStream_t st);
+
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef float floatx2 __attribute__((ext_vector_type(2)));
+typedef float floatx16 __attribute__((ext_vector_type(16)));
+
+constexpr uint32_t kB16M = 256;     // codes per workgroup tile (= threads of a workgroup)
+constexpr uint32_t kB16N = 128;     // most queries per workgroup tile; the rows of the query table are padded to it
+constexpr uint32_t kB16Pad = 64;    // the query table covers whole stages of either length
+constexpr uint32_t kB16Queue = 128; // records a wave gathers in LDS before it asks for room in the queries' lists
+
+template <int KIND>
+struct B16Layout {
+    static constexpr bool kSplit = KIND == VSAG_AMD_KIND_FP32;           // the code has a low part too
+    static constexpr uint32_t kSlots = kSplit ? 4 : 8;                   // eight dimensions each, per stage
+    static constexpr uint32_t kParts = kSplit ? 2 : 1;
+    static constexpr uint32_t kGranules = KIND == VSAG_AMD_KIND_FP32 ? 8 : KIND == VSAG_AMD_KIND_SQ8 ? 4 : 2;  // per stage
+};
+
+// sq8_uniform / sq4_uniform / rabitq stores have integer passes of their own.
+bool
+prefilter_b16_supports(const vsag_amd_store* s) {
+    return (s->kind == VSAG_AMD_KIND_FP32 || s->kind == VSAG_AMD_KIND_SQ8 || s->kind == VSAG_AMD_KIND_SQ4) &&
+           s->pf_term != nullptr && s->pf_ymax != nullptr;
+}
+
+static uint64_t
+b16_query_rows(uint64_t nq) {
+    return round_up(nq + 1, static_cast<uint64_t>(kB16N));  // (the row of a pair that does not exist is a row of zeros)
+}
+static uint32_t
+b16_slots(const vsag_amd_store* s) {
+    return static_cast<uint32_t>(round_up(s->dpad, kB16Pad) / 8);
+}
+static size_t
+b16_plane_bytes(const vsag_amd_store* s, uint64_t nq) {
+    return static_cast<size_t>(b16_slots(s)) * 2 * b16_query_rows(nq) * 16;
+}
+
+// Eight floats as their two bf16 parts.
+__device__ inline void
+b16_split8(const float (&x)[8], uint4* hi, uint4* lo) {
+    uint32_t h[4], l[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const bf16x2 hh = __builtin_convertvector((floatx2{x[2 * i], x[2 * i + 1]}), bf16x2);
+        h[i] = __builtin_bit_cast(uint32_t, hh);
+        const float r0 = x[2 * i] - __uint_as_float(h[i] << 16);
+        const float r1 = x[2 * i + 1] - __uint_as_float(h[i] & 0xFFFF0000U);
+        l[i] = __builtin_bit_cast(uint32_t, __builtin_convertvector((floatx2{r0, r1}), bf16x2));
+    }
+    *hi = make_uint4(h[0], h[1], h[2], h[3]);
+    *lo = make_uint4(l[0], l[1], l[2], l[3]);
+}
+
+// The two low bytes (bits 0..7, 8..15 of w) as bf16: a float of at most eight significant bits is its own upper half.
+__device__ inline uint32_t
+b16_two_bytes(uint32_t w, int at) {
+    const uint32_t a = __float_as_uint(static_cast<float>((w >> (8 * at)) & 0xffU));
+    const uint32_t b = __float_as_uint(static_cast<float>((w >> (8 * at + 8)) & 0xffU));
+    return __builtin_amdgcn_perm(b, a, 0x07060302U);
+}
+// An sq4 word (byte b: dimension 2 b in the low, 2 b + 1 in the high nibble) as the slot of its eight dimensions.
+__device__ inline uint4
+b16_nibbles(uint32_t w) {
+    const uint32_t lo = w & 0x0F0F0F0FU, hi = (w >> 4) & 0x0F0F0F0FU;
+    uint32_t out[4];
+#pragma unroll
+    for (int b = 0; b < 4; ++b) {
+        const uint32_t x = __float_as_uint(static_cast<float>((lo >> (8 * b)) & 0xffU));
+        const uint32_t y = __float_as_uint(static_cast<float>((hi >> (8 * b)) & 0xffU));
+        out[b] = __builtin_amdgcn_perm(y, x, 0x07060302U);
+    }
+    return make_uint4(out[0], out[1], out[2], out[3]);
+}
+
+// What a query's v can be off by: distance = v + constant, |v + constant - streaming distance| <= fixed + stream(D), with
+// stream(D) = root sqrt(D) + slope D the part that grows with the distance.
+struct B16Error {
+    float constant, fixed, root, slope;
+};
+
+struct B16QueryArgs {
+    const float* qtab;   // processed queries, zero beyond the dimension
+    uint32_t qstride;
+    uint32_t kdim;
+    const float* scale;  // sq8 / sq4 under l2: per dimension; null: ones
+    uint64_t nq, rows;
+    uint32_t slots;
+    uint4* planes;
+    const uint32_t* ymax_bits;  // largest |y| of the store (l2: scaled codes; ip: raw codes; fp32: the vectors)
+    float cmax;          // largest code value: 255, 15; fp32: 0
+    int is_l2;
+    const float* qmeta;  // sq8 / sq4, ip: sum q_d lb_d per query
+    uint32_t qmeta_stride;
+    B16Error* error;     // per query
+    // posting lists: thresholds from the queries' bounds
+    const uint32_t* bound;
+    float* tau;
+    float* magnitude;    // residual lists: the query's magnitudes (see IvfF32Args in prefilter.hip), or null
+};
+
+// One wave per row of the query table (rows at or beyond nq: zeros).
+__global__ void __launch_bounds__(64)
+b16_query_kernel(B16QueryArgs p) {
+    const uint64_t q = blockIdx.x;
+    const uint32_t lane = threadIdx.x;
+    const bool real = q < p.nq;
+    const float* row = p.qtab + q * p.qstride;
+    double a2 = 0.0, a1 = 0.0;               // of the processed query
+    double r1 = 0.0, r2 = 0.0, l2 = 0.0;     // the remainders and the low parts of b
+    for (uint32_t s = lane; s < p.slots; s += kWave) {
+        float x[8];
+        double exact[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            const uint32_t d = 8 * s + i;
+            const bool in = real && d < p.kdim;
+            const double a = in ? static_cast<double>(row[d]) : 0.0;
+            exact[i] = a * (in && p.scale != nullptr ? static_cast<double>(p.scale[d]) : 1.0);
+            x[i] = static_cast<float>(exact[i]);
+            a2 += a * a;
+            a1 += fabs(a);
+        }
+        uint4 hi, lo;
+        b16_split8(x, &hi, &lo);
+        p.planes[(static_cast<uint64_t>(s) * 2) * p.rows + q] = hi;
+        p.planes[(static_cast<uint64_t>(s) * 2 + 1) * p.rows + q] = lo;
+        const uint32_t hw[4] = {hi.x, hi.y, hi.z, hi.w}, lw[4] = {lo.x, lo.y, lo.z, lo.w};
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            const float h = __uint_as_float((i & 1) != 0 ? hw[i >> 1] & 0xFFFF0000U : hw[i >> 1] << 16);
+            const float l = __uint_as_float((i & 1) != 0 ? lw[i >> 1] & 0xFFFF0000U : lw[i >> 1] << 16);
+            const double left = exact[i] - static_cast<double>(h) - static_cast<double>(l);
+            r1 += fabs(left);
+            r2 += left * left;
+            l2 += static_cast<double>(l) * static_cast<double>(l);
+        }
+    }
+    for (int off = 32; off > 0; off >>= 1) {
+        a2 += __shfl_xor(a2, off);
+        a1 += __shfl_xor(a1, off);
+        r1 += __shfl_xor(r1, off);
+        r2 += __shfl_xor(r2, off);
+        l2 += __shfl_xor(l2, off);
+    }
+    if (lane != 0 || !real) {
+        return;
+    }
+    constexpr double kU = 5.9604644775390625e-8;  // 2^-24, the unit roundoff of fp32
+    const double kd = static_cast<double>(p.kdim);
+    const double ymax = static_cast<double>(__uint_as_float(*p.ymax_bits)) * (1.0 + 1.0e-6);
+    const double an = sqrt(a2);
+    const double dots = an * ymax;  // sum |b_d c_d| of any code, by Cauchy and Schwarz
+    const bool fp32 = p.cmax == 0.0F;
+    const double sums = fp32 || p.is_l2 ? dots : fmin(static_cast<double>(p.cmax) * a1, dots);
+    const double factor = p.is_l2 ? 2.0 : 1.0;
+    // Left out: the remainders of the query against a code (codes of bytes lie in [0, cmax]); of an fp32 code at most 2^-18
+    // of it against the query, and its low part (2^-9 of it) against the query's.
+    const double split = fp32 ? ymax * (sqrt(r2) + 3.9e-6 * an + 1.97e-3 * sqrt(l2)) : static_cast<double>(p.cmax) * r1;
+    // The accumulation: four roundings of the absolute sum per instruction (two or three per sixteen dimensions).
+    const double rounding = 4.0 * kU * ((fp32 ? 3.0 : 2.0) * kd / 16.0 + 4.0) * sums;
+    // Operands below the normal range taken as zero; fl(term + fl(factor acc)) of the test itself and |y|^2 rounded once.
+    const double flushed = kd * 4.7e-38 * (an + ymax + 1.0);
+    const double test = 6.0 * kU * ((p.is_l2 ? ymax * ymax : 0.0) + factor * dots);
+    double fixed = factor * (split + rounding) + flushed + test;
+    double root = 0.0, slope = 0.0;
+    double constant = a2;
+    if (p.is_l2) {
+        // The streaming kernel's fp32 sum of squares: every term (fl(c s) - a)^2 is off by two or three roundings of itself
+        // and, for codes of bytes, by the rounding of c s; then kdim roundings of the sum.
+        slope = (kd + 4.0) * kU;
+        root = fp32 ? 0.0 : 2.0 * kU * ymax;
+    } else {
+        // 1 - (fl(sum) + qmeta): kdim roundings of sum |terms|, then the closing operations.
+        const double qm = p.qmeta != nullptr ? static_cast<double>(p.qmeta[q * p.qmeta_stride]) : 0.0;
+        fixed += (kd + 2.0) * kU * sums + 4.0 * kU * (sums + fabs(qm) + 1.0);
+        constant = 1.0 - qm;
+    }
+    B16Error e;
+    e.constant = static_cast<float>(constant);
+    e.fixed = static_cast<float>(fixed) * 1.000001F + 1.0e-37F;
+    e.root = static_cast<float>(root) * 1.000001F;
+    e.slope = static_cast<float>(slope) * 1.000001F;
+    if (p.error != nullptr) {
+        p.error[q] = e;
+    }
+    if (p.tau == nullptr) {
+        return;
+    }
+    const uint32_t b = p.bound[q];
+    const double bd = static_cast<double>(ordered_to_float(b));
+    const double t = bd - constant + fixed + 1.01 * (root * sqrt(fabs(bd)) + slope * fabs(bd)) +
+                     1.0e-6 * (fabs(bd) + fabs(constant));
+    const float tf = static_cast<float>(t);
+    const float up = tf + fabsf(tf) * 1.2e-7F + 1.0e-37F;
+    // no bound yet, or entries that are not finite: everything is a candidate (and the query overflows)
+    const bool open = b == 0xFFFFFFFFU || !(up < 3.0e38F);
+    p.tau[q] = open ? 3.0e38F : up;
+    if (p.magnitude != nullptr) {
+        const double magnitude = fabs(bd) + fabs(constant) + (p.is_l2 ? ymax * ymax : 0.0) + factor * dots;
+        p.magnitude[q] = open ? 0.0F : static_cast<float>(magnitude) * 1.000001F;
+    }
+}
+
+struct B16TauArgs {
+    const float* least;     // nq x groups: the least v of every group of sampled codes
+    uint32_t groups, k;
+    const B16Error* error;
+    float* tau;
+    float* slack;           // twice what v can be off by, at the distances that matter
+    uint32_t* cand_cnt;     // zeroed
+    uint32_t* gate;         // zeroed
+    uint32_t* partial_cnt;  // nslots a query, zeroed
+    uint32_t nslots;
+};
+
+// One wave per query.
+__global__ void __launch_bounds__(64)
+b16_tau_kernel(B16TauArgs p) {
+    __shared__ uint32_t hist[256];
+    const uint64_t q = blockIdx.x;
+    const uint32_t lane = threadIdx.x;
+    const float* least = p.least + q * p.groups;
+    const float kth = kth_value_or_above([&](uint32_t i) { return least[i]; }, p.groups, p.k, hist, lane);
+    for (uint32_t i = lane; i < p.nslots; i += kWave) {
+        p.partial_cnt[q * p.nslots + i] = 0;
+    }
+    if (lane != 0) {
+        return;
+    }
+    p.cand_cnt[q] = 0;
+    p.gate[q] = 0;
+    const B16Error e = p.error[q];
+    // The k codes at or below kth have distances of at most D; so has whoever is among the k best.
+    const float far = fmaxf(kth + e.constant, 0.0F) * 1.00001F + 2.0F * e.fixed;
+    const float slack = 2.0F * e.fixed + 2.05F * (e.root * sqrtf(far) + e.slope * far);
+    const float tau = kth + slack;
+    const float up = tau + fabsf(tau) * 2.4e-7F + 1.0e-37F;
+    // fewer than k codes sampled, or values that are not finite: everything is a candidate
+    const bool open = !(up < 3.0e38F) || !(kth > -3.0e38F);
+    p.tau[q] = open ? 3.0e38F : up;
+    p.slack[q] = open ? 3.0e38F : slack;
+}
+
+struct PrefilterB16Args {
+    const uint4* tiles;
+    uint32_t G;
+    const uint4* planes;
+    uint64_t nq, rows;
+    uint32_t slots;
+    const float* term;  // per slot |y|^2
+    int is_l2;
+    const float* tau;
+    // flat stores
+    uint64_t ntiles, n;
+    uint64_t mstep;     // code tiles of four storage tiles: 0, mstep, 2 mstep, ... (1: all of them)
+    float* least;       // a sampling pass: nq x groups values, and no records; else null
+    uint32_t groups;
+    uint64_t* cand;     // nq x cap records: v as its ordered bits above the slot
+    uint32_t* cand_cnt;
+    uint32_t cap;
+    const uint32_t* deny;
+    // posting lists (as IvfF32Args in prefilter.hip)
+    const float* res_bias;
+    const float* res_term;
+    const float* magnitude;
+    const uint32_t* ymax_bits;
+    float res_cmax;
+    const uint32_t* ids;
+    const uint32_t* list_tile;
+    const uint32_t* pair_off;
+    const uint32_t* item_off;
+    const uint32_t* sorted_pair;
+    uint32_t nlist, nprobe;
+    uint32_t k;
+    uint64_t* partial;
+    uint32_t* partial_cnt;
+    uint32_t* gate;
+};
+
+constexpr uint32_t kIvfB16ChunkTiles = 32;  // as ivf_i8.hip: kIvfI8ChunkTiles, kIvfI8Chunks
+constexpr uint32_t kIvfB16Chunks = 4;
+
+template <int KIND, bool LISTS, int IB, int JB, int WN>
+__global__ void __launch_bounds__(256, IB * JB <= (KIND == VSAG_AMD_KIND_FP32 ? 4 : 2) ? 3 : 2)
+prefilter_b16_kernel(PrefilterB16Args p) {
+    using L = B16Layout<KIND>;
+    constexpr uint32_t N = WN * JB * 32;
+    static_assert((4 / WN) * IB * 32 == kB16M, "the waves cover the codes of a tile");
+    __shared__ uint4 sa[L::kSlots][L::kParts][kB16M];
+    __shared__ uint4 sb[L::kSlots][2][N];
+    __shared__ float code_term[kB16M];
+    __shared__ uint64_t queue_key[4][kB16Queue];
+    __shared__ uint32_t queue_col[4][kB16Queue];
+    const uint32_t tid = threadIdx.x;
+    const uint32_t lane = tid & 63;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const uint32_t wm = wave / WN, wn = wave % WN;
+    const uint32_t half = lane >> 5;
+    const uint32_t l32 = lane & 31;
+    const uint32_t stages = (p.G + L::kGranules - 1) / L::kGranules;
+
+    // What this workgroup walks: code tiles first, first + step, ... below mtiles (of four storage tiles from tile_begin
+    // on), against the query rows of its N columns.
+    uint64_t tile_begin = 0, tile_end, first = 0, step = 1;
+    uint64_t q0 = 0;
+    uint32_t pbeg = 0, pend = 0, chunk = 0;
+    if constexpr (LISTS) {
+        const uint32_t item = blockIdx.x;
+        const cu32_p ioff = as_const(p.item_off);
+        if (item >= ioff[p.nlist]) {
+            return;  // the whole workgroup
+        }
+        uint32_t lo_b = 0, hi_b = p.nlist;
+        while (hi_b - lo_b > 1) {
+            const uint32_t mid = (lo_b + hi_b) >> 1;
+            if (ioff[mid] <= item) {
+                lo_b = mid;
+            } else {
+                hi_b = mid;
+            }
+        }
+        const uint32_t list_begin = as_const(p.list_tile)[2 * lo_b], list_end = as_const(p.list_tile)[2 * lo_b + 1];
+        uint32_t chunks = (list_end - list_begin + kIvfB16ChunkTiles - 1) / kIvfB16ChunkTiles;
+        chunks = chunks < kIvfB16Chunks ? chunks : kIvfB16Chunks;
+        if (chunks == 0) {
+            return;
+        }
+        const uint32_t per = (list_end - list_begin + chunks - 1) / chunks;
+        chunk = (item - ioff[lo_b]) % chunks;
+        const uint32_t group = (item - ioff[lo_b]) / chunks;
+        uint32_t tb = list_begin + chunk * per;
+        tb = tb < list_end ? tb : list_end;
+        tile_begin = tb;
+        tile_end = tb + per < list_end ? tb + per : list_end;
+        pbeg = as_const(p.pair_off)[lo_b] + group * N;
+        pend = as_const(p.pair_off)[lo_b + 1];
+        if (tile_begin >= tile_end || pbeg >= pend) {
+            return;
+        }
+    } else {
+        tile_end = p.ntiles;
+        first = blockIdx.x * p.mstep;
+        step = gridDim.x * p.mstep;
+        q0 = static_cast<uint64_t>(blockIdx.y) * N;
+    }
+    const uint64_t mtiles = (tile_end - tile_begin + 3) / 4;
+
+    // Verdict side: the columns l32 of this wave's JB blocks.
+    float tau_n[JB];
+#pragma unroll
+    for (int j = 0; j < JB; ++j) {
+        const uint32_t col = wn * JB * 32 + j * 32 + l32;
+        if constexpr (LISTS) {
+            const uint32_t at = pbeg + col;
+            const uint32_t pair = at < pend ? as_const(p.sorted_pair)[at] : 0U;
+            const uint32_t query = pair / p.nprobe;
+            tau_n[j] = at < pend ? p.tau[query] : -__builtin_inff();
+            if (p.res_term != nullptr && at < pend) {
+                const float rt = p.res_term[pair];
+                // |bias| = |2 <c, y> + |c|^2| (l2; inner product has none); five more roundings stand between this test
+                // and the streaming result: 2e-6 of the magnitudes is several times their sum
+                const float bias_max =
+                    p.res_bias != nullptr ? (2.0F * __uint_as_float(*p.ymax_bits) + p.res_cmax) * p.res_cmax : 0.0F;
+                tau_n[j] = tau_n[j] + rt + 2.0e-6F * (p.magnitude[query] + fabsf(rt) + bias_max);
+            }
+        } else {
+            tau_n[j] = q0 + col < p.nq && p.least == nullptr ? p.tau[q0 + col] : -__builtin_inff();
+        }
+    }
+    // A wave none of whose columns holds a query only helps to fetch.
+    const bool busy = LISTS ? pbeg + wn * JB * 32 < pend : q0 + wn * JB * 32 < p.nq;
+
+    // Query loader: (slot, part) pairs x N rows per stage, consecutive threads on consecutive rows.
+    constexpr uint32_t kQueryRegs = L::kSlots * 2 * N / 256;
+    constexpr uint32_t kRowStep = 256 / N;  // (slot, part) pairs that one round of the workgroup covers
+    const uint32_t qr = tid % N;
+    uint64_t qsrc;
+    if constexpr (LISTS) {
+        const uint32_t at = pbeg + qr;
+        qsrc = at < pend ? as_const(p.sorted_pair)[at] / p.nprobe : p.nq;  // p.nq: a row of zeros
+    } else {
+        qsrc = q0 + qr;  // below p.rows: the table covers whole tiles of rows
+    }
+    // (Separate variables, not arrays: an array ended up in scratch memory.)
+    uint4 rc0, rc1, rc2, rc3, rc4, rc5, rc6, rc7, rq0, rq1, rq2, rq3, rq4, rq5, rq6, rq7;
+    const uint4* const qsrc_row = p.planes + static_cast<uint64_t>(tid / N) * p.rows + qsrc;
+    auto query_slot = [&](uint32_t st, uint32_t r) __attribute__((always_inline)) {
+        return qsrc_row[(static_cast<uint64_t>(st) * 2 * L::kSlots + kRowStep * r) * p.rows];
+    };
+    // No load stands behind a branch.  Granules past a code's end repeat its last one (the query's values there are zeros),
+    // tiles past the end repeat the first (their terms are infinite).
+    auto fetch = [&](uint64_t mt, uint32_t st) __attribute__((always_inline)) {
+        uint64_t tile = tile_begin + 4 * mt + wave;
+        tile = tile < tile_end ? tile : tile_begin;
+        const uint4* src = p.tiles + tile * p.G * kWave;
+        const uint32_t last = p.G - 1;
+        auto granule = [&](uint32_t u) __attribute__((always_inline)) {
+            const uint32_t j = L::kGranules * st + u < last ? L::kGranules * st + u : last;
+            return src[j * kWave + lane];
+        };
+        rc0 = granule(0);
+        rc1 = granule(1);
+        if constexpr (L::kGranules > 2) {
+            rc2 = granule(2);
+            rc3 = granule(3);
+        }
+        if constexpr (L::kGranules > 4) {
+            rc4 = granule(4);
+            rc5 = granule(5);
+            rc6 = granule(6);
+            rc7 = granule(7);
+        }
+        rq0 = query_slot(st, 0);
+        if constexpr (kQueryRegs > 1) {
+            rq1 = query_slot(st, 1);
+        }
+        if constexpr (kQueryRegs > 2) {
+            rq2 = query_slot(st, 2);
+            rq3 = query_slot(st, 3);
+        }
+        if constexpr (kQueryRegs > 4) {
+            rq4 = query_slot(st, 4);
+            rq5 = query_slot(st, 5);
+            rq6 = query_slot(st, 6);
+            rq7 = query_slot(st, 7);
+        }
+    };
+    auto park_floats = [&](uint32_t s, uint4 v, uint4 w) __attribute__((always_inline)) {
+        const float x[8] = {__uint_as_float(v.x), __uint_as_float(v.y), __uint_as_float(v.z), __uint_as_float(v.w),
+                            __uint_as_float(w.x), __uint_as_float(w.y), __uint_as_float(w.z), __uint_as_float(w.w)};
+        uint4 hi, lo;
+        b16_split8(x, &hi, &lo);
+        sa[s][0][tid] = hi;
+        sa[s][L::kParts - 1][tid] = lo;
+    };
+    auto park_bytes = [&](uint32_t s, uint4 v) __attribute__((always_inline)) {
+        sa[s][0][tid] = make_uint4(b16_two_bytes(v.x, 0), b16_two_bytes(v.x, 2), b16_two_bytes(v.y, 0), b16_two_bytes(v.y, 2));
+        sa[s + 1][0][tid] =
+            make_uint4(b16_two_bytes(v.z, 0), b16_two_bytes(v.z, 2), b16_two_bytes(v.w, 0), b16_two_bytes(v.w, 2));
+    };
+    auto park_nibbles = [&](uint32_t s, uint4 v) __attribute__((always_inline)) {
+        sa[s][0][tid] = b16_nibbles(v.x);
+        sa[s + 1][0][tid] = b16_nibbles(v.y);
+        sa[s + 2][0][tid] = b16_nibbles(v.z);
+        sa[s + 3][0][tid] = b16_nibbles(v.w);
+    };
+    auto park_query = [&](uint32_t r, uint4 v) __attribute__((always_inline)) {
+        const uint32_t sp = tid / N + kRowStep * r;
+        sb[sp >> 1][sp & 1][qr] = v;
+    };
+    auto park = [&]() __attribute__((always_inline)) {
+        if constexpr (KIND == VSAG_AMD_KIND_FP32) {
+            park_floats(0, rc0, rc1);
+            park_floats(1, rc2, rc3);
+            park_floats(2, rc4, rc5);
+            park_floats(3, rc6, rc7);
+        } else if constexpr (KIND == VSAG_AMD_KIND_SQ8) {
+            park_bytes(0, rc0);
+            park_bytes(2, rc1);
+            park_bytes(4, rc2);
+            park_bytes(6, rc3);
+        } else {
+            park_nibbles(0, rc0);
+            park_nibbles(4, rc1);
+        }
+        park_query(0, rq0);
+        if constexpr (kQueryRegs > 1) {
+            park_query(1, rq1);
+        }
+        if constexpr (kQueryRegs > 2) {
+            park_query(2, rq2);
+            park_query(3, rq3);
+        }
+        if constexpr (kQueryRegs > 4) {
+            park_query(4, rq4);
+            park_query(5, rq5);
+            park_query(6, rq6);
+            park_query(7, rq7);
+        }
+    };
+    // Records wait in the wave's queue (a query's counter is an atomic a microsecond away: asked for one record at a time it
+    // cost half of the pass), until it might overflow or the walk is over.
+    uint64_t* const keys = queue_key[wave];
+    uint32_t* const cols = queue_col[wave];
+    uint32_t waiting = 0;
+    auto flush = [&]() __attribute__((always_inline)) {
+        wave_lds_fence();
+        for (uint32_t i = lane; i < waiting; i += kWave) {
+            const uint64_t key = keys[i];
+            if constexpr (LISTS) {
+                // private list of the pair: chunk, which half of the 256 codes (the upper word)
+                const uint32_t pair = as_const(p.sorted_pair)[pbeg + cols[i]];
+                const uint64_t list =
+                    (static_cast<uint64_t>(pair) * kIvfB16Chunks + chunk) * 2 + static_cast<uint32_t>(key >> 32);
+                const uint32_t pos = atomicAdd(&p.partial_cnt[list], 1U);
+                if (pos < p.k) {
+                    p.partial[list * p.k + pos] = static_cast<uint32_t>(key);
+                } else if (pos == p.k) {
+                    if (atomicExch(&p.gate[pair / p.nprobe], 1U) == 0U) {
+                        atomicAdd(&p.gate[p.nq], 1U);
+                    }
+                }
+            } else {
+                const uint64_t q = q0 + cols[i];
+                const uint32_t pos = atomicAdd(&p.cand_cnt[q], 1U);
+                if (pos < p.cap) {
+                    p.cand[q * p.cap + pos] = key;
+                }
+            }
+        }
+        waiting = 0;
+        wave_lds_fence();
+    };
+
+    if (first < mtiles) {
+        fetch(first, 0);
+    }
+    for (uint64_t mt = first; mt < mtiles; mt += step) {
+        floatx16 acc[IB][JB];
+#pragma unroll
+        for (int i = 0; i < IB; ++i) {
+#pragma unroll
+            for (int j = 0; j < JB; ++j) {
+#pragma unroll
+                for (int e = 0; e < 16; ++e) {
+                    acc[i][j][e] = 0.0F;
+                }
+            }
+        }
+        const uint64_t slot0 = (tile_begin + 4 * mt) * kWave;
+        park();  // the stage is free: the previous tile's contraction ended with a barrier
+        float my_term;
+        {
+            const uint64_t slot = slot0 + tid;
+            bool real = tile_begin + 4 * mt + (tid >> 6) < tile_end;
+            if constexpr (LISTS) {
+                // (a padding slot is all zeros: under inner product, and with a residual bias, that is a good distance)
+                real = real && p.ids[slot] != VSAG_AMD_INVALID_ID;
+            } else {
+                real = real && slot < p.n && !denied(p.deny, slot);
+            }
+            my_term = real ? (p.is_l2 ? p.term[slot] : 0.0F) : __builtin_inff();
+            if (LISTS && real && p.res_bias != nullptr) {
+                my_term -= p.res_bias[slot];
+            }
+        }
+        __syncthreads();
+        for (uint32_t st = 0; st < stages; ++st) {
+            {
+                // the next stage of this tile, or the first of the next tile (of this one once more behind the last)
+                const bool more = st + 1 < stages;
+                fetch(more || mt + step >= mtiles ? mt : mt + step, more ? st + 1 : 0);
+            }
+            if (busy) {
+#pragma nounroll
+                for (uint32_t ks = 0; ks < L::kSlots / 2; ++ks) {
+                    const uint32_t slot = 2 * ks + half;
+                    bf16x8 bh[JB], bl[JB];
+#pragma unroll
+                    for (int j = 0; j < JB; ++j) {
+                        bh[j] = __builtin_bit_cast(bf16x8, sb[slot][0][wn * JB * 32 + j * 32 + l32]);
+                        bl[j] = __builtin_bit_cast(bf16x8, sb[slot][1][wn * JB * 32 + j * 32 + l32]);
+                    }
+#pragma unroll
+                    for (int i = 0; i < IB; ++i) {
+                        const uint32_t row = wm * IB * 32 + i * 32 + l32;
+                        const bf16x8 ah = __builtin_bit_cast(bf16x8, sa[slot][0][row]);
+                        if constexpr (L::kSplit) {
+                            const bf16x8 al = __builtin_bit_cast(bf16x8, sa[slot][L::kParts - 1][row]);
+#pragma unroll
+                            for (int j = 0; j < JB; ++j) {
+                                acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(al, bh[j], acc[i][j], 0, 0, 0);
+                            }
+                        }
+#pragma unroll
+                        for (int j = 0; j < JB; ++j) {
+                            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ah, bl[j], acc[i][j], 0, 0, 0);
+                        }
+#pragma unroll
+                        for (int j = 0; j < JB; ++j) {
+                            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ah, bh[j], acc[i][j], 0, 0, 0);
+                        }
+                    }
+                }
+            }
+            if (st + 1 == stages) {
+                // every wave is past this tile's first barrier, hence out of the previous tile's epilogue
+                code_term[tid] = my_term;
+            }
+            __syncthreads();  // every wave has read the stage
+            if (st + 1 < stages) {
+                park();
+                __syncthreads();
+            }
+        }
+        if (!busy) {
+            continue;
+        }
+        // Nearly nothing passes: sixteen products of a lane share a verdict (their least value), and only where a lane's
+        // passes are they looked at one by one.
+        const float dot_factor = p.is_l2 ? -2.0F : -1.0F;
+        float group_least[JB];
+#pragma unroll
+        for (int j = 0; j < JB; ++j) {
+            group_least[j] = __builtin_inff();
+        }
+#pragma unroll
+        for (int i = 0; i < IB; ++i) {
+            const uint32_t m0 = wm * IB * 32 + i * 32 + 4 * half;
+            float term[16];
+#pragma unroll
+            for (int e4 = 0; e4 < 4; ++e4) {
+                const float4 t4 = *reinterpret_cast<const float4*>(code_term + m0 + 8 * e4);
+                term[4 * e4] = t4.x;
+                term[4 * e4 + 1] = t4.y;
+                term[4 * e4 + 2] = t4.z;
+                term[4 * e4 + 3] = t4.w;
+            }
+#pragma unroll
+            for (int j = 0; j < JB; ++j) {
+                float v[16];
+                float least = __builtin_inff();
+#pragma unroll
+                for (int e = 0; e < 16; ++e) {
+                    v[e] = fmaf(dot_factor, acc[i][j][e], term[e]);
+                    least = fminf(least, v[e]);
+                }
+                group_least[j] = fminf(group_least[j], least);
+                if (__ballot(least <= tau_n[j]) == 0) {
+                    continue;
+                }
+                uint32_t hits = 0;
+#pragma unroll
+                for (int e = 0; e < 16; ++e) {
+                    hits |= (v[e] <= tau_n[j] ? 1U : 0U) << e;
+                }
+                hits = tau_n[j] > -__builtin_inff() ? hits : 0U;  // (a column without a query)
+                while (__ballot(hits != 0) != 0) {
+                    const bool hit = hits != 0;
+                    const uint64_t mask = __ballot(hit);
+                    const uint32_t np = static_cast<uint32_t>(__popcll(mask));
+                    if (waiting + np > kB16Queue) {
+                        flush();
+                    }
+                    if (hit) {
+                        const uint32_t e = static_cast<uint32_t>(__builtin_ctz(hits));
+                        hits &= hits - 1;
+                        const uint32_t at = waiting + mask_rank(mask);
+                        const uint32_t ml = m0 + 8 * (e >> 2) + (e & 3);
+                        const uint32_t slot = static_cast<uint32_t>(slot0) + ml;
+                        if constexpr (LISTS) {
+                            keys[at] = (static_cast<uint64_t>(ml >> 7) << 32) | slot;
+                        } else {
+                            float value = v[0];
+#pragma unroll
+                            for (int u = 1; u < 16; ++u) {
+                                value = e == static_cast<uint32_t>(u) ? v[u] : value;
+                            }
+                            keys[at] = make_key(value, slot);
+                        }
+                        cols[at] = wn * JB * 32 + j * 32 + l32;
+                    }
+                    waiting += np;
+                }
+            }
+        }
+        if constexpr (!LISTS) {
+            if (p.least != nullptr) {
+                // the codes of a lane: 16 IB of the tile's 256, one group
+#pragma unroll
+                for (int j = 0; j < JB; ++j) {
+                    const uint64_t q = q0 + wn * JB * 32 + j * 32 + l32;
+                    const uint32_t group = (static_cast<uint32_t>(mt / p.mstep) * (4 / WN) + wm) * 2 + half;
+                    if (q < p.nq) {
+                        p.least[q * p.groups + group] = group_least[j];
+                    }
+                }
+            }
+        }
+    }
+    if (waiting != 0) {
+        flush();
+    }
+}
+
+static void
+b16_query_args(const vsag_amd_store* s, const ScanArgs& a, uint64_t nq, B16QueryArgs* qa) {
+    const bool l2 = s->metric == VSAG_AMD_METRIC_L2;
+    const bool fp32 = s->kind == VSAG_AMD_KIND_FP32;
+    *qa = B16QueryArgs{};
+    qa->qtab = reinterpret_cast<const float*>(a.qtab);
+    qa->qstride = a.qstride;
+    qa->kdim = s->dpad;
+    qa->scale = !fp32 && l2 ? s->scale_dev : nullptr;
+    qa->nq = nq;
+    qa->rows = b16_query_rows(nq);
+    qa->slots = b16_slots(s);
+    qa->ymax_bits = s->pf_ymax;
+    qa->cmax = fp32 ? 0.0F : s->kind == VSAG_AMD_KIND_SQ8 ? 255.0F : 15.0F;
+    qa->is_l2 = l2 ? 1 : 0;
+    qa->qmeta = !fp32 && !l2 ? a.qmeta : nullptr;
+    qa->qmeta_stride = a.qmeta_stride;
+}
+
+template <int KIND>
+static void
+launch_b16_flat(uint64_t nq, uint32_t cus, PrefilterB16Args p, hipStream_t st) {
+    const uint32_t per = nq <= 32 ? 32 : nq <= 64 ? 64 : kB16N;
+    const uint64_t qtiles = div_up(nq, static_cast<uint64_t>(per));
+    const uint64_t mtiles = div_up(div_up(p.ntiles, 4), p.mstep);
+    // Two rounds of the workgroups that fit a compute unit (two or three) and not one more: a few left over would run a
+    // third round alone.  A workgroup walks every gridDim.x-th tile.
+    uint64_t groups = static_cast<uint64_t>(cus) * (per == kB16N ? 4 : 6) / qtiles;
+    groups = std::max<uint64_t>(1, std::min<uint64_t>(groups, mtiles));
+    const dim3 grid(static_cast<uint32_t>(groups), static_cast<uint32_t>(qtiles));
+    if (per == 32) {
+        hipLaunchKernelGGL((prefilter_b16_kernel<KIND, false, 2, 1, 1>), grid, dim3(256), 0, st, p);
+    } else if (per == 64) {
+        hipLaunchKernelGGL((prefilter_b16_kernel<KIND, false, 2, 2, 1>), grid, dim3(256), 0, st, p);
+    } else {
+        hipLaunchKernelGGL((prefilter_b16_kernel<KIND, false, 4, 2, 2>), grid, dim3(256), 0, st, p);
+    }
+}
+
+static void
+launch_b16_kind(const vsag_amd_store* s, uint64_t nq, const PrefilterB16Args& p, hipStream_t st) {
+    const uint32_t cus = static_cast<uint32_t>(device_cu_count());
+    if (s->kind == VSAG_AMD_KIND_FP32) {
+        launch_b16_flat<VSAG_AMD_KIND_FP32>(nq, cus, p, st);
+    } else if (s->kind == VSAG_AMD_KIND_SQ8) {
+        launch_b16_flat<VSAG_AMD_KIND_SQ8>(nq, cus, p, st);
+    } else {
+        launch_b16_flat<VSAG_AMD_KIND_SQ4>(nq, cus, p, st);
+    }
+}
+
+// The sample of a call: every step-th code tile of 256.  With s of n codes sampled, about k n / s codes lie at or below the
+// k-th smallest of the sample: kB16Expect of them (4 k where that is more), an eighth of the room a query has (a quarter).
+// Each sampled tile gives four groups at least, and four times as many groups as k keep their k-th least close to the k-th
+// of the sample.
+constexpr uint64_t kB16Expect = 256;
+constexpr uint32_t kB16Records = 2048;
+
+uint32_t
+prefilter_b16_cap(uint32_t k) {
+    return std::max<uint32_t>(kB16Records, 16 * k);
+}
+
+static uint64_t
+b16_sample_step(const vsag_amd_store* s, uint32_t k) {
+    const uint64_t mtiles = div_up(s->ntiles, 4);
+    const uint64_t expect = std::max<uint64_t>(kB16Expect, 4ull * k);
+    const uint64_t want = std::max<uint64_t>({16, k, div_up(mtiles * k, expect)});
+    return std::max<uint64_t>(1, mtiles / want);
+}
+static uint32_t
+b16_sample_groups(const vsag_amd_store* s, uint64_t nq, uint32_t k) {
+    const uint64_t tiles = div_up(div_up(s->ntiles, 4), b16_sample_step(s, k));
+    return static_cast<uint32_t>(tiles * (nq <= 64 ? 8 : 4));
+}
+
+// Scratch: the queries' parts, then their errors, thresholds, slacks and what the sample leaves.
+struct B16Scratch {
+    uint4* planes;
+    B16Error* error;
+    float* tau;
+    float* slack;
+    float* least;
+};
+static size_t
+carve_b16(Carver& c, const vsag_amd_store* s, uint64_t nq, uint32_t k, B16Scratch* b) {
+    b->planes = reinterpret_cast<uint4*>(c.take<uint8_t>(b16_plane_bytes(s, nq)));
+    b->error = c.take<B16Error>(nq);
+    b->tau = c.take<float>(nq);
+    b->slack = c.take<float>(nq);
+    b->least = c.take<float>(nq * b16_sample_groups(s, nq, k));
+    return c.used;
+}
+size_t
+prefilter_b16_scratch_bytes(const vsag_amd_store* s, uint64_t nq, uint32_t k) {
+    Carver c(nullptr, 0);
+    B16Scratch b;
+    return carve_b16(c, s, nq, k, &b);
+}
+
+int launch_rescore_valued(const vsag_amd_store* s, const ScanArgs& a, uint64_t nq, uint32_t k, uint32_t S, uint32_t* bound,
+                          const uint64_t* valued, const float* slack, const uint32_t* cand_cnt, uint32_t cap,
+                          uint64_t* partial, uint32_t* partial_cnt, uint32_t nslots, uint32_t out_slot, uint32_t* gate,
+                          hipStream_t st);
+
+// The flat scan of the header comment: list 0 of every query's nslots partial lists holds its k best, the others are empty,
+// and the gate of a query that has to stream is up.  `bound` holds what a search starts from.
+int
+launch_scan_b16(const vsag_amd_store* s, const ScanArgs& a, uint64_t nq, uint32_t k, uint32_t S, uint32_t* bound,
+                uint8_t* scratch, uint64_t* cand, uint32_t* cand_cnt, uint32_t cap, const uint32_t* deny, uint64_t* partial,
+                uint32_t* partial_cnt, uint32_t nslots, uint32_t* gate, hipStream_t st) {
+    Carver c(scratch, ~size_t{0});
+    B16Scratch b;
+    carve_b16(c, s, nq, k, &b);
+    B16QueryArgs qa;
+    b16_query_args(s, a, nq, &qa);
+    qa.planes = b.planes;
+    qa.error = b.error;
+    hipLaunchKernelGGL(b16_query_kernel, dim3(static_cast<uint32_t>(qa.rows)), dim3(kWave), 0, st, qa);
+    PrefilterB16Args p{};
+    p.tiles = s->tiles;
+    p.G = s->G;
+    p.planes = b.planes;
+    p.nq = nq;
+    p.rows = qa.rows;
+    p.slots = qa.slots;
+    p.term = s->pf_term;
+    p.is_l2 = qa.is_l2;
+    p.tau = b.tau;
+    p.ntiles = s->ntiles;
+    p.n = s->n;
+    p.deny = deny;
+    p.mstep = b16_sample_step(s, k);
+    p.least = b.least;
+    p.groups = b16_sample_groups(s, nq, k);
+    launch_b16_kind(s, nq, p, st);
+    B16TauArgs ta{b.least, p.groups, k, b.error, b.tau, b.slack, cand_cnt, gate, partial_cnt, nslots};
+    hipLaunchKernelGGL(b16_tau_kernel, dim3(static_cast<uint32_t>(nq)), dim3(kWave), 0, st, ta);
+    p.mstep = 1;
+    p.least = nullptr;
+    p.cand = cand;
+    p.cand_cnt = cand_cnt;
+    p.cap = cap;
+    timing_begin(st);
+    launch_b16_kind(s, nq, p, st);
+    timing_end(st);
+    VA_HIP(hipGetLastError());
+    return launch_rescore_valued(s, a, nq, k, S, bound, cand, b.slack, cand_cnt, cap, partial, partial_cnt, nslots, 0, gate, st);
+}
+
+bool
+ivf_b16_supports(const vsag_amd_store* s) {
+    return s->kind == VSAG_AMD_KIND_FP32 && s->nlist > 0 && s->pf_term != nullptr && s->pf_ymax != nullptr &&
+           s->ids_dev != nullptr && (s->residual_centroids_dev == nullptr || s->metric != VSAG_AMD_METRIC_COSINE);
+}
+
+uint32_t
+ivf_b16_pairs_per_item() {
+    return kB16N;
+}
+size_t
+ivf_b16_scratch_bytes(const vsag_amd_store* s, uint64_t nq) {
+    return b16_plane_bytes(s, nq);
+}
+
+// The candidates of probe columns [p0, nprobe) grouped by list (pair_off, sorted_pair; item_off counted with
+// ivf_b16_pairs_per_item() pairs per item) into the private lists (pair * 8 + chunk * 2 + half of the code tile) of
+// kcand records in `partial`; partial_cnt zero before.  tau: 2 nq + 1 floats; gate: nq + 2 words.
+int
+launch_ivf_b16(const vsag_amd_store* s, const ScanArgs& a, uint64_t nq, uint32_t nprobe, uint32_t p0, const uint32_t* pair_off,
+               const uint32_t* item_off, const uint32_t* sorted_pair, const uint32_t* bound, uint32_t kcand, float* tau,
+               uint8_t* scratch, uint64_t* partial, uint32_t* partial_cnt, uint32_t* gate, const float* res_term,
+               hipStream_t st) {
+    B16QueryArgs qa;
+    b16_query_args(s, a, nq, &qa);
+    qa.planes = reinterpret_cast<uint4*>(scratch);
+    qa.bound = bound;
+    qa.tau = tau;
+    qa.magnitude = res_term != nullptr ? tau + nq + 1 : nullptr;
+    hipLaunchKernelGGL(b16_query_kernel, dim3(static_cast<uint32_t>(qa.rows)), dim3(kWave), 0, st, qa);
+    PrefilterB16Args p{};
+    p.tiles = s->tiles;
+    p.G = s->G;
+    p.planes = qa.planes;
+    p.nq = nq;
+    p.rows = qa.rows;
+    p.slots = qa.slots;
+    p.term = s->pf_term;
+    p.is_l2 = qa.is_l2;
+    p.tau = tau;
+    if (res_term != nullptr) {
+        p.res_term = res_term;
+        p.res_bias = s->residual_bias_dev;
+        p.magnitude = qa.magnitude;
+        p.ymax_bits = s->pf_ymax;
+        p.res_cmax = s->residual_cmax;
+    }
+    p.ids = s->ids_dev;
+    p.list_tile = s->list_tile_dev;
+    p.pair_off = pair_off;
+    p.item_off = item_off;
+    p.sorted_pair = sorted_pair;
+    p.nlist = s->nlist;
+    p.nprobe = nprobe;
+    p.k = kcand;
+    p.partial = partial;
+    p.partial_cnt = partial_cnt;
+    p.gate = gate;
+    const uint64_t pairs = nq * (nprobe - p0);
+    const uint64_t max_items =
+        (div_up(pairs, static_cast<uint64_t>(kB16N)) + std::min<uint64_t>(s->nlist, pairs)) * kIvfB16Chunks;
+    timing_begin(st);
+    hipLaunchKernelGGL((prefilter_b16_kernel<VSAG_AMD_KIND_FP32, true, 4, 2, 2>), dim3(static_cast<uint32_t>(max_items)),
+                       dim3(256), 0, st, p);
+    timing_end(st);
+    VA_HIP(hipGetLastError());
+    return 0;
+}
+
+}  // namespace vsag_amd

@@ -1,22 +1,12 @@
 // Flat scan with fused per-query top-k (BruteForce::SearchWithRequest hot loop,
 // src/algorithm/bruteforce/bruteforce.cpp:481-597; FlattenDataCell::query,
-// src/datacell/flatten_datacell.h:334-440), batched over queries.
-//
-// Work decomposition.  Grid x = query tile (T queries), y = chunk of code tiles.  A workgroup has up to
-// four waves; wave w walks tiles chunk_begin + w, + W, ... with the next granule group already in flight,
-// and keeps one LDS selector per query of the tile.  Workgroups that are resident together have
-// consecutive x and the same y, so they stream the same chunk of codes at about the same time.
-//
-// Selection.  Every (wave, query) has a selector in LDS (topk.h).  Chunks and waves of one query share a
-// per-query bound in global memory (the k-th best distance any of them has proven so far), so later
-// work drops almost everything with one compare.  Each (chunk, wave) leaves a short counted list of the
-// survivors that the bound still admits; a merge kernel picks the k best per query.  All waves of a query
-// share a handful of addresses (its bound, its seed row), and atomics on one address serialise in L2, so
-// every atomicMin is preceded by a plain load and issued only when it would lower the value.
+// src/datacell/flatten_datacell.h:334-440), batched over queries: the plan of a call, the merge of the partial lists,
+// and the routes around the streaming kernel (scan_flat.hip).
 #include <atomic>
 #include <mutex>
 
 #include "distance.h"
+#include "scan_flat.h"
 #include "store.h"
 #include "topk.h"
 
@@ -67,217 +57,6 @@ reset_queries_kernel(uint32_t* bound, uint32_t bound0, uint64_t nq, uint32_t* se
     }
     if (i < nseed) {
         seed[i] = 0xFFFFFFFFU;
-    }
-}
-
-struct FlatArgs {
-    uint64_t n;
-    uint64_t tile0;         // the launch covers tiles [tile0, tile_end)
-    uint64_t tile_end;
-    uint64_t tiles_per_chunk;
-    uint64_t nq;
-    uint32_t k;
-    uint32_t S;
-    uint32_t nslots;        // partial lists per query (all launches of the call)
-    uint32_t slot0;         // first list of this launch
-    const uint32_t* gate;   // per query: 0 = this launch leaves the query alone; null = every query
-    uint32_t* bound;        // per query: ordered distance that k candidates are known to reach
-    uint64_t* partial;      // nq x nslots x k keys
-    uint32_t* partial_cnt;  // nq x nslots
-    uint32_t* seed;         // nq x k smallest first-tile distances by wave class, or null (see kSeedTiles)
-    const uint32_t* deny;   // filtered-out inner ids as a bit mask, or null
-};
-
-// Cold start.  A wave that begins without a bound would have to sort its first tiles just to learn a
-// threshold.  Instead every such wave publishes the smallest distance of its first tile into slot
-// (global wave index mod k) of its query's seed row; waves own disjoint codes, so once all k slots are
-// filled their maximum is a distance that k different codes reach -- a valid bound, usually far tighter
-// than anything one wave could find alone.  A cold wave re-reads the row after each of its first
-// kSeedTiles tiles; the host enables seeding only when there are at least 2k waves per query.
-constexpr uint32_t kSeedTiles = 6;
-
-template <int KIND, int METRIC, int T, bool SEED>
-__global__ void __launch_bounds__(256)
-flat_scan_kernel(ScanArgs a, FlatArgs f) {
-    extern __shared__ uint64_t lds[];
-    const uint32_t lane = threadIdx.x & 63;
-    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const uint32_t nwaves = blockDim.x >> 6;
-    const uint32_t S = f.S, k = f.k;
-    uint64_t* sel = lds + static_cast<size_t>(wave) * T * S;
-
-    uint32_t qidx[T];
-    uint32_t thr[T];   // a candidate passes when its ordered distance is below thr
-    uint32_t cnt[T];
-    uint32_t cold[T];  // tiles after which this wave still looks at the seed row
-    bool live[T];      // a real query that this launch serves
-    bool any_live = false;
-#pragma unroll
-    for (int t = 0; t < T; ++t) {
-        qidx[t] = blockIdx.x * T + t;
-        cnt[t] = 0;
-        live[t] = qidx[t] < f.nq && (f.gate == nullptr || as_const(f.gate)[qidx[t]] != 0);
-        any_live = any_live || live[t];
-        uint32_t bs = live[t] ? __builtin_amdgcn_readfirstlane(__atomic_load_n(&f.bound[qidx[t]], __ATOMIC_RELAXED))
-                              : 0xFFFFFFFFU;
-        thr[t] = !live[t] ? 0U : bs == 0xFFFFFFFFU ? bs : bs + 1;
-        cold[t] = SEED && live[t] && bs == 0xFFFFFFFFU ? kSeedTiles : 0;
-    }
-    if (!any_live) {
-        return;
-    }
-    for (uint32_t i = lane; i < T * S; i += kWave) {
-        sel[i] = kInfKey;
-    }
-    wave_lds_fence();
-    const uint32_t seed_slot = (blockIdx.y * nwaves + wave) % k;
-
-    const uint64_t tile_begin = f.tile0 + static_cast<uint64_t>(blockIdx.y) * f.tiles_per_chunk;
-    uint64_t tile_end = tile_begin + f.tiles_per_chunk;
-    if (tile_end > f.tile_end) {
-        tile_end = f.tile_end;
-    }
-    // Software pipeline over granule groups: the loads of group g+1 (possibly of the next tile) are
-    // issued before group g is consumed, so every wave keeps GROUP KiB in flight.  Two register buffers
-    // alternate; the loop body is written out twice so that both are addressed statically.
-    const QueryRows<T> qrows = query_rows<T>(a, qidx);
-    constexpr int GROUP = GroupOf<T>::value;
-    // RaBitQ codes have G = dim / 128 granules, often no multiple of the group (768 dimensions: 6).
-    constexpr bool OVERLAP = KIND == VSAG_AMD_KIND_RABITQ || KIND == kKindRabitqF32;
-    TileStream<GROUP, OVERLAP> cur{a.tiles, lane, tile_begin + wave, tile_end, nwaves, 0, a.G};
-    TileStream<GROUP, OVERLAP> nxt = cur;
-    uint4 buf_a[GROUP], buf_b[GROUP];
-    if (cur.valid()) {
-        cur.load(buf_a, cur.tile);
-    }
-    Acc<KIND, T> acc;
-    acc_reset(acc);
-
-    const uint32_t pend = selector_base(S, k);  // where a selector's pending keys start
-    // Sorts selector t and folds its k-th key and the shared bound into thr[t].
-    auto flush = [&](int t) __attribute__((always_inline)) {
-        uint64_t* keys = sel + t * S;
-        uint64_t th = selector_flush(keys, S, k, cnt[t], lane);
-        cnt[t] = 0;
-        cold[t] = 0;
-        uint32_t tl = static_cast<uint32_t>(th >> 32);  // 0xFFFFFFFF while fewer than k seen
-        uint32_t bs = 0xFFFFFFFFU;
-        if (live[t]) {
-            bs = lower_shared(&f.bound[qidx[t]], tl, lane);  // tl = 0xFFFFFFFF lowers nothing
-        }
-        uint32_t tb = bs == 0xFFFFFFFFU ? bs : bs + 1;
-        thr[t] = tl < tb ? tl : tb;
-    };
-
-    // What a cold wave reads of its queries' seed rows (largest entry over this lane's share): fetched when a tile
-    // begins, looked at when its distances are done, so that the read waits under the tile's arithmetic.
-    uint32_t seed_seen[T];
-    auto consume = [&](const uint4(&regs)[GROUP]) __attribute__((always_inline)) {
-        const uint32_t first = cur.first();
-        if (SEED && cur.j0 == 0) {
-#pragma unroll
-            for (int t = 0; t < T; ++t) {
-                seed_seen[t] = 0;
-                if (cold[t] != 0) {
-                    const uint32_t* row = f.seed + static_cast<uint64_t>(qidx[t]) * k;
-                    for (uint32_t i = lane; i < k; i += kWave) {
-                        const uint32_t v = __atomic_load_n(&row[i], __ATOMIC_RELAXED);
-                        seed_seen[t] = v > seed_seen[t] ? v : seed_seen[t];
-                    }
-                }
-            }
-        }
-#pragma unroll
-        for (int u = 0; u < GROUP; ++u) {
-            const uint32_t g = first + u;
-            if (g >= cur.j0 && g < a.G) {
-                accumulate_granule<KIND, METRIC, T>(a, qrows, g, regs[u], acc);
-            }
-        }
-        if (cur.j0 + GROUP < a.G) {
-            return;
-        }
-        const uint64_t id = cur.tile * kWave + lane;
-        float d[T];
-        finish_distances<KIND, METRIC, T>(a, qidx, id, acc, d);
-        acc_reset(acc);
-        const bool valid = id < f.n && !denied(f.deny, id);
-#pragma unroll
-        for (int t = 0; t < T; ++t) {
-            // Inner ids grow along the scan, so "ordered distance < thr" is exactly the (distance, id)
-            // order against the wave's own k-th key, and "<= bound" against the shared bound.
-            uint32_t od = float_to_ordered(d[t]);
-            if (SEED && cold[t] != 0) {
-                uint32_t* row = f.seed + static_cast<uint64_t>(qidx[t]) * k;
-                if (cold[t] == kSeedTiles) {
-                    // This wave's entry (its own first look at the row came before it, the next one will see it).
-                    uint32_t m = wave_min_u32(valid ? od : 0xFFFFFFFFU);
-                    lower_shared(&row[seed_slot], m, lane);
-                }
-                --cold[t];
-                const uint32_t mx = wave_max_u32(seed_seen[t]);
-                if (mx != 0xFFFFFFFFU) {
-                    // Every slot filled: k different codes reach mx.
-                    cold[t] = 0;
-                    const uint32_t b = lower_shared(&f.bound[qidx[t]], mx, lane);
-                    thr[t] = b + 1 < thr[t] ? b + 1 : thr[t];
-                }
-            }
-            bool pass = valid && od < thr[t];
-            uint64_t mask = __ballot(pass);
-            if (mask != 0) {
-                uint32_t np = __popcll(mask);
-                if (pend + cnt[t] + np > S) {
-                    flush(t);
-                }
-                if (pass) {
-                    sel[t * S + pend + cnt[t] + mask_rank(mask)] = (static_cast<uint64_t>(od) << 32) | static_cast<uint32_t>(id);
-                }
-                cnt[t] += np;
-            }
-        }
-    };
-
-    while (cur.valid()) {
-        nxt.advance();
-        nxt.load(buf_b, cur.tile);
-        consume(buf_a);
-        cur = nxt;
-        if (!cur.valid()) {
-            break;
-        }
-        nxt.advance();
-        nxt.load(buf_a, cur.tile);
-        consume(buf_b);
-        cur = nxt;
-    }
-
-    const uint32_t slot = f.slot0 + blockIdx.y * nwaves + wave;
-#pragma unroll
-    for (int t = 0; t < T; ++t) {
-        if (!live[t]) {
-            continue;
-        }
-        // Whatever lies above the shared bound is beaten by k candidates of other waves.  What remains is
-        // usually less than k keys, which go out as they are; only a wave left with more sorts once more.
-        uint64_t* keys = sel + t * S;
-        wave_lds_fence();
-        uint32_t bs = __builtin_amdgcn_readfirstlane(__atomic_load_n(&f.bound[qidx[t]], __ATOMIC_RELAXED));
-        uint32_t total = pend + cnt[t];
-        uint32_t admitted = selector_count_admitted(keys, total, bs, lane);
-        if (admitted > k) {
-            uint64_t th = selector_flush(keys, S, k, cnt[t], lane);
-            bs = lower_shared(&f.bound[qidx[t]], static_cast<uint32_t>(th >> 32), lane);
-            total = k;
-            admitted = selector_count_admitted(keys, total, bs, lane);
-        }
-        const uint64_t list = static_cast<uint64_t>(qidx[t]) * f.nslots + slot;
-        if (lane == 0) {
-            f.partial_cnt[list] = admitted;
-        }
-        if (admitted != 0) {
-            selector_copy_admitted(keys, total, bs, f.partial + list * k, lane);
-        }
     }
 }
 
@@ -807,6 +586,10 @@ struct CallPlan {
     uint64_t level_begin[kMaxLevels + 1] = {};
     bool int8 = false;         // the int8 matrix cores pre-select (sq8, at most 128 dimensions)
     bool rb = false;           // RaBitQ store: 1-bit codes x 4-bit queries on the int8 matrix cores
+    // fp32 stores, and sq8 / sq4 ones under a deny mask: the bf16 matrix cores, which need neither a prefix nor levels
+    // (prefilter_b16.hip); the streaming launch behind covers all tiles.
+    bool b16 = false;
+    size_t b16_scratch = 0;
     size_t h16_scratch = 0;    // sq8 beyond 128 dimensions: bytes of the fp16 query planes (0: the fp32 matrix cores)
     uint32_t cap = 0;          // candidates per query and level
     uint32_t sub_lists[kMaxLevels] = {};  // int8: private candidate lists per query ...
@@ -850,6 +633,12 @@ bool prefilter_rb_supports(const vsag_amd_store* s);
 size_t prefilter_rb_scratch_bytes(const vsag_amd_store* s, uint64_t nq);
 bool prefilter_h16_supports(const vsag_amd_store* s);
 size_t prefilter_h16_scratch_bytes(const vsag_amd_store* s, uint64_t nq);
+bool prefilter_b16_supports(const vsag_amd_store* s);
+size_t prefilter_b16_scratch_bytes(const vsag_amd_store* s, uint64_t nq, uint32_t k);
+uint32_t prefilter_b16_cap(uint32_t k);
+int launch_scan_b16(const vsag_amd_store* s, const ScanArgs& a, uint64_t nq, uint32_t k, uint32_t S, uint32_t* bound,
+                    uint8_t* scratch, uint64_t* cand, uint32_t* cand_cnt, uint32_t cap, const uint32_t* deny,
+                    uint64_t* partial, uint32_t* partial_cnt, uint32_t nslots, uint32_t* gate, hipStream_t st);
 uint32_t prefilter_rb_sub_lists(uint64_t nq, uint64_t span);
 
 // Whether a call goes through the table of approximate distances (see CallPlan::table).
@@ -865,13 +654,14 @@ small_store_table(const vsag_amd_store* s, uint64_t nq, uint32_t k) {
 // no room in the workspace.
 constexpr uint64_t kListsOptionalBelow = 512;
 
+// masked: the call has a deny mask.
 static void
-make_call_plan(const vsag_amd_store* s, uint64_t nq, uint32_t k, CallPlan* c) {
+make_call_plan(const vsag_amd_store* s, uint64_t nq, uint32_t k, bool masked, CallPlan* c) {
     make_plan(s, nq, k, s->ntiles, &c->all);
     c->nslots = static_cast<uint32_t>(c->all.chunks * c->all.waves);
     c->any_seeded = c->all.seeded;
     c->contraction = false;
-    c->table = small_store_table(s, nq, k);
+    c->table = !masked && small_store_table(s, nq, k);
     c->table_ld = c->table ? round_up(s->ntiles * kWave, 64) : 0;
     if (c->table) {
         return;
@@ -888,6 +678,20 @@ make_call_plan(const vsag_amd_store* s, uint64_t nq, uint32_t k, CallPlan* c) {
     // (The tuning knobs are the streaming kernel's: a batch that either route could serve streams where one is set.)
     const bool tuned = nq < kListsOptionalBelow && (tile_override(s) > 0 || chunk_override(s) > 0);
     if (!forced && (tuned || k > (rb ? 256U : 128U) || s->ntiles < 1024 || !prefilter_pays(s, nq, k))) {
+        return;
+    }
+    if (prefilter_mode(s) != 2 && prefilter_b16_supports(s) && (s->kind == VSAG_AMD_KIND_FP32 || masked)) {
+        const uint64_t cap = prefilter_b16_cap(k);
+        if (nq * cap * 8 > (2ull << 30) || s->ntiles == 0) {
+            return;
+        }
+        c->contraction = c->b16 = true;
+        c->cap = static_cast<uint32_t>(cap);
+        c->b16_scratch = prefilter_b16_scratch_bytes(s, nq, k);
+        c->nslots += 1;
+        return;
+    }
+    if (masked) {
         return;
     }
     // Candidate buffers: at most 2 GiB in all, 1024 to 4096 candidates per query (RaBitQ stores are searched with
@@ -985,11 +789,11 @@ make_call_plan(const vsag_amd_store* s, uint64_t nq, uint32_t k, CallPlan* c) {
 
 static bool
 drop_candidate_lists(const vsag_amd_store* s, uint64_t nq, CallPlan* c) {
-    if (!c->contraction || nq >= kListsOptionalBelow || prefilter_mode(s) != 0) {
+    if (!c->contraction || (nq >= kListsOptionalBelow && !c->b16) || prefilter_mode(s) != 0) {
         return false;
     }
-    c->contraction = c->int8 = c->rb = false;
-    c->h16_scratch = 0;
+    c->contraction = c->int8 = c->rb = c->b16 = false;
+    c->h16_scratch = c->b16_scratch = 0;
     c->nslots = static_cast<uint32_t>(c->all.chunks * c->all.waves);
     c->any_seeded = c->all.seeded;
     return true;
@@ -1033,102 +837,21 @@ carve_scan(Carver& c, const CallPlan& cp, uint64_t nq, uint32_t k, ScanBuffers* 
     }
     b->partial = c.take<uint64_t>(nq * cp.nslots * k);
     const uint64_t nq_pad8 = prefilter_i8_query_bytes(nq) / 256;  // whole workgroups of the int8 prefilter
-    b->tau = c.take<float>(cp.contraction ? nq_pad8 : 0);
+    b->tau = c.take<float>(cp.contraction && !cp.b16 ? nq_pad8 : 0);
     b->q8_u = c.take<float>(cp.int8 ? prefilter_i8_scalar_floats(nq) : 0);
-    b->q8 = c.take<uint8_t>(cp.int8 ? prefilter_i8_query_bytes(nq) : (cp.rb ? cp.rb_scratch : cp.h16_scratch));
-    if (!cp.int8 && !cp.rb && cp.h16_scratch == 0) {
+    b->q8 = c.take<uint8_t>(cp.int8 ? prefilter_i8_query_bytes(nq) : cp.rb ? cp.rb_scratch : cp.b16 ? cp.b16_scratch : cp.h16_scratch);
+    if (!cp.int8 && !cp.rb && !cp.b16 && cp.h16_scratch == 0) {
         b->q8 = nullptr;
     }
     b->cand_cnt = c.take<uint32_t>(cp.contraction ? nq * std::max<uint32_t>(1, cp.max_lists) : 0);
     b->gate = c.take<uint32_t>(cp.contraction ? nq : 0);
-    b->cand = c.take<uint32_t>(cp.contraction ? nq * cp.cap : 0);
+    b->cand = c.take<uint32_t>(cp.contraction ? nq * cp.cap * (cp.b16 ? 2 : 1) : 0);
     b->table = c.take<float>(cp.table ? nq * cp.table_ld : 0);
     b->table_rows = c.take<float>(cp.table ? cp.table_ld * p.ql.qstride : 0);
     b->table_norms = c.take<float>(cp.table ? cp.table_ld + 64 : 0);
     b->one_mins = c.take<uint64_t>(cp.one ? cp.one_runs : 0);
     b->one_dist = c.take<uint32_t>(cp.one ? cp.one_tiles * kWave : 0);
     return c.used;
-}
-
-template <int KIND, int METRIC, int T>
-static void
-launch_flat_s(dim3 grid, dim3 block, size_t lds, hipStream_t st, const ScanArgs& a, const FlatArgs& f) {
-    if (f.seed != nullptr) {
-        hipLaunchKernelGGL((flat_scan_kernel<KIND, METRIC, T, true>), grid, block, lds, st, a, f);
-    } else {
-        hipLaunchKernelGGL((flat_scan_kernel<KIND, METRIC, T, false>), grid, block, lds, st, a, f);
-    }
-}
-
-template <int KIND, int METRIC>
-static void
-launch_flat_t(int T, dim3 grid, dim3 block, size_t lds, hipStream_t st, const ScanArgs& a, const FlatArgs& f) {
-    switch (T) {
-        case 1:
-            launch_flat_s<KIND, METRIC, 1>(grid, block, lds, st, a, f);
-            break;
-        case 2:
-            launch_flat_s<KIND, METRIC, 2>(grid, block, lds, st, a, f);
-            break;
-        case 4:
-            launch_flat_s<KIND, METRIC, 4>(grid, block, lds, st, a, f);
-            break;
-        default:
-            launch_flat_s<KIND, METRIC, 8>(grid, block, lds, st, a, f);
-            break;
-    }
-}
-
-template <int KIND>
-static void
-launch_flat_m(int metric, int T, dim3 grid, dim3 block, size_t lds, hipStream_t st, const ScanArgs& a,
-              const FlatArgs& f) {
-    // Cosine stores hold normalised vectors and scan as inner product (RaBitQ has its own formula).
-    if (metric == VSAG_AMD_METRIC_L2) {
-        launch_flat_t<KIND, VSAG_AMD_METRIC_L2>(T, grid, block, lds, st, a, f);
-    } else if (metric == VSAG_AMD_METRIC_COSINE && (KIND == VSAG_AMD_KIND_RABITQ || KIND == kKindRabitqF32)) {
-        launch_flat_t<KIND, VSAG_AMD_METRIC_COSINE>(T, grid, block, lds, st, a, f);
-    } else {
-        launch_flat_t<KIND, VSAG_AMD_METRIC_IP>(T, grid, block, lds, st, a, f);
-    }
-}
-
-static int
-launch_flat(const vsag_amd_store* s, const ScanPlan& p, const ScanArgs& a, const FlatArgs& f, hipStream_t st) {
-    dim3 grid(static_cast<uint32_t>(p.groups), static_cast<uint32_t>(p.chunks));
-    dim3 block(p.waves * kWave);
-    size_t lds = p.lds_bytes;
-    switch (s->kind) {
-        case VSAG_AMD_KIND_FP32:
-            launch_flat_m<VSAG_AMD_KIND_FP32>(s->metric, p.T, grid, block, lds, st, a, f);
-            break;
-        case VSAG_AMD_KIND_SQ8:
-            launch_flat_m<VSAG_AMD_KIND_SQ8>(s->metric, p.T, grid, block, lds, st, a, f);
-            break;
-        case VSAG_AMD_KIND_SQ4:
-            launch_flat_m<VSAG_AMD_KIND_SQ4>(s->metric, p.T, grid, block, lds, st, a, f);
-            break;
-        case VSAG_AMD_KIND_SQ4_UNIFORM:
-            launch_flat_m<VSAG_AMD_KIND_SQ4_UNIFORM>(s->metric, p.T, grid, block, lds, st, a, f);
-            break;
-        case VSAG_AMD_KIND_SQ8_UNIFORM:
-            launch_flat_m<VSAG_AMD_KIND_SQ8_UNIFORM>(s->metric, p.T, grid, block, lds, st, a, f);
-            break;
-        case VSAG_AMD_KIND_PQFS:
-            launch_flat_m<VSAG_AMD_KIND_PQFS>(s->metric, p.T, grid, block, lds, st, a, f);
-            break;
-        case VSAG_AMD_KIND_RABITQ:
-            if (s->query_bits == 32) {
-                launch_flat_m<kKindRabitqF32>(s->metric, p.T, grid, block, lds, st, a, f);
-            } else {
-                launch_flat_m<VSAG_AMD_KIND_RABITQ>(s->metric, p.T, grid, block, lds, st, a, f);
-            }
-            break;
-        default:
-            return fail(VSAG_AMD_INVALID_ARGUMENT, "unknown store kind %d", s->kind);
-    }
-    VA_HIP(hipGetLastError());
-    return 0;
 }
 
 // ---- many queries against a small fp32 store: selection from a table of approximate distances ------------------
@@ -1402,6 +1125,16 @@ launch_table_select(uint64_t codes, dim3 grid, hipStream_t st, const ScanArgs& a
     }
 }
 
+// Workspace of a call, with or without a deny mask.
+static size_t
+plan_bytes(const vsag_amd_store* s, uint64_t nq, uint32_t k, bool masked) {
+    CallPlan cp;
+    make_call_plan(s, nq, k, masked, &cp);
+    Carver c(nullptr, 0);
+    ScanBuffers b;
+    return carve_scan(c, cp, nq, k, &b) + 256;
+}
+
 static int
 check_scan_call(const vsag_amd_store* s, uint64_t nq, uint32_t k) {
     VA_CHECK_ARG(s != nullptr, "store is null");
@@ -1420,11 +1153,7 @@ vsag_amd_flat_scan_workspace_bytes(const vsag_amd_store_t* s, uint64_t nq, uint3
     if (check_scan_call(s, nq, k) != 0 || ensure_init() != 0) {
         return 0;
     }
-    CallPlan cp;
-    make_call_plan(s, nq, k, &cp);
-    Carver c(nullptr, 0);
-    ScanBuffers b;
-    return carve_scan(c, cp, nq, k, &b) + 256;
+    return std::max(plan_bytes(s, nq, k, false), plan_bytes(s, nq, k, true));
 }
 
 extern "C" int
@@ -1462,7 +1191,8 @@ run_streaming(const vsag_amd_store* s, const ScanPlan& p, const ScanArgs& a, con
     f.partial_cnt = b.partial_cnt;
     f.seed = p.seeded ? b.seed : nullptr;
     f.deny = options != nullptr ? options->deny_bits_dev : nullptr;
-    return launch_flat(s, p, a, f, st);
+    return launch_flat(s, p.T, dim3(static_cast<uint32_t>(p.groups), static_cast<uint32_t>(p.chunks)), dim3(p.waves * kWave),
+                       p.lds_bytes, a, f, st);
 }
 
 }  // namespace
@@ -1486,8 +1216,11 @@ flat_scan_call(const vsag_amd_store_t* s, const float* queries_dev, uint64_t nq,
     VA_CHECK_ARG(s->nlist == 0, "flat scan on a posting-list store");
     VA_CHECK_ARG(queries_dev && ids_dev && dists_dev, "null query / output pointer");
     hipStream_t st = static_cast<hipStream_t>(stream);
+    // A radius goes the streaming way (no pre-selection knows it), a pre-filter to the one that does.
+    const bool masked = options != nullptr && options->deny_bits_dev != nullptr;
+    const bool ranged = options != nullptr && options->use_radius != 0;
     CallPlan cp;
-    make_call_plan(s, nq, k, &cp);
+    make_call_plan(s, nq, k, masked, &cp);
     Carver c(workspace_dev, workspace_bytes);
     ScanBuffers b;
     carve_scan(c, cp, nq, k, &b);
@@ -1504,9 +1237,8 @@ flat_scan_call(const vsag_amd_store_t* s, const float* queries_dev, uint64_t nq,
         carve_scan(c, cp, nq, k, &b);
     }
     VA_CHECK_ARG(c.ok(), "workspace too small: need %zu bytes, got %zu", c.used, workspace_bytes);
-    // A pre-filter or a radius goes the streaming way (the prefilter knows neither).
-    const bool plain = options == nullptr || (options->deny_bits_dev == nullptr && options->use_radius == 0);
-    const bool contraction = cp.contraction && plain;
+    const bool plain = !masked && !ranged;
+    const bool contraction = cp.contraction && !ranged;
     const ScanPlan& p = cp.all;
 
     VA_TRY(prepare_queries(s, queries_dev, nq, p.nq_pad, p.ql, b.qtab, b.qmeta, b.qcodes, st));
@@ -1558,6 +1290,14 @@ flat_scan_call(const vsag_amd_store_t* s, const float* queries_dev, uint64_t nq,
         timing_end(st);
         tl_last_tile = p.T;
         tl_last_passes = p.groups;
+    } else if (cp.b16) {
+        nslots = 1 + static_cast<uint32_t>(p.chunks * p.waves);
+        VA_TRY(launch_scan_b16(s, a, nq, k, p.S, b.bound, b.q8, reinterpret_cast<uint64_t*>(b.cand), b.cand_cnt, cp.cap,
+                               masked ? options->deny_bits_dev : nullptr, b.partial, b.partial_cnt, nslots, b.gate, st));
+        // the queries whose records found no room
+        VA_TRY(run_streaming(s, p, a, b, nq, k, options, 0, s->ntiles, 1, nslots, b.gate, st));
+        tl_last_tile = 128;  // queries per pass
+        tl_last_passes = div_up(nq, 128);
     } else {
         const uint32_t slots_prefix = static_cast<uint32_t>(cp.prefix.chunks * cp.prefix.waves);
         const uint32_t slots_rest = static_cast<uint32_t>(cp.rest.chunks * cp.rest.waves);
@@ -1597,7 +1337,7 @@ flat_scan_call(const vsag_amd_store_t* s, const float* queries_dev, uint64_t nq,
     }
     VA_TRY(launch_merge_partials(b.partial, b.partial_cnt, b.bound, nslots, nslots, k, p.S, nq, ids_dev, dists_dev, st));
     // Code bytes under the timed kernel: the whole store, or the last (by far the largest) level of the contraction.
-    const uint64_t timed_tiles = contraction ? s->ntiles - cp.level_begin[cp.levels - 1] : s->ntiles;
+    const uint64_t timed_tiles = contraction && !cp.b16 ? s->ntiles - cp.level_begin[cp.levels - 1] : s->ntiles;
     tl_last_bytes = timed_tiles * s->G * kWave * kGranule;
     return 0;
 }
@@ -1658,10 +1398,11 @@ vsag_amd_flat_scan_topk_noalloc(const vsag_amd_store_t* s, const float* queries_
         VA_TRY(static_scratch_setup(device));
     }
     void* const scratch_dev = g_scratch_ptr[device].load(std::memory_order_acquire);
-    size_t need = vsag_amd_flat_scan_workspace_bytes(s, nq, k);
+    const bool masked = options != nullptr && options->deny_bits_dev != nullptr;
+    size_t need = plan_bytes(s, nq, k, masked);
     if (need > kStaticScratchBytes) {
         CallPlan cp;
-        make_call_plan(s, nq, k, &cp);
+        make_call_plan(s, nq, k, masked, &cp);
         if (drop_candidate_lists(s, nq, &cp)) {
             Carver c(nullptr, 0);
             ScanBuffers b;
