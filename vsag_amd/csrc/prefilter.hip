@@ -17,6 +17,7 @@
 // (no bound yet, masses of equal distances) is flagged and served by the streaming kernel over the remaining
 // tiles instead.
 #include "distance.h"
+#include "kth_value.h"
 #include "store.h"
 #include "topk.h"
 
@@ -403,8 +404,8 @@ struct RescoreArgs {
     uint32_t sub_lists, sub_cap, gather;
     const uint4* rows;  // the codes a row per code (store.h), or null: read the tiles
     uint32_t row_granules;  // granules of a row: G, or G + 1 with the code's metadata words behind the code
-    // VALUED: records of the approximate distance's ordered bits above the slot, cap a query, and per query twice what the
-    // approximation can be off by.
+    // VALUED: records of the approximate distance's ordered bits above the slot, cap a query (their counts 32 words apart),
+    // and per query twice what the approximation can be off by.
     const uint64_t* valued;
     const float* slack;
 };
@@ -428,7 +429,7 @@ rescore_kernel(ScanArgs a, RescoreArgs r) {
     const uint32_t q = blockIdx.x;
     const uint64_t list = static_cast<uint64_t>(q) * r.nslots + r.out_slot;
     bool overflow = false;
-    const uint32_t* counts = r.cand_cnt + static_cast<uint64_t>(q) * (r.sub_lists != 0 ? r.sub_lists : 1);
+    const uint32_t* counts = r.cand_cnt + static_cast<uint64_t>(q) * (VALUED ? 32 : r.sub_lists != 0 ? r.sub_lists : 1);
     if (r.sub_lists == 0) {
         overflow = as_const(counts)[0] > r.cap;
     } else {
@@ -535,7 +536,7 @@ rescore_kernel(ScanArgs a, RescoreArgs r) {
         uint32_t waiting = 0;
         for (uint32_t base = 0; base < total; base += kWave) {
             const uint64_t key = base + lane < total ? valued[base + lane] : kInfKey;
-            const bool take = base + lane < total && ordered_to_float(static_cast<uint32_t>(key >> 32)) <= limit;
+            const bool take = base + lane < total && !(ordered_to_float(static_cast<uint32_t>(key >> 32)) > limit);
             const uint64_t mask = __ballot(take);
             if (take) {
                 pick[waiting + mask_rank(mask)] = static_cast<uint32_t>(key);

@@ -12,27 +12,28 @@
 // fp32: no operand needs a scale, and what is below the normal range may be taken as zero.
 //
 // A flat scan (launch_scan_b16) needs no exact distance before the end:
-//   1. a sample of the code tiles, spread over the store, leaves the least v of every 64 (32) codes; k of those lie at or
+//   1. a sample of the code tiles, spread over the store, leaves the least v of every 64 codes; k of those lie at or
 //      below the k-th smallest, m;
 //   2. whoever is among the k best has v <= m + 2 e: the pass over all codes records (v, slot) of those, a few hundred a
 //      query (b16_tau_kernel says how many are expected);
 //   3. of the records only those within 2 e of their own k-th smallest are rescored with the streaming kernel's arithmetic
 //      (rescore_kernel): k and a handful, and the result is the streaming result, bit for bit.
-// A query with more records than there is room for is gated and streams.  A deny mask takes part in 1 and 2 as an infinite
-// |y|^2.  100k x 128 fp32, 1000 queries, k 10 (fp32 matrix cores, an exact prefix and levels before: 460 us): 209 us.
+// A query with more records than there is room for is gated and streams.  A deny mask takes part in 1 and 2 as a |y|^2
+// beyond every threshold.  100k x 128 fp32, 1000 queries, k 10 (fp32 matrix cores, an exact prefix and levels before: 460 us): 209 us.
 // 100k x 768 fp32, 32 queries (streamed before: 684 us on the device): MEASURED_B.  500k x 100 sq8 under a deny mask, 200
 // queries, k 100 (streamed before: 664 us): 209 us.
 //
 // What bounds it: with 128 queries per workgroup the matrix cores beside the splitting of the codes and the verdicts; with
 // few queries the bytes of the codes, each read once per 32, 64 or 128 queries.
 //
-// Work split: a workgroup of four waves takes 256 codes (four storage tiles) and 128, 64 or 32 queries (kernel
-// parameters IB, JB, WN: a wave has IB x JB blocks of 32 x 32, WN waves stand side by side along the queries) in
-// stages of 32 dimensions (sq8, sq4: 64).  A stage sits in LDS as 16-byte slots of eight bf16 values [eight
-// dimensions][part][row], the operand order of the instruction (lane % 32 = row, lane / 32 = which eight of sixteen
-// dimensions).  The codes are split while they are parked in LDS (a thread owns a code), the queries once per call into a
-// table in slot order.
+// Work split: a workgroup of four waves takes 256 codes, a storage tile a wave, and 128, 64 or 32 queries (JB blocks of
+// 32), so a code is read by one wave alone and goes from memory into the registers of the lanes that multiply it (lane %
+// 32 = code, lane / 32 = which eight of sixteen dimensions): a load instruction covers two runs of 512 bytes.  It is split
+// there, a stage of 32 dimensions (sq8, sq4: 64) at a time, while the loads of the next stage are under way.  The queries
+// are split once per call into a table of 16-byte slots [eight dimensions][part][row]; a workgroup stages them in LDS
+// twice 16 KB at a time (sq8, sq4 with 128 queries: 32), one barrier each.
 #include "distance.h"
+#include "kth_value.h"
 #include "store.h"
 #include "topk.h"
 
@@ -46,16 +47,17 @@ typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef float floatx2 __attribute__((ext_vector_type(2)));
 typedef float floatx16 __attribute__((ext_vector_type(16)));
 
-constexpr uint32_t kB16M = 256;     // codes per workgroup tile (= threads of a workgroup)
 constexpr uint32_t kB16N = 128;     // most queries per workgroup tile; the rows of the query table are padded to it
 constexpr uint32_t kB16Pad = 64;    // the query table covers whole stages of either length
+constexpr float kB16Absent = 3.3e38F;  // |y|^2 of a slot that cannot be found: above every threshold (3e38 at most), and no
+                                       // infinity, which four other low bits would make a NaN that hides the fifteen others
+constexpr uint32_t kB16CountStride = 32;  // words between the queries' record counters: atomics on one memory line take turns
 constexpr uint32_t kB16Queue = 128; // records a wave gathers in LDS before it asks for room in the queries' lists
 
 template <int KIND>
 struct B16Layout {
     static constexpr bool kSplit = KIND == VSAG_AMD_KIND_FP32;           // the code has a low part too
     static constexpr uint32_t kSlots = kSplit ? 4 : 8;                   // eight dimensions each, per stage
-    static constexpr uint32_t kParts = kSplit ? 2 : 1;
     static constexpr uint32_t kGranules = KIND == VSAG_AMD_KIND_FP32 ? 8 : KIND == VSAG_AMD_KIND_SQ8 ? 4 : 2;  // per stage
 };
 
@@ -202,9 +204,9 @@ b16_query_kernel(B16QueryArgs p) {
     const double split = fp32 ? ymax * (sqrt(r2) + 3.9e-6 * an + 1.97e-3 * sqrt(l2)) : static_cast<double>(p.cmax) * r1;
     // The accumulation: four roundings of the absolute sum per instruction (two or three per sixteen dimensions).
     const double rounding = 4.0 * kU * ((fp32 ? 3.0 : 2.0) * kd / 16.0 + 4.0) * sums;
-    // Operands below the normal range taken as zero; fl(term + fl(factor acc)) of the test itself and |y|^2 rounded once.
+    // Operands below the normal range taken as zero; fma(factor, acc, term) and |y|^2 rounded, the low four bits cut off.
     const double flushed = kd * 4.7e-38 * (an + ymax + 1.0);
-    const double test = 6.0 * kU * ((p.is_l2 ? ymax * ymax : 0.0) + factor * dots);
+    const double test = 36.0 * kU * ((p.is_l2 ? ymax * ymax : 0.0) + factor * dots);
     double fixed = factor * (split + rounding) + flushed + test;
     double root = 0.0, slope = 0.0;
     double constant = a2;
@@ -271,9 +273,10 @@ b16_tau_kernel(B16TauArgs p) {
     if (lane != 0) {
         return;
     }
-    p.cand_cnt[q] = 0;
-    p.gate[q] = 0;
     const B16Error e = p.error[q];
+    // (a query whose sums can leave fp32, or with entries that are not finite, streams: more records than there is room for)
+    p.cand_cnt[q * kB16CountStride] = e.fixed < 1.0e37F ? 0U : 0x40000000U;
+    p.gate[q] = 0;
     // The k codes at or below kth have distances of at most D; so has whoever is among the k best.
     const float far = fmaxf(kth + e.constant, 0.0F) * 1.00001F + 2.0F * e.fixed;
     const float slack = 2.0F * e.fixed + 2.05F * (e.root * sqrtf(far) + e.slope * far);
@@ -324,27 +327,90 @@ struct PrefilterB16Args {
 constexpr uint32_t kIvfB16ChunkTiles = 32;  // as ivf_i8.hip: kIvfI8ChunkTiles, kIvfI8Chunks
 constexpr uint32_t kIvfB16Chunks = 4;
 
-template <int KIND, bool LISTS, int IB, int JB, int WN>
-__global__ void __launch_bounds__(256, IB * JB <= (KIND == VSAG_AMD_KIND_FP32 ? 4 : 2) ? 3 : 2)
+// The codes of one stage of a wave, in registers: of both blocks of 32 codes, the granules this lane multiplies.
+template <int KIND>
+struct B16Codes {
+    static constexpr int kLoads = B16Layout<KIND>::kGranules / 2;  // per block
+    uint4 g[2][kLoads];
+};
+
+// Granules past a code's end repeat its last one (the query's values there are zeros): no load stands behind a branch.
+template <int KIND>
+__device__ __forceinline__ void
+b16_fetch_codes(B16Codes<KIND>& c, const uint4* tile, uint32_t G, uint32_t st, uint32_t half, uint32_t l32) {
+    using L = B16Layout<KIND>;
+#pragma unroll
+    for (int u = 0; u < B16Codes<KIND>::kLoads; ++u) {
+        // fp32: the two granules of the eight dimensions that this half multiplies in step u / 2; sq8, sq4: one granule
+        // holds this half's dimensions of two (four) steps
+        uint32_t j = L::kGranules * st + (KIND == VSAG_AMD_KIND_FP32 ? 4 * (u / 2) + 2 * half + (u & 1) : 2 * u + half);
+        j = j < G ? j : G - 1;
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            c.g[i][u] = tile[j * kWave + 32 * i + l32];
+        }
+    }
+}
+
+// The operand of step ks: eight dimensions of the code of this lane.
+template <int KIND>
+__device__ __forceinline__ void
+b16_operand(const B16Codes<KIND>& c, int i, int ks, bf16x8* hi, bf16x8* lo) {
+    if constexpr (KIND == VSAG_AMD_KIND_FP32) {
+        const uint4 v = c.g[i][2 * ks], w = c.g[i][2 * ks + 1];
+        const float x[8] = {__uint_as_float(v.x), __uint_as_float(v.y), __uint_as_float(v.z), __uint_as_float(v.w),
+                            __uint_as_float(w.x), __uint_as_float(w.y), __uint_as_float(w.z), __uint_as_float(w.w)};
+        uint4 h, l;
+        b16_split8(x, &h, &l);
+        *hi = __builtin_bit_cast(bf16x8, h);
+        *lo = __builtin_bit_cast(bf16x8, l);
+    } else if constexpr (KIND == VSAG_AMD_KIND_SQ8) {
+        const uint4 v = c.g[i][ks / 2];
+        const uint32_t a = (ks & 1) != 0 ? v.z : v.x, b = (ks & 1) != 0 ? v.w : v.y;
+        *hi = __builtin_bit_cast(bf16x8, make_uint4(b16_two_bytes(a, 0), b16_two_bytes(a, 2), b16_two_bytes(b, 0),
+                                                    b16_two_bytes(b, 2)));
+    } else {
+        const uint4 v = c.g[i][0];
+        *hi = __builtin_bit_cast(bf16x8, b16_nibbles(ks == 0 ? v.x : ks == 1 ? v.y : ks == 2 ? v.z : v.w));
+    }
+}
+
+// The slot (eight dimensions) of the query table that lines up with a half's operand of step ks of stage st.
+template <int KIND>
+__device__ __forceinline__ uint32_t
+b16_slot(uint32_t ks, uint32_t half) {
+    if constexpr (KIND == VSAG_AMD_KIND_FP32) {
+        return 2 * ks + half;
+    } else if constexpr (KIND == VSAG_AMD_KIND_SQ8) {
+        return 4 * (ks >> 1) + 2 * half + (ks & 1);
+    } else {
+        return 4 * half + ks;
+    }
+}
+
+template <int KIND, bool LISTS, int JB>
+__global__ void __launch_bounds__(256, JB == 4 || (JB == 2 && KIND == VSAG_AMD_KIND_FP32) ? 2 : 3)
 prefilter_b16_kernel(PrefilterB16Args p) {
     using L = B16Layout<KIND>;
-    constexpr uint32_t N = WN * JB * 32;
-    static_assert((4 / WN) * IB * 32 == kB16M, "the waves cover the codes of a tile");
-    __shared__ uint4 sa[L::kSlots][L::kParts][kB16M];
-    __shared__ uint4 sb[L::kSlots][2][N];
-    __shared__ float code_term[kB16M];
+    constexpr uint32_t N = JB * 32;
+    constexpr uint32_t kSteps = L::kSlots / 2;
+    constexpr uint32_t kRound = JB * L::kSlots >= 16 ? 1 : 16 / (JB * L::kSlots);  // stages of codes per stage of queries
+    constexpr uint32_t kSlotsB = kRound * L::kSlots;       // slots of a stage of queries
+    constexpr uint32_t kQueryRegs = kSlotsB * 2 * N / 256;
+    constexpr uint32_t kRowStep = 256 / N;                 // (slot, part) pairs that one round of the workgroup covers
+    __shared__ uint4 sb[2][kSlotsB][2][N];
+    __shared__ float code_term[4][kWave];
     __shared__ uint64_t queue_key[4][kB16Queue];
     __shared__ uint32_t queue_col[4][kB16Queue];
     const uint32_t tid = threadIdx.x;
     const uint32_t lane = tid & 63;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const uint32_t wm = wave / WN, wn = wave % WN;
     const uint32_t half = lane >> 5;
     const uint32_t l32 = lane & 31;
     const uint32_t stages = (p.G + L::kGranules - 1) / L::kGranules;
 
     // What this workgroup walks: code tiles first, first + step, ... below mtiles (of four storage tiles from tile_begin
-    // on), against the query rows of its N columns.
+    // on, one a wave), against the query rows of its N columns.
     uint64_t tile_begin = 0, tile_end, first = 0, step = 1;
     uint64_t q0 = 0;
     uint32_t pbeg = 0, pend = 0, chunk = 0;
@@ -388,17 +454,20 @@ prefilter_b16_kernel(PrefilterB16Args p) {
         q0 = static_cast<uint64_t>(blockIdx.y) * N;
     }
     const uint64_t mtiles = (tile_end - tile_begin + 3) / 4;
+    if (first >= mtiles) {
+        return;  // the whole workgroup
+    }
 
-    // Verdict side: the columns l32 of this wave's JB blocks.
+    // Verdict side: the columns l32 of the JB blocks.
     float tau_n[JB];
 #pragma unroll
     for (int j = 0; j < JB; ++j) {
-        const uint32_t col = wn * JB * 32 + j * 32 + l32;
+        const uint32_t col = j * 32 + l32;
         if constexpr (LISTS) {
             const uint32_t at = pbeg + col;
             const uint32_t pair = at < pend ? as_const(p.sorted_pair)[at] : 0U;
             const uint32_t query = pair / p.nprobe;
-            tau_n[j] = at < pend ? p.tau[query] : -__builtin_inff();
+            tau_n[j] = at < pend ? p.tau[query] : __builtin_nanf("");
             if (p.res_term != nullptr && at < pend) {
                 const float rt = p.res_term[pair];
                 // |bias| = |2 <c, y> + |c|^2| (l2; inner product has none); five more roundings stand between this test
@@ -408,15 +477,11 @@ prefilter_b16_kernel(PrefilterB16Args p) {
                 tau_n[j] = tau_n[j] + rt + 2.0e-6F * (p.magnitude[query] + fabsf(rt) + bias_max);
             }
         } else {
-            tau_n[j] = q0 + col < p.nq && p.least == nullptr ? p.tau[q0 + col] : -__builtin_inff();
+            tau_n[j] = q0 + col < p.nq && p.least == nullptr ? p.tau[q0 + col] : __builtin_nanf("");  // no verdict passes
         }
     }
-    // A wave none of whose columns holds a query only helps to fetch.
-    const bool busy = LISTS ? pbeg + wn * JB * 32 < pend : q0 + wn * JB * 32 < p.nq;
 
-    // Query loader: (slot, part) pairs x N rows per stage, consecutive threads on consecutive rows.
-    constexpr uint32_t kQueryRegs = L::kSlots * 2 * N / 256;
-    constexpr uint32_t kRowStep = 256 / N;  // (slot, part) pairs that one round of the workgroup covers
+    // Query loader: (slot, part) pairs x N rows per stage of queries, consecutive threads on consecutive rows.
     const uint32_t qr = tid % N;
     uint64_t qsrc;
     if constexpr (LISTS) {
@@ -425,101 +490,62 @@ prefilter_b16_kernel(PrefilterB16Args p) {
     } else {
         qsrc = q0 + qr;  // below p.rows: the table covers whole tiles of rows
     }
-    // (Separate variables, not arrays: an array ended up in scratch memory.)
-    uint4 rc0, rc1, rc2, rc3, rc4, rc5, rc6, rc7, rq0, rq1, rq2, rq3, rq4, rq5, rq6, rq7;
-    const uint4* const qsrc_row = p.planes + static_cast<uint64_t>(tid / N) * p.rows + qsrc;
-    auto query_slot = [&](uint32_t st, uint32_t r) __attribute__((always_inline)) {
-        return qsrc_row[(static_cast<uint64_t>(st) * 2 * L::kSlots + kRowStep * r) * p.rows];
-    };
-    // No load stands behind a branch.  Granules past a code's end repeat its last one (the query's values there are zeros),
-    // tiles past the end repeat the first (their terms are infinite).
-    auto fetch = [&](uint64_t mt, uint32_t st) __attribute__((always_inline)) {
-        uint64_t tile = tile_begin + 4 * mt + wave;
-        tile = tile < tile_end ? tile : tile_begin;
-        const uint4* src = p.tiles + tile * p.G * kWave;
-        const uint32_t last = p.G - 1;
-        auto granule = [&](uint32_t u) __attribute__((always_inline)) {
-            const uint32_t j = L::kGranules * st + u < last ? L::kGranules * st + u : last;
-            return src[j * kWave + lane];
+    // (Separate variables, not an array: that ended up in scratch memory.)
+    uint4 rq0, rq1, rq2, rq3, rq4, rq5, rq6, rq7;
+    static_assert(kQueryRegs == 4 || kQueryRegs == 8, "what the loaders below move");
+    auto fetch_queries = [&](uint32_t st) __attribute__((always_inline)) {
+        auto slot = [&](uint32_t r) __attribute__((always_inline)) {
+            uint32_t sp = st * 2 * L::kSlots + tid / N + kRowStep * r;
+            sp = sp < 2 * p.slots ? sp : 2 * p.slots - 1;  // (of no stage that is multiplied)
+            return p.planes[static_cast<uint64_t>(sp) * p.rows + qsrc];
         };
-        rc0 = granule(0);
-        rc1 = granule(1);
-        if constexpr (L::kGranules > 2) {
-            rc2 = granule(2);
-            rc3 = granule(3);
-        }
-        if constexpr (L::kGranules > 4) {
-            rc4 = granule(4);
-            rc5 = granule(5);
-            rc6 = granule(6);
-            rc7 = granule(7);
-        }
-        rq0 = query_slot(st, 0);
-        if constexpr (kQueryRegs > 1) {
-            rq1 = query_slot(st, 1);
-        }
-        if constexpr (kQueryRegs > 2) {
-            rq2 = query_slot(st, 2);
-            rq3 = query_slot(st, 3);
-        }
-        if constexpr (kQueryRegs > 4) {
-            rq4 = query_slot(st, 4);
-            rq5 = query_slot(st, 5);
-            rq6 = query_slot(st, 6);
-            rq7 = query_slot(st, 7);
+        rq0 = slot(0);
+        rq1 = slot(1);
+        rq2 = slot(2);
+        rq3 = slot(3);
+        if constexpr (kQueryRegs == 8) {
+            rq4 = slot(4);
+            rq5 = slot(5);
+            rq6 = slot(6);
+            rq7 = slot(7);
         }
     };
-    auto park_floats = [&](uint32_t s, uint4 v, uint4 w) __attribute__((always_inline)) {
-        const float x[8] = {__uint_as_float(v.x), __uint_as_float(v.y), __uint_as_float(v.z), __uint_as_float(v.w),
-                            __uint_as_float(w.x), __uint_as_float(w.y), __uint_as_float(w.z), __uint_as_float(w.w)};
-        uint4 hi, lo;
-        b16_split8(x, &hi, &lo);
-        sa[s][0][tid] = hi;
-        sa[s][L::kParts - 1][tid] = lo;
+    auto park_queries = [&](uint32_t buf) __attribute__((always_inline)) {
+        auto put = [&](uint32_t r, uint4 v) __attribute__((always_inline)) {
+            const uint32_t sp = tid / N + kRowStep * r;
+            sb[buf][sp >> 1][sp & 1][qr] = v;
+        };
+        put(0, rq0);
+        put(1, rq1);
+        put(2, rq2);
+        put(3, rq3);
+        if constexpr (kQueryRegs == 8) {
+            put(4, rq4);
+            put(5, rq5);
+            put(6, rq6);
+            put(7, rq7);
+        }
     };
-    auto park_bytes = [&](uint32_t s, uint4 v) __attribute__((always_inline)) {
-        sa[s][0][tid] = make_uint4(b16_two_bytes(v.x, 0), b16_two_bytes(v.x, 2), b16_two_bytes(v.y, 0), b16_two_bytes(v.y, 2));
-        sa[s + 1][0][tid] =
-            make_uint4(b16_two_bytes(v.z, 0), b16_two_bytes(v.z, 2), b16_two_bytes(v.w, 0), b16_two_bytes(v.w, 2));
-    };
-    auto park_nibbles = [&](uint32_t s, uint4 v) __attribute__((always_inline)) {
-        sa[s][0][tid] = b16_nibbles(v.x);
-        sa[s + 1][0][tid] = b16_nibbles(v.y);
-        sa[s + 2][0][tid] = b16_nibbles(v.z);
-        sa[s + 3][0][tid] = b16_nibbles(v.w);
-    };
-    auto park_query = [&](uint32_t r, uint4 v) __attribute__((always_inline)) {
-        const uint32_t sp = tid / N + kRowStep * r;
-        sb[sp >> 1][sp & 1][qr] = v;
-    };
-    auto park = [&]() __attribute__((always_inline)) {
-        if constexpr (KIND == VSAG_AMD_KIND_FP32) {
-            park_floats(0, rc0, rc1);
-            park_floats(1, rc2, rc3);
-            park_floats(2, rc4, rc5);
-            park_floats(3, rc6, rc7);
-        } else if constexpr (KIND == VSAG_AMD_KIND_SQ8) {
-            park_bytes(0, rc0);
-            park_bytes(2, rc1);
-            park_bytes(4, rc2);
-            park_bytes(6, rc3);
+
+    auto record = [&](uint32_t col, uint64_t key) __attribute__((always_inline)) {
+        if constexpr (LISTS) {
+            // private list of the pair: chunk, which half of the 256 codes (the upper word)
+            const uint32_t pair = as_const(p.sorted_pair)[pbeg + col];
+            const uint64_t list = (static_cast<uint64_t>(pair) * kIvfB16Chunks + chunk) * 2 + static_cast<uint32_t>(key >> 32);
+            const uint32_t pos = atomicAdd(&p.partial_cnt[list], 1U);
+            if (pos < p.k) {
+                p.partial[list * p.k + pos] = static_cast<uint32_t>(key);
+            } else if (pos == p.k) {
+                if (atomicExch(&p.gate[pair / p.nprobe], 1U) == 0U) {
+                    atomicAdd(&p.gate[p.nq], 1U);
+                }
+            }
         } else {
-            park_nibbles(0, rc0);
-            park_nibbles(4, rc1);
-        }
-        park_query(0, rq0);
-        if constexpr (kQueryRegs > 1) {
-            park_query(1, rq1);
-        }
-        if constexpr (kQueryRegs > 2) {
-            park_query(2, rq2);
-            park_query(3, rq3);
-        }
-        if constexpr (kQueryRegs > 4) {
-            park_query(4, rq4);
-            park_query(5, rq5);
-            park_query(6, rq6);
-            park_query(7, rq7);
+            const uint64_t q = q0 + col;
+            const uint32_t pos = atomicAdd(&p.cand_cnt[q * kB16CountStride], 1U);
+            if (pos < p.cap) {
+                p.cand[q * p.cap + pos] = key;
+            }
         }
     };
     // Records wait in the wave's queue (a query's counter is an atomic a microsecond away: asked for one record at a time it
@@ -530,39 +556,27 @@ prefilter_b16_kernel(PrefilterB16Args p) {
     auto flush = [&]() __attribute__((always_inline)) {
         wave_lds_fence();
         for (uint32_t i = lane; i < waiting; i += kWave) {
-            const uint64_t key = keys[i];
-            if constexpr (LISTS) {
-                // private list of the pair: chunk, which half of the 256 codes (the upper word)
-                const uint32_t pair = as_const(p.sorted_pair)[pbeg + cols[i]];
-                const uint64_t list =
-                    (static_cast<uint64_t>(pair) * kIvfB16Chunks + chunk) * 2 + static_cast<uint32_t>(key >> 32);
-                const uint32_t pos = atomicAdd(&p.partial_cnt[list], 1U);
-                if (pos < p.k) {
-                    p.partial[list * p.k + pos] = static_cast<uint32_t>(key);
-                } else if (pos == p.k) {
-                    if (atomicExch(&p.gate[pair / p.nprobe], 1U) == 0U) {
-                        atomicAdd(&p.gate[p.nq], 1U);
-                    }
-                }
-            } else {
-                const uint64_t q = q0 + cols[i];
-                const uint32_t pos = atomicAdd(&p.cand_cnt[q], 1U);
-                if (pos < p.cap) {
-                    p.cand[q * p.cap + pos] = key;
-                }
-            }
+            record(cols[i], keys[i]);
         }
         waiting = 0;
         wave_lds_fence();
     };
 
-    if (first < mtiles) {
-        fetch(first, 0);
-    }
+    auto tile_of = [&](uint64_t mt) __attribute__((always_inline)) {
+        const uint64_t tile = tile_begin + 4 * mt + wave;
+        return p.tiles + (tile < tile_end ? tile : tile_begin) * p.G * kWave;  // (slots past the end count as absent)
+    };
+    B16Codes<KIND> codes;
+    const uint4* tile = tile_of(first);
+    b16_fetch_codes<KIND>(codes, tile, p.G, 0, half, l32);
+    fetch_queries(0);
+    park_queries(0);
+    __syncthreads();
+    uint32_t buf = 0;  // where the queries of the current stage are
     for (uint64_t mt = first; mt < mtiles; mt += step) {
-        floatx16 acc[IB][JB];
+        floatx16 acc[2][JB];
 #pragma unroll
-        for (int i = 0; i < IB; ++i) {
+        for (int i = 0; i < 2; ++i) {
 #pragma unroll
             for (int j = 0; j < JB; ++j) {
 #pragma unroll
@@ -571,77 +585,86 @@ prefilter_b16_kernel(PrefilterB16Args p) {
                 }
             }
         }
-        const uint64_t slot0 = (tile_begin + 4 * mt) * kWave;
-        park();  // the stage is free: the previous tile's contraction ended with a barrier
+        const uint64_t slot0 = (tile_begin + 4 * mt + wave) * kWave;
+        const bool more_tiles = mt + step < mtiles;
         float my_term;
         {
-            const uint64_t slot = slot0 + tid;
-            bool real = tile_begin + 4 * mt + (tid >> 6) < tile_end;
+            const uint64_t slot = slot0 + lane;
+            bool real = tile_begin + 4 * mt + wave < tile_end;
             if constexpr (LISTS) {
                 // (a padding slot is all zeros: under inner product, and with a residual bias, that is a good distance)
                 real = real && p.ids[slot] != VSAG_AMD_INVALID_ID;
             } else {
                 real = real && slot < p.n && !denied(p.deny, slot);
             }
-            my_term = real ? (p.is_l2 ? p.term[slot] : 0.0F) : __builtin_inff();
+            my_term = real ? p.term[slot] : kB16Absent;
+            if (!p.is_l2 && my_term < 3.0e38F) {
+                my_term = 0.0F;
+            } else if (!p.is_l2 && real && p.least == nullptr) {
+                // A code whose norm leaves fp32 (under l2 it stands behind all others) may have any inner product: a
+                // record of every query, and as its value is no number it is always rescored.
+                const uint32_t cols_here =
+                    LISTS ? (pend - pbeg < N ? pend - pbeg : N) : static_cast<uint32_t>(p.nq - q0 < N ? p.nq - q0 : N);
+                for (uint32_t col = 0; col < cols_here; ++col) {
+                    record(col, LISTS ? (static_cast<uint64_t>(wave >> 1) << 32) | static_cast<uint32_t>(slot)
+                                      : (0xFFFFFFFFULL << 32) | static_cast<uint32_t>(slot));
+                }
+                my_term = kB16Absent;
+            } else if (!(my_term < 3.0e38F)) {
+                my_term = kB16Absent;
+            }
             if (LISTS && real && p.res_bias != nullptr) {
                 my_term -= p.res_bias[slot];
             }
         }
-        __syncthreads();
         for (uint32_t st = 0; st < stages; ++st) {
-            {
-                // the next stage of this tile, or the first of the next tile (of this one once more behind the last)
-                const bool more = st + 1 < stages;
-                fetch(more || mt + step >= mtiles ? mt : mt + step, more ? st + 1 : 0);
+            // The operands of this stage, then the loads of the next one (of the next tile behind the last).
+            bf16x8 ah[2][kSteps], al[2][L::kSplit ? kSteps : 1];
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+#pragma unroll
+                for (uint32_t ks = 0; ks < kSteps; ++ks) {
+                    b16_operand<KIND>(codes, i, static_cast<int>(ks), &ah[i][ks], &al[i][L::kSplit ? ks : 0]);
+                }
             }
-            if (busy) {
-#pragma nounroll
-                for (uint32_t ks = 0; ks < L::kSlots / 2; ++ks) {
-                    const uint32_t slot = 2 * ks + half;
-                    bf16x8 bh[JB], bl[JB];
+            const bool last = st + 1 == stages;
+            if (last) {
+                tile = more_tiles ? tile_of(mt + step) : tile;
+            }
+            b16_fetch_codes<KIND>(codes, tile, p.G, last ? 0 : st + 1, half, l32);
+            // The queries of the next round of stages: fetched as this round begins, parked as it ends.
+            const uint32_t within = st % kRound;
+            if (within == 0) {
+                const uint32_t next = st + kRound;
+                fetch_queries(next < stages ? next : 0);
+            }
 #pragma unroll
-                    for (int j = 0; j < JB; ++j) {
-                        bh[j] = __builtin_bit_cast(bf16x8, sb[slot][0][wn * JB * 32 + j * 32 + l32]);
-                        bl[j] = __builtin_bit_cast(bf16x8, sb[slot][1][wn * JB * 32 + j * 32 + l32]);
-                    }
+            for (uint32_t ks = 0; ks < kSteps; ++ks) {
+                const uint32_t slot = within * L::kSlots + b16_slot<KIND>(ks, half);
 #pragma unroll
-                    for (int i = 0; i < IB; ++i) {
-                        const uint32_t row = wm * IB * 32 + i * 32 + l32;
-                        const bf16x8 ah = __builtin_bit_cast(bf16x8, sa[slot][0][row]);
+                for (int j = 0; j < JB; ++j) {
+                    const bf16x8 bh = __builtin_bit_cast(bf16x8, sb[buf][slot][0][j * 32 + l32]);
+                    const bf16x8 bl = __builtin_bit_cast(bf16x8, sb[buf][slot][1][j * 32 + l32]);
+#pragma unroll
+                    for (int i = 0; i < 2; ++i) {
                         if constexpr (L::kSplit) {
-                            const bf16x8 al = __builtin_bit_cast(bf16x8, sa[slot][L::kParts - 1][row]);
-#pragma unroll
-                            for (int j = 0; j < JB; ++j) {
-                                acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(al, bh[j], acc[i][j], 0, 0, 0);
-                            }
+                            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(al[i][ks], bh, acc[i][j], 0, 0, 0);
                         }
-#pragma unroll
-                        for (int j = 0; j < JB; ++j) {
-                            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ah, bl[j], acc[i][j], 0, 0, 0);
-                        }
-#pragma unroll
-                        for (int j = 0; j < JB; ++j) {
-                            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ah, bh[j], acc[i][j], 0, 0, 0);
-                        }
+                        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ah[i][ks], bl, acc[i][j], 0, 0, 0);
+                        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ah[i][ks], bh, acc[i][j], 0, 0, 0);
                     }
                 }
             }
-            if (st + 1 == stages) {
-                // every wave is past this tile's first barrier, hence out of the previous tile's epilogue
-                code_term[tid] = my_term;
-            }
-            __syncthreads();  // every wave has read the stage
-            if (st + 1 < stages) {
-                park();
+            if (within + 1 == kRound || last) {
+                // (the other buffer's readers passed the barrier before this round)
+                buf ^= 1;
+                park_queries(buf);
                 __syncthreads();
             }
         }
-        if (!busy) {
-            continue;
-        }
-        // Nearly nothing passes: sixteen products of a lane share a verdict (their least value), and only where a lane's
-        // passes are they looked at one by one.
+        // Nearly nothing passes: sixteen products of a lane share a verdict (their least value).
+        code_term[wave][lane] = my_term;
+        wave_lds_fence();
         const float dot_factor = p.is_l2 ? -2.0F : -1.0F;
         float group_least[JB];
 #pragma unroll
@@ -649,12 +672,12 @@ prefilter_b16_kernel(PrefilterB16Args p) {
             group_least[j] = __builtin_inff();
         }
 #pragma unroll
-        for (int i = 0; i < IB; ++i) {
-            const uint32_t m0 = wm * IB * 32 + i * 32 + 4 * half;
+        for (int i = 0; i < 2; ++i) {
+            const uint32_t m0 = i * 32 + 4 * half;
             float term[16];
 #pragma unroll
             for (int e4 = 0; e4 < 4; ++e4) {
-                const float4 t4 = *reinterpret_cast<const float4*>(code_term + m0 + 8 * e4);
+                const float4 t4 = *reinterpret_cast<const float4*>(&code_term[wave][m0 + 8 * e4]);
                 term[4 * e4] = t4.x;
                 term[4 * e4 + 1] = t4.y;
                 term[4 * e4 + 2] = t4.z;
@@ -662,61 +685,50 @@ prefilter_b16_kernel(PrefilterB16Args p) {
             }
 #pragma unroll
             for (int j = 0; j < JB; ++j) {
+                // The low four bits of a value say which of the sixteen it is.
                 float v[16];
                 float least = __builtin_inff();
 #pragma unroll
                 for (int e = 0; e < 16; ++e) {
-                    v[e] = fmaf(dot_factor, acc[i][j][e], term[e]);
+                    const float d = fmaf(dot_factor, acc[i][j][e], term[e]);
+                    v[e] = __uint_as_float((__float_as_uint(d) & ~15U) | static_cast<uint32_t>(e));
                     least = fminf(least, v[e]);
                 }
                 group_least[j] = fminf(group_least[j], least);
-                if (__ballot(least <= tau_n[j]) == 0) {
-                    continue;
-                }
-                uint32_t hits = 0;
-#pragma unroll
-                for (int e = 0; e < 16; ++e) {
-                    hits |= (v[e] <= tau_n[j] ? 1U : 0U) << e;
-                }
-                hits = tau_n[j] > -__builtin_inff() ? hits : 0U;  // (a column without a query)
-                while (__ballot(hits != 0) != 0) {
-                    const bool hit = hits != 0;
+                while (__ballot(least <= tau_n[j]) != 0) {
+                    const bool hit = least <= tau_n[j];
                     const uint64_t mask = __ballot(hit);
                     const uint32_t np = static_cast<uint32_t>(__popcll(mask));
                     if (waiting + np > kB16Queue) {
                         flush();
                     }
                     if (hit) {
-                        const uint32_t e = static_cast<uint32_t>(__builtin_ctz(hits));
-                        hits &= hits - 1;
+                        const uint32_t e = __float_as_uint(least) & 15U;
                         const uint32_t at = waiting + mask_rank(mask);
-                        const uint32_t ml = m0 + 8 * (e >> 2) + (e & 3);
-                        const uint32_t slot = static_cast<uint32_t>(slot0) + ml;
-                        if constexpr (LISTS) {
-                            keys[at] = (static_cast<uint64_t>(ml >> 7) << 32) | slot;
-                        } else {
-                            float value = v[0];
-#pragma unroll
-                            for (int u = 1; u < 16; ++u) {
-                                value = e == static_cast<uint32_t>(u) ? v[u] : value;
-                            }
-                            keys[at] = make_key(value, slot);
-                        }
-                        cols[at] = wn * JB * 32 + j * 32 + l32;
+                        const uint32_t slot = static_cast<uint32_t>(slot0) + m0 + 8 * (e >> 2) + (e & 3);
+                        keys[at] = LISTS ? (static_cast<uint64_t>(wave >> 1) << 32) | slot : make_key(least, slot);
+                        cols[at] = j * 32 + l32;
                     }
                     waiting += np;
+                    // the next of this lane's sixteen (they differ: in the low four bits at least)
+                    const float last = least;
+                    least = __builtin_inff();
+#pragma unroll
+                    for (int e = 0; e < 16; ++e) {
+                        least = fminf(least, v[e] > last ? v[e] : __builtin_inff());
+                    }
                 }
             }
         }
         if constexpr (!LISTS) {
             if (p.least != nullptr) {
-                // the codes of a lane: 16 IB of the tile's 256, one group
+                // the codes of this wave, one group
 #pragma unroll
                 for (int j = 0; j < JB; ++j) {
-                    const uint64_t q = q0 + wn * JB * 32 + j * 32 + l32;
-                    const uint32_t group = (static_cast<uint32_t>(mt / p.mstep) * (4 / WN) + wm) * 2 + half;
-                    if (q < p.nq) {
-                        p.least[q * p.groups + group] = group_least[j];
+                    const float least = fminf(group_least[j], __shfl_xor(group_least[j], 32));
+                    const uint64_t q = q0 + j * 32 + l32;
+                    if (half == 0 && q < p.nq) {
+                        p.least[q * p.groups + static_cast<uint32_t>(mt / p.mstep) * 4 + wave] = least;
                     }
                 }
             }
@@ -754,15 +766,15 @@ launch_b16_flat(uint64_t nq, uint32_t cus, PrefilterB16Args p, hipStream_t st) {
     const uint64_t mtiles = div_up(div_up(p.ntiles, 4), p.mstep);
     // Two rounds of the workgroups that fit a compute unit (two or three) and not one more: a few left over would run a
     // third round alone.  A workgroup walks every gridDim.x-th tile.
-    uint64_t groups = static_cast<uint64_t>(cus) * (per == kB16N ? 4 : 6) / qtiles;
+    uint64_t groups = static_cast<uint64_t>(cus) * (per == 32 || (per == 64 && KIND != VSAG_AMD_KIND_FP32) ? 6 : 4) / qtiles;
     groups = std::max<uint64_t>(1, std::min<uint64_t>(groups, mtiles));
     const dim3 grid(static_cast<uint32_t>(groups), static_cast<uint32_t>(qtiles));
     if (per == 32) {
-        hipLaunchKernelGGL((prefilter_b16_kernel<KIND, false, 2, 1, 1>), grid, dim3(256), 0, st, p);
+        hipLaunchKernelGGL((prefilter_b16_kernel<KIND, false, 1>), grid, dim3(256), 0, st, p);
     } else if (per == 64) {
-        hipLaunchKernelGGL((prefilter_b16_kernel<KIND, false, 2, 2, 1>), grid, dim3(256), 0, st, p);
+        hipLaunchKernelGGL((prefilter_b16_kernel<KIND, false, 2>), grid, dim3(256), 0, st, p);
     } else {
-        hipLaunchKernelGGL((prefilter_b16_kernel<KIND, false, 4, 2, 2>), grid, dim3(256), 0, st, p);
+        hipLaunchKernelGGL((prefilter_b16_kernel<KIND, false, 4>), grid, dim3(256), 0, st, p);
     }
 }
 
@@ -779,10 +791,10 @@ launch_b16_kind(const vsag_amd_store* s, uint64_t nq, const PrefilterB16Args& p,
 }
 
 // The sample of a call: every step-th code tile of 256.  With s of n codes sampled, about k n / s codes lie at or below the
-// k-th smallest of the sample: kB16Expect of them (4 k where that is more), an eighth of the room a query has (a quarter).
-// Each sampled tile gives four groups at least, and four times as many groups as k keep their k-th least close to the k-th
+// k-th smallest of the sample: kB16Expect of them (4 k where that is more), a sixteenth of the room a query has (a quarter).
+// Each sampled tile gives four groups, and four times as many groups as k keep their k-th least close to the k-th
 // of the sample.
-constexpr uint64_t kB16Expect = 256;
+constexpr uint64_t kB16Expect = 128;
 constexpr uint32_t kB16Records = 2048;
 
 uint32_t
@@ -798,9 +810,8 @@ b16_sample_step(const vsag_amd_store* s, uint32_t k) {
     return std::max<uint64_t>(1, mtiles / want);
 }
 static uint32_t
-b16_sample_groups(const vsag_amd_store* s, uint64_t nq, uint32_t k) {
-    const uint64_t tiles = div_up(div_up(s->ntiles, 4), b16_sample_step(s, k));
-    return static_cast<uint32_t>(tiles * (nq <= 64 ? 8 : 4));
+b16_sample_groups(const vsag_amd_store* s, uint32_t k) {
+    return static_cast<uint32_t>(div_up(div_up(s->ntiles, 4), b16_sample_step(s, k)) * 4);
 }
 
 // Scratch: the queries' parts, then their errors, thresholds, slacks and what the sample leaves.
@@ -817,7 +828,7 @@ carve_b16(Carver& c, const vsag_amd_store* s, uint64_t nq, uint32_t k, B16Scratc
     b->error = c.take<B16Error>(nq);
     b->tau = c.take<float>(nq);
     b->slack = c.take<float>(nq);
-    b->least = c.take<float>(nq * b16_sample_groups(s, nq, k));
+    b->least = c.take<float>(nq * b16_sample_groups(s, k));
     return c.used;
 }
 size_t
@@ -861,7 +872,7 @@ launch_scan_b16(const vsag_amd_store* s, const ScanArgs& a, uint64_t nq, uint32_
     p.deny = deny;
     p.mstep = b16_sample_step(s, k);
     p.least = b.least;
-    p.groups = b16_sample_groups(s, nq, k);
+    p.groups = b16_sample_groups(s, k);
     launch_b16_kind(s, nq, p, st);
     B16TauArgs ta{b.least, p.groups, k, b.error, b.tau, b.slack, cand_cnt, gate, partial_cnt, nslots};
     hipLaunchKernelGGL(b16_tau_kernel, dim3(static_cast<uint32_t>(nq)), dim3(kWave), 0, st, ta);
@@ -939,7 +950,7 @@ launch_ivf_b16(const vsag_amd_store* s, const ScanArgs& a, uint64_t nq, uint32_t
     const uint64_t max_items =
         (div_up(pairs, static_cast<uint64_t>(kB16N)) + std::min<uint64_t>(s->nlist, pairs)) * kIvfB16Chunks;
     timing_begin(st);
-    hipLaunchKernelGGL((prefilter_b16_kernel<VSAG_AMD_KIND_FP32, true, 4, 2, 2>), dim3(static_cast<uint32_t>(max_items)),
+    hipLaunchKernelGGL((prefilter_b16_kernel<VSAG_AMD_KIND_FP32, true, 4>), dim3(static_cast<uint32_t>(max_items)),
                        dim3(256), 0, st, p);
     timing_end(st);
     VA_HIP(hipGetLastError());

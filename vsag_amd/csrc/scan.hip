@@ -843,7 +843,7 @@ carve_scan(Carver& c, const CallPlan& cp, uint64_t nq, uint32_t k, ScanBuffers* 
     if (!cp.int8 && !cp.rb && !cp.b16 && cp.h16_scratch == 0) {
         b->q8 = nullptr;
     }
-    b->cand_cnt = c.take<uint32_t>(cp.contraction ? nq * std::max<uint32_t>(1, cp.max_lists) : 0);
+    b->cand_cnt = c.take<uint32_t>(cp.contraction ? nq * (cp.b16 ? 32U : std::max<uint32_t>(1, cp.max_lists)) : 0);
     b->gate = c.take<uint32_t>(cp.contraction ? nq : 0);
     b->cand = c.take<uint32_t>(cp.contraction ? nq * cp.cap * (cp.b16 ? 2 : 1) : 0);
     b->table = c.take<float>(cp.table ? nq * cp.table_ld : 0);
