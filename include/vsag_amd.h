@@ -324,8 +324,9 @@ VSAG_AMD_API int vsag_amd_flat_scan_topk_noalloc(const vsag_amd_store_t* store, 
  * Posting lists of sq4_uniform codes of at most 128 dimensions (any metric) scan the probe columns behind the first on the
  * int8 matrix cores when a batch has at least 8192 (query, list) groups (same results; off with mode -1).
  * sq8 and sq4 stores of at most 128 dimensions pre-select on the int8 matrix cores (queries split into two int8 planes
- * with a rigorous bound on the remainder), those beyond on the fp16 and fp32 stores on the fp32 matrix cores.
- * mode: 0 = when it pays (default: >= 512 queries, or 16 and more against enough codes, k <= 128, >= 65536 codes; below 512
+ * with a rigorous bound on the remainder), those beyond on the fp16 matrix cores; fp32 stores, and sq8 / sq4 ones under a
+ * deny mask or in small batches, on the bf16 matrix cores.
+ * mode: 0 = when it pays (default: >= 512 queries, or 4 and more against enough codes, k <= 128, >= 65536 codes; below 512
  * not where a query tile or a number of chunks is set, see the tuning knobs), 1 = whenever the store and k
  * allow it, 2 = like 1 but always on the fp32 matrix cores, -1 = never.  Process-wide; affects
  * vsag_amd_flat_scan_workspace_bytes as well.  No counterpart in the reference (it scans one query at a time). */
@@ -341,9 +342,10 @@ VSAG_AMD_API int vsag_amd_set_scan_tuning(int query_tile, int base_chunks);
  * counterpart in the reference. */
 VSAG_AMD_API int vsag_amd_store_set_scan_contraction(vsag_amd_store_t* store, int mode);
 VSAG_AMD_API int vsag_amd_store_set_scan_tuning(vsag_amd_store_t* store, int query_tile, int base_chunks);
-/* What the last flat scan on this thread used: query tile (128 / 256: the batch went through the fp32 / int8
- * matrix cores), passes over the code array, bytes of codes one pass reads.  After a posting-list scan: query tile
- * only (256: the columns behind the first went through the int8 matrix cores). */
+/* What the last flat scan on this thread used: query tile (128 / 256: a large batch went through the
+ * bf16, fp16 or fp32 / int8 matrix cores; 64: a smaller one through the bf16 or fp32 ones), passes over the code array,
+ * bytes of codes one pass reads.  After a posting-list scan: query tile only (256: the columns behind the first went through
+ * the int8 matrix cores). */
 VSAG_AMD_API int vsag_amd_last_scan_info(int* query_tile, uint64_t* passes, uint64_t* bytes_per_pass);
 
 /* Measurement hook: when enabled, a call records HIP events on its stream around the launch of its

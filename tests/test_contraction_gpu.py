@@ -134,6 +134,30 @@ def test_small_batches_of_every_kind_and_metric(lib, modes, kind, metric, n, d, 
     st.destroy()
 
 
+@pytest.mark.parametrize("kind,metric,n,d,k,streamed", [
+    ("fp32", orc.L2, 81857, 64, 10, 4), ("fp32", orc.COSINE, 82000, 30, 21, 7), ("sq8", orc.L2, 81857, 100, 20, 3),
+    ("sq8", orc.IP, 90001, 17, 128, 5), ("sq4", orc.COSINE, 81900, 129, 1, 3), ("sq8", orc.COSINE, 81857, 300, 21, 5)])
+def test_smallest_batches_on_the_bf16_matrix_cores(lib, modes, kind, metric, n, d, k, streamed):
+    """A handful of queries against 1280 tiles of codes: the largest batch that streams, and from the next one on the bf16
+    matrix cores with 32, 64 and 128 queries per workgroup, with the streaming kernel's ids and distance bits."""
+    rng = np.random.default_rng(n + d)
+    x, means = gaussian_mixture(rng, n, d, 60, 0.05)
+    q, _ = gaussian_mixture(rng, 129, d, 60, 0.05, means=means)
+    q[1] = x[5]
+    st = _store_of(kind, metric, x, rng)
+    for nq in (streamed, streamed + 1, 32, 33, 64, 65, 129):
+        plain, auto, tile = modes(st, q[:nq], k, 0)
+        assert same(plain, auto), nq
+        assert (tile >= 64) == (nq > streamed), (nq, tile)
+    st.destroy()
+    # one tile fewer: as before
+    if n == 81857:
+        st = _store_of(kind, metric, x[:n - 1], rng)
+        plain, auto, tile = modes(st, q[:16], k, 0)
+        assert same(plain, auto) and tile < 64
+        st.destroy()
+
+
 @pytest.mark.parametrize("kind,bits", [("sq8", 8), ("sq4", 4)])
 def test_fp16_preselection_keeps_few_candidates_under_cosine(lib, modes, kind, bits):
     """The thresholds of a cosine batch are as narrow as its distances: no query overflows its candidates (every query did,

@@ -1220,14 +1220,13 @@ prefilter_supports(const vsag_amd_store* s) {
     return s->nlist == 0 && (s->kind == VSAG_AMD_KIND_FP32 || s->kind == VSAG_AMD_KIND_SQ8) && s->pf_term != nullptr;
 }
 
-// Whether a batch of nq queries is pre-selected (stores of at least 1024 tiles).  From 512 queries on always; below, the
-// dozen launches, the exact prefix and the rescoring (which grows with k) have to be less than the streaming kernel's time,
-// which grows with queries x codes x dimensions.  Measured on Gaussian mixtures with the plan that the default mode makes,
-// under L2, us per call, streaming -> pre-selected, beside the line:
-//   fp32 (fp32 matrix cores): 100k x 128, k 10, 64 queries 291 -> 208 (32: 236 -> 182, not taken); 1M x 100, k 100, 128
-//     queries 1759 -> 831; 100k x 768, k 100, 64 queries 955 -> 1075, 128 1406 -> 1154 (not taken); 600k x 960, k 10, 256
-//     queries 12109 -> 3907.  Their time hardly depends on the dimension's share of the work from 128 on: both sides grow
-//     with it.
+// Whether a batch of nq queries is a large one: pre-selected level by level where prefilter_b16_pays does not take it
+// (stores of at least 1024 tiles), and reported as such where it does.  From 512 queries on always; below, the dozen
+// launches, the exact prefix and the rescoring (which grows with k) have to be less than the streaming kernel's time, which
+// grows with queries x codes x dimensions.  Measured on Gaussian mixtures, under L2, us per call, streaming -> pre-selected,
+// beside the line:
+//   fp32 (fp32 matrix cores, as batches that find no room on the bf16 ones still take them): 100k x 128, k 10, 64 queries
+//     291 -> 208; 1M x 100, k 100, 128 queries 1759 -> 831; 600k x 960, k 10, 256 queries 12109 -> 3907.
 //   sq8 / sq4 on the int8 matrix cores: 1M x 100, k 10, 32 queries 474 -> 358, 16 269 -> 333 (not taken); k 100, 64 queries
 //     752 -> 606; 100k x 128, k 10, 256 queries 314 -> 243, 128 224 -> 237 (not taken).
 //   sq8 / sq4 on the fp16 matrix cores: 200k x 768, k 10, 32 queries 849 -> 462, 16 458 -> 450 (not taken); k 100, 128

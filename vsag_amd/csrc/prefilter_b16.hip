@@ -19,9 +19,9 @@
 //   3. of the records only those within 2 e of their own k-th smallest are rescored with the streaming kernel's arithmetic
 //      (rescore_kernel): k and a handful, and the result is the streaming result, bit for bit.
 // A query with more records than there is room for is gated and streams.  A deny mask takes part in 1 and 2 as a |y|^2
-// beyond every threshold.  100k x 128 fp32, 1000 queries, k 10 (fp32 matrix cores, an exact prefix and levels before: 460 us): 209 us.
-// 100k x 768 fp32, 32 queries (streamed before: 684 us on the device): MEASURED_B.  500k x 100 sq8 under a deny mask, 200
-// queries, k 100 (streamed before: 664 us): 209 us.
+// beyond every threshold.  100k x 128 fp32, 1000 queries, k 10 (fp32 matrix cores, an exact prefix and levels before: 460 us): 150 us.
+// 100k x 768 fp32, 32 queries (streamed before: 684 us on the device): 141 us.  500k x 100 sq8 under a deny mask, 200
+// queries, k 100 (streamed before: 664 us): 160 us.
 //
 // What bounds it: with 128 queries per workgroup the matrix cores beside the splitting of the codes and the verdicts; with
 // few queries the bytes of the codes, each read once per 32, 64 or 128 queries.
@@ -66,6 +66,33 @@ bool
 prefilter_b16_supports(const vsag_amd_store* s) {
     return (s->kind == VSAG_AMD_KIND_FP32 || s->kind == VSAG_AMD_KIND_SQ8 || s->kind == VSAG_AMD_KIND_SQ4) &&
            s->pf_term != nullptr && s->pf_ymax != nullptr;
+}
+
+// Whether a batch takes this route of its own accord, measured on Gaussian mixtures against what served it before (us per
+// call, other -> this).
+//   Streaming passes serve four or eight queries at a time: fp32 100k x 768, k 10 4 queries 131 -> 140 (cosine; not taken), 5:
+//   153 -> 139, 8: 281 -> 141, 32: 686 -> 141; k 100 6: 161 -> 234 (not taken), 8: 294 -> 212; sq8 500k x 100 cosine, k 10
+//   2: 62 -> 69 (not taken), 4: 93 -> 68; k 100 4: 79 -> 91 (not taken), 6: 110 -> 92; 1M x 128 16: 259 -> 87.
+//   sq8 / sq4 up to 128 dimensions have the int8 matrix cores, twice as fast a product behind a prefix and four levels: 1M x
+//   128, k 10 512 queries 415 -> 362 (not taken from 508 on), 1000 532 -> 653 (not taken); k 100 600 710 -> 568, 1000 802 ->
+//   828 (not taken); k 1 600 370 -> 407 (not taken); 300k 1000 318 -> 269 (not taken), 2000 402 -> 456 (not taken); 100k, k 10
+//   512 231 -> 112, 2000 300 -> 238 (not taken), 4000 354 -> 410 (not taken), k 100 4000 704 -> 490.
+//   Beyond, the fp16 ones, one product where this takes two: sq4 200k x 512 cosine, k 10 1000 508 -> 456, 2000 792 -> 856
+//   (not taken); sq8 600k x 960 ip 256 798 -> 629, 1000 1825 -> 2265 (not taken); 200k x 768, k 100 1000 1504 -> 879.
+//   A deny mask leaves the streaming kernel alone as the other side.
+// Smaller stores than 81920 codes would gain as well (sq8 70000 x 200, 512 queries 263 -> 121; 70000 x 32, 8 60 -> 47), but
+// the records of a query take 16 KB, several times the streaming kernel's workspace there: batches of those keep it.
+bool
+prefilter_b16_pays(const vsag_amd_store* s, uint64_t nq, uint32_t k, bool masked) {
+    const bool fp32 = s->kind == VSAG_AMD_KIND_FP32;
+    if (s->ntiles < 1280 || nq < (fp32 ? (k <= 20 ? 5U : 8U) : (k <= 20 ? 4U : 6U))) {
+        return false;
+    }
+    if (fp32 || masked || nq <= 64) {
+        return true;
+    }
+    const double n = static_cast<double>(s->n), work = static_cast<double>(nq) * n * s->dim;
+    return work <= (s->dim <= 128 ? 2.0e10 + 5.0e8 * k + 4.0e10 * log10(n * 1.0e-5) : 1.4e11 + 2.0e9 * k);
 }
 
 static uint64_t

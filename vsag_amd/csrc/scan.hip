@@ -586,9 +586,10 @@ struct CallPlan {
     uint64_t level_begin[kMaxLevels + 1] = {};
     bool int8 = false;         // the int8 matrix cores pre-select (sq8, at most 128 dimensions)
     bool rb = false;           // RaBitQ store: 1-bit codes x 4-bit queries on the int8 matrix cores
-    // fp32 stores, and sq8 / sq4 ones under a deny mask: the bf16 matrix cores, which need neither a prefix nor levels
-    // (prefilter_b16.hip); the streaming launch behind covers all tiles.
+    // fp32 stores, and sq8 / sq4 ones in small batches or under a deny mask: the bf16 matrix cores, which need neither a
+    // prefix nor levels (prefilter_b16.hip); the streaming launch behind covers all tiles.
     bool b16 = false;
+    bool large = false;  // (b16) what vsag_amd_last_scan_info tells large batches by: prefilter_pays
     size_t b16_scratch = 0;
     size_t h16_scratch = 0;    // sq8 beyond 128 dimensions: bytes of the fp16 query planes (0: the fp32 matrix cores)
     uint32_t cap = 0;          // candidates per query and level
@@ -634,6 +635,7 @@ size_t prefilter_rb_scratch_bytes(const vsag_amd_store* s, uint64_t nq);
 bool prefilter_h16_supports(const vsag_amd_store* s);
 size_t prefilter_h16_scratch_bytes(const vsag_amd_store* s, uint64_t nq);
 bool prefilter_b16_supports(const vsag_amd_store* s);
+bool prefilter_b16_pays(const vsag_amd_store* s, uint64_t nq, uint32_t k, bool masked);
 size_t prefilter_b16_scratch_bytes(const vsag_amd_store* s, uint64_t nq, uint32_t k);
 uint32_t prefilter_b16_cap(uint32_t k);
 int launch_scan_b16(const vsag_amd_store* s, const ScanArgs& a, uint64_t nq, uint32_t k, uint32_t S, uint32_t* bound,
@@ -677,18 +679,24 @@ make_call_plan(const vsag_amd_store* s, uint64_t nq, uint32_t k, bool masked, Ca
     const bool rb = prefilter_rb_supports(s);
     // (The tuning knobs are the streaming kernel's: a batch that either route could serve streams where one is set.)
     const bool tuned = nq < kListsOptionalBelow && (tile_override(s) > 0 || chunk_override(s) > 0);
-    if (!forced && (tuned || k > (rb ? 256U : 128U) || s->ntiles < 1024 || !prefilter_pays(s, nq, k))) {
+    if (!forced && (tuned || k > (rb ? 256U : 128U))) {
         return;
     }
-    if (prefilter_mode(s) != 2 && prefilter_b16_supports(s) && (s->kind == VSAG_AMD_KIND_FP32 || masked)) {
+    const bool large = forced || (s->ntiles >= 1024 && prefilter_pays(s, nq, k));
+    if (prefilter_mode(s) != 2 && prefilter_b16_supports(s) && s->ntiles != 0 &&
+        ((large && (s->kind == VSAG_AMD_KIND_FP32 || masked)) || (!forced && prefilter_b16_pays(s, nq, k, masked)))) {
         const uint64_t cap = prefilter_b16_cap(k);
-        if (nq * cap * 8 > (2ull << 30) || s->ntiles == 0) {
+        if (nq * cap * 8 <= (2ull << 30)) {
+            c->contraction = c->b16 = true;
+            c->large = large;
+            c->cap = static_cast<uint32_t>(cap);
+            c->b16_scratch = prefilter_b16_scratch_bytes(s, nq, k);
+            c->nslots += 1;
             return;
         }
-        c->contraction = c->b16 = true;
-        c->cap = static_cast<uint32_t>(cap);
-        c->b16_scratch = prefilter_b16_scratch_bytes(s, nq, k);
-        c->nslots += 1;
+        // (a batch without room for that many records: shorter lists, level by level)
+    }
+    if (!large) {
         return;
     }
     if (masked) {
@@ -1296,7 +1304,7 @@ flat_scan_call(const vsag_amd_store_t* s, const float* queries_dev, uint64_t nq,
                                masked ? options->deny_bits_dev : nullptr, b.partial, b.partial_cnt, nslots, b.gate, st));
         // the queries whose records found no room
         VA_TRY(run_streaming(s, p, a, b, nq, k, options, 0, s->ntiles, 1, nslots, b.gate, st));
-        tl_last_tile = 128;  // queries per pass
+        tl_last_tile = cp.large ? 128 : 64;
         tl_last_passes = div_up(nq, 128);
     } else {
         const uint32_t slots_prefix = static_cast<uint32_t>(cp.prefix.chunks * cp.prefix.waves);
