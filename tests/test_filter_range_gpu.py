@@ -77,6 +77,31 @@ def test_masked_batches_on_the_bf16_matrix_cores(lib, kind, metric, n, d, nq, k,
     st.destroy()
 
 
+def test_denied_codes_stay_hidden_where_products_overflow(lib):
+    """Products of denied codes with a query leave fp32: they must not pass for the best of all."""
+    rng = np.random.default_rng(5)
+    n, d, nq, k = 20000, 40, 33, 10
+    x = rng.standard_normal((n, d)).astype(np.float32)
+    q = rng.standard_normal((nq, d)).astype(np.float32)
+    deny = np.ones(n, bool)
+    deny[::20] = False
+    x[7::2000] = np.float32(1e20)
+    q[5] = np.float32(1e20)
+    st = Store(capi.KIND_FP32, orc.IP, d)
+    st.append(x.view(np.uint8).reshape(n, -1))
+    res = []
+    try:
+        for mode in (-1, 1):
+            capi.check(st.lib.vsag_amd_set_scan_contraction(mode))
+            res.append(st.flat_scan(q, k, deny=deny))
+    finally:
+        capi.check(st.lib.vsag_amd_set_scan_contraction(0))
+    assert not deny[res[1][0]].any()
+    assert np.array_equal(res[0][0], res[1][0])
+    assert np.array_equal(res[0][1].view(np.uint32), res[1][1].view(np.uint32))
+    st.destroy()
+
+
 @pytest.mark.parametrize("metric", [orc.L2, orc.IP])
 def test_flat_scan_with_radius(lib, metric):
     rng = np.random.default_rng(91)

@@ -234,7 +234,8 @@ b16_query_kernel(B16QueryArgs p) {
     // Operands below the normal range taken as zero; fma(factor, acc, term) and |y|^2 rounded, the low four bits cut off.
     const double flushed = kd * 4.7e-38 * (an + ymax + 1.0);
     const double test = 36.0 * kU * ((p.is_l2 ? ymax * ymax : 0.0) + factor * dots);
-    double fixed = factor * (split + rounding) + flushed + test;
+    // (A product that can leave fp32 would carry a slot that cannot be found past its |y|^2: such a query streams.)
+    double fixed = factor * dots < 1.0e37 ? factor * (split + rounding) + flushed + test : 1.0e39;
     double root = 0.0, slope = 0.0;
     double constant = a2;
     if (p.is_l2) {
