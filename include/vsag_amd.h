@@ -317,7 +317,7 @@ VSAG_AMD_API int vsag_amd_flat_scan_topk_noalloc(const vsag_amd_store_t* store, 
                                     uint32_t k, const vsag_amd_search_options_t* options, uint32_t* ids_dev,
                                     float* dists_dev, void* stream);
 
-/* Large batches on flat fp32 / sq8 / sq4 / sq8_uniform / sq4_uniform (the uniform kinds: at most 128 dimensions) / rabitq stores are served by a matrix-core contraction that pre-selects
+/* Large batches on flat fp32 / sq8 / sq4 / sq8_uniform / sq4_uniform / rabitq stores are served by a matrix-core contraction that pre-selects
  * candidates, which are then recomputed and selected exactly as the streaming scan does (same results, bit for bit).
  * rabitq stores with 4-bit queries and at most 1024 dimensions (L2, inner product) expand code bits to fp4 and query nibbles
  * to fp6 for the scaled matrix instruction (the integer product is exact; k up to 256 by default).
@@ -325,7 +325,7 @@ VSAG_AMD_API int vsag_amd_flat_scan_topk_noalloc(const vsag_amd_store_t* store, 
  * int8 matrix cores when a batch has at least 8192 (query, list) groups (same results; off with mode -1).
  * sq8 and sq4 stores of at most 128 dimensions pre-select on the int8 matrix cores (queries split into two int8 planes
  * with a rigorous bound on the remainder), those beyond on the fp16 matrix cores; fp32 stores, and sq8 / sq4 ones under a
- * deny mask or in small batches, on the bf16 matrix cores.
+ * deny mask or in small batches, and the uniform kinds beyond 128 dimensions, on the bf16 matrix cores.
  * mode: 0 = when it pays (default: >= 512 queries, or 4 and more against enough codes, k <= 128, >= 65536 codes; below 512
  * not where a query tile or a number of chunks is set, see the tuning knobs), 1 = whenever the store and k
  * allow it, 2 = like 1 but always on the fp32 matrix cores, -1 = never.  Process-wide; affects

@@ -136,7 +136,8 @@ def test_small_batches_of_every_kind_and_metric(lib, modes, kind, metric, n, d, 
 
 @pytest.mark.parametrize("kind,metric,n,d,k,streamed", [
     ("fp32", orc.L2, 81857, 64, 10, 4), ("fp32", orc.COSINE, 82000, 30, 21, 7), ("sq8", orc.L2, 81857, 100, 20, 3),
-    ("sq8", orc.IP, 90001, 17, 128, 5), ("sq4", orc.COSINE, 81900, 129, 1, 3), ("sq8", orc.COSINE, 81857, 300, 21, 5)])
+    ("sq8", orc.IP, 90001, 17, 128, 8), ("sq4", orc.COSINE, 81900, 129, 1, 3), ("sq8", orc.L2, 81857, 300, 21, 5),
+    ("sq8_uniform", orc.IP, 81857, 130, 21, 8), ("sq4_uniform", orc.L2, 82001, 64, 20, 4)])
 def test_smallest_batches_on_the_bf16_matrix_cores(lib, modes, kind, metric, n, d, k, streamed):
     """A handful of queries against 1280 tiles of codes: the largest batch that streams, and from the next one on the bf16
     matrix cores with 32, 64 and 128 queries per workgroup, with the streaming kernel's ids and distance bits."""
@@ -155,6 +156,49 @@ def test_smallest_batches_on_the_bf16_matrix_cores(lib, modes, kind, metric, n, 
         st = _store_of(kind, metric, x[:n - 1], rng)
         plain, auto, tile = modes(st, q[:16], k, 0)
         assert same(plain, auto) and tile < 64
+        st.destroy()
+
+
+@pytest.mark.parametrize("metric", [orc.L2, orc.IP, orc.COSINE])
+@pytest.mark.parametrize("kind,n,d,nq,k", [("sq8_uniform", 30001, 130, 40, 10), ("sq8_uniform", 9000, 960, 129, 100),
+                                           ("sq4_uniform", 20011, 161, 65, 1), ("sq4_uniform", 7000, 300, 5, 20),
+                                           ("sq8_uniform", 82001, 33, 64, 10), ("sq4_uniform", 90000, 128, 33, 50)])
+def test_uniform_codes_on_the_bf16_matrix_cores(lib, modes, kind, metric, n, d, nq, k):
+    """Byte and nibble rows as one bf16 part: beyond 128 dimensions, in small batches, and under a deny mask, with the
+    streaming kernel's ids and distance bits."""
+    rng = np.random.default_rng(n + d)
+    x, means = gaussian_mixture(rng, n, d, 30, 0.05)
+    q, _ = gaussian_mixture(rng, nq, d, 30, 0.05, means=means)
+    q[0] = x[3]
+    q[1] = -1e3
+    st = _store_of(kind, metric, x, rng)
+    plain, fast, tile = modes(st, q, k, 1 if d > 128 else 0)
+    assert tile in (64, 128), "the bf16 pass did not run"
+    assert same(plain, fast)
+    deny = rng.random(n) < 0.6
+    res = []
+    for mode in (-1, 1):
+        capi.check(st.lib.vsag_amd_store_set_scan_contraction(st.handle, mode))
+        res.append(st.flat_scan(q, k, deny=deny))
+    assert same(*res)
+    st.destroy()
+
+
+@pytest.mark.parametrize("bounds", [[0.0, 0.0], [3.0, 1e-30], [-1e18, 1e19], [0.0, -2.0]])
+def test_uniform_bounds_out_of_range_stream(lib, modes, bounds):
+    """A rate of zero, one that makes every distance a denormal number, one whose distances leave fp32: what streaming
+    returns."""
+    rng = np.random.default_rng(3)
+    n, d, nq, k = 5000, 160, 20, 10
+    x = rng.random((n, d), dtype=np.float32)
+    q = rng.random((nq, d), dtype=np.float32)
+    for metric in (orc.L2, orc.IP):
+        codes = orc.squ_encode(x, 8, 0.0, 1.0, metric)
+        st = Store(capi.KIND_SQ8_UNIFORM, metric, d, bounds=bounds)
+        st.append(codes)
+        plain, fast, _ = modes(st, q, k, 1)
+        assert np.array_equal(plain[1].view(np.uint32), fast[1].view(np.uint32))
+        assert np.array_equal(plain[0], fast[0])
         st.destroy()
 
 

@@ -1201,6 +1201,7 @@ int launch_prefilter_rb(const vsag_amd_store* s, const ScanArgs& a, uint64_t nq,
                         uint32_t sub_cap, hipStream_t st);
 
 bool prefilter_i8_supports(const vsag_amd_store* s);
+bool prefilter_b16_supports(const vsag_amd_store* s);
 bool prefilter_h16_supports(const vsag_amd_store* s);
 int launch_prefilter_h16(const vsag_amd_store* s, const ScanArgs& a, uint64_t nq, uint64_t tile_begin, uint64_t tile_end,
                          const uint32_t* bound, float* tau, uint8_t* scratch, uint32_t* cand, uint32_t* cand_cnt,
@@ -1215,7 +1216,7 @@ prefilter_supports(const vsag_amd_store* s) {
         return prefilter_i8_supports(s) || prefilter_h16_supports(s);  // int8 up to 128 dimensions, fp16 beyond
     }
     if (s->kind == VSAG_AMD_KIND_SQ8_UNIFORM || s->kind == VSAG_AMD_KIND_SQ4_UNIFORM) {
-        return prefilter_i8_supports(s);  // the int8 matrix cores or nothing
+        return prefilter_i8_supports(s) || (s->nlist == 0 && prefilter_b16_supports(s));  // bf16 alone beyond 128 dimensions
     }
     return s->nlist == 0 && (s->kind == VSAG_AMD_KIND_FP32 || s->kind == VSAG_AMD_KIND_SQ8) && s->pf_term != nullptr;
 }
@@ -1266,13 +1267,24 @@ prefilter_pays(const vsag_amd_store* s, uint64_t nq, uint32_t k) {
     }
 }
 
-// sq8_uniform: the per-code term of the int8 test, from the code's stored scalar (prefilter_i8.hip).
+// sq8_uniform, sq4_uniform: the per-code term of the tests, from the code's stored scalar (prefilter_i8.hip), and the bits of
+// the largest magnitude among them (prefilter_b16.hip).
 __global__ void __launch_bounds__(256)
-uniform_term_kernel(const uint32_t* meta, uint64_t first, uint64_t count, int is_l2, float lb, float* term) {
+uniform_term_kernel(const uint32_t* meta, uint64_t first, uint64_t count, int is_l2, float lb, float* term, uint32_t* most) {
     const uint64_t i = static_cast<uint64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+    uint32_t bits = 0;
     if (i < count) {
         const float m = __uint_as_float(meta[first + i]);
-        term[first + i] = is_l2 ? m : -(lb * m);
+        const float t = is_l2 ? m : -(lb * m);
+        term[first + i] = t;
+        bits = __float_as_uint(fabsf(t));
+    }
+    for (int off = 32; off > 0; off >>= 1) {
+        const uint32_t o = __shfl_xor(bits, off);
+        bits = o > bits ? o : bits;
+    }
+    if ((threadIdx.x & 63) == 0 && bits > __atomic_load_n(most, __ATOMIC_RELAXED)) {
+        atomicMax(most, bits);
     }
 }
 
@@ -1286,7 +1298,7 @@ launch_code_terms(vsag_amd_store* s, uint64_t first, uint64_t count, hipStream_t
     dim3 grid(static_cast<uint32_t>(div_up(count, 256)));
     if (s->kind == VSAG_AMD_KIND_SQ8_UNIFORM || s->kind == VSAG_AMD_KIND_SQ4_UNIFORM) {
         hipLaunchKernelGGL(uniform_term_kernel, grid, dim3(256), 0, st, s->meta, first, count,
-                           s->metric == VSAG_AMD_METRIC_L2 ? 1 : 0, s->ulb, s->pf_term);
+                           s->metric == VSAG_AMD_METRIC_L2 ? 1 : 0, s->ulb, s->pf_term, s->pf_ymax);
     } else if (s->kind == VSAG_AMD_KIND_SQ8) {
         const float* scale = s->metric == VSAG_AMD_METRIC_L2 ? s->scale_dev : nullptr;
         hipLaunchKernelGGL(code_term_kernel<VSAG_AMD_KIND_SQ8>, grid, dim3(256), 0, st, s->tiles, s->G, scale, first,
@@ -1387,7 +1399,11 @@ launch_rescore_valued(const vsag_amd_store* s, const ScanArgs& a, uint64_t nq, u
     r.row_granules = s->row_granules;
     const dim3 grid(static_cast<uint32_t>(nq));
     const size_t lds = S * 8 + (128 + 256) * 4;
-    if (s->kind == VSAG_AMD_KIND_SQ8) {
+    if (s->kind == VSAG_AMD_KIND_SQ8_UNIFORM) {
+        launch_rescore_m<VSAG_AMD_KIND_SQ8_UNIFORM, true>(s->metric, grid, lds, st, a, r);
+    } else if (s->kind == VSAG_AMD_KIND_SQ4_UNIFORM) {
+        launch_rescore_m<VSAG_AMD_KIND_SQ4_UNIFORM, true>(s->metric, grid, lds, st, a, r);
+    } else if (s->kind == VSAG_AMD_KIND_SQ8) {
         launch_rescore_m<VSAG_AMD_KIND_SQ8, true>(s->metric, grid, lds, st, a, r);
     } else if (s->kind == VSAG_AMD_KIND_SQ4) {
         launch_rescore_m<VSAG_AMD_KIND_SQ4, true>(s->metric, grid, lds, st, a, r);

@@ -1,13 +1,15 @@
-// Pre-selection for query batches on the bf16 matrix cores: flat fp32, sq8 and sq4 stores, fp32 posting lists.
+// Pre-selection for query batches on the bf16 matrix cores: flat fp32, sq8, sq4, sq8_uniform and sq4_uniform stores, fp32
+// posting lists.
 //
 // The inner product <b, c> of a query with a code is formed from two bf16 values per operand, x = h + l + r with h =
 // bf16(x), l = bf16(x - h) and |r| <= 2^-18 |x| (bf16 keeps eight bits, rounded to nearest).  A code byte or nibble is one
 // bf16 value exactly, so
 //   sq8, sq4   <b, c>  ~  <h_b, c> + <l_b, c>                        (b: the query with the scale folded in)
 //   fp32       <a, y>  ~  <h_a, h_y> + <l_a, h_y> + <h_a, l_y>
-// two or three v_mfma_f32_32x32x16_bf16 for sixteen dimensions.  The products are exact in the fp32 accumulator; what is
+//   uniform    <b, c>  =  the integer product of two rows of bytes: one part each
+// one to three v_mfma_f32_32x32x16_bf16 for sixteen dimensions.  The products are exact in the fp32 accumulator; what is
 // left out is known (the remainders of the query are summed, those of an fp32 code are at most 2^-18 of it), so the value
-//   v = |y|^2 - 2 <b, c>  (inner product: -<b, c>)
+//   v = |y|^2 - 2 <b, c>  (inner product: -<b, c>; uniform kinds: -lb sum(c) - rate <b, c>)
 // stands within a bound e of the streaming kernel's distance less the query's constant.  bf16 has the exponent range of
 // fp32: no operand needs a scale, and what is below the normal range may be taken as zero.
 //
@@ -61,38 +63,59 @@ struct B16Layout {
     static constexpr uint32_t kGranules = KIND == VSAG_AMD_KIND_FP32 ? 8 : KIND == VSAG_AMD_KIND_SQ8 ? 4 : 2;  // per stage
 };
 
-// sq8_uniform / sq4_uniform / rabitq stores have integer passes of their own.
+static bool
+b16_uniform(const vsag_amd_store* s) {
+    return s->kind == VSAG_AMD_KIND_SQ8_UNIFORM || s->kind == VSAG_AMD_KIND_SQ4_UNIFORM;
+}
+
+// Posting lists of sq8 / sq4 / uniform codes and rabitq stores have passes of their own.  (Uniform codes: the product of two
+// rows fits the streaming kernel's 32-bit integer.)
 bool
 prefilter_b16_supports(const vsag_amd_store* s) {
-    return (s->kind == VSAG_AMD_KIND_FP32 || s->kind == VSAG_AMD_KIND_SQ8 || s->kind == VSAG_AMD_KIND_SQ4) &&
-           s->pf_term != nullptr && s->pf_ymax != nullptr;
+    const bool kind = s->kind == VSAG_AMD_KIND_FP32 || s->kind == VSAG_AMD_KIND_SQ8 || s->kind == VSAG_AMD_KIND_SQ4 ||
+                      (b16_uniform(s) && s->nlist == 0 && s->dpad <= 8192);
+    return kind && s->pf_term != nullptr && s->pf_ymax != nullptr;
 }
 
 // Whether a batch takes this route of its own accord, measured on Gaussian mixtures against what served it before (us per
 // call, other -> this).
 //   Streaming passes serve four or eight queries at a time: fp32 100k x 768, k 10 4 queries 131 -> 140 (cosine; not taken), 5:
 //   153 -> 139, 8: 281 -> 141, 32: 686 -> 141; k 100 6: 161 -> 234 (not taken), 8: 294 -> 212; sq8 500k x 100 cosine, k 10
-//   2: 62 -> 69 (not taken), 4: 93 -> 68; k 100 4: 79 -> 91 (not taken), 6: 110 -> 92; 1M x 128 16: 259 -> 87.
+//   2: 62 -> 69 (not taken), 4: 93 -> 68; sq4 100k x 960 cosine, k 100 8: 133 -> 143 (not taken), 64: 543 -> 159; sq8 600k x
+//   960 l2, k 100 6: 930 -> 274; 1M x 128 16: 259 -> 87; sq8_uniform (cheap to stream) 200k x 768, k 10 4: 97 -> 102 (not
+//   taken), 6: 108 -> 102, 64: 337 -> 116; k 100 8: 121 -> 138 (not taken), 10: 164 -> 139.
 //   sq8 / sq4 up to 128 dimensions have the int8 matrix cores, twice as fast a product behind a prefix and four levels: 1M x
 //   128, k 10 512 queries 415 -> 362 (not taken from 508 on), 1000 532 -> 653 (not taken); k 100 600 710 -> 568, 1000 802 ->
 //   828 (not taken); k 1 600 370 -> 407 (not taken); 300k 1000 318 -> 269 (not taken), 2000 402 -> 456 (not taken); 100k, k 10
 //   512 231 -> 112, 2000 300 -> 238 (not taken), 4000 354 -> 410 (not taken), k 100 4000 704 -> 490.
 //   Beyond, the fp16 ones, one product where this takes two: sq4 200k x 512 cosine, k 10 1000 508 -> 456, 2000 792 -> 856
 //   (not taken); sq8 600k x 960 ip 256 798 -> 629, 1000 1825 -> 2265 (not taken); 200k x 768, k 100 1000 1504 -> 879.
+//   The uniform kinds take one product here as well: 1M x 128, k 10 1000 queries 517 -> 507 (not taken from 914 on), 100k x
+//   128, 2000 279 -> 172; beyond 128 dimensions they have nothing else (200k x 768, 2000 queries 4221 -> 854; 600k x 960
+//   sq4_uniform, 1000 5790 -> 1312).
 //   A deny mask leaves the streaming kernel alone as the other side.
 // Smaller stores than 81920 codes would gain as well (sq8 70000 x 200, 512 queries 263 -> 121; 70000 x 32, 8 60 -> 47), but
 // the records of a query take 16 KB, several times the streaming kernel's workspace there: batches of those keep it.
 bool
 prefilter_b16_pays(const vsag_amd_store* s, uint64_t nq, uint32_t k, bool masked) {
     const bool fp32 = s->kind == VSAG_AMD_KIND_FP32;
-    if (s->ntiles < 1280 || nq < (fp32 ? (k <= 20 ? 5U : 8U) : (k <= 20 ? 4U : 6U))) {
+    const uint32_t least = fp32             ? (k <= 20 ? 5 : 8)
+                           : b16_uniform(s) ? (k <= 20 ? 5 : 9)
+                                            : (k <= 20 ? 4 : s->metric == VSAG_AMD_METRIC_L2 ? 6 : 9);
+    if (s->ntiles < 1280 || nq < least) {
         return false;
     }
     if (fp32 || masked || nq <= 64) {
         return true;
     }
+    if (b16_uniform(s) && s->dpad > 128) {
+        return true;
+    }
     const double n = static_cast<double>(s->n), work = static_cast<double>(nq) * n * s->dim;
-    return work <= (s->dim <= 128 ? 2.0e10 + 5.0e8 * k + 4.0e10 * log10(n * 1.0e-5) : 1.4e11 + 2.0e9 * k);
+    if (s->dim > 128) {
+        return work <= 1.4e11 + 2.0e9 * k;
+    }
+    return work <= (b16_uniform(s) ? 1.8 : 1.0) * (2.0e10 + 5.0e8 * k + 4.0e10 * log10(n * 1.0e-5));
 }
 
 static uint64_t
@@ -159,9 +182,13 @@ struct B16QueryArgs {
     uint64_t nq, rows;
     uint32_t slots;
     uint4* planes;
-    const uint32_t* ymax_bits;  // largest |y| of the store (l2: scaled codes; ip: raw codes; fp32: the vectors)
+    const uint32_t* ymax_bits;  // largest |y| of the store (l2: scaled codes; ip: raw codes; fp32: the vectors; uniform kinds:
+                                // largest term)
     float cmax;          // largest code value: 255, 15; fp32: 0
     int is_l2;
+    // uniform kinds: qtab holds the query's bytes (nibbles: per eight dimensions a word of the even ones, one of the odd)
+    int uniform, nibbles;
+    float lb, rate;
     const float* qmeta;  // sq8 / sq4, ip: sum q_d lb_d per query
     uint32_t qmeta_stride;
     B16Error* error;     // per query
@@ -187,7 +214,14 @@ b16_query_kernel(B16QueryArgs p) {
         for (int i = 0; i < 8; ++i) {
             const uint32_t d = 8 * s + i;
             const bool in = real && d < p.kdim;
-            const double a = in ? static_cast<double>(row[d]) : 0.0;
+            double a = 0.0;
+            if (in && p.uniform != 0) {
+                const uint32_t* words = reinterpret_cast<const uint32_t*>(row);
+                a = p.nibbles != 0 ? (words[2 * (d >> 3) + (d & 1)] >> (8 * ((d >> 1) & 3))) & 255U
+                                   : (words[d >> 2] >> (8 * (d & 3))) & 255U;
+            } else if (in) {
+                a = static_cast<double>(row[d]);
+            }
             exact[i] = a * (in && p.scale != nullptr ? static_cast<double>(p.scale[d]) : 1.0);
             x[i] = static_cast<float>(exact[i]);
             a2 += a * a;
@@ -220,6 +254,29 @@ b16_query_kernel(B16QueryArgs p) {
     }
     constexpr double kU = 5.9604644775390625e-8;  // 2^-24, the unit roundoff of fp32
     const double kd = static_cast<double>(p.kdim);
+    if (p.uniform != 0) {
+        // No remainders.  l2: v + norm_q is the distance over the rate, whose sign and range keep the order; both forms round
+        // a few times at these magnitudes, and the low four bits of v are cut off.
+        const double qm = static_cast<double>(p.qmeta[q * p.qmeta_stride]);
+        const double term = static_cast<double>(__uint_as_float(*p.ymax_bits)) * (1.0 + 1.0e-6);
+        double sums = static_cast<double>(p.cmax) * a1;  // most <b, c>
+        if (p.is_l2) {
+            sums = fmin(sums, sqrt(a2 * term));  // (|c|^2 is the term)
+        }
+        const double rate = static_cast<double>(p.rate), lb = static_cast<double>(p.lb);
+        const double factor = p.is_l2 ? 2.0 : fabs(rate);
+        // (an integer below 2^24 is exact in the accumulator)
+        const double rounding = sums < 16777216.0 ? 0.0 : 4.0 * kU * (kd / 16.0 + 4.0) * sums;
+        const double magnitude = term + factor * sums + (p.is_l2 ? fabs(qm) : fabs(lb * qm) + lb * lb + 1.0);
+        const double fixed = factor * rounding + 48.0 * kU * magnitude;
+        const bool ordered = p.is_l2 ? rate > 1.0e-30 && rate < 1.0e28 : true;
+        B16Error e;
+        e.constant = static_cast<float>(p.is_l2 ? qm : 1.0 - lb * qm - lb * lb);
+        e.fixed = ordered && magnitude < 1.0e37 ? static_cast<float>(fixed) * 1.000001F + 1.0e-37F : 1.0e38F;
+        e.root = e.slope = 0.0F;
+        p.error[q] = e;
+        return;
+    }
     const double ymax = static_cast<double>(__uint_as_float(*p.ymax_bits)) * (1.0 + 1.0e-6);
     const double an = sqrt(a2);
     const double dots = an * ymax;  // sum |b_d c_d| of any code, by Cauchy and Schwarz
@@ -322,8 +379,9 @@ struct PrefilterB16Args {
     const uint4* planes;
     uint64_t nq, rows;
     uint32_t slots;
-    const float* term;  // per slot |y|^2
-    int is_l2;
+    const float* term;  // per slot |y|^2 (uniform kinds: launch_code_terms)
+    int terms;          // whether v has it: l2, uniform kinds
+    float factor;       // of <b, c> in v
     const float* tau;
     // flat stores
     uint64_t ntiles, n;
@@ -416,7 +474,8 @@ b16_slot(uint32_t ks, uint32_t half) {
     }
 }
 
-template <int KIND, bool LISTS, int JB>
+// ONE: the query has no low part (uniform kinds; KIND says how the codes lie).
+template <int KIND, bool LISTS, int JB, bool ONE = false>
 __global__ void __launch_bounds__(256, JB == 4 || (JB == 2 && KIND == VSAG_AMD_KIND_FP32) ? 2 : 3)
 prefilter_b16_kernel(PrefilterB16Args p) {
     using L = B16Layout<KIND>;
@@ -626,9 +685,9 @@ prefilter_b16_kernel(PrefilterB16Args p) {
                 real = real && slot < p.n && !denied(p.deny, slot);
             }
             my_term = real ? p.term[slot] : kB16Absent;
-            if (!p.is_l2 && my_term < 3.0e38F) {
+            if (p.terms == 0 && my_term < 3.0e38F) {
                 my_term = 0.0F;
-            } else if (!p.is_l2 && real && p.least == nullptr) {
+            } else if (p.terms == 0 && real && p.least == nullptr) {
                 // A code whose norm leaves fp32 (under l2 it stands behind all others) may have any inner product: a
                 // record of every query, and as its value is no number it is always rescored.
                 const uint32_t cols_here =
@@ -672,13 +731,15 @@ prefilter_b16_kernel(PrefilterB16Args p) {
 #pragma unroll
                 for (int j = 0; j < JB; ++j) {
                     const bf16x8 bh = __builtin_bit_cast(bf16x8, sb[buf][slot][0][j * 32 + l32]);
-                    const bf16x8 bl = __builtin_bit_cast(bf16x8, sb[buf][slot][1][j * 32 + l32]);
 #pragma unroll
                     for (int i = 0; i < 2; ++i) {
                         if constexpr (L::kSplit) {
                             acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(al[i][ks], bh, acc[i][j], 0, 0, 0);
                         }
-                        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ah[i][ks], bl, acc[i][j], 0, 0, 0);
+                        if constexpr (!ONE) {
+                            const bf16x8 bl = __builtin_bit_cast(bf16x8, sb[buf][slot][1][j * 32 + l32]);
+                            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ah[i][ks], bl, acc[i][j], 0, 0, 0);
+                        }
                         acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ah[i][ks], bh, acc[i][j], 0, 0, 0);
                     }
                 }
@@ -693,7 +754,6 @@ prefilter_b16_kernel(PrefilterB16Args p) {
         // Nearly nothing passes: sixteen products of a lane share a verdict (their least value).
         code_term[wave][lane] = my_term;
         wave_lds_fence();
-        const float dot_factor = p.is_l2 ? -2.0F : -1.0F;
         float group_least[JB];
 #pragma unroll
         for (int j = 0; j < JB; ++j) {
@@ -718,7 +778,7 @@ prefilter_b16_kernel(PrefilterB16Args p) {
                 float least = __builtin_inff();
 #pragma unroll
                 for (int e = 0; e < 16; ++e) {
-                    const float d = fmaf(dot_factor, acc[i][j][e], term[e]);
+                    const float d = fmaf(p.factor, acc[i][j][e], term[e]);
                     v[e] = __uint_as_float((__float_as_uint(d) & ~15U) | static_cast<uint32_t>(e));
                     least = fminf(least, v[e]);
                 }
@@ -780,13 +840,18 @@ b16_query_args(const vsag_amd_store* s, const ScanArgs& a, uint64_t nq, B16Query
     qa->rows = b16_query_rows(nq);
     qa->slots = b16_slots(s);
     qa->ymax_bits = s->pf_ymax;
-    qa->cmax = fp32 ? 0.0F : s->kind == VSAG_AMD_KIND_SQ8 ? 255.0F : 15.0F;
+    qa->cmax = fp32 ? 0.0F : s->kind == VSAG_AMD_KIND_SQ8 || s->kind == VSAG_AMD_KIND_SQ8_UNIFORM ? 255.0F : 15.0F;
     qa->is_l2 = l2 ? 1 : 0;
-    qa->qmeta = !fp32 && !l2 ? a.qmeta : nullptr;
+    qa->uniform = b16_uniform(s) ? 1 : 0;
+    qa->nibbles = s->kind == VSAG_AMD_KIND_SQ4_UNIFORM ? 1 : 0;
+    qa->lb = s->ulb;
+    qa->rate = s->scalar_rate;
+    qa->scale = b16_uniform(s) ? nullptr : qa->scale;
+    qa->qmeta = (!fp32 && !l2) || b16_uniform(s) ? a.qmeta : nullptr;
     qa->qmeta_stride = a.qmeta_stride;
 }
 
-template <int KIND>
+template <int KIND, bool ONE = false>
 static void
 launch_b16_flat(uint64_t nq, uint32_t cus, PrefilterB16Args p, hipStream_t st) {
     const uint32_t per = nq <= 32 ? 32 : nq <= 64 ? 64 : kB16N;
@@ -798,11 +863,11 @@ launch_b16_flat(uint64_t nq, uint32_t cus, PrefilterB16Args p, hipStream_t st) {
     groups = std::max<uint64_t>(1, std::min<uint64_t>(groups, mtiles));
     const dim3 grid(static_cast<uint32_t>(groups), static_cast<uint32_t>(qtiles));
     if (per == 32) {
-        hipLaunchKernelGGL((prefilter_b16_kernel<KIND, false, 1>), grid, dim3(256), 0, st, p);
+        hipLaunchKernelGGL((prefilter_b16_kernel<KIND, false, 1, ONE>), grid, dim3(256), 0, st, p);
     } else if (per == 64) {
-        hipLaunchKernelGGL((prefilter_b16_kernel<KIND, false, 2>), grid, dim3(256), 0, st, p);
+        hipLaunchKernelGGL((prefilter_b16_kernel<KIND, false, 2, ONE>), grid, dim3(256), 0, st, p);
     } else {
-        hipLaunchKernelGGL((prefilter_b16_kernel<KIND, false, 4>), grid, dim3(256), 0, st, p);
+        hipLaunchKernelGGL((prefilter_b16_kernel<KIND, false, 4, ONE>), grid, dim3(256), 0, st, p);
     }
 }
 
@@ -813,6 +878,10 @@ launch_b16_kind(const vsag_amd_store* s, uint64_t nq, const PrefilterB16Args& p,
         launch_b16_flat<VSAG_AMD_KIND_FP32>(nq, cus, p, st);
     } else if (s->kind == VSAG_AMD_KIND_SQ8) {
         launch_b16_flat<VSAG_AMD_KIND_SQ8>(nq, cus, p, st);
+    } else if (s->kind == VSAG_AMD_KIND_SQ8_UNIFORM) {
+        launch_b16_flat<VSAG_AMD_KIND_SQ8, true>(nq, cus, p, st);
+    } else if (s->kind == VSAG_AMD_KIND_SQ4_UNIFORM) {
+        launch_b16_flat<VSAG_AMD_KIND_SQ4, true>(nq, cus, p, st);
     } else {
         launch_b16_flat<VSAG_AMD_KIND_SQ4>(nq, cus, p, st);
     }
@@ -893,7 +962,8 @@ launch_scan_b16(const vsag_amd_store* s, const ScanArgs& a, uint64_t nq, uint32_
     p.rows = qa.rows;
     p.slots = qa.slots;
     p.term = s->pf_term;
-    p.is_l2 = qa.is_l2;
+    p.terms = qa.is_l2 != 0 || qa.uniform != 0 ? 1 : 0;
+    p.factor = qa.is_l2 != 0 ? -2.0F : qa.uniform != 0 ? -qa.rate : -1.0F;
     p.tau = b.tau;
     p.ntiles = s->ntiles;
     p.n = s->n;
@@ -954,7 +1024,8 @@ launch_ivf_b16(const vsag_amd_store* s, const ScanArgs& a, uint64_t nq, uint32_t
     p.rows = qa.rows;
     p.slots = qa.slots;
     p.term = s->pf_term;
-    p.is_l2 = qa.is_l2;
+    p.terms = qa.is_l2;
+    p.factor = qa.is_l2 != 0 ? -2.0F : -1.0F;
     p.tau = tau;
     if (res_term != nullptr) {
         p.res_term = res_term;

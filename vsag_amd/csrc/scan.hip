@@ -682,9 +682,12 @@ make_call_plan(const vsag_amd_store* s, uint64_t nq, uint32_t k, bool masked, Ca
     if (!forced && (tuned || k > (rb ? 256U : 128U))) {
         return;
     }
+    // (beyond 128 dimensions the uniform kinds have the bf16 route alone)
+    const bool long_uniform =
+        (s->kind == VSAG_AMD_KIND_SQ8_UNIFORM || s->kind == VSAG_AMD_KIND_SQ4_UNIFORM) && !prefilter_i8_supports(s);
     const bool large = forced || (s->ntiles >= 1024 && prefilter_pays(s, nq, k));
     if (prefilter_mode(s) != 2 && prefilter_b16_supports(s) && s->ntiles != 0 &&
-        ((large && (s->kind == VSAG_AMD_KIND_FP32 || masked)) || (!forced && prefilter_b16_pays(s, nq, k, masked)))) {
+        ((large && (s->kind == VSAG_AMD_KIND_FP32 || masked || long_uniform)) || (!forced && prefilter_b16_pays(s, nq, k, masked)))) {
         const uint64_t cap = prefilter_b16_cap(k);
         if (nq * cap * 8 <= (2ull << 30)) {
             c->contraction = c->b16 = true;
@@ -696,7 +699,7 @@ make_call_plan(const vsag_amd_store* s, uint64_t nq, uint32_t k, bool masked, Ca
         }
         // (a batch without room for that many records: shorter lists, level by level)
     }
-    if (!large) {
+    if (!large || long_uniform) {
         return;
     }
     if (masked) {

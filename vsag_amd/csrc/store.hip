@@ -232,8 +232,11 @@ relocate_tiles_kernel(RelocateArgs a) {
 // Stores whose large batches are pre-selected on the matrix cores and rescored (prefilter.hip).
 static bool
 keeps_rows(const vsag_amd_store* s) {
-    // Not fp32 stores: the copy would double the largest of all stores for the smallest gain.
-    return (s->pf_ymax != nullptr && s->kind != VSAG_AMD_KIND_FP32) ||
+    // Not fp32 stores: the copy would double the largest of all stores for the smallest gain.  Nor uniform codes beyond 128
+    // dimensions, of which a few dozen per query are rescored (prefilter_b16.hip).
+    const bool long_uniform =
+        (s->kind == VSAG_AMD_KIND_SQ8_UNIFORM || s->kind == VSAG_AMD_KIND_SQ4_UNIFORM) && s->dpad > 128;
+    return (s->pf_ymax != nullptr && s->kind != VSAG_AMD_KIND_FP32 && !long_uniform) ||
            (s->kind == VSAG_AMD_KIND_RABITQ && s->query_bits == 4);
 }
 
@@ -692,7 +695,7 @@ vsag_amd_store_create(const vsag_amd_store_params_t* p, vsag_amd_store_t** out) 
     }
     // Stores the matrix cores can pre-select on keep a per-code term (and the largest norm, where a threshold needs it).
     if (p->kind == VSAG_AMD_KIND_FP32 || p->kind == VSAG_AMD_KIND_SQ8 || p->kind == VSAG_AMD_KIND_SQ4 ||
-        ((p->kind == VSAG_AMD_KIND_SQ8_UNIFORM || p->kind == VSAG_AMD_KIND_SQ4_UNIFORM) && s->dpad <= 128)) {
+        p->kind == VSAG_AMD_KIND_SQ8_UNIFORM || p->kind == VSAG_AMD_KIND_SQ4_UNIFORM) {
         if (hipMalloc(&s->pf_ymax, 4) != hipSuccess || hipMemset(s->pf_ymax, 0, 4) != hipSuccess) {
             return fail_free(fail(VSAG_AMD_NO_ENOUGH_MEMORY, "hipMalloc of the norm scalar failed"));
         }
