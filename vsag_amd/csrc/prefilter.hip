@@ -386,6 +386,40 @@ prefilter_tau_kernel(const float* qtab, uint32_t qstride, uint32_t kdim, const f
     }
 }
 
+// One candidate per lane against one query: the granules of its code, AHEAD fetched before the first is used.  Whole groups
+// go without a condition on any granule: each condition was a branch, behind which the query's scalars were waited for alone
+// (rescore_kernel, 100k x 768 fp32 cosine, 32 queries: 60 -> 42 us, the call 222 -> 211; 100k x 128 fp32, 1000 queries: 19.4
+// -> 17.9 us).
+template <int KIND, int METRIC, uint32_t AHEAD>
+__device__ __forceinline__ void
+accumulate_code(const ScanArgs& a, const QueryRows<1>& q, const uint4* code, uint32_t stride, Acc<KIND, 1>& acc) {
+    uint4 c[AHEAD];
+    uint32_t j0 = 0;
+    for (; j0 + AHEAD <= a.G; j0 += AHEAD) {
+#pragma unroll
+        for (uint32_t u = 0; u < AHEAD; ++u) {
+            c[u] = code[static_cast<size_t>(j0 + u) * stride];
+        }
+#pragma unroll
+        for (uint32_t u = 0; u < AHEAD; ++u) {
+            accumulate_granule<KIND, METRIC, 1>(a, q, j0 + u, c[u], acc);
+        }
+    }
+    if (j0 < a.G) {
+#pragma unroll
+        for (uint32_t u = 0; u < AHEAD; ++u) {
+            const uint32_t j = j0 + u < a.G ? j0 + u : a.G - 1;
+            c[u] = code[static_cast<size_t>(j) * stride];
+        }
+#pragma unroll
+        for (uint32_t u = 0; u < AHEAD; ++u) {
+            if (j0 + u < a.G) {
+                accumulate_granule<KIND, METRIC, 1>(a, q, j0 + u, c[u], acc);
+            }
+        }
+    }
+}
+
 struct RescoreArgs {
     const uint32_t* cand;
     const uint32_t* cand_cnt;
@@ -475,20 +509,8 @@ rescore_kernel(ScanArgs a, RescoreArgs r) {
             constexpr uint32_t kAhead = VALUED && KIND == VSAG_AMD_KIND_FP32 ? 16
                                        : KIND == VSAG_AMD_KIND_SQ4 ? (METRIC == VSAG_AMD_METRIC_L2 ? 1 : 2)
                                        : (KIND == VSAG_AMD_KIND_SQ8 && METRIC == VSAG_AMD_METRIC_L2 ? 2 : 4);
-            for (uint32_t j0 = 0; j0 < a.G; j0 += kAhead) {
-                uint4 c[kAhead];
-#pragma unroll
-                for (uint32_t u = 0; u < kAhead; ++u) {
-                    const uint32_t j = j0 + u < a.G ? j0 + u : a.G - 1;
-                    c[u] = row != nullptr ? row[j] : a.tiles[(tile * a.G + j) * kWave + ln];
-                }
-#pragma unroll
-                for (uint32_t u = 0; u < kAhead; ++u) {
-                    if (j0 + u < a.G) {
-                        accumulate_granule<KIND, METRIC, 1>(a, qrows, j0 + u, c[u], acc);
-                    }
-                }
-            }
+            accumulate_code<KIND, METRIC, kAhead>(a, qrows, row != nullptr ? row : a.tiles + tile * a.G * kWave + ln,
+                                                  row != nullptr ? 1 : kWave, acc);
             float d[1];
             if (r.row_granules > a.G) {
                 // The metadata words of the code sit behind it in the row: the same words in the same arithmetic, but one
@@ -720,20 +742,7 @@ ivf_rescore_kernel(ScanArgs a, IvfRescoreArgs r) {
             acc_reset(acc);
             constexpr uint32_t kAhead = KIND == VSAG_AMD_KIND_SQ4 ? (METRIC == VSAG_AMD_METRIC_L2 ? 1 : 2)
                                        : (KIND == VSAG_AMD_KIND_SQ8 && METRIC == VSAG_AMD_METRIC_L2 ? 2 : 4);
-            for (uint32_t j0 = 0; j0 < a.G; j0 += kAhead) {
-                uint4 c4[kAhead];
-#pragma unroll
-                for (uint32_t u = 0; u < kAhead; ++u) {
-                    const uint32_t j = j0 + u < a.G ? j0 + u : a.G - 1;
-                    c4[u] = a.tiles[(tile * a.G + j) * kWave + ln];
-                }
-#pragma unroll
-                for (uint32_t u = 0; u < kAhead; ++u) {
-                    if (j0 + u < a.G) {
-                        accumulate_granule<KIND, METRIC, 1>(a, qrows, j0 + u, c4[u], acc);
-                    }
-                }
-            }
+            accumulate_code<KIND, METRIC, kAhead>(a, qrows, a.tiles + tile * a.G * kWave + ln, kWave, acc);
             float d[1];
             finish_distances<KIND, METRIC, 1>(a, qidx, slot, acc, d);
             if (r.res_term != nullptr && have) {
