@@ -331,6 +331,37 @@ def test_residual_lists_match_oracle(lib, kind, metric, mname):
     st.destroy()
 
 
+@pytest.mark.parametrize("nlist,nq,nprobe", [(3, 1, 1), (1024, 341, 24), (1025, 1024, 8), (1500, 1025, 8), (8192, 680, 12),
+                                             (8193, 680, 12)])
+def test_small_batches_are_grouped_in_one_workgroup(lib, nlist, nq, nprobe):
+    """Fewer than 8192 work items: one workgroup groups the pairs by list, with its counters in LDS up to 8192 lists; missing
+    and unknown buckets among them, and pairs that just fill, and just exceed, what the workgroup loads at a time."""
+    rng = np.random.default_rng(nlist + nq)
+    n, d, kcand = 20000, 16, 10
+    x = rng.random((n, d), dtype=np.float32)
+    q = rng.random((nq, d), dtype=np.float32)
+    labels = rng.integers(0, nlist, n).astype(np.int32)
+    labels[:400] = nlist // 2  # a list that is cut into chunks
+    offsets, order = orc.ivf_build_lists(labels, nlist)
+    l, dd = orc.sq_train_uniform(x, 4, orc.L2, mode=3)
+    codes = orc.squ_encode(x, 4, l, dd, orc.L2)
+    st = Store(capi.KIND_SQ4_UNIFORM, orc.L2, d, bounds=[l, dd])
+    st.set_lists(codes, labels, nlist)
+    first = rng.integers(0, nlist, nq)
+    first[::5] = nlist // 2
+    buckets = ((first[:, None] + np.arange(nprobe) * max(1, nlist // nprobe)) % nlist).astype(np.int32)
+    buckets[3::7, nprobe // 2] = -1
+    buckets[4::7, nprobe // 2] = -1
+    unknown = buckets.copy()
+    unknown[4::7, nprobe // 2] = nlist  # no list of that number
+    ids, ds = st.ivf_scan(q, unknown, kcand)
+    rids, rds = orc.ivf_scan(orc.SQ4U, orc.L2, d, codes[order], offsets, order, orc.squ_encode(q, 4, l, dd, orc.L2), buckets,
+                             kcand, lb=l, diff=dd)
+    assert np.array_equal(ds.view(np.uint32), rds.view(np.uint32))
+    assert_topk_close(ids, ds, rids, rds, rtol=0, atol=0, tie_rtol=0, label="small batch")
+    st.destroy()
+
+
 @pytest.mark.parametrize("nq,kcand", [(40, 32), (40, 33), (6000, 32), (6000, 7)])
 def test_a_list_probed_twice_brings_every_key_twice(lib, nq, kcand):
     """Injected buckets may name a list twice; then every (distance, id) key exists twice, also the k-th one, and the
