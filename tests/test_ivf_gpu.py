@@ -362,6 +362,30 @@ def test_small_batches_are_grouped_in_one_workgroup(lib, nlist, nq, nprobe):
     st.destroy()
 
 
+@pytest.mark.parametrize("kind,metric", [("fp32", orc.L2), ("fp32", orc.IP), ("sq8", orc.IP)])
+@pytest.mark.parametrize("nq,kcand", [(1949, 20), (1950, 20), (1950, 1), (1950, 256), (1950, 257)])
+def test_middling_batches_of_finer_items(lib, kind, metric, nq, kcand):
+    """15 600 pairs and more cut their lists finer: a batch's rows equal those of the same queries a few at a time."""
+    rng = np.random.default_rng(kcand)
+    n, d, nlist, nprobe = 40000, 20, 64, 8
+    x, q, cent, labels = _ivf_case(rng, n, d, nlist, nq)
+    if kind == "sq8":
+        lb, diff = orc.sq_train(x, 8, metric)
+        codes = orc.sq_encode(x, 8, lb, diff, metric)
+        st = Store(capi.KIND_SQ8, metric, d, lb=lb, diff=diff)
+    else:
+        codes = x.view(np.uint8).reshape(n, 4 * d)
+        st = Store(capi.KIND_FP32, metric, d)
+    st.set_lists(codes, labels, nlist)
+    buckets, _ = orc.ivf_route(cent, q, nprobe)
+    ids, ds = st.ivf_scan(q, buckets, kcand)
+    for i in range(0, nq, 650):
+        part = slice(i, i + 64)
+        few, fd = st.ivf_scan(q[part], buckets[part], kcand)
+        assert np.array_equal(ids[part], few) and np.array_equal(ds[part].view(np.uint32), fd.view(np.uint32))
+    st.destroy()
+
+
 @pytest.mark.parametrize("nq,kcand", [(40, 32), (40, 33), (6000, 32), (6000, 7)])
 def test_a_list_probed_twice_brings_every_key_twice(lib, nq, kcand):
     """Injected buckets may name a list twice; then every (distance, id) key exists twice, also the k-th one, and the

@@ -598,7 +598,7 @@ struct IvfBuffers {
 constexpr uint32_t kGatedPairsCap = 32768;
 
 static void
-plan_ivf(const vsag_amd_store* s, uint64_t nq, uint32_t nprobe, uint32_t kcand, ScanPlanIvf* p) {
+plan_ivf(const vsag_amd_store* s, uint64_t nq, uint32_t nprobe, uint32_t kcand, ScanPlanIvf* p, bool fine = true) {
     p->S = selector_slots(kcand);
     uint64_t npairs = nq * nprobe;
     uint64_t avg = s->nlist ? npairs / s->nlist : 1;
@@ -620,13 +620,20 @@ plan_ivf(const vsag_amd_store* s, uint64_t nq, uint32_t nprobe, uint32_t kcand, 
     // Enough (list, query group) items to fill the machine: every item walks its whole list, the nearest list
     // of every query goes first.  Otherwise lists are cut into chunks of at least four tiles for about 4096 items in all (a probed
     // list is taken as twice the average length), at most 64 chunks per list and 256 MiB of partial lists.
+    // fp32 and sq8 codes against four queries an item make long items of many registers: from some 15 600 pairs on four times
+    // as many keep the machine evenly busy to the end (fp32 l2 200k x 200, 512 lists, k 20, 1000 queries x 24: 480 -> 414 us,
+    // k 100 568 -> 497; 200k x 768 1471 -> 1245; ip 1M x 96 459 -> 372; sq8 ip 200k x 200, 80 candidates, 457 -> 415; 42
+    // points of these kinds, 1.02 times slower at most).  Fewer pairs lose (200k x 768, 1000 x 8: 646 -> 731), and so do two queries an
+    // item (sq8 l2 1M x 96, 200 candidates, 2000 x 8: 1046 -> 1139; rabitq 590 -> 668) and sq4_uniform codes (533 -> 595).
     const uint64_t groups = div_up(npairs, static_cast<uint64_t>(t));
     p->chunked = groups < 8192 && s->max_list_tiles > 2;
     p->tiles_per_item = 0xFFFFFFFFU;
     p->chunks_max = 1;
     if (p->chunked) {
         const uint64_t avg_tiles = std::max<uint64_t>(1, s->nlist ? s->ntiles / s->nlist : 1);
-        const uint64_t tpi = std::max<uint64_t>(4, div_up(groups * avg_tiles * 2, 4096));
+        const bool four = fine && t == 4 && groups >= 3900 && kcand <= 256 &&
+                          (s->kind == VSAG_AMD_KIND_FP32 || s->kind == VSAG_AMD_KIND_SQ8);
+        const uint64_t tpi = std::max<uint64_t>(4, div_up(groups * avg_tiles * 2, four ? 16384 : 4096));
         uint64_t cap = std::min<uint64_t>(64, div_up(s->max_list_tiles, tpi));
         while (cap > 1 && npairs * cap * kcand * 8 > (256ull << 20)) {
             cap /= 2;
@@ -765,6 +772,11 @@ vsag_amd_ivf_scan_topk_ex(const vsag_amd_store_t* s, const float* queries_dev, u
     Carver c(workspace_dev, workspace_bytes);
     IvfBuffers b;
     carve_ivf(c, s, p, nq, kcand, &b);
+    if (!c.ok()) {  // (sized for another batch: without room for four times the chunks)
+        plan_ivf(s, nq, nprobe, kcand, &p, false);
+        c = Carver(workspace_dev, workspace_bytes);
+        carve_ivf(c, s, p, nq, kcand, &b);
+    }
     VA_CHECK_ARG(c.ok(), "workspace too small: need %zu bytes, got %zu", c.used, workspace_bytes);
 
     // Row nq of the query tables is the all-zero row that idle slots of a query tile point at.
