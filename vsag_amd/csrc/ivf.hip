@@ -622,7 +622,7 @@ plan_ivf(const vsag_amd_store* s, uint64_t nq, uint32_t nprobe, uint32_t kcand, 
     // list is taken as twice the average length), at most 64 chunks per list and 256 MiB of partial lists.
     // fp32 and sq8 codes against four queries an item make long items of many registers: from some 15 600 pairs on four times
     // as many keep the machine evenly busy to the end (fp32 l2 200k x 200, 512 lists, k 20, 1000 queries x 24: 480 -> 414 us,
-    // k 100 568 -> 497; 200k x 768 1471 -> 1245; ip 1M x 96 459 -> 372; sq8 ip 200k x 200, 80 candidates, 457 -> 415; 42
+    // k 100 568 -> 497; 200k x 768 1471 -> 1245; ip 1M x 96 459 -> 372; sq8 ip 200k x 200, 80 candidates, 457 -> 415; 60
     // points of these kinds, 1.02 times slower at most).  Fewer pairs lose (200k x 768, 1000 x 8: 646 -> 731), and so do two queries an
     // item (sq8 l2 1M x 96, 200 candidates, 2000 x 8: 1046 -> 1139; rabitq 590 -> 668) and sq4_uniform codes (533 -> 595).
     const uint64_t groups = div_up(npairs, static_cast<uint64_t>(t));
