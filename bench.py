@@ -457,14 +457,18 @@ def run_c1(env):
             "algorithmic_bytes_per_launch": algo, "flops_per_launch": 2.0 * n * d * nq,
             "tflops": 2.0 * n * d * nq / (kms * 1e-3) / 1e12}
     if tile >= 64:
-        # The timed kernel is the last level of the contraction: bpp bytes of fp32 codes against every query.
+        # The timed kernel is the contraction (its last level): bpp bytes of fp32 codes against every query.
         codes = bpp / (4.0 * d)
         tf = 2.0 * codes * d * nq / (kms * 1e-3) / 1e12
-        roof = {"bound": "mfma", "achieved": tf, "peak": MFMA_F32_PEAK_TFLOPS, "unit": "TFLOP/s",
-                "frac": tf / MFMA_F32_PEAK_TFLOPS,
+        # (the bf16 matrix cores, three products a pair, over all codes, unless --contraction 2 keeps the fp32 ones)
+        bf16 = args.contraction != 2
+        peak = MFMA_F16_PEAK_TFLOPS if bf16 else MFMA_F32_PEAK_TFLOPS
+        roof = {"bound": "mfma", "achieved": tf, "peak": peak, "unit": "TFLOP/s", "frac": tf / peak,
+                "executed_frac": (3.0 if bf16 else 1.0) * tf / peak,
                 # rocprofv3 --pmc FETCH_SIZE (x 2.00) + WRITE_SIZE of this launch: profiles/prefilter_fp32_c1.md
-                "traffic": 87735.7 * 2.00 * 1024 + 23281.8 * 1024 if (n, d, nq, k) == (100000, 128, 1000, 10) else None,
-                "kernel": "prefilter_kernel<fp32> (fp32 MFMA, last level)", "kernel_ms": kms,
+                "traffic": 87735.7 * 2.00 * 1024 + 23281.8 * 1024 if not bf16 and (n, d, nq, k) == (100000, 128, 1000, 10) else None,
+                "kernel": "prefilter_b16_kernel<fp32> (bf16 MFMA, all codes)" if bf16 else
+                          "prefilter_kernel<fp32> (fp32 MFMA, last level)", "kernel_ms": kms,
                 "flops_per_launch": 2.0 * codes * d * nq, "codes_per_launch": codes}
     return env.base_line("QPS @ recall@10 (100k x 128 fp32 brute force)", "queries/s", nq / sec, sec, "f32",
                          "configs[0]: brute_force fp32 L2, N=%d, d=%d, %d queries, k=%d" % (n, d, nq, k),
@@ -807,19 +811,20 @@ def run_c4(env):
         tops = ops / (kms * 1e-3) / 1e12
         # (sq8 lists beyond 128 dimensions: the fp16 matrix cores, unless --contraction 2 keeps the fp32 ones)
         h16 = per_dim and d > 128 and bits == 8 and args.contraction != 2
-        peak = (MFMA_F16_PEAK_TFLOPS if h16 else MFMA_F32_PEAK_TFLOPS if raw32 or (per_dim and d > 128) else
+        b16 = raw32 and args.contraction != 2  # fp32 lists: three bf16 products a pair
+        peak = (MFMA_F16_PEAK_TFLOPS if h16 or b16 else MFMA_F32_PEAK_TFLOPS if raw32 or (per_dim and d > 128) else
                 MFMA_F6F4_PEAK_TFLOPS if one_bit else MFMA_I8_PEAK_TOPS)
         roof = {"bound": "mfma", "achieved": tops, "peak": peak, "unit": "TOP/s" if peak == MFMA_I8_PEAK_TOPS else "TFLOP/s",
                 "frac": tops / peak,
                 # rocprofv3 --pmc FETCH_SIZE (x 2.00) + WRITE_SIZE of this launch: profiles/ivf_i8_sq4u_c4.md
                 "traffic": 491061.0 * 2.00 * 1024 + 73550.7 * 1024
                 if (n, d, nq, k, nlist, bits) == (10000000, 128, 10000, 10, 4096, 4) else None,
-                "kernel": "%s<%s> (%s MFMA, probe columns 1..%d)" % ("ivf_h16_kernel" if h16 else
+                "kernel": "%s<%s> (%s MFMA, probe columns 1..%d)" % ("ivf_h16_kernel" if h16 else "prefilter_b16_kernel<lists>" if b16 else
                                                                         "ivf_f32_kernel" if peak == MFMA_F32_PEAK_TFLOPS else
                                                                         "ivf_pq_kernel" if pqfs else
                                                                         "prefilter_rb_kernel<lists>" if one_bit else
                                                                         "ivf_sq8_i8_kernel" if per_dim else "ivf_i8_kernel",
-                                                                        kind_name, "fp16" if h16 else
+                                                                        kind_name, "fp16" if h16 else "bf16" if b16 else
                                                                         "fp32" if peak == MFMA_F32_PEAK_TFLOPS else
                                                                         "fp4 x fp6" if one_bit else "int8",
                                                                         nprobe - 1), "kernel_ms": kms,
