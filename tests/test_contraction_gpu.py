@@ -427,6 +427,33 @@ def test_fp32_on_the_bf16_matrix_cores(lib, modes, metric, n, d, nq, k):
         st.destroy()
 
 
+def _near_one(units):
+    return np.float32(1 + units * 2.0 ** -16)
+
+
+@pytest.mark.parametrize("metric", [orc.L2, orc.IP])
+@pytest.mark.parametrize("d", [16, 20, 48, 64, 128])
+def test_rows_that_two_bf16_values_miss_by_as_much_as_they_can(lib, modes, metric, d):
+    """1 + 254.5 units of 2^-16 loses nearly 2^-17 of itself and has a low part of nearly 2^-8, and so, with the other sign,
+    has what lies as far below 1 + 2^-7.  The best row's products come out too small in every dimension, the others' too
+    large: the best must still be among the records."""
+    n, nq = 1500, 40
+    x = np.full((n, d), _near_one(512 - 254.5), np.float32)
+    q = np.full((nq, d), _near_one(254), np.float32)
+    x[700] = _near_one(254.5)
+    if metric == orc.IP:
+        q[:, -1] = 1
+        x[:, -1] = 0
+        lead = (x[0, :-1].astype(np.float64) - x[700, :-1]) @ q[0, :-1].astype(np.float64)
+        x[700, -1] = np.float16(1.05 * lead)  # (no more bits than a bf16 value's two parts hold)
+    st = Store(capi.KIND_FP32, metric, d)
+    st.append(x.view(np.uint8).reshape(n, -1))
+    plain, fast, tile = modes(st, q, 1)
+    assert tile == 128, "the contraction path did not run"
+    assert np.all(plain[0] == 700) and same(plain, fast)
+    st.destroy()
+
+
 @pytest.mark.parametrize("kind", ["fp32", "sq8"])
 def test_many_short_tiles_per_workgroup(lib, modes, kind):
     """100000 x 128 against 1000 queries: every workgroup walks many code tiles with a short contraction each, so

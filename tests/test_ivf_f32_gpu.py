@@ -145,3 +145,22 @@ def test_residual_lists_on_the_matrix_cores_equal_streaming(lib, metric, kind, n
         direct.destroy()
     cb.free()
     st.destroy()
+
+
+@pytest.mark.parametrize("metric,d", [(orc.L2, 16), (orc.L2, 64), (orc.L2, 128), (orc.IP, 16), (orc.IP, 32)])
+def test_rows_that_two_bf16_values_miss_by_as_much_as_they_can(lib, metric, d):
+    """The first list gives the bound, a little behind the best row, which the second list holds: 1 + 254.5 units of 2^-16
+    loses nearly 2^-17 of itself in the split and has a low part of nearly 2^-8, and its products come out too small in every
+    dimension.  (One more row there would overflow the records of one candidate, and the query would stream.)"""
+    near = lambda units: np.float32(1 + units * 2.0 ** -16)  # noqa: E731
+    n, nq = 80, 64
+    x = np.full((n, d), 0.1, np.float32)
+    labels = np.where(np.arange(n) < 40, 0, 1).astype(np.int32)
+    q = np.full((nq, d), near(254), np.float32)
+    x[0] = near(253.45) if metric == orc.L2 else near(254.4)
+    x[50] = near(254.5)
+    st = Store(capi.KIND_FP32, metric, d)
+    st.set_lists(x.view(np.uint8).reshape(n, 4 * d), labels, 2)
+    plain, fast = _both(lib, st, q, np.tile(np.int32([0, 1]), (nq, 1)), 1)
+    assert np.all(plain[0] == 50) and _same(plain, fast)
+    st.destroy()

@@ -2,13 +2,14 @@
 // posting lists.
 //
 // The inner product <b, c> of a query with a code is formed from two bf16 values per operand, x = h + l + r with h =
-// bf16(x), l = bf16(x - h) and |r| <= 2^-18 |x| (bf16 keeps eight bits, rounded to nearest).  A code byte or nibble is one
-// bf16 value exactly, so
+// bf16(x), l = bf16(x - h), |l| <= 2^-8 |x| and |r| <= 2^-17 |x| (bf16 keeps eight bits, rounded to nearest: half a unit in
+// the last place is 2^-8 of the power of two below x, and of l at most 2^-9 of 2^-8).  A code byte or nibble is one bf16
+// value exactly, so
 //   sq8, sq4   <b, c>  ~  <h_b, c> + <l_b, c>                        (b: the query with the scale folded in)
 //   fp32       <a, y>  ~  <h_a, h_y> + <l_a, h_y> + <h_a, l_y>
 //   uniform    <b, c>  =  the integer product of two rows of bytes: one part each
 // one to three v_mfma_f32_32x32x16_bf16 for sixteen dimensions.  The products are exact in the fp32 accumulator; what is
-// left out is known (the remainders of the query are summed, those of an fp32 code are at most 2^-18 of it), so the value
+// left out is known (the remainders of the query are summed, those of an fp32 code are at most 2^-17 of it), so the value
 //   v = |y|^2 - 2 <b, c>  (inner product: -<b, c>; uniform kinds: -lb sum(c) - rate <b, c>)
 // stands within a bound e of the streaming kernel's distance less the query's constant.  bf16 has the exponent range of
 // fp32: no operand needs a scale, and what is below the normal range may be taken as zero.
@@ -54,6 +55,9 @@ constexpr uint32_t kB16Pad = 64;    // the query table covers whole stages of ei
 constexpr float kB16Absent = 3.3e38F;  // |y|^2 of a slot that cannot be found: above every threshold (3e38 at most), and no
                                        // infinity, which four other low bits would make a NaN that hides the fifteen others
 constexpr uint32_t kB16CountStride = 32;  // words between the queries' record counters: atomics on one memory line take turns
+// What the two parts of a value can miss of it, and its low part: 2^-17 and 2^-8, and a little for their own rounding.
+constexpr double kB16Left = 7.7e-6;
+constexpr double kB16Low = 3.92e-3;
 constexpr uint32_t kB16Queue = 128; // records a wave gathers in LDS before it asks for room in the queries' lists
 
 template <int KIND>
@@ -283,9 +287,9 @@ b16_query_kernel(B16QueryArgs p) {
     const bool fp32 = p.cmax == 0.0F;
     const double sums = fp32 || p.is_l2 ? dots : fmin(static_cast<double>(p.cmax) * a1, dots);
     const double factor = p.is_l2 ? 2.0 : 1.0;
-    // Left out: the remainders of the query against a code (codes of bytes lie in [0, cmax]); of an fp32 code at most 2^-18
-    // of it against the query, and its low part (2^-9 of it) against the query's.
-    const double split = fp32 ? ymax * (sqrt(r2) + 3.9e-6 * an + 1.97e-3 * sqrt(l2)) : static_cast<double>(p.cmax) * r1;
+    // Left out: the remainders of the query against a code (codes of bytes lie in [0, cmax]); of an fp32 code at most
+    // kB16Left of it against the query, and its low part (kB16Low of it) against the query's.
+    const double split = fp32 ? ymax * (sqrt(r2) + kB16Left * an + kB16Low * sqrt(l2)) : static_cast<double>(p.cmax) * r1;
     // The accumulation: four roundings of the absolute sum per instruction (two or three per sixteen dimensions).
     const double rounding = 4.0 * kU * ((fp32 ? 3.0 : 2.0) * kd / 16.0 + 4.0) * sums;
     // Operands below the normal range taken as zero; fma(factor, acc, term) and |y|^2 rounded, the low four bits cut off.
