@@ -164,3 +164,28 @@ def test_rows_that_two_bf16_values_miss_by_as_much_as_they_can(lib, metric, d):
     plain, fast = _both(lib, st, q, np.tile(np.int32([0, 1]), (nq, 1)), 1)
     assert np.all(plain[0] == 50) and _same(plain, fast)
     st.destroy()
+
+
+@pytest.mark.parametrize("metric", [orc.L2, orc.IP])
+@pytest.mark.parametrize("kcand", [3, 50, 70])
+def test_products_that_leave_fp32(lib, metric, kcand):
+    """Queries whose products with a stored row are no fp32 numbers any more: infinite distances of either sign and no
+    numbers come out as the streaming scan has them, every row once.  (70 candidates: the lists are too short to overflow.)"""
+    rng = np.random.default_rng(3)
+    n, d, nq = 100, 24, 64
+    x = rng.standard_normal((n, d)).astype(np.float32)
+    labels = np.where(np.arange(n) < 50, 0, 1).astype(np.int32)
+    x[51:57, 0] = 1e19
+    x[60:63, :2] = 1e19
+    x[70:75, 1] = 1e38   # a norm whose square is no fp32 number
+    q = rng.standard_normal((nq, d)).astype(np.float32)
+    q[::2, 0] = 1e25
+    q[1::4, 0] = -1e25
+    q[::8, 1] = -1e25    # inf - inf against rows 60 to 62
+    q[3::8, 1] = 2
+    st = Store(capi.KIND_FP32, metric, d)
+    st.set_lists(x.view(np.uint8).reshape(n, 4 * d), labels, 2)
+    plain, fast = _both(lib, st, q, np.tile(np.int32([0, 1]), (nq, 1)), kcand)
+    assert np.array_equal(plain[0], fast[0])
+    assert np.array_equal(plain[1].view(np.uint32), fast[1].view(np.uint32))
+    st.destroy()

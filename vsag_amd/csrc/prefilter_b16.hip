@@ -52,13 +52,18 @@ typedef float floatx16 __attribute__((ext_vector_type(16)));
 
 constexpr uint32_t kB16N = 128;     // most queries per workgroup tile; the rows of the query table are padded to it
 constexpr uint32_t kB16Pad = 64;    // the query table covers whole stages of either length
-constexpr float kB16Absent = 3.3e38F;  // |y|^2 of a slot that cannot be found: above every threshold (3e38 at most), and no
-                                       // infinity, which four other low bits would make a NaN that hides the fifteen others
+// |y|^2 of a slot that cannot be found: a quiet NaN, which no product carries below a threshold, no minimum takes and four
+// other low bits leave a quiet NaN.  (A number above every threshold comes down with a large enough product, and the slots
+// past a list's end, which multiply the codes of another, lie outside the store.)
+constexpr float kB16Absent = __builtin_nanf("");
 constexpr uint32_t kB16CountStride = 32;  // words between the queries' record counters: atomics on one memory line take turns
 // What the two parts of a value can miss of it, and its low part: 2^-17 and 2^-8, and a little for their own rounding.
 constexpr double kB16Left = 7.7e-6;
 constexpr double kB16Low = 3.92e-3;
 constexpr uint32_t kB16Queue = 128; // records a wave gathers in LDS before it asks for room in the queries' lists
+
+constexpr uint32_t kIvfB16ChunkTiles = 32;  // as ivf_i8.hip: kIvfI8ChunkTiles, kIvfI8Chunks
+constexpr uint32_t kIvfB16Chunks = 4;
 
 template <int KIND>
 struct B16Layout {
@@ -200,6 +205,10 @@ struct B16QueryArgs {
     const uint32_t* bound;
     float* tau;
     float* magnitude;    // residual lists: the query's magnitudes (see IvfF32Args in prefilter.hip), or null
+    // queries that stream: their flags, then how many; their pairs' first private list of k records is marked as overflowed
+    uint32_t* gate;
+    uint32_t* partial_cnt;
+    uint32_t p0, nprobe, k;
 };
 
 // One wave per row of the query table (rows at or beyond nq: zeros).
@@ -295,7 +304,7 @@ b16_query_kernel(B16QueryArgs p) {
     // Operands below the normal range taken as zero; fma(factor, acc, term) and |y|^2 rounded, the low four bits cut off.
     const double flushed = kd * 4.7e-38 * (an + ymax + 1.0);
     const double test = 36.0 * kU * ((p.is_l2 ? ymax * ymax : 0.0) + factor * dots);
-    // (A product that can leave fp32 would carry a slot that cannot be found past its |y|^2: such a query streams.)
+    // (Where a product can leave fp32, or with entries that are not finite, the query streams.)
     double fixed = factor * dots < 1.0e37 ? factor * (split + rounding) + flushed + test : 1.0e39;
     double root = 0.0, slope = 0.0;
     double constant = a2;
@@ -321,13 +330,24 @@ b16_query_kernel(B16QueryArgs p) {
     if (p.tau == nullptr) {
         return;
     }
+    if (!(fixed < 1.0e37)) {
+        // Nothing passes, and the query streams.  (A product beyond fp32 would be an infinity with other low bits: a NaN, and
+        // the code lost.)
+        p.tau[q] = kB16Absent;
+        p.gate[q] = 1;
+        atomicAdd(&p.gate[p.nq], 1U);
+        for (uint32_t c = p.p0; c < p.nprobe; ++c) {
+            p.partial_cnt[(q * p.nprobe + c) * 2 * kIvfB16Chunks] = p.k + 1;
+        }
+        return;
+    }
     const uint32_t b = p.bound[q];
     const double bd = static_cast<double>(ordered_to_float(b));
     const double t = bd - constant + fixed + 1.01 * (root * sqrt(fabs(bd)) + slope * fabs(bd)) +
                      1.0e-6 * (fabs(bd) + fabs(constant));
     const float tf = static_cast<float>(t);
     const float up = tf + fabsf(tf) * 1.2e-7F + 1.0e-37F;
-    // no bound yet, or entries that are not finite: everything is a candidate (and the query overflows)
+    // no bound yet: everything is a candidate (and the query overflows, or its lists are short)
     const bool open = b == 0xFFFFFFFFU || !(up < 3.0e38F);
     p.tau[q] = open ? 3.0e38F : up;
     if (p.magnitude != nullptr) {
@@ -413,9 +433,6 @@ struct PrefilterB16Args {
     uint32_t* partial_cnt;
     uint32_t* gate;
 };
-
-constexpr uint32_t kIvfB16ChunkTiles = 32;  // as ivf_i8.hip: kIvfI8ChunkTiles, kIvfI8Chunks
-constexpr uint32_t kIvfB16Chunks = 4;
 
 // The codes of one stage of a wave, in registers: of both blocks of 32 codes, the granules this lane multiplies.
 template <int KIND>
@@ -689,9 +706,9 @@ prefilter_b16_kernel(PrefilterB16Args p) {
                 real = real && slot < p.n && !denied(p.deny, slot);
             }
             my_term = real ? p.term[slot] : kB16Absent;
-            if (p.terms == 0 && my_term < 3.0e38F) {
-                my_term = 0.0F;
-            } else if (p.terms == 0 && real && p.least == nullptr) {
+            const bool found = my_term < 3.0e38F;
+            my_term = !found ? kB16Absent : p.terms == 0 ? 0.0F : my_term;
+            if (real && !found && p.terms == 0 && p.least == nullptr) {
                 // A code whose norm leaves fp32 (under l2 it stands behind all others) may have any inner product: a
                 // record of every query, and as its value is no number it is always rescored.
                 const uint32_t cols_here =
@@ -700,9 +717,6 @@ prefilter_b16_kernel(PrefilterB16Args p) {
                     record(col, LISTS ? (static_cast<uint64_t>(wave >> 1) << 32) | static_cast<uint32_t>(slot)
                                       : (0xFFFFFFFFULL << 32) | static_cast<uint32_t>(slot));
                 }
-                my_term = kB16Absent;
-            } else if (!(my_term < 3.0e38F)) {
-                my_term = kB16Absent;
             }
             if (LISTS && real && p.res_bias != nullptr) {
                 my_term -= p.res_bias[slot];
@@ -1007,7 +1021,7 @@ ivf_b16_scratch_bytes(const vsag_amd_store* s, uint64_t nq) {
 
 // The candidates of probe columns [p0, nprobe) grouped by list (pair_off, sorted_pair; item_off counted with
 // ivf_b16_pairs_per_item() pairs per item) into the private lists (pair * 8 + chunk * 2 + half of the code tile) of
-// kcand records in `partial`; partial_cnt zero before.  tau: 2 nq + 1 floats; gate: nq + 2 words.
+// kcand records in `partial`; partial_cnt and gate zero before.  tau: 2 nq + 1 floats; gate: nq + 2 words.
 int
 launch_ivf_b16(const vsag_amd_store* s, const ScanArgs& a, uint64_t nq, uint32_t nprobe, uint32_t p0, const uint32_t* pair_off,
                const uint32_t* item_off, const uint32_t* sorted_pair, const uint32_t* bound, uint32_t kcand, float* tau,
@@ -1018,6 +1032,11 @@ launch_ivf_b16(const vsag_amd_store* s, const ScanArgs& a, uint64_t nq, uint32_t
     qa.planes = reinterpret_cast<uint4*>(scratch);
     qa.bound = bound;
     qa.tau = tau;
+    qa.gate = gate;
+    qa.partial_cnt = partial_cnt;
+    qa.p0 = p0;
+    qa.nprobe = nprobe;
+    qa.k = kcand;
     qa.magnitude = res_term != nullptr ? tau + nq + 1 : nullptr;
     hipLaunchKernelGGL(b16_query_kernel, dim3(static_cast<uint32_t>(qa.rows)), dim3(kWave), 0, st, qa);
     PrefilterB16Args p{};
