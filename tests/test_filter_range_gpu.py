@@ -77,6 +77,34 @@ def test_masked_batches_on_the_bf16_matrix_cores(lib, kind, metric, n, d, nq, k,
     st.destroy()
 
 
+@pytest.mark.parametrize("metric", [orc.L2, orc.IP])
+@pytest.mark.parametrize("value", [5e18, 1e30, np.inf, np.nan])
+def test_allowed_rows_whose_squared_norm_leaves_fp32_are_found(lib, metric, value):
+    """Three ordinary rows and six far ones are allowed, ten are asked for: all nine come out, as by streaming."""
+    rng = np.random.default_rng(9)
+    n, d, nq, k = 5000, 24, 40, 10
+    x = rng.standard_normal((n, d)).astype(np.float32)
+    q = rng.standard_normal((nq, d)).astype(np.float32)
+    far = np.arange(100, 106)
+    x[far] = value
+    deny = np.ones(n, bool)
+    deny[far] = False
+    deny[[7, 400, 4999]] = False
+    st = Store(capi.KIND_FP32, metric, d)
+    st.append(x.view(np.uint8).reshape(n, -1))
+    res = []
+    try:
+        for mode in (-1, 1):
+            capi.check(st.lib.vsag_amd_set_scan_contraction(mode))
+            res.append(st.flat_scan(q, k, deny=deny))
+    finally:
+        capi.check(st.lib.vsag_amd_set_scan_contraction(0))
+    assert all(set(far) <= set(ids) for ids in res[0][0])
+    assert np.array_equal(res[0][0], res[1][0])
+    assert np.array_equal(res[0][1].view(np.uint32), res[1][1].view(np.uint32))
+    st.destroy()
+
+
 def test_denied_codes_stay_hidden_where_products_overflow(lib):
     """Products of denied codes with a query leave fp32: they must not pass for the best of all."""
     rng = np.random.default_rng(5)

@@ -189,3 +189,20 @@ def test_products_that_leave_fp32(lib, metric, kcand):
     assert np.array_equal(plain[0], fast[0])
     assert np.array_equal(plain[1].view(np.uint32), fast[1].view(np.uint32))
     st.destroy()
+
+
+@pytest.mark.parametrize("metric", [orc.L2, orc.IP])
+@pytest.mark.parametrize("value", [5e18, np.inf, np.nan])
+def test_rows_whose_squared_norm_leaves_fp32_are_found(lib, metric, value):
+    """Fewer ordinary rows than are asked for: the far ones of the second list come out behind them, as by streaming."""
+    rng = np.random.default_rng(4)
+    n, d, nq, kcand = 100, 24, 64, 95
+    x = rng.standard_normal((n, d)).astype(np.float32)
+    labels = np.where(np.arange(n) < 50, 0, 1).astype(np.int32)
+    x[50:60] = value
+    q = rng.standard_normal((nq, d)).astype(np.float32)
+    st = Store(capi.KIND_FP32, metric, d)
+    st.set_lists(x.view(np.uint8).reshape(n, 4 * d), labels, 2)
+    plain, fast = _both(lib, st, q, np.tile(np.int32([0, 1]), (nq, 1)), kcand)
+    assert _same(plain, fast)
+    st.destroy()

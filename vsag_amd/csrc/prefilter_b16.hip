@@ -57,6 +57,10 @@ constexpr uint32_t kB16Pad = 64;    // the query table covers whole stages of ei
 // past a list's end, which multiply the codes of another, lie outside the store.)
 constexpr float kB16Absent = __builtin_nanf("");
 constexpr uint32_t kB16CountStride = 32;  // words between the queries' record counters: atomics on one memory line take turns
+// Thresholds end at kB16Closed: a code of |y|^2 from 3e38 on (l2) is further than that, with products of 1e37 at most.  Beyond
+// it, and where nothing bounds a query, a threshold is kB16Open, and every code that can be found is a candidate.
+constexpr float kB16Closed = 2.8e38F;
+constexpr float kB16Open = 3.0e38F;
 // What the two parts of a value can miss of it, and its low part: 2^-17 and 2^-8, and a little for their own rounding.
 constexpr double kB16Left = 7.7e-6;
 constexpr double kB16Low = 3.92e-3;
@@ -348,8 +352,8 @@ b16_query_kernel(B16QueryArgs p) {
     const float tf = static_cast<float>(t);
     const float up = tf + fabsf(tf) * 1.2e-7F + 1.0e-37F;
     // no bound yet: everything is a candidate (and the query overflows, or its lists are short)
-    const bool open = b == 0xFFFFFFFFU || !(up < 3.0e38F);
-    p.tau[q] = open ? 3.0e38F : up;
+    const bool open = b == 0xFFFFFFFFU || !(up < kB16Closed);
+    p.tau[q] = open ? kB16Open : up;
     if (p.magnitude != nullptr) {
         const double magnitude = fabs(bd) + fabs(constant) + (p.is_l2 ? ymax * ymax : 0.0) + factor * dots;
         p.magnitude[q] = open ? 0.0F : static_cast<float>(magnitude) * 1.000001F;
@@ -392,8 +396,8 @@ b16_tau_kernel(B16TauArgs p) {
     const float tau = kth + slack;
     const float up = tau + fabsf(tau) * 2.4e-7F + 1.0e-37F;
     // fewer than k codes sampled, or values that are not finite: everything is a candidate
-    const bool open = !(up < 3.0e38F) || !(kth > -3.0e38F);
-    p.tau[q] = open ? 3.0e38F : up;
+    const bool open = !(up < kB16Closed) || !(kth > -3.0e38F);
+    p.tau[q] = open ? kB16Open : up;
     p.slack[q] = open ? 3.0e38F : slack;
 }
 
@@ -708,12 +712,15 @@ prefilter_b16_kernel(PrefilterB16Args p) {
             my_term = real ? p.term[slot] : kB16Absent;
             const bool found = my_term < 3.0e38F;
             my_term = !found ? kB16Absent : p.terms == 0 ? 0.0F : my_term;
-            if (real && !found && p.terms == 0 && p.least == nullptr) {
-                // A code whose norm leaves fp32 (under l2 it stands behind all others) may have any inner product: a
-                // record of every query, and as its value is no number it is always rescored.
+            if (real && !found && p.least == nullptr) {
+                // A code whose squared norm leaves fp32 may have any inner product: a record of every query.  Under l2 it
+                // stands behind every threshold but an open one.  Its value is no number, so it is always rescored.
                 const uint32_t cols_here =
                     LISTS ? (pend - pbeg < N ? pend - pbeg : N) : static_cast<uint32_t>(p.nq - q0 < N ? p.nq - q0 : N);
                 for (uint32_t col = 0; col < cols_here; ++col) {
+                    if (p.terms != 0 && !(p.tau[LISTS ? as_const(p.sorted_pair)[pbeg + col] / p.nprobe : q0 + col] >= kB16Open)) {
+                        continue;
+                    }
                     record(col, LISTS ? (static_cast<uint64_t>(wave >> 1) << 32) | static_cast<uint32_t>(slot)
                                       : (0xFFFFFFFFULL << 32) | static_cast<uint32_t>(slot));
                 }
