@@ -232,6 +232,43 @@ def test_fp16_preselection_keeps_few_candidates_under_cosine(lib, modes, kind, b
     st.destroy()
 
 
+def _times(st, q, k, rounds=8):
+    """The best time of a call that streams and of one on the route the library takes, in turn."""
+    nq = len(q)
+    qb, ids, ds = dev(q), capi.DeviceBuffer(nq * k * 4), capi.DeviceBuffer(nq * k * 4)
+    best = {-1: 1e9, 0: 1e9}
+    for _ in range(rounds):
+        for mode in best:
+            capi.check(st.lib.vsag_amd_store_set_scan_contraction(st.handle, mode))
+            wsb = st.lib.vsag_amd_flat_scan_workspace_bytes(st.handle, nq, k)
+            ws = capi.DeviceBuffer(wsb)
+            capi.synchronize()
+            t0 = time.perf_counter()
+            capi.check(st.lib.vsag_amd_flat_scan_topk(st.handle, qb.ptr, nq, k, ids.ptr, ds.ptr, ws.ptr, wsb, None))
+            capi.synchronize()
+            best[mode] = min(best[mode], time.perf_counter() - t0)
+            ws.free()
+    capi.check(st.lib.vsag_amd_store_set_scan_contraction(st.handle, -2))
+    return best
+
+
+@pytest.mark.parametrize("size", [1e30, 1e37])
+def test_queries_that_stream_leave_no_records(lib, modes, size):
+    """Queries whose distances, or products, leave fp32 stream; every code of the store was a record of theirs first (seven
+    times the streaming kernel's time; three times is the line here)."""
+    rng = np.random.default_rng(6)
+    n, d, nq, k = 100000, 128, 8, 10
+    x = rng.random((n, d), dtype=np.float32)
+    q = (1 + rng.random((nq, d), dtype=np.float32)) * np.float32(size)
+    st = Store(capi.KIND_FP32, orc.L2, d)
+    st.append(x.view(np.uint8).reshape(n, -1))
+    plain, fast, tile = modes(st, q, k, 0)
+    assert tile == 64 and same(plain, fast)
+    best = _times(st, q, k)
+    assert best[0] < 3.0 * best[-1], best
+    st.destroy()
+
+
 @pytest.mark.parametrize("tile,chunks", [(2, -1), (8, 0), (-1, 7), (0, 7)])
 def test_tuning_knobs_ask_for_the_streaming_kernel(lib, modes, tile, chunks):
     """A query tile or a number of chunks set by hand: a batch of fewer than 512 queries that would be pre-selected streams
