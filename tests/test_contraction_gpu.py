@@ -90,6 +90,37 @@ def test_small_batches_equal_streaming(lib, modes, kind, d, nq, k, pre):
     st.destroy()
 
 
+@pytest.mark.parametrize("nq", [40, 600])
+def test_workspace_between_the_routes(lib, modes, nq):
+    """A workspace that has room for a streaming scan and for some, not all, of the bf16 route's records: the level-by-level
+    pre-selection where that fits (600 queries), streaming otherwise, the same results."""
+    rng = np.random.default_rng(nq)
+    n, d, k = 82000, 40, 10
+    x, means = gaussian_mixture(rng, n, d, 30, 0.05)
+    q, _ = gaussian_mixture(rng, nq, d, 30, 0.05, means=means)
+    st = Store(capi.KIND_FP32, orc.L2, d)
+    st.append(x.view(np.uint8).reshape(n, -1))
+    L = st.lib
+    plain, auto, tile = modes(st, q, k, 0)
+    assert same(plain, auto) and tile == (64 if nq == 40 else 128)
+    need = L.vsag_amd_flat_scan_workspace_bytes(st.handle, nq, k)
+    capi.check(L.vsag_amd_store_set_scan_contraction(st.handle, -1))
+    streaming = L.vsag_amd_flat_scan_workspace_bytes(st.handle, nq, k)
+    capi.check(L.vsag_amd_store_set_scan_contraction(st.handle, -2))
+    assert need > streaming
+    qb, ids, ds, room = dev(q), capi.DeviceBuffer(nq * k * 4), capi.DeviceBuffer(nq * k * 4), capi.DeviceBuffer(need)
+    used = capi.C.c_int()
+    for size, tile_expected in ((need, tile), (need - 4096, None), (streaming + 4096, None), (streaming, 8)):
+        capi.check(L.vsag_amd_flat_scan_topk(st.handle, qb.ptr, nq, k, ids.ptr, ds.ptr, room.ptr, size, None))
+        L.vsag_amd_last_scan_info(capi.C.byref(used), None, None)
+        if tile_expected is None:
+            tile_expected = 128 if nq == 600 and size > streaming + 4096 else 8
+        assert used.value == tile_expected, (size, used.value)
+        assert np.array_equal(ids.to_numpy(np.uint32, (nq, k)), plain[0].view(np.uint32))
+        assert np.array_equal(ds.to_numpy(np.uint32, (nq, k)), plain[1].view(np.uint32))
+    st.destroy()
+
+
 def _store_of(kind, metric, x, rng):
     """A store of the rows' codes, quantizer trained on the first of them."""
     d = x.shape[1]

@@ -101,6 +101,31 @@ def test_noalloc_flat_scan_equals_workspace_scan(lib):
     store.destroy()
 
 
+def test_noalloc_batches_without_room_for_the_bf16_records(lib):
+    """33 MiB of records and partial lists do not fit the array, the shorter lists of the level-by-level pre-selection do: the
+    batch takes those and does not stream, and streams where they do not fit either or a mask leaves nothing else."""
+    l = capi.load_library()
+    rng = np.random.default_rng(7)
+    n, d, k = 100000, 128, 10
+    x, means = gaussian_mixture(rng, n, d, 100, 0.05)
+    q, _ = gaussian_mixture(rng, 1400, d, 100, 0.05, means=means)
+    store = Store(capi.KIND_FP32, capi.METRIC_L2, d)
+    store.append(x.view(np.uint8).reshape(n, 4 * d))
+    deny = rng.random(n) < 0.5
+    opt, keep = store._options(deny, None)
+    tile = C.c_int()
+    for nq, with_mask, tile_expected in ((1250, False, 128), (1300, False, 128), (1400, False, 8), (1300, True, 8)):
+        room = l.vsag_amd_flat_scan_workspace_bytes(store.handle, nq, k)
+        assert (room > 32 << 20) == (nq > 1250)
+        got = noalloc_scan(l, store, q[:nq], k, opt if with_mask else None, count_memory=False)
+        l.vsag_amd_last_scan_info(C.byref(tile), None, None)
+        assert tile.value == tile_expected, (nq, tile.value)
+        assert same(got, store.flat_scan(q[:nq], k, deny=deny if with_mask else None))
+    for b in keep:
+        b.free()
+    store.destroy()
+
+
 def _rotation(rng, d):
     g = rng.standard_normal((d, d))
     q, r = np.linalg.qr(g)

@@ -591,6 +591,7 @@ struct CallPlan {
     bool b16 = false;
     bool large = false;  // (b16) what vsag_amd_last_scan_info tells large batches by: prefilter_pays
     size_t b16_scratch = 0;
+    bool without_b16 = false;  // the plan of a workspace that has no room for the bf16 route's records
     size_t h16_scratch = 0;    // sq8 beyond 128 dimensions: bytes of the fp16 query planes (0: the fp32 matrix cores)
     uint32_t cap = 0;          // candidates per query and level
     uint32_t sub_lists[kMaxLevels] = {};  // int8: private candidate lists per query ...
@@ -686,7 +687,7 @@ make_call_plan(const vsag_amd_store* s, uint64_t nq, uint32_t k, bool masked, Ca
     const bool long_uniform =
         (s->kind == VSAG_AMD_KIND_SQ8_UNIFORM || s->kind == VSAG_AMD_KIND_SQ4_UNIFORM) && !prefilter_i8_supports(s);
     const bool large = forced || (s->ntiles >= 1024 && prefilter_pays(s, nq, k));
-    if (prefilter_mode(s) != 2 && prefilter_b16_supports(s) && s->ntiles != 0 &&
+    if (!c->without_b16 && prefilter_mode(s) != 2 && prefilter_b16_supports(s) && s->ntiles != 0 &&
         ((large && (s->kind == VSAG_AMD_KIND_FP32 || masked || long_uniform)) || (!forced && prefilter_b16_pays(s, nq, k, masked)))) {
         const uint64_t cap = prefilter_b16_cap(k);
         if (nq * cap * 8 <= (2ull << 30)) {
@@ -798,13 +799,22 @@ make_call_plan(const vsag_amd_store* s, uint64_t nq, uint32_t k, bool masked, Ca
     c->any_seeded = c->any_seeded || c->prefix.seeded || c->rest.seeded;
 }
 
+// The plan that a workspace too small for *c may have room for, false where there is none: level by level (shorter lists than
+// the bf16 route's records: 1300 queries against 100k x 128 fp32 take 28 MiB where those take 33, and pre-select), then
+// streaming.
 static bool
-drop_candidate_lists(const vsag_amd_store* s, uint64_t nq, CallPlan* c) {
-    if (!c->contraction || (nq >= kListsOptionalBelow && !c->b16) || prefilter_mode(s) != 0) {
+smaller_plan(const vsag_amd_store* s, uint64_t nq, uint32_t k, bool masked, CallPlan* c) {
+    if (c->b16) {
+        *c = CallPlan{};
+        c->without_b16 = true;
+        make_call_plan(s, nq, k, masked, c);
+        return true;
+    }
+    if (!c->contraction || (nq >= kListsOptionalBelow && !c->without_b16) || prefilter_mode(s) != 0) {
         return false;
     }
-    c->contraction = c->int8 = c->rb = c->b16 = false;
-    c->h16_scratch = c->b16_scratch = 0;
+    c->contraction = c->int8 = c->rb = false;
+    c->h16_scratch = 0;
     c->nslots = static_cast<uint32_t>(c->all.chunks * c->all.waves);
     c->any_seeded = c->all.seeded;
     return true;
@@ -1242,7 +1252,7 @@ flat_scan_call(const vsag_amd_store_t* s, const float* queries_dev, uint64_t nq,
         c = Carver(workspace_dev, workspace_bytes);
         carve_scan(c, cp, nq, k, &b);
     }
-    if (!c.ok() && drop_candidate_lists(s, nq, &cp)) {
+    while (!c.ok() && smaller_plan(s, nq, k, masked, &cp)) {
         // Nor does a workspace without the candidate lists keep a small batch from being served.
         c = Carver(workspace_dev, workspace_bytes);
         carve_scan(c, cp, nq, k, &b);
@@ -1414,7 +1424,7 @@ vsag_amd_flat_scan_topk_noalloc(const vsag_amd_store_t* s, const float* queries_
     if (need > kStaticScratchBytes) {
         CallPlan cp;
         make_call_plan(s, nq, k, masked, &cp);
-        if (drop_candidate_lists(s, nq, &cp)) {
+        while (need > kStaticScratchBytes && smaller_plan(s, nq, k, masked, &cp)) {
             Carver c(nullptr, 0);
             ScanBuffers b;
             need = carve_scan(c, cp, nq, k, &b) + 256;
