@@ -475,9 +475,10 @@ rescore_kernel(ScanArgs a, RescoreArgs r) {
     if (overflow || as_const(r.gate)[q] != 0) {
         // The streaming kernel will scan every tile behind the prefix for this query: the lists of the levels so
         // far must not contribute the same codes a second time.
-        const uint32_t nlev = r.out_slot - r.first_slot + 1;
-        if (lane < nlev) {
-            r.partial_cnt[static_cast<uint64_t>(q) * r.nslots + r.first_slot + lane] = 0;
+        // (VALUED: all of the query's lists, which nothing has cleared so far.)
+        const uint32_t nlev = VALUED ? r.nslots : r.out_slot - r.first_slot + 1;
+        for (uint32_t i = lane; i < nlev; i += kWave) {
+            r.partial_cnt[static_cast<uint64_t>(q) * r.nslots + r.first_slot + i] = 0;
         }
         if (lane == 0) {
             r.gate[q] = 1;

@@ -15,13 +15,15 @@
 // fp32: no operand needs a scale, and what is below the normal range may be taken as zero.
 //
 // A flat scan (launch_scan_b16) needs no exact distance before the end:
-//   1. a sample of the code tiles, spread over the store, leaves the least v of every 64 codes; k of those lie at or
+//   1. a sample of the storage tiles, spread over the store, leaves the least v of every 64 codes; k of those lie at or
 //      below the k-th smallest, m;
 //   2. whoever is among the k best has v <= m + 2 e: the pass over all codes records (v, slot) of those, a few hundred a
-//      query (b16_tau_kernel says how many are expected);
+//      query (b16_sample_count says how many are expected);
 //   3. of the records only those within 2 e of their own k-th smallest are rescored with the streaming kernel's arithmetic
 //      (rescore_kernel): k and a handful, and the result is the streaming result, bit for bit.
-// A query with more records than there is room for is gated and streams.  A deny mask takes part in 1 and 2 as a |y|^2
+// Rows stored in the order of their clusters, or a mask over one run of them, make a poor sample, and more records than there
+// is room for: those that found room are a second sample, its k-th smallest a second threshold, and the queries concerned
+// pass over the codes once more.  One that overflows again is gated and streams.  A deny mask takes part in 1 and 2 as a |y|^2
 // beyond every threshold.  100k x 128 fp32, 1000 queries, k 10 (fp32 matrix cores, an exact prefix and levels before: 460 us): 150 us.
 // 100k x 768 fp32, 32 queries (streamed before: 684 us on the device): 141 us.  500k x 100 sq8 under a deny mask, 200
 // queries, k 100 (streamed before: 664 us): 160 us.
@@ -61,6 +63,8 @@ constexpr uint32_t kB16CountStride = 32;  // words between the queries' record c
 // it, and where nothing bounds a query, a threshold is kB16Open, and every code that can be found is a candidate.
 constexpr float kB16Closed = 2.8e38F;
 constexpr float kB16Open = 3.0e38F;
+constexpr uint32_t kB16Held = 2048;       // values of the sample that b16_tau_kernel keeps in LDS
+constexpr uint32_t kB16Streams = 0x40000000;  // the record counter of a query that streams whatever it finds
 // What the two parts of a value can miss of it, and its low part: 2^-17 and 2^-8, and a little for their own rounding.
 constexpr double kB16Left = 7.7e-6;
 constexpr double kB16Low = 3.92e-3;
@@ -208,11 +212,17 @@ struct B16QueryArgs {
     // posting lists: thresholds from the queries' bounds
     const uint32_t* bound;
     float* tau;
+    // flat scans: what a search starts from, bound0 (and no seeds, unless seed is null), and no query to pass over again
+    uint32_t* start;
+    uint32_t bound0;
+    uint32_t* seed;
+    uint32_t* again;
     float* magnitude;    // residual lists: the query's magnitudes (see IvfF32Args in prefilter.hip), or null
     // queries that stream: their flags, then how many; their pairs' first private list of k records is marked as overflowed
     uint32_t* gate;
     uint32_t* partial_cnt;
-    uint32_t p0, nprobe, k;
+    uint32_t p0, nprobe;
+    uint32_t k;
 };
 
 // One wave per row of the query table (rows at or beyond nq: zeros).
@@ -266,8 +276,17 @@ b16_query_kernel(B16QueryArgs p) {
         r2 += __shfl_xor(r2, off);
         l2 += __shfl_xor(l2, off);
     }
+    if (real && p.seed != nullptr) {
+        for (uint32_t i = lane; i < p.k; i += kWave) {
+            p.seed[q * p.k + i] = 0xFFFFFFFFU;
+        }
+    }
     if (lane != 0 || !real) {
         return;
+    }
+    if (p.start != nullptr) {
+        p.start[q] = p.bound0;
+        p.again[q] = 0;
     }
     constexpr double kU = 5.9604644775390625e-8;  // 2^-24, the unit roundoff of fp32
     const double kd = static_cast<double>(p.kdim);
@@ -368,40 +387,101 @@ struct B16TauArgs {
     float* slack;           // twice what v can be off by, at the distances that matter
     uint32_t* cand_cnt;     // zeroed
     uint32_t* gate;         // zeroed
-    uint32_t* partial_cnt;  // nslots a query, zeroed
-    uint32_t nslots;
 };
+
+struct B16Threshold {
+    float tau, slack;  // not below the k best values; twice what a value can be off by there
+};
+
+// The k codes at or below kth have distances of at most D; so has whoever is among the k best.
+__device__ inline B16Threshold
+b16_threshold(const B16Error& e, float kth) {
+    const float far = fmaxf(kth + e.constant, 0.0F) * 1.00001F + 2.0F * e.fixed;
+    const float slack = 2.0F * e.fixed + 2.05F * (e.root * sqrtf(far) + e.slope * far);
+    const float tau = kth + slack;
+    return {tau + fabsf(tau) * 2.4e-7F + 1.0e-37F, slack};
+}
 
 // One wave per query.
 __global__ void __launch_bounds__(64)
 b16_tau_kernel(B16TauArgs p) {
     __shared__ uint32_t hist[256];
+    __shared__ float held[kB16Held];
     const uint64_t q = blockIdx.x;
     const uint32_t lane = threadIdx.x;
     const float* least = p.least + q * p.groups;
-    const float kth = kth_value_or_above([&](uint32_t i) { return least[i]; }, p.groups, p.k, hist, lane);
-    for (uint32_t i = lane; i < p.nslots; i += kWave) {
-        p.partial_cnt[q * p.nslots + i] = 0;
+    // (asked for three times: from LDS as far as they fit)
+    for (uint32_t i = lane; i < p.groups && i < kB16Held; i += kWave) {
+        held[i] = least[i];
     }
+    wave_lds_fence();
+    const float kth =
+        kth_value_or_above([&](uint32_t i) { return i < kB16Held ? held[i] : least[i]; }, p.groups, p.k, hist, lane);
     if (lane != 0) {
         return;
     }
     const B16Error e = p.error[q];
-    // The k codes at or below kth have distances of at most D; so has whoever is among the k best.
-    const float far = fmaxf(kth + e.constant, 0.0F) * 1.00001F + 2.0F * e.fixed;
-    const float slack = 2.0F * e.fixed + 2.05F * (e.root * sqrtf(far) + e.slope * far);
-    const float tau = kth + slack;
-    const float up = tau + fabsf(tau) * 2.4e-7F + 1.0e-37F;
+    const B16Threshold t = b16_threshold(e, kth);
     // fewer than k codes sampled: everything is a candidate
     const bool open = !(kth < 3.0e38F);
     // A query whose sums can leave fp32, with entries that are not finite, or so far out that the threshold is, streams: more
     // records than there is room for, and nothing passes (8 queries of 1e30 against 100k x 128 fp32, every code a record of
     // each: 1367 us a call, now 234).
-    const bool streams = !(e.fixed < 1.0e37F) || (!open && !(up < kB16Closed));
-    p.cand_cnt[q * kB16CountStride] = streams ? 0x40000000U : 0U;
+    const bool streams = !(e.fixed < 1.0e37F) || (!open && !(t.tau < kB16Closed));
+    p.cand_cnt[q * kB16CountStride] = streams ? kB16Streams : 0U;
     p.gate[q] = 0;
-    p.tau[q] = streams ? kB16Absent : open ? kB16Open : up;
-    p.slack[q] = streams || open ? 3.0e38F : slack;
+    p.tau[q] = streams ? kB16Absent : open ? kB16Open : t.tau;
+    p.slack[q] = streams || open ? 3.0e38F : t.slack;
+}
+
+struct B16AgainArgs {
+    const uint64_t* cand;
+    uint32_t cap, k;
+    const B16Error* error;
+    float* tau;
+    float* slack;
+    uint32_t* cand_cnt;
+    uint32_t* again;   // per query tile of `columns`: whether one of its queries passes over the codes once more
+    uint32_t columns;
+};
+
+// One wave per query, behind the pass: a threshold from the records that found room, where some did not.
+__global__ void __launch_bounds__(64)
+b16_again_kernel(B16AgainArgs p) {
+    __shared__ uint32_t hist[256];
+    const uint64_t q = blockIdx.x;
+    const uint32_t lane = threadIdx.x;
+    const uint32_t count = as_const(p.cand_cnt)[q * kB16CountStride];
+    B16Threshold t{kB16Absent, 0.0F};  // nothing passes
+    if (count > p.cap && count < kB16Streams) {
+        const uint64_t* cand = p.cand + q * p.cap;
+        auto value = [&](uint32_t i) { return ordered_to_float(static_cast<uint32_t>(cand[i] >> 32)); };
+        // (Once more among what is left: the bins of the first span other clusters, in which the query's own is a bin or two.)
+        float kth = kth_value_or_above(value, p.cap, p.k, hist, lane);
+        const float first = kth;
+        wave_lds_fence();
+        kth = kth_value_or_above([&](uint32_t i) { const float v = value(i); return v <= first ? v : __builtin_inff(); }, p.cap, p.k,
+                                 hist, lane);
+        t = b16_threshold(p.error[q], kth);
+        // As many of all as of those here will pass.  (Thousands of equal distances: nothing helps.)
+        uint32_t pass = 0;
+        for (uint32_t i = lane; i < p.cap; i += kWave) {
+            pass += ordered_to_float(static_cast<uint32_t>(cand[i] >> 32)) <= t.tau ? 1U : 0U;
+        }
+        for (int off = 32; off > 0; off >>= 1) {
+            pass += __shfl_xor(pass, off);
+        }
+        const bool fits = static_cast<uint64_t>(pass) * count <= static_cast<uint64_t>(p.cap) * p.cap;
+        t.tau = t.tau < kB16Closed && fits ? t.tau : kB16Absent;
+    }
+    if (lane == 0) {
+        p.tau[q] = t.tau;
+        if (t.tau < kB16Closed) {
+            p.slack[q] = t.slack;
+            p.cand_cnt[q * kB16CountStride] = 0;
+            p.again[q / p.columns] = 1;
+        }
+    }
 }
 
 struct PrefilterB16Args {
@@ -416,9 +496,10 @@ struct PrefilterB16Args {
     const float* tau;
     // flat stores
     uint64_t ntiles, n;
-    uint64_t mstep;     // code tiles of four storage tiles: 0, mstep, 2 mstep, ... (1: all of them)
     float* least;       // a sampling pass: nq x groups values, and no records; else null
-    uint32_t groups;
+    uint32_t groups;    // the storage tiles of the sample: tile (i spread) >> 32 for i = 0 .. groups - 1
+    uint64_t spread;
+    const uint32_t* again;  // a second pass: the query tiles it is for; else null
     uint64_t* cand;     // nq x cap records: v as its ordered bits above the slot
     uint32_t* cand_cnt;
     uint32_t cap;
@@ -517,6 +598,7 @@ prefilter_b16_kernel(PrefilterB16Args p) {
     __shared__ float code_term[4][kWave];
     __shared__ uint64_t queue_key[4][kB16Queue];
     __shared__ uint32_t queue_col[4][kB16Queue];
+    __shared__ uint32_t col_count[LISTS ? 1 : 4][LISTS ? 1 : N];
     const uint32_t tid = threadIdx.x;
     const uint32_t lane = tid & 63;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -564,11 +646,15 @@ prefilter_b16_kernel(PrefilterB16Args p) {
         }
     } else {
         tile_end = p.ntiles;
-        first = blockIdx.x * p.mstep;
-        step = gridDim.x * p.mstep;
+        first = blockIdx.x;
+        step = gridDim.x;
         q0 = static_cast<uint64_t>(blockIdx.y) * N;
+        if (p.again != nullptr && as_const(p.again)[blockIdx.y] == 0) {
+            return;  // the whole workgroup
+        }
     }
-    const uint64_t mtiles = (tile_end - tile_begin + 3) / 4;
+    const bool sampling = !LISTS && p.least != nullptr;
+    const uint64_t mtiles = sampling ? p.groups / 4 : (tile_end - tile_begin + 3) / 4;
     if (first >= mtiles) {
         return;  // the whole workgroup
     }
@@ -642,6 +728,20 @@ prefilter_b16_kernel(PrefilterB16Args p) {
         }
     };
 
+    // Once a query's list is full, record number pos takes a place with probability cap / (pos + 1): what is there in the end
+    // is a sample of all its records, whatever order the codes are in (b16_again_kernel).  (Scrambled twice: places spread as
+    // evenly as one product spreads them leave nothing of the first records.)
+    auto place = [&](uint64_t q, uint32_t pos, uint64_t key) __attribute__((always_inline)) {
+        uint32_t at = pos;
+        if (pos >= p.cap) {
+            uint32_t h = pos * 0x9E3779B1U;
+            h = (h ^ (h >> 15)) * 0x85EBCA77U;
+            at = __umulhi(h ^ (h >> 13), pos + 1);
+        }
+        if (at < p.cap) {
+            p.cand[q * p.cap + at] = key;
+        }
+    };
     auto record = [&](uint32_t col, uint64_t key) __attribute__((always_inline)) {
         if constexpr (LISTS) {
             // private list of the pair: chunk, which half of the 256 codes (the upper word)
@@ -657,28 +757,59 @@ prefilter_b16_kernel(PrefilterB16Args p) {
             }
         } else {
             const uint64_t q = q0 + col;
-            const uint32_t pos = atomicAdd(&p.cand_cnt[q * kB16CountStride], 1U);
-            if (pos < p.cap) {
-                p.cand[q * p.cap + pos] = key;
-            }
+            place(q, atomicAdd(&p.cand_cnt[q * kB16CountStride], 1U), key);
         }
     };
     // Records wait in the wave's queue (a query's counter is an atomic a microsecond away: asked for one record at a time it
-    // cost half of the pass), until it might overflow or the walk is over.
+    // cost half of the pass), until it might overflow or the walk is over.  Flat: the queue asks once for all records of a
+    // column, a lane per column (a few queries that admit thousands of codes each otherwise wait for their own counters: 5
+    // against 100k x 128 fp32 in the order of its clusters: 147 -> 91 us).
     uint64_t* const keys = queue_key[wave];
     uint32_t* const cols = queue_col[wave];
     uint32_t waiting = 0;
     auto flush = [&]() __attribute__((always_inline)) {
         wave_lds_fence();
-        for (uint32_t i = lane; i < waiting; i += kWave) {
-            record(cols[i], keys[i]);
+        if constexpr (LISTS) {
+            for (uint32_t i = lane; i < waiting; i += kWave) {
+                record(cols[i], keys[i]);
+            }
+        } else {
+            uint32_t* const counts = col_count[wave];
+            for (uint32_t c = lane; c < N; c += kWave) {
+                counts[c] = 0;
+            }
+            wave_lds_fence();
+            uint32_t rank[kB16Queue / kWave];
+#pragma unroll
+            for (uint32_t r = 0; r < kB16Queue / kWave; ++r) {
+                const uint32_t i = r * kWave + lane;
+                rank[r] = i < waiting ? atomicAdd(&counts[cols[i]], 1U) : 0U;
+            }
+            wave_lds_fence();
+            for (uint32_t c = lane; c < N; c += kWave) {
+                if (counts[c] != 0) {
+                    counts[c] = atomicAdd(&p.cand_cnt[(q0 + c) * kB16CountStride], counts[c]);
+                }
+            }
+            wave_lds_fence();
+#pragma unroll
+            for (uint32_t r = 0; r < kB16Queue / kWave; ++r) {
+                const uint32_t i = r * kWave + lane;
+                if (i < waiting) {
+                    place(q0 + cols[i], counts[cols[i]] + rank[r], keys[i]);
+                }
+            }
         }
         waiting = 0;
         wave_lds_fence();
     };
 
+    auto tile_at = [&](uint64_t mt) __attribute__((always_inline)) {
+        const uint64_t i = tile_begin + 4 * mt + wave;
+        return sampling ? (i * p.spread) >> 32 : i;
+    };
     auto tile_of = [&](uint64_t mt) __attribute__((always_inline)) {
-        const uint64_t tile = tile_begin + 4 * mt + wave;
+        const uint64_t tile = tile_at(mt);
         return p.tiles + (tile < tile_end ? tile : tile_begin) * p.G * kWave;  // (slots past the end count as absent)
     };
     B16Codes<KIND> codes;
@@ -700,12 +831,12 @@ prefilter_b16_kernel(PrefilterB16Args p) {
                 }
             }
         }
-        const uint64_t slot0 = (tile_begin + 4 * mt + wave) * kWave;
+        const uint64_t slot0 = tile_at(mt) * kWave;
         const bool more_tiles = mt + step < mtiles;
         float my_term;
         {
             const uint64_t slot = slot0 + lane;
-            bool real = tile_begin + 4 * mt + wave < tile_end;
+            bool real = tile_at(mt) < tile_end;
             if constexpr (LISTS) {
                 // (a padding slot is all zeros: under inner product, and with a residual bias, that is a good distance)
                 real = real && p.ids[slot] != VSAG_AMD_INVALID_ID;
@@ -845,7 +976,7 @@ prefilter_b16_kernel(PrefilterB16Args p) {
                     const float least = fminf(group_least[j], __shfl_xor(group_least[j], 32));
                     const uint64_t q = q0 + j * 32 + l32;
                     if (half == 0 && q < p.nq) {
-                        p.least[q * p.groups + static_cast<uint32_t>(mt / p.mstep) * 4 + wave] = least;
+                        p.least[q * p.groups + static_cast<uint32_t>(mt) * 4 + wave] = least;
                     }
                 }
             }
@@ -880,15 +1011,22 @@ b16_query_args(const vsag_amd_store* s, const ScanArgs& a, uint64_t nq, B16Query
     qa->qmeta_stride = a.qmeta_stride;
 }
 
+// Queries per workgroup.
+static uint32_t
+b16_columns(uint64_t nq) {
+    return nq <= 32 ? 32 : nq <= 64 ? 64 : kB16N;
+}
+
 template <int KIND, bool ONE = false>
 static void
 launch_b16_flat(uint64_t nq, uint32_t cus, PrefilterB16Args p, hipStream_t st) {
-    const uint32_t per = nq <= 32 ? 32 : nq <= 64 ? 64 : kB16N;
+    const uint32_t per = b16_columns(nq);
     const uint64_t qtiles = div_up(nq, static_cast<uint64_t>(per));
-    const uint64_t mtiles = div_up(div_up(p.ntiles, 4), p.mstep);
+    const uint64_t mtiles = p.least != nullptr ? p.groups / 4 : div_up(p.ntiles, 4);
     // Two rounds of the workgroups that fit a compute unit (two or three) and not one more: a few left over would run a
-    // third round alone.  A workgroup walks every gridDim.x-th tile.
-    uint64_t groups = static_cast<uint64_t>(cus) * (per == 32 || (per == 64 && KIND != VSAG_AMD_KIND_FP32) ? 6 : 4) / qtiles;
+    // third round alone.  A workgroup walks every gridDim.x-th tile.  (One round where most of them return at once.)
+    const uint32_t rounds = p.again != nullptr ? 1 : 2;
+    uint64_t groups = static_cast<uint64_t>(cus) * rounds * (per == 32 || (per == 64 && KIND != VSAG_AMD_KIND_FP32) ? 3 : 2) / qtiles;
     groups = std::max<uint64_t>(1, std::min<uint64_t>(groups, mtiles));
     const dim3 grid(static_cast<uint32_t>(groups), static_cast<uint32_t>(qtiles));
     if (per == 32) {
@@ -916,10 +1054,9 @@ launch_b16_kind(const vsag_amd_store* s, uint64_t nq, const PrefilterB16Args& p,
     }
 }
 
-// The sample of a call: every step-th code tile of 256.  With s of n codes sampled, about k n / s codes lie at or below the
-// k-th smallest of the sample: kB16Expect of them (4 k where that is more), a sixteenth of the room a query has (a quarter).
-// Each sampled tile gives four groups, and four times as many groups as k keep their k-th least close to the k-th
-// of the sample.
+// The sample of a call, in storage tiles spread evenly over the store.  With s of n codes sampled, about k n / s codes lie at or
+// below the k-th smallest of the sample: kB16Expect of them (4 k where that is more), a sixteenth of the room a query has (a
+// quarter).  Four times as many groups as k keep their k-th least close to the k-th of the sample.
 constexpr uint64_t kB16Expect = 128;
 constexpr uint32_t kB16Records = 2048;
 
@@ -928,16 +1065,20 @@ prefilter_b16_cap(uint32_t k) {
     return std::max<uint32_t>(kB16Records, 16 * k);
 }
 
-static uint64_t
-b16_sample_step(const vsag_amd_store* s, uint32_t k) {
+// A multiple of four, the tiles of whole workgroups.  (A small store's sample is all of its tiles, and up to three behind them
+// that hold nothing.)
+static uint32_t
+b16_sample_groups(const vsag_amd_store* s, uint32_t k) {
     const uint64_t mtiles = div_up(s->ntiles, 4);
     const uint64_t expect = std::max<uint64_t>(kB16Expect, 4ull * k);
     const uint64_t want = std::max<uint64_t>({16, k, div_up(mtiles * k, expect)});
-    return std::max<uint64_t>(1, mtiles / want);
+    return static_cast<uint32_t>(4 * div_up(mtiles, std::max<uint64_t>(1, mtiles / want)));
 }
-static uint32_t
-b16_sample_groups(const vsag_amd_store* s, uint32_t k) {
-    return static_cast<uint32_t>(div_up(div_up(s->ntiles, 4), b16_sample_step(s, k)) * 4);
+// No two of the sample's tiles are the same.
+static uint64_t
+b16_sample_spread(const vsag_amd_store* s, uint32_t k) {
+    const uint64_t groups = b16_sample_groups(s, k);
+    return groups < s->ntiles ? (s->ntiles << 32) / groups : 1ull << 32;
 }
 
 // Scratch: the queries' parts, then their errors, thresholds, slacks and what the sample leaves.
@@ -946,6 +1087,7 @@ struct B16Scratch {
     B16Error* error;
     float* tau;
     float* slack;
+    uint32_t* again;
     float* least;
 };
 static size_t
@@ -954,6 +1096,7 @@ carve_b16(Carver& c, const vsag_amd_store* s, uint64_t nq, uint32_t k, B16Scratc
     b->error = c.take<B16Error>(nq);
     b->tau = c.take<float>(nq);
     b->slack = c.take<float>(nq);
+    b->again = c.take<uint32_t>(nq);
     b->least = c.take<float>(nq * b16_sample_groups(s, k));
     return c.used;
 }
@@ -969,11 +1112,12 @@ int launch_rescore_valued(const vsag_amd_store* s, const ScanArgs& a, uint64_t n
                           uint64_t* partial, uint32_t* partial_cnt, uint32_t nslots, uint32_t out_slot, uint32_t* gate,
                           hipStream_t st);
 
-// The flat scan of the header comment: list 0 of every query's nslots partial lists holds its k best, the others are empty,
-// and the gate of a query that has to stream is up.  `bound` holds what a search starts from.
+// The flat scan of the header comment: list 0 of every query's nslots partial lists holds its k best, or, where the query has
+// to stream, its gate is up and all its lists are empty.  (The other lists of the others hold nothing.)  `bound` and `seed` (or null) are what a search starts from: bound0, and no
+// seeds.
 int
 launch_scan_b16(const vsag_amd_store* s, const ScanArgs& a, uint64_t nq, uint32_t k, uint32_t S, uint32_t* bound,
-                uint8_t* scratch, uint64_t* cand, uint32_t* cand_cnt, uint32_t cap, const uint32_t* deny, uint64_t* partial,
+                uint32_t bound0, uint32_t* seed, uint8_t* scratch, uint64_t* cand, uint32_t* cand_cnt, uint32_t cap, const uint32_t* deny, uint64_t* partial,
                 uint32_t* partial_cnt, uint32_t nslots, uint32_t* gate, hipStream_t st) {
     Carver c(scratch, ~size_t{0});
     B16Scratch b;
@@ -982,6 +1126,11 @@ launch_scan_b16(const vsag_amd_store* s, const ScanArgs& a, uint64_t nq, uint32_
     b16_query_args(s, a, nq, &qa);
     qa.planes = b.planes;
     qa.error = b.error;
+    qa.start = bound;
+    qa.bound0 = bound0;
+    qa.seed = seed;
+    qa.k = k;
+    qa.again = b.again;
     hipLaunchKernelGGL(b16_query_kernel, dim3(static_cast<uint32_t>(qa.rows)), dim3(kWave), 0, st, qa);
     PrefilterB16Args p{};
     p.tiles = s->tiles;
@@ -997,13 +1146,12 @@ launch_scan_b16(const vsag_amd_store* s, const ScanArgs& a, uint64_t nq, uint32_
     p.ntiles = s->ntiles;
     p.n = s->n;
     p.deny = deny;
-    p.mstep = b16_sample_step(s, k);
     p.least = b.least;
     p.groups = b16_sample_groups(s, k);
+    p.spread = b16_sample_spread(s, k);
     launch_b16_kind(s, nq, p, st);
-    B16TauArgs ta{b.least, p.groups, k, b.error, b.tau, b.slack, cand_cnt, gate, partial_cnt, nslots};
+    B16TauArgs ta{b.least, p.groups, k, b.error, b.tau, b.slack, cand_cnt, gate};
     hipLaunchKernelGGL(b16_tau_kernel, dim3(static_cast<uint32_t>(nq)), dim3(kWave), 0, st, ta);
-    p.mstep = 1;
     p.least = nullptr;
     p.cand = cand;
     p.cand_cnt = cand_cnt;
@@ -1011,6 +1159,10 @@ launch_scan_b16(const vsag_amd_store* s, const ScanArgs& a, uint64_t nq, uint32_
     timing_begin(st);
     launch_b16_kind(s, nq, p, st);
     timing_end(st);
+    B16AgainArgs aa{cand, cap, k, b.error, b.tau, b.slack, cand_cnt, b.again, b16_columns(nq)};
+    hipLaunchKernelGGL(b16_again_kernel, dim3(static_cast<uint32_t>(nq)), dim3(kWave), 0, st, aa);
+    p.again = b.again;
+    launch_b16_kind(s, nq, p, st);
     VA_HIP(hipGetLastError());
     return launch_rescore_valued(s, a, nq, k, S, bound, cand, b.slack, cand_cnt, cap, partial, partial_cnt, nslots, 0, gate, st);
 }

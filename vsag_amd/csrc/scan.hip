@@ -190,12 +190,15 @@ block_bitonic_sort(uint64_t* keys, uint32_t P) {
 // an LDS pool; a radix selection finds the k-th smallest of the pool, the keys up to it are compacted and
 // sorted.  When the pool overflows (long runs of nearly equal distances), the k-th smallest of what did fit
 // -- an upper bound of the k-th smallest of all -- becomes the admission key of another round.
+// gate: null, or per query whether lists beyond the first hold anything (the bf16 route: hundreds of counts that are all
+// zero unless the query streamed were read for nothing, and written before).
 constexpr uint32_t kPoolKeys = 4096;       // few queries per call: every wave started without a bound
 constexpr uint32_t kPoolKeysBatch = 2048;  // batches: the bound is known, and twice the workgroups fit a compute unit
 
 __global__ void __launch_bounds__(1024)
 merge_partials_kernel(const uint64_t* partial, const uint32_t* partial_cnt, const uint32_t* bound, uint32_t nslots,
-                      uint32_t stride, uint32_t k, uint32_t S, uint32_t pool_keys, uint32_t* ids, float* dists) {
+                      uint32_t stride, uint32_t k, uint32_t S, uint32_t pool_keys, const uint32_t* gate, uint32_t* ids,
+                      float* dists) {
     extern __shared__ uint64_t lds[];  // S output keys, then the pool
     __shared__ uint32_t npool;
     __shared__ uint32_t nout;
@@ -205,6 +208,7 @@ merge_partials_kernel(const uint64_t* partial, const uint32_t* partial_cnt, cons
     __shared__ uint32_t long_slot[kLongLists];
     uint64_t* pool = lds + S;
     const uint64_t q = blockIdx.x;
+    nslots = gate != nullptr && as_const(gate)[q] == 0 ? 1 : nslots;
     const uint32_t* cnts = partial_cnt + q * stride;  // the first nslots of the query's `stride` lists
     const uint64_t* src = partial + q * stride * k;
     uint64_t admit = (static_cast<uint64_t>(as_const(bound)[q]) << 32) | 0xFFFFFFFFULL;
@@ -378,10 +382,11 @@ constexpr uint32_t kSmallMergeKeys = 512;
 
 __global__ void __launch_bounds__(64)
 merge_small_kernel(const uint64_t* partial, const uint32_t* partial_cnt, const uint32_t* bound, uint32_t nslots,
-                   uint32_t stride, uint32_t k, uint32_t* ids, float* dists) {
+                   uint32_t stride, uint32_t k, const uint32_t* gate, uint32_t* ids, float* dists) {
     __shared__ uint64_t pool[kSmallMergeKeys];
     const uint32_t lane = threadIdx.x;
     const uint64_t q = blockIdx.x;
+    nslots = gate != nullptr && as_const(gate)[q] == 0 ? 1 : nslots;
     const uint32_t* cnts = partial_cnt + q * stride;
     const uint64_t* src = partial + q * stride * k;
     const uint64_t admit = (static_cast<uint64_t>(as_const(bound)[q]) << 32) | 0xFFFFFFFFULL;
@@ -440,13 +445,12 @@ merge_small_kernel(const uint64_t* partial, const uint32_t* partial_cnt, const u
 }
 
 // ------------------------------------------------------------------ host side
-int
-launch_merge_partials(const uint64_t* partial, const uint32_t* partial_cnt, const uint32_t* bound, uint32_t nslots,
-                      uint32_t stride, uint32_t k, uint32_t S, uint64_t nq, uint32_t* ids, float* dists,
-                      hipStream_t st) {
+static int
+launch_gated_merge(const uint64_t* partial, const uint32_t* partial_cnt, const uint32_t* bound, uint32_t nslots, uint32_t stride,
+                   uint32_t k, uint32_t S, uint64_t nq, const uint32_t* gate, uint32_t* ids, float* dists, hipStream_t st) {
     if (nslots <= kWave && static_cast<uint64_t>(nslots) * k <= kSmallMergeKeys && nq > 256) {
         hipLaunchKernelGGL(merge_small_kernel, dim3(static_cast<uint32_t>(nq)), dim3(kWave), 0, st, partial, partial_cnt,
-                           bound, nslots, stride, k, ids, dists);
+                           bound, nslots, stride, k, gate, ids, dists);
         VA_HIP(hipGetLastError());
         return 0;
     }
@@ -454,9 +458,16 @@ launch_merge_partials(const uint64_t* partial, const uint32_t* partial_cnt, cons
     const uint32_t threads = nq <= 256 ? 1024 : 256;
     const uint32_t pool_keys = nq <= 256 ? kPoolKeys : kPoolKeysBatch;
     hipLaunchKernelGGL(merge_partials_kernel, dim3(static_cast<uint32_t>(nq)), dim3(threads), (S + pool_keys) * 8, st,
-                       partial, partial_cnt, bound, nslots, stride, k, S, pool_keys, ids, dists);
+                       partial, partial_cnt, bound, nslots, stride, k, S, pool_keys, gate, ids, dists);
     VA_HIP(hipGetLastError());
     return 0;
+}
+
+int
+launch_merge_partials(const uint64_t* partial, const uint32_t* partial_cnt, const uint32_t* bound, uint32_t nslots,
+                      uint32_t stride, uint32_t k, uint32_t S, uint64_t nq, uint32_t* ids, float* dists,
+                      hipStream_t st) {
+    return launch_gated_merge(partial, partial_cnt, bound, nslots, stride, k, S, nq, nullptr, ids, dists, st);
 }
 
 static int g_tile_override = 0;
@@ -640,7 +651,7 @@ bool prefilter_b16_pays(const vsag_amd_store* s, uint64_t nq, uint32_t k, bool m
 size_t prefilter_b16_scratch_bytes(const vsag_amd_store* s, uint64_t nq, uint32_t k);
 uint32_t prefilter_b16_cap(uint32_t k);
 int launch_scan_b16(const vsag_amd_store* s, const ScanArgs& a, uint64_t nq, uint32_t k, uint32_t S, uint32_t* bound,
-                    uint8_t* scratch, uint64_t* cand, uint32_t* cand_cnt, uint32_t cap, const uint32_t* deny,
+                    uint32_t bound0, uint32_t* seed, uint8_t* scratch, uint64_t* cand, uint32_t* cand_cnt, uint32_t cap, const uint32_t* deny,
                     uint64_t* partial, uint32_t* partial_cnt, uint32_t nslots, uint32_t* gate, hipStream_t st);
 uint32_t prefilter_rb_sub_lists(uint64_t nq, uint64_t span);
 
@@ -1298,8 +1309,10 @@ flat_scan_call(const vsag_amd_store_t* s, const float* queries_dev, uint64_t nq,
         return 0;
     }
     const uint64_t nseed = b.seed != nullptr ? nq * k : 0;
-    hipLaunchKernelGGL(reset_queries_kernel, dim3(static_cast<uint32_t>(div_up(nq > nseed ? nq : nseed, 256))), dim3(256),
-                       0, st, b.bound, initial_bound(options), nq, b.seed, nseed);
+    if (!contraction || !cp.b16 || s->ntiles == 0) {  // (that route's first launch does it)
+        hipLaunchKernelGGL(reset_queries_kernel, dim3(static_cast<uint32_t>(div_up(nq > nseed ? nq : nseed, 256))), dim3(256),
+                           0, st, b.bound, initial_bound(options), nq, b.seed, nseed);
+    }
     ScanArgs a = make_scan_args(s, p.ql, b.qtab, b.qmeta);
     uint32_t nslots = 0;
     if (s->ntiles == 0) {
@@ -1313,8 +1326,8 @@ flat_scan_call(const vsag_amd_store_t* s, const float* queries_dev, uint64_t nq,
         tl_last_passes = p.groups;
     } else if (cp.b16) {
         nslots = 1 + static_cast<uint32_t>(p.chunks * p.waves);
-        VA_TRY(launch_scan_b16(s, a, nq, k, p.S, b.bound, b.q8, reinterpret_cast<uint64_t*>(b.cand), b.cand_cnt, cp.cap,
-                               masked ? options->deny_bits_dev : nullptr, b.partial, b.partial_cnt, nslots, b.gate, st));
+        VA_TRY(launch_scan_b16(s, a, nq, k, p.S, b.bound, initial_bound(options), b.seed, b.q8,
+                               reinterpret_cast<uint64_t*>(b.cand), b.cand_cnt, cp.cap, masked ? options->deny_bits_dev : nullptr, b.partial, b.partial_cnt, nslots, b.gate, st));
         // the queries whose records found no room
         VA_TRY(run_streaming(s, p, a, b, nq, k, options, 0, s->ntiles, 1, nslots, b.gate, st));
         tl_last_tile = cp.large ? 128 : 64;
@@ -1356,7 +1369,8 @@ flat_scan_call(const vsag_amd_store_t* s, const float* queries_dev, uint64_t nq,
         tl_last_tile = cp.int8 ? 256 : 128;  // queries per pass of the contraction
         tl_last_passes = div_up(nq, cp.int8 ? 256 : 128);
     }
-    VA_TRY(launch_merge_partials(b.partial, b.partial_cnt, b.bound, nslots, nslots, k, p.S, nq, ids_dev, dists_dev, st));
+    VA_TRY(launch_gated_merge(b.partial, b.partial_cnt, b.bound, nslots, nslots, k, p.S, nq,
+                              contraction && cp.b16 ? b.gate : nullptr, ids_dev, dists_dev, st));
     // Code bytes under the timed kernel: the whole store, or the last (by far the largest) level of the contraction.
     const uint64_t timed_tiles = contraction && !cp.b16 ? s->ntiles - cp.level_begin[cp.levels - 1] : s->ntiles;
     tl_last_bytes = timed_tiles * s->G * kWave * kGranule;
