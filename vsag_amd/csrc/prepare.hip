@@ -1,6 +1,7 @@
 // Query preparation for the scans: ProcessQueryImpl of every store kind, written into the tables the
 // distance loops read through scalar loads (one row per query, rows aligned to 64 bytes).
 #include "distance.h"
+#include "prepare_rows.h"
 #include "store.h"
 
 namespace vsag_amd {
@@ -8,79 +9,9 @@ namespace vsag_amd {
 // ------------------------------------------------------------------ query preparation
 // One workgroup (256 threads) per query row; rows >= nq are written as zeros so that a partly filled
 // query tile computes harmless values.
-__device__ inline float
-block_sum(float v, float* red) {
-    for (int off = 32; off > 0; off >>= 1) {
-        v += __shfl_down(v, off);
-    }
-    uint32_t wave = threadIdx.x >> 6;
-    if ((threadIdx.x & 63) == 0) {
-        red[wave] = v;
-    }
-    __syncthreads();
-    float s = 0;
-    for (uint32_t i = 0; i < (blockDim.x >> 6); ++i) {
-        s += red[i];
-    }
-    __syncthreads();
-    return s;
-}
-
-// fp32 / sq8 / sq4 tables (ProcessQueryImpl of fp32_quantizer.cpp:216-233 and scalar_quantizer.cpp:154-171
-// keep the query in fp32, normalised for cosine; the per-dimension constants are folded in here).
 __global__ void __launch_bounds__(256)
-prepare_float_queries(const float* q, uint64_t nq, uint32_t dim, int kind, int metric, const float* scale,
-                      const float* lb, float* qtab, uint32_t qstride, float* qmeta, uint32_t qmeta_stride) {
-    __shared__ float red[4];
-    uint64_t row = blockIdx.x;
-    float* out = qtab + row * qstride;
-    if (row >= nq) {
-        for (uint32_t d = threadIdx.x; d < qstride; d += blockDim.x) {
-            out[d] = 0.0F;
-        }
-        if (threadIdx.x < qmeta_stride) {
-            qmeta[row * qmeta_stride + threadIdx.x] = 0.0F;
-        }
-        return;
-    }
-    const float* src = q + row * dim;
-    float inv_norm = 1.0F;
-    bool cosine = metric == VSAG_AMD_METRIC_COSINE;
-    if (cosine) {
-        float s = 0;
-        for (uint32_t d = threadIdx.x; d < dim; d += blockDim.x) {
-            s += src[d] * src[d];
-        }
-        s = block_sum(s, red);
-        inv_norm = sqrtf(s);
-        if (inv_norm == 0.0F) {
-            inv_norm = 1.0F;  // DivScalarImpl (src/simd/kernels/scalar_op.h:40-42): a zero norm divides by 1
-        }
-    }
-    float bias = 0;
-    for (uint32_t d = threadIdx.x; d < qstride; d += blockDim.x) {
-        float v = 0.0F;
-        if (d < dim) {
-            float x = cosine ? src[d] / inv_norm : src[d];
-            if (kind == VSAG_AMD_KIND_FP32) {
-                v = x;
-            } else if (metric == VSAG_AMD_METRIC_L2) {
-                v = x - lb[d];
-            } else {
-                v = x * scale[d];
-                bias += x * lb[d];
-            }
-        }
-        out[d] = v;
-    }
-    if (kind != VSAG_AMD_KIND_FP32 && metric != VSAG_AMD_METRIC_L2) {
-        bias = block_sum(bias, red);
-        if (threadIdx.x == 0) {
-            qmeta[row * qmeta_stride] = bias;
-        }
-    } else if (threadIdx.x < qmeta_stride) {
-        qmeta[row * qmeta_stride + threadIdx.x] = 0.0F;
-    }
+prepare_float_queries(FloatQueryArgs p) {
+    prepare_float_row(p, blockIdx.x);
 }
 
 // Uniform kinds: the query has been encoded with the base encoder (ProcessQueryImpl = EncodeOneImpl,
@@ -335,8 +266,7 @@ prepare_queries(const vsag_amd_store* s, const float* queries, uint64_t nq, uint
         case VSAG_AMD_KIND_FP32:
         case VSAG_AMD_KIND_SQ8:
         case VSAG_AMD_KIND_SQ4:
-            hipLaunchKernelGGL(prepare_float_queries, grid, dim3(256), 0, st, queries, nq, s->dim, s->kind, s->metric,
-                               s->scale_dev, s->lb_dev, reinterpret_cast<float*>(qtab), ql.qstride, qmeta, ql.qmeta);
+            hipLaunchKernelGGL(prepare_float_queries, grid, dim3(256), 0, st, float_query_args(s, queries, nq, ql, qtab, qmeta));
             break;
         case VSAG_AMD_KIND_SQ4_UNIFORM:
         case VSAG_AMD_KIND_SQ8_UNIFORM: {

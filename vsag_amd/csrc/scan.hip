@@ -6,6 +6,7 @@
 #include <mutex>
 
 #include "distance.h"
+#include "prepare_rows.h"
 #include "scan_flat.h"
 #include "store.h"
 #include "topk.h"
@@ -650,7 +651,8 @@ bool prefilter_b16_supports(const vsag_amd_store* s);
 bool prefilter_b16_pays(const vsag_amd_store* s, uint64_t nq, uint32_t k, bool masked);
 size_t prefilter_b16_scratch_bytes(const vsag_amd_store* s, uint64_t nq, uint32_t k);
 uint32_t prefilter_b16_cap(uint32_t k);
-int launch_scan_b16(const vsag_amd_store* s, const ScanArgs& a, uint64_t nq, uint32_t k, uint32_t S, uint32_t* bound,
+int launch_scan_b16(const vsag_amd_store* s, const ScanArgs& a, const FloatQueryArgs& raw, uint64_t nq_pad, uint64_t nq, uint32_t k,
+                    uint32_t S, uint32_t* bound,
                     uint32_t bound0, uint32_t* seed, uint8_t* scratch, uint64_t* cand, uint32_t* cand_cnt, uint32_t cap, const uint32_t* deny,
                     uint64_t* partial, uint32_t* partial_cnt, uint32_t nslots, uint32_t* gate, hipStream_t st);
 uint32_t prefilter_rb_sub_lists(uint64_t nq, uint64_t span);
@@ -1273,7 +1275,13 @@ flat_scan_call(const vsag_amd_store_t* s, const float* queries_dev, uint64_t nq,
     const bool contraction = cp.contraction && !ranged;
     const ScanPlan& p = cp.all;
 
-    VA_TRY(prepare_queries(s, queries_dev, nq, p.nq_pad, p.ql, b.qtab, b.qmeta, b.qcodes, st));
+    FloatQueryArgs raw{};
+    if (contraction && cp.b16 && !cp.one &&
+        (s->kind == VSAG_AMD_KIND_FP32 || s->kind == VSAG_AMD_KIND_SQ8 || s->kind == VSAG_AMD_KIND_SQ4)) {
+        raw = float_query_args(s, queries_dev, nq, p.ql, b.qtab, b.qmeta);  // (that route's first launch prepares them)
+    } else {
+        VA_TRY(prepare_queries(s, queries_dev, nq, p.nq_pad, p.ql, b.qtab, b.qmeta, b.qcodes, st));
+    }
     if (cp.table && plain) {
         const ScanArgs ta = make_scan_args(s, p.ql, b.qtab, b.qmeta);
         const uint64_t slots = cp.table_ld;
@@ -1326,7 +1334,7 @@ flat_scan_call(const vsag_amd_store_t* s, const float* queries_dev, uint64_t nq,
         tl_last_passes = p.groups;
     } else if (cp.b16) {
         nslots = 1 + static_cast<uint32_t>(p.chunks * p.waves);
-        VA_TRY(launch_scan_b16(s, a, nq, k, p.S, b.bound, initial_bound(options), b.seed, b.q8,
+        VA_TRY(launch_scan_b16(s, a, raw, p.nq_pad, nq, k, p.S, b.bound, initial_bound(options), b.seed, b.q8,
                                reinterpret_cast<uint64_t*>(b.cand), b.cand_cnt, cp.cap, masked ? options->deny_bits_dev : nullptr, b.partial, b.partial_cnt, nslots, b.gate, st));
         // the queries whose records found no room
         VA_TRY(run_streaming(s, p, a, b, nq, k, options, 0, s->ntiles, 1, nslots, b.gate, st));
