@@ -215,21 +215,24 @@ def test_uniform_codes_on_the_bf16_matrix_cores(lib, modes, kind, metric, n, d, 
     st.destroy()
 
 
-@pytest.mark.parametrize("bounds", [[0.0, 0.0], [3.0, 1e-30], [-1e18, 1e19], [0.0, -2.0]])
-def test_uniform_bounds_out_of_range_stream(lib, modes, bounds):
-    """A rate of zero, one that makes every distance a denormal number, one whose distances leave fp32: what streaming
-    returns."""
+@pytest.mark.parametrize("bounds", [[0.0, 0.0], [3.0, 1e-30], [0.0, 1e-20], [-1e18, 1e19], [0.0, -2.0]])
+def test_uniform_bounds_at_the_ends_of_fp32(lib, modes, bounds):
+    """A rate of zero (every distance the same: the first ids), one that makes the distances denormal numbers, of which many
+    are the same, one whose distances leave fp32, a negative width: what streaming returns.  Fewer codes than a query has
+    room for records, so none of them streams only because its records overflow."""
     rng = np.random.default_rng(3)
-    n, d, nq, k = 5000, 160, 20, 10
+    n, d, nq, k = 1500, 160, 20, 10
     x = rng.random((n, d), dtype=np.float32)
     q = rng.random((nq, d), dtype=np.float32)
     for metric in (orc.L2, orc.IP):
         codes = orc.squ_encode(x, 8, 0.0, 1.0, metric)
         st = Store(capi.KIND_SQ8_UNIFORM, metric, d, bounds=bounds)
         st.append(codes)
-        plain, fast, _ = modes(st, q, k, 1)
-        assert np.array_equal(plain[1].view(np.uint32), fast[1].view(np.uint32))
-        assert np.array_equal(plain[0], fast[0])
+        plain, fast, tile = modes(st, q, k, 1)
+        assert tile == 128, "the contraction path did not run"
+        if metric == orc.L2 and bounds[1] == 0.0:
+            assert np.all(plain[0] == np.arange(k))
+        assert same(plain, fast)
         st.destroy()
 
 
