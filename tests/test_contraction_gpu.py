@@ -543,6 +543,18 @@ def test_fp32_contraction_equals_streaming(lib, modes, metric, n, d, nq, k):
     st.destroy()
 
 
+@pytest.mark.parametrize("kind,d", [("sq8_uniform", 8192), ("sq8_uniform", 8193), ("sq4_uniform", 8192), ("sq4_uniform", 8200)])
+def test_longest_uniform_codes(lib, modes, kind, d):
+    """Up to 8192 dimensions on the bf16 matrix cores, beyond by streaming."""
+    rng = np.random.default_rng(d)
+    n, nq, k = 700, 9, 5
+    x = rng.random((n, d), dtype=np.float32)
+    st = _store_of(kind, orc.L2, x, rng)
+    plain, fast, tile = modes(st, x[:nq] + np.float32(0.1), k, 1)
+    assert (tile == 128) == (d <= 8192) and same(plain, fast)
+    st.destroy()
+
+
 @pytest.mark.parametrize("metric", [orc.L2, orc.IP, orc.COSINE])
 @pytest.mark.parametrize("n,d,nq,k", [(1500, 17, 1, 1), (2049, 32, 31, 5), (4097, 36, 33, 10), (5003, 130, 64, 10),
                                       (3001, 64, 65, 20), (6000, 260, 129, 3)])

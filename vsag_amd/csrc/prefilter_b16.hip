@@ -86,12 +86,11 @@ b16_uniform(const vsag_amd_store* s) {
     return s->kind == VSAG_AMD_KIND_SQ8_UNIFORM || s->kind == VSAG_AMD_KIND_SQ4_UNIFORM;
 }
 
-// Posting lists of sq8 / sq4 / uniform codes and rabitq stores have passes of their own.  (Uniform codes: the product of two
-// rows fits the streaming kernel's 32-bit integer.)
+// Posting lists of sq8 / sq4 / uniform codes and rabitq stores have passes of their own.
 bool
 prefilter_b16_supports(const vsag_amd_store* s) {
     const bool kind = s->kind == VSAG_AMD_KIND_FP32 || s->kind == VSAG_AMD_KIND_SQ8 || s->kind == VSAG_AMD_KIND_SQ4 ||
-                      (b16_uniform(s) && s->nlist == 0 && s->dpad <= 8192);
+                      (b16_uniform(s) && s->nlist == 0 && s->dpad <= kUniformTermDims);
     return kind && s->pf_term != nullptr && s->pf_ymax != nullptr;
 }
 

@@ -121,6 +121,10 @@ constexpr uint32_t kRbMaxG = 8;  // granules per code (1024 dimensions) of the r
 constexpr float kRbMaxA = 64.0F;
 constexpr float kRbMaxB = 4096.0F;
 
+// Largest dpad of the uniform kinds at which a pre-selection takes them (the product of two rows fits the streaming kernel's
+// 32-bit integer); stores beyond it keep no per-code term.
+constexpr uint32_t kUniformTermDims = 8192;
+
 struct QueryLayout {
     uint32_t qstride;  // 4-byte words per query in the main table
     uint32_t qmeta;    // floats per query in the scalar table
