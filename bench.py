@@ -465,8 +465,9 @@ def run_c1(env):
         peak = MFMA_F16_PEAK_TFLOPS if bf16 else MFMA_F32_PEAK_TFLOPS
         roof = {"bound": "mfma", "achieved": tf, "peak": peak, "unit": "TFLOP/s", "frac": tf / peak,
                 "executed_frac": (3.0 if bf16 else 1.0) * tf / peak,
-                # rocprofv3 --pmc FETCH_SIZE (x 2.00) + WRITE_SIZE of this launch: profiles/prefilter_fp32_c1.md
-                "traffic": 87735.7 * 2.00 * 1024 + 23281.8 * 1024 if not bf16 and (n, d, nq, k) == (100000, 128, 1000, 10) else None,
+                # rocprofv3 --pmc FETCH_SIZE (x 2.00) + WRITE_SIZE of this launch: profiles/prefilter_b16.md, prefilter_fp32_c1.md
+                "traffic": None if (n, d, nq, k) != (100000, 128, 1000, 10) else
+                           (85968.2 * 2.00 + 6329.1) * 1024 if bf16 else (87735.7 * 2.00 + 23281.8) * 1024,
                 "kernel": "prefilter_b16_kernel<fp32> (bf16 MFMA, all codes)" if bf16 else
                           "prefilter_kernel<fp32> (fp32 MFMA, last level)", "kernel_ms": kms,
                 "flops_per_launch": 2.0 * codes * d * nq, "codes_per_launch": codes}

@@ -38,8 +38,9 @@ struct ScanPlanIvf {
     bool pq;                  // ... with pqfs codes: one-hot centroid indices against the byte tables (ivf_pq.hip)
     bool h16;                 // ... sq8 codes beyond 128 dimensions: the fp16 matrix cores, records rescored
     bool f32;                 // ... with fp32 codes (sq8 beyond 128 dimensions): the fp32 matrix cores, records rescored
-    bool b16;                 // ... fp32 codes on the bf16 matrix cores instead, two bf16 values per operand
                               // (prefilter.hip)
+    bool b16;                 // ... fp32 codes on the bf16 matrix cores instead, two bf16 values per operand
+                              // (prefilter_b16.hip)
 };
 
 uint64_t rabitq_query_code_size(uint32_t dim, int metric, int query_bits);

@@ -26,10 +26,12 @@
 // pass over the codes once more.  One that overflows again is gated and streams.  A deny mask takes part in 1 and 2 as a |y|^2
 // beyond every threshold.  100k x 128 fp32, 1000 queries, k 10 (fp32 matrix cores, an exact prefix and levels before: 460 us): 150 us.
 // 100k x 768 fp32, 32 queries (streamed before: 684 us on the device): 141 us.  500k x 100 sq8 under a deny mask, 200
-// queries, k 100 (streamed before: 664 us): 160 us.
+// queries, k 100 (streamed before: 664 us): 157 us.  100k x 128 fp32, 1000 queries, rows in the order of their clusters: 469 us.
 //
-// What bounds it: with 128 queries per workgroup the matrix cores beside the splitting of the codes and the verdicts; with
-// few queries the bytes of the codes, each read once per 32, 64 or 128 queries.
+// What bounds it: with 128 queries per workgroup the matrix cores beside the splitting of the codes and the verdicts (100k x
+// 128 fp32, 1000 queries: matrix pipe busy 34 % of the pass, vector instructions issued 38 %, a third of the waves' time spent
+// waiting; no bank conflicts to speak of); with few queries the bytes of the codes, each read once per 32, 64 or 128 queries
+// (100k x 768 fp32, 32 queries: 6.0 TB/s, matrix pipe 10 %).
 //
 // Work split: a workgroup of four waves takes 256 codes, a storage tile a wave, and 128, 64 or 32 queries (JB blocks of
 // 32), so a code is read by one wave alone and goes from memory into the registers of the lanes that multiply it (lane %
@@ -111,6 +113,9 @@ prefilter_b16_supports(const vsag_amd_store* s) {
 //   128, 2000 279 -> 172; beyond 128 dimensions they have nothing else (200k x 768, 2000 queries 4221 -> 854; 600k x 960
 //   sq4_uniform, 1000 5790 -> 1312).
 //   A deny mask leaves the streaming kernel alone as the other side.
+// Rows in the order of their clusters take the second pass (us, streaming -> this): fp32 100k x 768 5 queries 178 -> 195, 8: 269
+// -> 261, 32: 683 -> 259; 100k x 128 5: 85 -> 90, 1000 (by levels before) 2676 -> 469; sq8 500k x 100, k 100 9: 186 -> 128.
+// Thousands of equal distances stream behind the pass: 100k x 128 of 40 distinct rows 8 queries 123 -> 192, 64 578 -> 409.
 // Smaller stores than 81920 codes would gain as well (sq8 70000 x 200, 512 queries 263 -> 121; 70000 x 32, 8 60 -> 47), but
 // the records of a query take 16 KB, several times the streaming kernel's workspace there: batches of those keep it.
 bool
@@ -345,7 +350,9 @@ b16_query_kernel(B16QueryArgs p) {
     // Left out: the remainders of the query against a code (codes of bytes lie in [0, cmax]); of an fp32 code at most
     // kB16Left of it against the query, and its low part (kB16Low of it) against the query's.
     const double split = fp32 ? ymax * (sqrt(r2) + kB16Left * an + kB16Low * sqrt(l2)) : static_cast<double>(p.cmax) * r1;
-    // The accumulation: four roundings of the absolute sum per instruction (two or three per sixteen dimensions).
+    // The accumulation, two or three instructions per sixteen dimensions.  One was measured to lose at most 2 units of 2^-24 of
+    // its accumulator and 8 of its largest product (it cuts off what it aligns: one product of 1 and fifteen just below 2^-24
+    // lose 7.9; random and crafted inputs): 2 n + 8 of the absolute sum over n instructions.  Twice that.
     const double rounding = 4.0 * kU * ((fp32 ? 3.0 : 2.0) * kd / 16.0 + 4.0) * sums;
     // Operands below the normal range taken as zero; fma(factor, acc, term) and |y|^2 rounded, the low four bits cut off.
     const double flushed = kd * 4.7e-38 * (an + ymax + 1.0);

@@ -8,7 +8,8 @@
 // v_mfma_f32_32x32x16_f16, which runs at sixteen times the rate of the fp32 instruction.  A pair is lost only if the
 // matrix cores' product comes out too small (it comes off the distance, and the codes are not negative): what the
 // fp16 values fall short of their b_d is summed per query in double precision, times the largest code value, and the
-// accumulation is allowed two roundings per instruction of the absolute sum.  Both go onto the query's threshold
+// accumulation is allowed two roundings per instruction of the absolute sum and eight more (what one was measured to lose:
+// at most 2 units of 2^-24 of its accumulator and 8 of its largest product).  Both go onto the query's threshold
 // (h16_split_kernel), next to what the streaming kernel's own fp32 arithmetic can be off by -- a multiple of the
 // distance, not of |q| |y|, since no fp32 contraction stands between the test and the truth here.  (A second fp16
 // part of the query would carry the 2^-12 the first misses; it doubles the matrix work and the LDS reads and saves
@@ -177,7 +178,7 @@ h16_split_kernel(H16SplitArgs p) {
         t = bd - 1.0 + qm + e_stream;
     }
     // every code value lies in [0, cmax]: what the fp16 value misses of b_d, and two roundings of the running absolute
-    // sum per matrix instruction (sixteen dimensions each) plus four for the closing operations
+    // sum per matrix instruction (sixteen dimensions each) plus eight for their largest products
     const double roundings = 2.0 * (p.kdim / 16.0 + 4.0) * kU;
     const double extra = fabs(static_cast<double>(p.dot_factor)) * static_cast<double>(p.cmax) * (miss + roundings * sum_abs);
     // the test itself: fl(term + fl(factor acc)) against the threshold rounded to fp32 (no term under ip: there

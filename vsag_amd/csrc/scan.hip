@@ -583,9 +583,10 @@ make_plan(const vsag_amd_store* s, uint64_t nq, uint32_t k, uint64_t ntiles, Sca
     p->qcode_bytes = query_staging_bytes(s, nq);
 }
 
-// A call is served either by one streaming launch over all tiles, or -- large batches on fp32 / sq8 stores
-// (prefilter.hip) -- by a streaming launch over a prefix, the matrix-core prefilter with exact rescoring over the
-// rest, and a streaming launch over the rest for the queries whose candidates overflowed.
+// A call is served by one streaming launch over all tiles; by the bf16 matrix cores over all tiles (prefilter_b16.hip), with
+// exact rescoring and a streaming launch for the queries whose records overflowed; by a streaming launch over a prefix, the
+// matrix-core prefilter with exact rescoring over the rest, level by level (prefilter.hip), and a streaming launch over the
+// rest for the queries whose candidates overflowed; or by one of the two small routes at the end of the plan.
 struct CallPlan {
     ScanPlan all;
     bool contraction = false;
