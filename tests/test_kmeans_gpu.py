@@ -414,3 +414,38 @@ def test_run_with_the_fp16_preselection_keeps_its_rows(lib, n, d, k, iters):
                                             L.vsag_amd_kmeans_update_workspace_bytes(n, d, k), None))
         assert (counts.to_numpy(np.int32, (k,)) > 0).all()
     assert np.array_equal(lab, last[0]) and loss.value == last[2]
+
+
+@pytest.mark.parametrize("n,k,kind", [(1, 1, "even"), (63, 2, "even"), (1023, 3, "even"), (1024, 64, "even"), (1025, 65, "even"),
+                                      (5000, 98, "skewed"), (5000, 98, "runs"), (40000, 4097, "even"), (40000, 16384, "even"),
+                                      (40000, 16385, "even"), (70000, 1000, "one")])
+def test_update_groups_the_rows_of_every_label(lib, n, k, kind):
+    """Rows grouped by label around the edges of the counting sort's units and label bits: every mean is the sequential fp32 sum
+    of the rows in row order, bit for bit, which holds only if the grouping is stable and complete."""
+    L = lib.load_library()
+    rng = np.random.default_rng(n * 7 + k)
+    labels = rng.integers(0, k, n).astype(np.int32)
+    if kind == "skewed":
+        labels = (k * rng.random(n) ** 6).astype(np.int32)
+    elif kind == "runs":
+        labels = np.sort(labels)
+    elif kind == "one":
+        labels[:] = k - 1
+    x = rng.standard_normal((n, 4)).astype(np.float32)
+    cent0 = rng.standard_normal((k, 4)).astype(np.float32)
+    xb, lb, cb, counts = dev(x), dev(labels), dev(cent0), capi.DeviceBuffer(k * 4)
+    wsb = L.vsag_amd_kmeans_update_workspace_bytes(n, 4, k)
+    ws = capi.DeviceBuffer(wsb)
+    capi.check(L.vsag_amd_kmeans_update(xb.ptr, lb.ptr, n, 4, k, cb.ptr, counts.ptr, ws.ptr, wsb, None))
+    sizes = np.bincount(labels, minlength=k)
+    want, order = cent0.copy(), np.argsort(labels, kind="stable")
+    begin = np.concatenate([[0], np.cumsum(sizes)])
+    for j in np.nonzero(sizes)[0]:
+        sums = np.cumsum(x[order[begin[j]:begin[j + 1]]], axis=0, dtype=np.float32)[-1]
+        want[j] = sums * (np.float32(1) / np.float32(sizes[j]))
+    assert np.array_equal(counts.to_numpy(np.int32, (k,)), sizes)
+    # below 65 centroids of 8 dimensions and fewer in all the sums are added block by block of 1024 rows
+    if k <= 64 and k * 4 <= 512 and n > 1024:
+        assert np.allclose(cb.to_numpy(np.float32, (k, 4)), want, rtol=1e-5, atol=1e-6)
+    else:
+        assert np.array_equal(cb.to_numpy(np.float32, (k, 4)), want)

@@ -563,24 +563,56 @@ fill_u64_kernel(unsigned long long* p, unsigned long long v, uint64_t n) {
     }
 }
 
-// ||row||^2 for every row; one wave per row.
+// ||row||^2 for every row.  It is a read of the rows and nothing else, so what counts is bytes in flight: 16 lanes take a
+// row in runs of 16 bytes each, four rows at once, and every component has a sum of its own (as many additions in a chain
+// as when a wave took a row).  904 914 x 416 rows: a wave per row and 4 bytes per lane 488 us (3.1 TB/s), this
+// 242 us (6.2 TB/s); 747 490 x 96: 150 -> 46 us.
+constexpr uint32_t kNormRows = 4;                       // rows of a group of 16 lanes
+constexpr uint32_t kNormBlock = 16 * kNormRows;         // rows of a workgroup
+typedef float float4_any __attribute__((ext_vector_type(4), aligned(4)));  // rows need not be 16-byte aligned
+
 __global__ void __launch_bounds__(256)
 row_sqnorm_kernel(const float* x, uint64_t n, uint32_t dim, float* out) {
-    uint64_t row = static_cast<uint64_t>(blockIdx.x) * 4 + (threadIdx.x >> 6);
-    uint32_t lane = threadIdx.x & 63;
-    if (row >= n) {
-        return;
+    const uint32_t l16 = threadIdx.x & 15;
+    const uint64_t row0 = static_cast<uint64_t>(blockIdx.x) * kNormBlock + (threadIdx.x >> 4) * kNormRows;
+    const float* rows[kNormRows];
+    float4_any sums[kNormRows];
+#pragma unroll
+    for (uint32_t r = 0; r < kNormRows; ++r) {  // (rows past the end repeat the last one)
+        rows[r] = x + (row0 + r < n ? row0 + r : n - 1) * dim;
+        sums[r] = float4_any{0.0F, 0.0F, 0.0F, 0.0F};
     }
-    const float* r = x + row * dim;
-    float s = 0.0F;
-    for (uint32_t d = lane; d < dim; d += 64) {
-        s = fmaf(r[d], r[d], s);
+    const uint32_t whole = dim & ~3U;
+    for (uint32_t d = 4 * l16; d < whole; d += 64) {
+        float4_any v[kNormRows];
+#pragma unroll
+        for (uint32_t r = 0; r < kNormRows; ++r) {
+            v[r] = *reinterpret_cast<const float4_any*>(rows[r] + d);
+        }
+#pragma unroll
+        for (uint32_t r = 0; r < kNormRows; ++r) {
+#pragma unroll
+            for (uint32_t e = 0; e < 4; ++e) {
+                sums[r][e] = fmaf(v[r][e], v[r][e], sums[r][e]);
+            }
+        }
     }
-    for (int off = 32; off > 0; off >>= 1) {
-        s += __shfl_down(s, off);
+    if (whole + l16 < dim) {
+#pragma unroll
+        for (uint32_t r = 0; r < kNormRows; ++r) {
+            const float v = rows[r][whole + l16];
+            sums[r][0] = fmaf(v, v, sums[r][0]);
+        }
     }
-    if (lane == 0) {
-        out[row] = s;
+#pragma unroll
+    for (uint32_t r = 0; r < kNormRows; ++r) {
+        float s = (sums[r][0] + sums[r][1]) + (sums[r][2] + sums[r][3]);
+        for (int off = 8; off > 0; off >>= 1) {
+            s += __shfl_down(s, off, 16);
+        }
+        if (l16 == 0 && row0 + r < n) {
+            out[row0 + r] = s;
+        }
     }
 }
 
@@ -659,7 +691,7 @@ count_labels_kernel(const int32_t* labels, uint64_t n, uint32_t k, uint32_t* cou
 // Exclusive prefix sum of k counts by one workgroup (k is a few thousand).
 __global__ void __launch_bounds__(1024)
 exclusive_scan_kernel(const uint32_t* counts, uint32_t k, uint32_t* offsets) {
-    __shared__ uint32_t sums[1024];
+    __shared__ uint32_t sums[16];
     uint32_t per = (k + blockDim.x - 1) / blockDim.x;
     uint32_t begin = threadIdx.x * per;
     uint32_t end = begin + per < k ? begin + per : k;
@@ -667,22 +699,154 @@ exclusive_scan_kernel(const uint32_t* counts, uint32_t k, uint32_t* offsets) {
     for (uint32_t i = begin; i < end; ++i) {
         s += counts[i];
     }
-    sums[threadIdx.x] = s;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        uint32_t run = 0;
-        for (uint32_t i = 0; i < blockDim.x; ++i) {
-            uint32_t t = sums[i];
-            sums[i] = run;
-            run += t;
-        }
-        offsets[k] = run;
+    uint32_t upto = s;  // inclusive sums: over the lanes of a wave, then over the waves
+    for (int off = 1; off < 64; off <<= 1) {
+        const uint32_t v = __shfl_up(upto, off);
+        upto += static_cast<int>(threadIdx.x & 63) >= off ? v : 0;
+    }
+    if ((threadIdx.x & 63) == 63) {
+        sums[threadIdx.x >> 6] = upto;
     }
     __syncthreads();
-    uint32_t run = sums[threadIdx.x];
+    uint32_t run = upto - s;
+    for (uint32_t w = 0; w < (threadIdx.x >> 6); ++w) {
+        run += sums[w];
+    }
+    if (threadIdx.x == blockDim.x - 1) {
+        offsets[k] = run + s;
+    }
     for (uint32_t i = begin; i < end; ++i) {
         offsets[i] = run;
         run += counts[i];
+    }
+}
+
+// The rows of every label, in row order: a stable counting sort.  A unit is a run of rows; the units' counts per label
+// stand in a table, a column of which is summed over the units, and one wave per unit then gives its rows their places.
+// (Every row counted by an atomic on its label's counter in memory, and the rows sorted by hipCUB in up to 20 launches,
+// took 1.41 ms for 904 914 rows of 98 labels, most of it the atomics that meet at a counter, and 0.15 ms for 1M rows of
+// 4096; this takes 32 us for the first, 24-35 us for anything between.)
+constexpr uint32_t kGroupMaxLabels = 16384;  // a unit's counters stand in 64 KB of LDS
+constexpr uint32_t kGroupMinRows = 1024;     // rows of a unit, at least
+constexpr uint32_t kGroupChunks = 16;        // parts of a column that are summed side by side
+
+struct GroupPlan {
+    uint32_t unit_rows, units;
+};
+
+// The table has units x k words and lies in the 2 n words of the buffers that the general sort keeps its pairs in.
+static GroupPlan
+group_plan(uint64_t n, uint32_t k) {
+    GroupPlan p;
+    p.unit_rows = static_cast<uint32_t>(round_up(k / 2 + 1 > kGroupMinRows ? k / 2 + 1 : kGroupMinRows, 64));
+    p.units = static_cast<uint32_t>(div_up(n, p.unit_rows));
+    return p;
+}
+
+static bool
+group_takes(uint64_t n, uint32_t k) {
+    return k <= kGroupMaxLabels && static_cast<uint64_t>(group_plan(n, k).units) * k <= 2 * n;
+}
+
+__global__ void __launch_bounds__(256)
+group_count_kernel(const int32_t* labels, uint64_t n, uint32_t k, uint32_t unit_rows, uint32_t* table) {
+    extern __shared__ uint32_t counters[];
+    for (uint32_t l = threadIdx.x; l < k; l += blockDim.x) {
+        counters[l] = 0;
+    }
+    __syncthreads();
+    const uint64_t first = static_cast<uint64_t>(blockIdx.x) * unit_rows;
+    const uint64_t last = first + unit_rows < n ? first + unit_rows : n;
+    for (uint64_t i = first + threadIdx.x; i < last; i += blockDim.x) {
+        const uint32_t l = static_cast<uint32_t>(labels[i]);
+        if (l < k) {  // (a negative label is a large one here: no row of any centroid)
+            atomicAdd(&counters[l], 1U);
+        }
+    }
+    __syncthreads();
+    for (uint32_t l = threadIdx.x; l < k; l += blockDim.x) {
+        table[static_cast<uint64_t>(blockIdx.x) * k + l] = counters[l];
+    }
+}
+
+// table[u][l] becomes the rows of label l in the units before u, counts[l] those of all units.  64 labels a workgroup (a
+// lane each: whole lines), a wave for each part of the column.
+__global__ void __launch_bounds__(64 * kGroupChunks)
+group_columns_kernel(uint32_t* table, uint32_t units, uint32_t k, uint32_t* counts) {
+    __shared__ uint32_t part[kGroupChunks][64];
+    const uint32_t lane = threadIdx.x & 63, chunk = threadIdx.x >> 6;
+    const uint32_t l = blockIdx.x * 64 + lane;
+    const uint32_t per = (units + kGroupChunks - 1) / kGroupChunks;
+    const uint32_t begin = chunk * per < units ? chunk * per : units;
+    const uint32_t end = begin + per < units ? begin + per : units;
+    uint32_t* column = table + (l < k ? l : k - 1);
+    uint32_t sum = 0;
+#pragma unroll 8
+    for (uint32_t u = begin; u < end; ++u) {
+        sum += column[static_cast<uint64_t>(u) * k];
+    }
+    part[chunk][lane] = sum;
+    __syncthreads();
+    uint32_t run = 0;
+    for (uint32_t c = 0; c < chunk; ++c) {
+        run += part[c][lane];
+    }
+    if (l >= k) {
+        return;
+    }
+    if (chunk == kGroupChunks - 1) {
+        counts[l] = run + sum;
+    }
+    for (uint32_t u0 = begin; u0 < end; u0 += 8) {  // eight loads on their way before the first store behind them
+        uint32_t c[8];
+#pragma unroll
+        for (uint32_t v = 0; v < 8; ++v) {
+            c[v] = column[static_cast<uint64_t>(u0 + v < end ? u0 + v : end - 1) * k];
+        }
+#pragma unroll
+        for (uint32_t v = 0; v < 8; ++v) {
+            if (u0 + v < end) {
+                column[static_cast<uint64_t>(u0 + v) * k] = run;
+                run += c[v];
+            }
+        }
+    }
+}
+
+// One wave per unit: 64 rows at a time find, ballot by ballot over the bits of their labels, the lanes that share theirs;
+// a row's place is its label's next one plus the lanes before it, and the last of them moves the label on.
+__global__ void __launch_bounds__(64)
+group_scatter_kernel(const int32_t* labels, uint64_t n, uint32_t k, uint32_t bits, uint32_t unit_rows,
+                     const uint32_t* table, const uint32_t* offsets, uint32_t* rows_out) {
+    extern __shared__ uint32_t next[];
+    const uint32_t lane = threadIdx.x;
+    for (uint32_t l = lane; l < k; l += 64) {
+        next[l] = offsets[l] + table[static_cast<uint64_t>(blockIdx.x) * k + l];
+    }
+    __syncthreads();
+    const uint64_t first = static_cast<uint64_t>(blockIdx.x) * unit_rows;
+    const uint64_t last = first + unit_rows < n ? first + unit_rows : n;
+    const uint64_t before = (1ull << lane) - 1;
+    uint32_t l = first + lane < last ? static_cast<uint32_t>(labels[first + lane]) : 0xFFFFFFFFU;
+    for (uint64_t i0 = first; i0 < last; i0 += 64) {
+        const uint64_t ahead = i0 + 64 + lane;
+        const uint32_t l_next = ahead < last ? static_cast<uint32_t>(labels[ahead]) : 0xFFFFFFFFU;
+        const bool valid = l < k;
+        uint64_t same = __ballot(valid);
+        for (uint32_t b = 0; b < bits; ++b) {
+            const bool bit = ((l >> b) & 1) != 0;
+            const uint64_t set = __ballot(bit);
+            same &= bit ? set : ~set;
+        }
+        if (valid) {
+            const uint32_t place = next[l] + static_cast<uint32_t>(__popcll(same & before));
+            rows_out[place] = static_cast<uint32_t>(i0 + lane);
+            if ((same >> lane) == 1) {  // the last lane of its label
+                next[l] = place + 1;
+            }
+        }
+        __syncthreads();  // (one wave: the next rows read what was written above)
+        l = l_next;
     }
 }
 
@@ -701,7 +865,6 @@ constexpr uint32_t kMeanDims = 64;
 constexpr uint32_t kMeanRows = 64;   // per stage
 constexpr uint32_t kMeanLoads = kMeanRows / 16;
 constexpr uint64_t kMeanGrid = 1ull << 22;
-typedef float float4_any __attribute__((ext_vector_type(4), aligned(4)));  // rows need not be 16-byte aligned
 
 // QUADS: the dimension is a multiple of 4, a run of four dimensions lies in one row.
 template <bool QUADS>
@@ -857,7 +1020,7 @@ max_norm_kernel(const float* out, uint64_t n, uint32_t* max_bits) {
 // ||row||^2 of nx rows and the largest of them (as float bits).
 int
 launch_row_sqnorms(const float* x, uint64_t nx, uint32_t dim, float* out, uint32_t* max_bits, hipStream_t st) {
-    hipLaunchKernelGGL(row_sqnorm_kernel, dim3(static_cast<uint32_t>(div_up(nx, 4))), dim3(256), 0, st, x, nx, dim, out);
+    hipLaunchKernelGGL(row_sqnorm_kernel, dim3(static_cast<uint32_t>(div_up(nx, kNormBlock))), dim3(256), 0, st, x, nx, dim, out);
     hipLaunchKernelGGL(max_norm_kernel, dim3(1), dim3(1024), 0, st, out, nx, max_bits);
     VA_HIP(hipGetLastError());
     return 0;
@@ -892,10 +1055,10 @@ carve_assign(Carver& c, uint64_t n, uint32_t dim, uint32_t k, bool preselect, As
 static int
 assign_launch(const float* x, uint64_t n, uint32_t dim, const float* cent, uint32_t k, int32_t* labels,
               float* min_dist, double* loss_dev, const AssignBuffers& b, int iteration, hipStream_t st) {
-    hipLaunchKernelGGL(row_sqnorm_kernel, dim3(static_cast<uint32_t>(div_up(k, 4))), dim3(256), 0, st, cent,
+    hipLaunchKernelGGL(row_sqnorm_kernel, dim3(static_cast<uint32_t>(div_up(k, kNormBlock))), dim3(256), 0, st, cent,
                        static_cast<uint64_t>(k), dim, b.ynorm);
     if (iteration == 0 && !b.h16) {  // (from the second Lloyd iteration on |x|^2 is there)
-        hipLaunchKernelGGL(row_sqnorm_kernel, dim3(static_cast<uint32_t>(div_up(n, 4))), dim3(256), 0, st, x, n, dim,
+        hipLaunchKernelGGL(row_sqnorm_kernel, dim3(static_cast<uint32_t>(div_up(n, kNormBlock))), dim3(256), 0, st, x, n, dim,
                            b.xnorm);
     }
     if (!b.h16) {
@@ -1012,8 +1175,8 @@ static size_t
 carve_update(Carver& c, uint64_t n, uint32_t k, UpdateBuffers* b) {
     b->counts = c.take<uint32_t>(k + 1);
     b->offsets = c.take<uint32_t>(k + 1);
-    b->rows_in = c.take<uint32_t>(n);
     b->rows_out = c.take<uint32_t>(n);
+    b->rows_in = c.take<uint32_t>(n);  // (with keys_out behind it: the counting sort's table)
     b->keys_out = c.take<int32_t>(n);
     b->sort_tmp_bytes = sort_temp_bytes(n);
     b->sort_tmp = c.take<uint8_t>(b->sort_tmp_bytes);
@@ -1097,19 +1260,31 @@ update_launch(const float* x, const int32_t* labels, uint64_t n, uint32_t dim, u
         VA_HIP(hipGetLastError());
         return 0;
     }
-    uint32_t blocks = static_cast<uint32_t>(div_up(n, 256));
-    hipLaunchKernelGGL(fill_u64_kernel, dim3((k / 2 + 1 + 255) / 256), dim3(256), 0, st,
-                       reinterpret_cast<unsigned long long*>(b.counts), 0ull, static_cast<uint64_t>(k / 2 + 1));
-    hipLaunchKernelGGL(count_labels_kernel, dim3(blocks), dim3(256), 0, st, labels, n, k, b.counts);
-    hipLaunchKernelGGL(exclusive_scan_kernel, dim3(1), dim3(1024), 0, st, b.counts, k, b.offsets);
-    hipLaunchKernelGGL(iota_u32_kernel, dim3(blocks), dim3(256), 0, st, b.rows_in, n);
     int end_bit = 1;
     while ((1ull << end_bit) < k) {
         ++end_bit;
     }
-    size_t tmp_bytes = b.sort_tmp_bytes;
-    VA_HIP(hipcub::DeviceRadixSort::SortPairs(b.sort_tmp, tmp_bytes, labels, b.keys_out, b.rows_in, b.rows_out,
-                                              static_cast<int>(n), 0, end_bit, st));
+    if (group_takes(n, k)) {
+        const GroupPlan p = group_plan(n, k);
+        hipLaunchKernelGGL(group_count_kernel, dim3(p.units), dim3(256), k * sizeof(uint32_t), st, labels, n, k, p.unit_rows,
+                           b.rows_in);
+        hipLaunchKernelGGL(group_columns_kernel, dim3((k + 63) / 64), dim3(64 * kGroupChunks), 0, st, b.rows_in, p.units, k,
+                           b.counts);
+        hipLaunchKernelGGL(exclusive_scan_kernel, dim3(1), dim3(1024), 0, st, b.counts, k, b.offsets);
+        hipLaunchKernelGGL(group_scatter_kernel, dim3(p.units), dim3(64), k * sizeof(uint32_t), st, labels, n, k,
+                           static_cast<uint32_t>(end_bit), p.unit_rows, b.rows_in, b.offsets, b.rows_out);
+    } else {
+        // more labels than a unit has counters for
+        uint32_t blocks = static_cast<uint32_t>(div_up(n, 256));
+        hipLaunchKernelGGL(fill_u64_kernel, dim3((k / 2 + 1 + 255) / 256), dim3(256), 0, st,
+                           reinterpret_cast<unsigned long long*>(b.counts), 0ull, static_cast<uint64_t>(k / 2 + 1));
+        hipLaunchKernelGGL(count_labels_kernel, dim3(blocks), dim3(256), 0, st, labels, n, k, b.counts);
+        hipLaunchKernelGGL(exclusive_scan_kernel, dim3(1), dim3(1024), 0, st, b.counts, k, b.offsets);
+        hipLaunchKernelGGL(iota_u32_kernel, dim3(blocks), dim3(256), 0, st, b.rows_in, n);
+        size_t tmp_bytes = b.sort_tmp_bytes;
+        VA_HIP(hipcub::DeviceRadixSort::SortPairs(b.sort_tmp, tmp_bytes, labels, b.keys_out, b.rows_in, b.rows_out,
+                                                  static_cast<int>(n), 0, end_bit, st));
+    }
     const uint64_t tasks = static_cast<uint64_t>(k) * div_up(dim, kMeanDims);
     const dim3 grid(static_cast<uint32_t>(tasks < kMeanGrid ? tasks : kMeanGrid));
     if ((dim & 3) == 0) {
