@@ -574,88 +574,99 @@ store_f32(uint8_t* p, float v) {
 }
 
 // Column means as running fp32 sums over the rows in order (rabitq_quantizer.cpp:224-241).  A workgroup owns 32
-// columns: all 1024 threads stage the next 256 rows of those columns in LDS while the first 32 threads add the
-// current 256 rows, one column each, in row order -- the additions stay sequential, the loads do not.
+// columns: eight waves stage the next 256 rows of those columns in LDS while a ninth adds the current 256, one column a
+// lane, in row order -- the additions stay sequential, the loads do not.
 //
-// What bounds it is one memory latency per stage in flight: four stages are, so that a latency is spread over 1024 rows (one
-// stage in flight: 6.9 ns a row, 5.0 ns now; the chain of adds itself is most of that).
+// What bounds it is the chain of adds.  Four stages are on their way, so that a memory latency is spread over 1024 rows, and
+// the adding wave does nothing else and goes first on its SIMD (168 787 x 128 rows: 849 us with a
+// wave that loads as well, 730 now: 4.3 ns a row).
 constexpr uint32_t kMeanCols = 32;
 constexpr uint32_t kMeanRows = 256;
 constexpr uint32_t kMeanAhead = 4;
+constexpr uint32_t kMeanLoaders = 512;
+constexpr uint32_t kMeanSlots = kMeanLoaders / kMeanCols;   // rows of a load
+constexpr uint32_t kMeanLoads = kMeanRows / kMeanSlots;     // loads of a stage
 
-__global__ void __launch_bounds__(1024)
+__global__ void __launch_bounds__(kMeanLoaders + kWave)
 column_mean_seq_kernel(const float* x, uint64_t n, uint32_t dim, float* mean) {
     __shared__ __align__(16) float stage[2][kMeanCols][kMeanRows + 4];  // a column's rows in a run: four of them a read
-    const uint32_t col = threadIdx.x & (kMeanCols - 1);
-    const uint32_t slot = threadIdx.x / kMeanCols;  // 0..31
-    const uint32_t d = blockIdx.x * kMeanCols + col;
-    const bool live = d < dim;
-    float regs[kMeanAhead][kMeanRows / 32];
-    // (no branch around a load: the wait for one stage must not become a wait for all that are in flight)
-    const uint32_t d_in = live ? d : dim - 1;
-    auto fetch = [&](uint64_t row0, float(&to)[kMeanRows / 32]) {
-#pragma unroll
-        for (uint32_t u = 0; u < kMeanRows / 32; ++u) {
-            const uint64_t r = row0 + u * 32 + slot;
-            to[u] = x[(r < n ? r : n - 1) * dim + d_in];
-        }
-    };
-#pragma unroll
-    for (uint32_t a = 0; a < kMeanAhead; ++a) {
-        fetch(static_cast<uint64_t>(a) * kMeanRows, regs[a]);
-    }
-    float s = 0.0F;
     static_assert(kMeanAhead % 2 == 0, "the two LDS buffers alternate within a round");
-    for (uint64_t base = 0; base < n; base += kMeanAhead * kMeanRows) {
+    if (threadIdx.x < kMeanLoaders) {
+        const uint32_t col = threadIdx.x & (kMeanCols - 1);
+        const uint32_t slot = threadIdx.x / kMeanCols;
+        const uint32_t d = blockIdx.x * kMeanCols + col;
+        float regs[kMeanAhead][kMeanLoads];
+        // (no branch around a load: the wait for one stage must not become a wait for all that are in flight)
+        const uint32_t d_in = d < dim ? d : dim - 1;
+        auto fetch = [&](uint64_t row0, float(&to)[kMeanLoads]) {
+#pragma unroll
+            for (uint32_t u = 0; u < kMeanLoads; ++u) {
+                const uint64_t r = row0 + u * kMeanSlots + slot;
+                to[u] = x[(r < n ? r : n - 1) * dim + d_in];
+            }
+        };
 #pragma unroll
         for (uint32_t a = 0; a < kMeanAhead; ++a) {
-            const uint64_t row0 = base + a * kMeanRows;
-            if (row0 >= n) {
-                break;
-            }
-            // Buffer a & 1 was last read two stages ago, a barrier ago.
+            fetch(static_cast<uint64_t>(a) * kMeanRows, regs[a]);
+        }
+        for (uint64_t base = 0; base < n; base += kMeanAhead * kMeanRows) {
 #pragma unroll
-            for (uint32_t u = 0; u < kMeanRows / 32; ++u) {
-                stage[a & 1U][col][u * 32 + slot] = regs[a][u];
+            for (uint32_t a = 0; a < kMeanAhead; ++a) {
+                const uint64_t row0 = base + a * kMeanRows;
+                if (row0 >= n) {
+                    break;
+                }
+                // Buffer a & 1 was last read two stages ago, a barrier ago.
+#pragma unroll
+                for (uint32_t u = 0; u < kMeanLoads; ++u) {
+                    stage[a & 1U][col][u * kMeanSlots + slot] = regs[a][u];
+                }
+                fetch(row0 + kMeanAhead * kMeanRows, regs[a]);
+                __syncthreads();
             }
-            fetch(row0 + kMeanAhead * kMeanRows, regs[a]);
-            __syncthreads();
-            if (slot == 0) {
-                const uint32_t m = n - row0 < kMeanRows ? static_cast<uint32_t>(n - row0) : kMeanRows;
-                const float* rows = stage[a & 1U][col];
-                if (m == kMeanRows) {
-                    // the LDS reads of the next 32 rows ahead of the adds of these: only the adds wait for each other
-                    float4 v[2][8];
+        }
+        return;
+    }
+    __builtin_amdgcn_s_setprio(3);
+    const uint32_t col = threadIdx.x & (kMeanCols - 1);  // (both halves of the wave add; the first one writes)
+    const uint32_t d = blockIdx.x * kMeanCols + col;
+    float s = 0.0F;
+    uint32_t a = 0;
+    for (uint64_t row0 = 0; row0 < n; row0 += kMeanRows, a ^= 1) {  // a barrier per stage, as above
+        __syncthreads();
+        const uint32_t m = n - row0 < kMeanRows ? static_cast<uint32_t>(n - row0) : kMeanRows;
+        const float* rows = stage[a][col];
+        if (m == kMeanRows) {
+            // the LDS reads of the next 32 rows ahead of the adds of these: only the adds wait for each other
+            float4 v[2][8];
+#pragma unroll
+            for (uint32_t u = 0; u < 8; ++u) {
+                v[0][u] = *reinterpret_cast<const float4*>(rows + 4 * u);
+            }
+#pragma unroll
+            for (uint32_t r = 0; r < kMeanRows; r += 32) {
+                if (r + 32 < kMeanRows) {
 #pragma unroll
                     for (uint32_t u = 0; u < 8; ++u) {
-                        v[0][u] = *reinterpret_cast<const float4*>(rows + 4 * u);
-                    }
-#pragma unroll
-                    for (uint32_t r = 0; r < kMeanRows; r += 32) {
-                        if (r + 32 < kMeanRows) {
-#pragma unroll
-                            for (uint32_t u = 0; u < 8; ++u) {
-                                v[(r / 32 + 1) & 1][u] = *reinterpret_cast<const float4*>(rows + r + 32 + 4 * u);
-                            }
-                        }
-#pragma unroll
-                        for (uint32_t u = 0; u < 8; ++u) {
-                            const float4 four = v[(r / 32) & 1][u];
-                            s += four.x;
-                            s += four.y;
-                            s += four.z;
-                            s += four.w;
-                        }
-                    }
-                } else {
-                    for (uint32_t r = 0; r < m; ++r) {
-                        s += rows[r];
+                        v[(r / 32 + 1) & 1][u] = *reinterpret_cast<const float4*>(rows + r + 32 + 4 * u);
                     }
                 }
+#pragma unroll
+                for (uint32_t u = 0; u < 8; ++u) {
+                    const float4 w = v[(r / 32) & 1][u];
+                    s += w.x;
+                    s += w.y;
+                    s += w.z;
+                    s += w.w;
+                }
+            }
+        } else {
+            for (uint32_t r = 0; r < m; ++r) {
+                s += rows[r];
             }
         }
     }
-    if (slot == 0 && live) {
+    if (threadIdx.x < kMeanLoaders + kMeanCols && d < dim) {
         mean[d] = s / static_cast<float>(n);
     }
 }
@@ -1810,8 +1821,8 @@ vsag_amd_rabitq_train(const float* x_dev, uint64_t n, uint32_t dim, const float*
     hipStream_t st = static_cast<hipStream_t>(stream);
     float* mean = nullptr;
     VA_HIP(hipMallocAsync(reinterpret_cast<void**>(&mean), dim * 4, st));
-    hipLaunchKernelGGL(column_mean_seq_kernel, dim3((dim + kMeanCols - 1) / kMeanCols), dim3(1024), 0, st, x_dev, n, dim,
-                       mean);
+    hipLaunchKernelGGL(column_mean_seq_kernel, dim3((dim + kMeanCols - 1) / kMeanCols), dim3(kMeanLoaders + kWave), 0,
+                       st, x_dev, n, dim, mean);
     int rc = gemm_nt_seq(mean, rotation_dev, centroid_dev, 1, dim, dim, st);
     VA_HIP(hipFreeAsync(mean, st));
     return rc;
