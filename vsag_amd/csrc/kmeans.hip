@@ -589,8 +589,9 @@ fill_u64_kernel(unsigned long long* p, unsigned long long v, uint64_t n) {
 }
 
 // ||row||^2 for every row.  It is a read of the rows and nothing else, so what counts is bytes in flight: 16 lanes take a
-// row in runs of 16 bytes each, four rows at once, and every component has a sum of its own (as many additions in a chain
-// as when a wave took a row).  904 914 x 416 rows: a wave per row and 4 bytes per lane 488 us (3.1 TB/s), this
+// row in runs of 16 bytes each, four rows at once, and every component has a sum of its own.  The sums are those of a wave
+// that takes dimension d in lane d % 64 and folds its lanes 32, 16, ... 1, bit for bit: with another order some rows between
+// two centroids change their label.  904 914 x 416 rows: a wave per row and 4 bytes per lane 488 us (3.1 TB/s), this
 // 242 us (6.2 TB/s); 747 490 x 96: 150 -> 46 us.
 constexpr uint32_t kNormRows = 4;                       // rows of a group of 16 lanes
 constexpr uint32_t kNormBlock = 16 * kNormRows;         // rows of a workgroup
@@ -622,21 +623,29 @@ row_sqnorm_kernel(const float* x, uint64_t n, uint32_t dim, float* out) {
             }
         }
     }
-    if (whole + l16 < dim) {
+    // Dimension d belongs to component d % 4 of lane (d % 64) / 4, behind those that the lane has summed above.
+    if (whole < dim && l16 == (whole & 63) >> 2) {
 #pragma unroll
         for (uint32_t r = 0; r < kNormRows; ++r) {
-            const float v = rows[r][whole + l16];
-            sums[r][0] = fmaf(v, v, sums[r][0]);
+#pragma unroll
+            for (uint32_t e = 0; e < 3; ++e) {
+                if (whole + e < dim) {
+                    const float v = rows[r][whole + e];
+                    sums[r][e] = fmaf(v, v, sums[r][e]);
+                }
+            }
         }
     }
 #pragma unroll
     for (uint32_t r = 0; r < kNormRows; ++r) {
-        float s = (sums[r][0] + sums[r][1]) + (sums[r][2] + sums[r][3]);
-        for (int off = 8; off > 0; off >>= 1) {
-            s += __shfl_down(s, off, 16);
+#pragma unroll
+        for (uint32_t e = 0; e < 4; ++e) {
+            for (int off = 8; off > 0; off >>= 1) {
+                sums[r][e] += __shfl_down(sums[r][e], off, 16);
+            }
         }
         if (l16 == 0 && row0 + r < n) {
-            out[row0 + r] = s;
+            out[row0 + r] = (sums[r][0] + sums[r][2]) + (sums[r][1] + sums[r][3]);
         }
     }
 }
