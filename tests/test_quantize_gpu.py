@@ -377,3 +377,42 @@ def test_sq_bounds_of_columns_that_are_not_finite(lib, bits, n, odd):
     assert np.array_equal(lb, lower, equal_nan=True)
     with np.errstate(invalid="ignore"):
         assert np.array_equal(diff, upper - lower, equal_nan=True)
+
+
+@pytest.mark.parametrize("bits", [8, 4])
+@pytest.mark.parametrize("metric", [orc.L2, orc.COSINE])
+@pytest.mark.parametrize("n,d", [(9, 2), (1, 1), (37, 100), (7001, 130), (3, 4096), (11, 4104), (301, 257), (77, 1023), (9, 1025)])
+def test_sq_encode_at_the_levels_edges(lib, bits, metric, n, d):
+    """Values a few units in the last place around every level's edge, columns whose diff lies at the ends of what is
+    multiplied by its reciprocal (2^-23, 2^100) and beyond, infinities and NaN: the codes are the divided ones."""
+    L = lib.load_library()
+    rng = np.random.default_rng(7 * n + d + bits)
+    special = np.array([1.2e-7, 1.19e-7, 1e-9, 0.0, 2.0 ** 100, 2.0 ** 101, 3e38, 0.1, 1.0 - 2.0 ** -24], dtype=np.float32)
+    diff = (2.0 ** rng.uniform(-20, 20, d)).astype(np.float32)
+    diff[:min(d, special.size)] = special[:min(d, special.size)]
+    lb = np.where(rng.random(d) < 0.5, 0.0, -0.37 * diff).astype(np.float32)
+    k = rng.integers(0, 2 ** bits, (n, d)).astype(np.float32) / np.float32(2 ** bits - 1)
+    x = (k * diff).astype(np.float32)
+    x = (x.view(np.int32) + rng.integers(-3, 4, (n, d)).astype(np.int32)).view(np.float32)
+    x = (x + lb).astype(np.float32)
+    if metric == orc.L2:
+        odd = rng.random((n, d)) < 0.01
+        x[odd] = rng.choice(np.array([np.inf, -np.inf, np.nan, 3.4e38, -3.4e38, 1e-40], dtype=np.float32), odd.sum())
+    else:
+        x = np.clip(np.nan_to_num(x, nan=1.0, posinf=1.0, neginf=-1.0), -1e6, 1e6).astype(np.float32)
+    code_size = (d * bits + 7) // 8
+    xb, lbb, dfb, out = dev(x), dev(lb), dev(diff), capi.DeviceBuffer(n * code_size)
+    capi.check(L.vsag_amd_sq_encode(xb.ptr, n, d, bits, metric, lbb.ptr, dfb.ptr, out.ptr, None))
+    assert np.array_equal(out.to_numpy(np.uint8, (n, code_size)), orc.sq_encode(x, bits, lb, diff, metric))
+
+
+@pytest.mark.parametrize("n", [32768, 32769, 65536, 65537, 100352, 100353])
+def test_sq_train_at_the_ends_of_the_register_tiers(lib, n):
+    rng = np.random.default_rng(n)
+    x = rng.standard_normal((n, 3)).astype(np.float32)
+    x[rng.random(n) < 0.5, 1] = 0.25   # one value many times: its bin is cut again
+    x[n // 2, 2] = np.inf              # no linear bins
+    for mode in (capi.SQ_TRAIN_TRUNC_BOUND, capi.SQ_TRAIN_CLASSIC):
+        lb, diff = _train(lib, x, 8, orc.L2, mode, max_sample=n)
+        rlb, rdiff = orc.sq_train(x, 8, orc.L2, mode=mode, max_sample=n)
+        assert np.array_equal(lb, rlb) and np.array_equal(diff, rdiff)

@@ -129,78 +129,119 @@ sq_level(float v, float lb, float diff, float levels) {
     return static_cast<uint8_t>(levels * clamp_delta(delta));
 }
 
+// 1 / diff where a division by diff can be replaced: a = v - lb, q = a * inv is two units in the last place off at most, a
+// first remainder brings it to within one, and from there a remainder and a correction give the rounded quotient if inv is
+// the rounded reciprocal (Markstein, IBM J. Res. Dev. 34, 1990), as long as nothing leaves the normal numbers: diff is held
+// to [2^-23, 2^100], and a quotient below 1/256 is level 0 however it is rounded.  0 elsewhere: such a column divides.
+__device__ inline float
+sq_inverse(float diff) {
+    return diff >= FLT_EPSILON && diff <= 0x1p100F ? 1.0F / diff : 0.0F;
+}
+
+// sq_level with inv = sq_inverse(diff): the same level for every v.
+__device__ inline uint32_t
+sq_level_by_inverse(float v, float lb, float diff, float inv, float levels) {
+    if (inv == 0.0F) {
+        return sq_level(v, lb, diff, levels);
+    }
+    const float a = v - lb;
+    const float q = a * inv;
+    float delta = fmaf(fmaf(-q, diff, a), inv, q);
+    delta = fmaf(fmaf(-delta, diff, a), inv, delta);
+    delta = q < 2.0F ? delta : q;  // (far above the range an infinity has no remainder)
+    return static_cast<uint8_t>(levels * clamp_delta(delta));
+}
+
 // Rows and codes as two flat arrays: where a row fills whole bytes (sq8; sq4 with an even dimension) neither has a gap, so
 // a thread turns 4 (sq8) or 8 (sq4) values in a run, wherever rows begin in it, into one code word: 16-byte loads and 4-byte
-// stores at any dimension.  Bound by memory (1M x 128 rows to sq8: 466 us with a thread per byte, 160 us, 4.0 TB/s of
-// rows and codes).  VEC: the dimension is a multiple of four, a run of four values lies in one row.
-template <int BITS, bool VEC>
-__global__ void __launch_bounds__(256)
+// stores at any dimension.  A workgroup of `blockDim` threads takes RUNS x blockDim consecutive runs; with RUNS > 1 blockDim
+// runs are whole rows, so a thread meets the same dimensions in each of its runs and keeps their bounds in registers, with
+// RUNS loads on their way.  What bounds it is memory: 1M x 128 rows to sq8 466 us with a thread per byte, 138 us with a run
+// per thread and a division per value, 132 us without the division, and 108 us with short workgroups of four runs a
+// thread that pass the caches by (2048 long-lived ones, loads and stores as they come: 132; the reading alone 72).
+template <int BITS, bool NORM, int RUNS>
+__global__ void __launch_bounds__(1024)
 sq_encode_kernel(const float* x, uint64_t total, uint32_t dim, const float* lb, const float* diff, const float* norms,
                  uint8_t* codes) {
     constexpr uint32_t kDims = 32 / BITS;  // per code word
-    const uint64_t first = static_cast<uint64_t>(blockIdx.x) * (256 * kDims);
-    const uint64_t at = first + threadIdx.x * kDims;
-    if (at >= total) {
+    const uint64_t first = static_cast<uint64_t>(blockIdx.x) * (blockDim.x * RUNS);  // of the workgroup
+    const uint64_t whole = total / kDims;
+    const uint64_t run = first + threadIdx.x;
+    if (run * kDims >= total) {
         return;
     }
-    // Row and dimension of the first value, from those of the workgroup (wave-uniform).
-    const uint64_t row0 = first / dim;
-    const uint32_t off = static_cast<uint32_t>(first - row0 * dim) + threadIdx.x * kDims;
-    uint64_t row = row0 + off / dim;
-    uint32_t d = off % dim;
-    const float levels = static_cast<float>((1 << BITS) - 1);
-    const bool whole = at + kDims <= total;
-    float v[kDims];
-    if (whole) {
+    typedef float float4_v __attribute__((ext_vector_type(4)));
+    float v[RUNS][kDims];
+#pragma unroll
+    for (uint32_t r = 0; r < RUNS; ++r) {
+        const uint64_t at = run + r * blockDim.x;
 #pragma unroll
         for (uint32_t e = 0; e < kDims; e += 4) {
-            const float4 a = *reinterpret_cast<const float4*>(x + at + e);
-            v[e] = a.x, v[e + 1] = a.y, v[e + 2] = a.z, v[e + 3] = a.w;
+            float4_v a = {0.0F, 0.0F, 0.0F, 0.0F};
+            if (at < whole) {
+                a = __builtin_nontemporal_load(reinterpret_cast<const float4_v*>(x + at * kDims + e));
+            }
+            v[r][e] = a.x, v[r][e + 1] = a.y, v[r][e + 2] = a.z, v[r][e + 3] = a.w;
         }
-    } else {
+    }
+    // Row and dimension of the first value, from those of the workgroup (wave-uniform).
+    const uint64_t row0 = first * kDims / dim;
+    const uint32_t off = static_cast<uint32_t>(first * kDims - row0 * dim) + threadIdx.x * kDims;
+    const uint64_t row = row0 + off / dim;
+    const uint64_t step_rows = static_cast<uint64_t>(blockDim.x) * kDims / dim;
+    float lo[kDims], df[kDims], inv[kDims];
+    uint32_t row_off[kDims];
+    {
+        uint32_t d = off % dim, r = 0;
 #pragma unroll
         for (uint32_t e = 0; e < kDims; ++e) {
-            v[e] = at + e < total ? x[at + e] : 0.0F;
+            lo[e] = lb[d];
+            df[e] = diff[d];
+            inv[e] = sq_inverse(df[e]);
+            row_off[e] = r;
+            ++d;
+            r += d == dim ? 1 : 0;
+            d = d == dim ? 0 : d;
         }
     }
-    uint32_t word = 0;
+    const float levels = static_cast<float>((1 << BITS) - 1);
 #pragma unroll
-    for (uint32_t e = 0; e < kDims; e += 4) {
-        float lo[4], df[4], nrm[4];
-        if constexpr (VEC) {
-            const float4 l4 = *reinterpret_cast<const float4*>(lb + d);
-            const float4 f4 = *reinterpret_cast<const float4*>(diff + d);
-            lo[0] = l4.x, lo[1] = l4.y, lo[2] = l4.z, lo[3] = l4.w;
-            df[0] = f4.x, df[1] = f4.y, df[2] = f4.z, df[3] = f4.w;
-            nrm[0] = nrm[1] = nrm[2] = nrm[3] = norms != nullptr && at + e < total ? norms[row] : 1.0F;
-            d += 4;
-            row += d == dim ? 1 : 0;
-            d = d == dim ? 0 : d;
+    for (uint32_t r = 0; r < RUNS; ++r) {
+        const uint64_t at = run + r * blockDim.x;
+        if (at * kDims >= total) {
+            break;
+        }
+        const uint32_t values = at < whole ? kDims : static_cast<uint32_t>(total - at * kDims);
+        uint32_t word = 0;
+#pragma unroll
+        for (uint32_t e = 0; e < kDims; ++e) {
+            float value = at < whole || e >= values ? v[r][e] : x[at * kDims + e];
+            if constexpr (NORM) {
+                value /= e < values ? norms[row + r * step_rows + row_off[e]] : 1.0F;
+            }
+            word |= sq_level_by_inverse(value, lo[e], df[e], inv[e], levels) << (e * BITS);
+        }
+        if (at < whole) {
+            __builtin_nontemporal_store(word, reinterpret_cast<uint32_t*>(codes) + at);
         } else {
-#pragma unroll
-            for (uint32_t u = 0; u < 4; ++u) {
-                lo[u] = lb[d];
-                df[u] = diff[d];
-                nrm[u] = norms != nullptr && at + e + u < total ? norms[row] : 1.0F;
-                ++d;
-                row += d == dim ? 1 : 0;
-                d = d == dim ? 0 : d;
+            for (uint32_t b = 0; b < values * BITS / 8; ++b) {
+                codes[at * kDims * BITS / 8 + b] = static_cast<uint8_t>(word >> (8 * b));
             }
         }
-#pragma unroll
-        for (uint32_t u = 0; u < 4; ++u) {
-            const float value = norms != nullptr ? v[e + u] / nrm[u] : v[e + u];
-            word |= sq_level(value, lo[u], df[u], levels) << ((e + u) * BITS);
-        }
     }
-    uint8_t* to = codes + at * BITS / 8;
-    if (whole) {
-        *reinterpret_cast<uint32_t*>(to) = word;
-    } else {
-        for (uint32_t b = 0; b < (total - at) * BITS / 8; ++b) {
-            to[b] = static_cast<uint8_t>(word >> (8 * b));
-        }
+}
+
+// The workgroup of the kernel above: threads, runs per thread.  After `period` runs the dimensions repeat; workgroups are
+// multiples of it with four runs where that makes at most 1024 threads, and one run otherwise (odd dimensions beyond 1024).
+static void
+sq_encode_shape(uint32_t dim, uint32_t kdims, uint32_t* threads, uint32_t* runs) {
+    uint32_t g = kdims;
+    while (dim % g != 0) {
+        g /= 2;
     }
+    const uint32_t period = dim / g;
+    *runs = period <= 1024 ? 4 : 1;
+    *threads = period > 1024 || period == 1 ? 256 : period > 256 ? period : 256 / period * period;
 }
 
 // The same with one thread per code byte: sq4 codes of an odd dimension (the last byte of a row holds one value), and
@@ -1424,6 +1465,49 @@ for_column(const float* vals, uint64_t count, F f) {
     }
 }
 
+// The values of a column, thread t of 1024 holding t, t + 1024, ...: REGS of them in registers, or none (0), where they are
+// read again for every pass over them.
+constexpr uint32_t kBoundThreads = 1024;
+
+template <uint32_t REGS>
+struct ColumnValues {
+    const float* vals;
+    uint64_t count;
+    float v[REGS > 0 ? REGS : 1];
+
+    __device__ inline void
+    load() {
+        if constexpr (REGS > 0) {
+#pragma unroll
+            for (uint32_t u = 0; u < REGS; ++u) {
+                const uint32_t i = threadIdx.x + u * kBoundThreads;
+                v[u] = vals[i < static_cast<uint32_t>(count) ? i : static_cast<uint32_t>(count) - 1];
+            }
+        }
+    }
+
+    template <typename F>
+    __device__ inline void
+    each(F f) {
+        if constexpr (REGS > 0) {
+            uint32_t end = static_cast<uint32_t>(count);
+            asm volatile("" : "+s"(end));
+#pragma unroll
+            for (uint32_t u = 0; u < REGS; ++u) {
+                // (opaque to the compiler, which would keep a mask and a key of every value from one pass to the next: more
+                // than there are registers)
+                asm volatile("" : "+v"(v[u]));
+                if (threadIdx.x + u * kBoundThreads < end) {
+                    f(v[u]);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        } else {
+            for_column(vals, count, f);
+        }
+    }
+};
+
 constexpr uint32_t kBins = 1024;
 constexpr uint32_t kFewKeys = 2048;
 
@@ -1538,25 +1622,30 @@ kth_key_in(const float* vals, uint64_t count, uint32_t base, uint32_t last, uint
 // One workgroup per dimension.  The range of the column's values is cut into 1024 equal bins -- any map that keeps the order
 // serves, and bins of the float's bits put nearly all values of a column into a few of them, where the atomics of a wave
 // wait for each other --; that one histogram places both order statistics in bins of a few hundred values, which are ranked
-// in LDS: three reads of the column in all, with 1024 threads (100 000 x 128: 980 us with eight reads by 256 threads, 47 us
-// now).
+// in LDS: three passes over the column, whose values stay in registers where 1024 threads hold them (up to REGS each: 98
+// for the default sample of 100 000) -- a workgroup per column leaves every second compute unit idle at 128 dimensions, and
+// the other half waited for the same 400 KB three times.  100 000 x 128: 980 us with eight reads by 256 threads, 50 us with
+// three reads by 1024, 37 us now.
 // A column with values beyond any such range (NaN, infinities) takes bins of the ordered bits.
-__global__ void __launch_bounds__(1024)
+template <uint32_t REGS>
+__global__ void __launch_bounds__(kBoundThreads)
 sq_bounds_kernel(const float* sample_t, uint64_t count, uint64_t ignore_count, float* lb, float* diff, float* upper_out,
                  float* lower_out) {
     __shared__ BoundScratch sc;
     const uint32_t d = blockIdx.x;
     const float* col = sample_t + static_cast<uint64_t>(d) * count;
     const uint64_t k = ignore_count < count ? ignore_count : count;
-    // Smallest and largest ordered bits of the values that `in` admits, in sc.lo / sc.hi.
-    auto range_of = [&](auto in) {
+    ColumnValues<REGS> column{col, count, {}};
+    column.load();
+    // Smallest and largest ordered bits of the values of `values` that `in` admits, in sc.lo / sc.hi.
+    auto range_of = [&](auto&& values, auto in) {
         if (threadIdx.x == 0) {
             sc.lo = 0xFFFFFFFFU;
             sc.hi = 0;
         }
         __syncthreads();
         uint32_t lo = 0xFFFFFFFFU, hi = 0;
-        for_column(col, count, [&](float v) {
+        values.each([&](float v) {
             if (in(v)) {
                 const uint32_t key = float_to_ordered(v);
                 lo = key < lo ? key : lo;
@@ -1577,7 +1666,7 @@ sq_bounds_kernel(const float* sample_t, uint64_t count, uint64_t ignore_count, f
     if (threadIdx.x < 2) {
         sc.fill[threadIdx.x] = 0;
     }
-    range_of([](float) { return true; });
+    range_of(column, [](float) { return true; });
     const uint32_t kmin = sc.lo, kmax = sc.hi;
     const float vmin = ordered_to_float(kmin), vmax = ordered_to_float(kmax);
     const float scale = static_cast<float>(kBins) / (vmax - vmin);
@@ -1592,7 +1681,7 @@ sq_bounds_kernel(const float* sample_t, uint64_t count, uint64_t ignore_count, f
         }
         return (float_to_ordered(v) - kmin) >> shift;
     };
-    for_column(col, count, [&](float v) { atomicAdd(&sc.hist[bin_of(v)], 1U); });
+    column.each([&](float v) { atomicAdd(&sc.hist[bin_of(v)], 1U); });
     __syncthreads();
     uint32_t bin[2], population[2];
     uint64_t rank[2] = {k, count - k + 1};
@@ -1604,7 +1693,7 @@ sq_bounds_kernel(const float* sample_t, uint64_t count, uint64_t ignore_count, f
         __syncthreads();
     }
     if (population[0] <= kFewKeys || population[1] <= kFewKeys) {
-        for_column(col, count, [&](float v) {
+        column.each([&](float v) {
             const uint32_t b = bin_of(v);
 #pragma unroll
             for (int s = 0; s < 2; ++s) {
@@ -1622,7 +1711,7 @@ sq_bounds_kernel(const float* sample_t, uint64_t count, uint64_t ignore_count, f
             key = kth_of_few(sc, s, rank[s]);
         } else {
             const uint32_t want = bin[s];
-            range_of([&](float v) { return bin_of(v) == want; });
+            range_of(ColumnValues<0>{col, count, {}}, [&](float v) { return bin_of(v) == want; });
             const uint32_t from = sc.lo, to = sc.hi;
             __syncthreads();
             key = kth_key_in(col, count, from, to, population[s], rank[s], sc);
@@ -1721,7 +1810,9 @@ sq_train_common(const float* x, uint64_t n, uint32_t dim, int bits, int metric, 
     }
     hipLaunchKernelGGL(sq_sample_kernel, dim3(static_cast<uint32_t>(div_up(p.sample_count, 4 * kWave))), dim3(256), 0, st,
                        x, n, dim, p.step, p.sample_count, norms, sample_t);
-    hipLaunchKernelGGL(sq_bounds_kernel, dim3(dim), dim3(1024), 0, st, sample_t, p.sample_count, p.ignore_count, lb, diff,
+    const uint64_t each = div_up(p.sample_count, kBoundThreads);
+    auto bounds = each <= 32 ? sq_bounds_kernel<32> : each <= 64 ? sq_bounds_kernel<64> : each <= 98 ? sq_bounds_kernel<98> : sq_bounds_kernel<0>;
+    hipLaunchKernelGGL(bounds, dim3(dim), dim3(kBoundThreads), 0, st, sample_t, p.sample_count, p.ignore_count, lb, diff,
                        upper, lower);
     if (uniform_out != nullptr) {
         hipLaunchKernelGGL(sq_uniform_reduce_kernel, dim3(1), dim3(64), 0, st, upper, lower, dim, mode, uniform_out);
@@ -1783,16 +1874,25 @@ vsag_amd_sq_encode(const float* x_dev, uint64_t n, uint32_t dim, int bits, int m
                       (reinterpret_cast<uintptr_t>(codes_dev) & 3U) == 0;
     const uint64_t threads = flat ? div_up(total, static_cast<uint64_t>(32 / bits)) : n * code_size;
     VA_CHECK_ARG(div_up(threads, 256) < (1ull << 31), "too many rows for one encode call");
-    const dim3 grid(static_cast<uint32_t>(div_up(threads, 256)));
     if (!flat) {
-        hipLaunchKernelGGL(sq_encode_bytes_kernel, grid, dim3(256), 0, st, x_dev, n, dim, bits, lower_bound_dev, diff_dev,
-                           norms, code_size, codes_dev);
+        hipLaunchKernelGGL(sq_encode_bytes_kernel, dim3(static_cast<uint32_t>(div_up(threads, 256))), dim3(256), 0, st, x_dev,
+                           n, dim, bits, lower_bound_dev, diff_dev, norms, code_size, codes_dev);
     } else {
-        const bool vec = (dim & 3U) == 0 && ((reinterpret_cast<uintptr_t>(lower_bound_dev) |
-                                              reinterpret_cast<uintptr_t>(diff_dev)) & 15U) == 0;
-        auto kernel = bits == 8 ? (vec ? sq_encode_kernel<8, true> : sq_encode_kernel<8, false>)
-                                : (vec ? sq_encode_kernel<4, true> : sq_encode_kernel<4, false>);
-        hipLaunchKernelGGL(kernel, grid, dim3(256), 0, st, x_dev, total, dim, lower_bound_dev, diff_dev, norms, codes_dev);
+        uint32_t block = 0, runs = 0;
+        sq_encode_shape(dim, 32U / bits, &block, &runs);
+        auto launch = [&](auto kernel) {
+            hipLaunchKernelGGL(kernel, dim3(static_cast<uint32_t>(div_up(threads, static_cast<uint64_t>(block) * runs))),
+                               dim3(block), 0, st, x_dev, total, dim, lower_bound_dev, diff_dev, norms, codes_dev);
+        };
+        if (bits == 8 && runs == 4) {
+            launch(norms != nullptr ? sq_encode_kernel<8, true, 4> : sq_encode_kernel<8, false, 4>);
+        } else if (bits == 8) {
+            launch(norms != nullptr ? sq_encode_kernel<8, true, 1> : sq_encode_kernel<8, false, 1>);
+        } else if (runs == 4) {
+            launch(norms != nullptr ? sq_encode_kernel<4, true, 4> : sq_encode_kernel<4, false, 4>);
+        } else {
+            launch(norms != nullptr ? sq_encode_kernel<4, true, 1> : sq_encode_kernel<4, false, 1>);
+        }
     }
     VA_HIP(hipGetLastError());
     if (norms != nullptr) {
