@@ -28,14 +28,15 @@
 // 67.9; 480k x 960, k 256 2.42 / 3.51 / 2.68; of a single slab (65536 x 128, k 512) 0.12 / 0.18 / 0.18.  Where nothing is
 // open, asking costs 0.5 to 1 %.
 //
-// 1M x 960 rows, 4096 centroids (one assignment): 63.3 -> 13.0 ms.  Of that the contraction takes 9.3 (7.9e12 flop: 847
-// TFLOP/s, 34 % of the fp16 peak; a workgroup waits at each of its fifteen stages for all eight waves), the rounding of
-// the rows 1.25 (5.8 GB at 4.6 TB/s) and the rescoring 2.8 (3.8 GB of rows, 0.8 GB of table, one to three centroids a
-// row).
+// 1M x 960 rows, 4096 centroids (one assignment): 63.3 -> 11.4 ms.  Of that the contraction takes 7.4 (7.9e12 flop: 1070
+// TFLOP/s, where matrix instructions on random operands in registers reach 1610 to 1690 and with their reads of LDS 1580,
+// all bound by power), the rounding of the rows 1.25 (5.8 GB at 4.6 TB/s) and the rescoring 2.8 (3.8 GB of rows, 0.8 GB of
+// table, one to three centroids a row).
 #include "kmeans_h16.h"
 
 #include <algorithm>
 #include <mutex>
+#include <type_traits>
 
 namespace vsag_amd {
 
@@ -375,6 +376,25 @@ kmeans_round_rows_kernel(const float* x, uint64_t rows, uint32_t dim, uint32_t d
     }
 }
 
+__device__ inline uint32_t
+lds_offset(const void* p) {
+    return static_cast<uint32_t>(reinterpret_cast<uintptr_t>(
+        (__attribute__((address_space(3))) const void*)p));  // NOLINT: an address-space cast
+}
+
+// Lane l's 16 bytes (touch_line: 4, for the sake of their line) at base + bytes go to LDS at to + 16 l (4 l); `to` is the same
+// in all lanes.  In assembly because the compiler would wait for all such loads before any read of LDS; who reads what they
+// bring waits for vmcnt and a barrier itself.
+__device__ inline void
+load_to_lds(const void* base, uint32_t bytes, uint32_t to) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" : : "s"(to), "v"(bytes), "s"(base) : "memory");
+}
+
+__device__ inline void
+touch_line(const void* base, uint32_t bytes, uint32_t to) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2" : : "s"(to), "v"(bytes), "s"(base) : "memory");
+}
+
 struct KmeansH16Args {
     const uint4* x16;  // [rows][dpad / 8]
     const uint4* c16;  // [k][dpad / 8]
@@ -391,8 +411,12 @@ struct KmeansH16Args {
 };
 
 // 256 centroids (the M side, so that a lane's sixteen results belong to one row) x 256 rows, eight waves of 128 x 64.  A
-// stage of 64 dimensions is 64 KB; two are in LDS, the next one's loads are in flight through registers while a stage is
-// multiplied, and there is one barrier per stage.
+// stage of 64 dimensions is 64 KB; two are in LDS, the next one's loads go straight there while a stage is multiplied, and
+// there is one barrier per stage, with the products of a stage's last step behind it, beside the reads of the next stage's
+// first operands.  The lines of the stage after that are touched, so that they are in the XCD's L2 when they are asked for.
+// Launch of 69 888 x 960 rows, k 4096, us: loads through registers, each stage's first reads exposed 628; as above without
+// the touch 536; with it 510.  (Two workgroups of four waves, 256 x 128 and stages of 32 dimensions three deep to a compute
+// unit, so that one looks through its products beside the other's contraction: 557; it moves half as much again.)
 //
 // LDS: 16-byte slots [row][8], slot s of row r at position s ^ ((r >> 1) & 7): the 16 consecutive rows that a
 // ds_read_b128 serves at a time fall on the sixteen 16-byte columns of the 64 banks, and a global line of a row stays one
@@ -428,46 +452,57 @@ kmeans_h16_kernel(KmeansH16Args p) {
     const uint32_t c0 = ct * kTile;
     const uint32_t stages = p.slots / kSlots;
 
-    // Loader: thread t moves slot t % 8 of rows t / 8 + 64 i of both sides; rows past the end repeat the last one.
-    const uint32_t lr = tid >> 3, ls = tid & 7;
+    // Loader: from memory into LDS without a stop in registers, 16 bytes a lane, eight rows a wave at a time; wave w brings
+    // rows 8 w + 64 i of both sides.  LDS takes the lanes' pieces in order, so the lane chooses the slot that belongs where
+    // it lands; rows past the end repeat the last one.
+    const uint32_t lr = tid >> 3, ls = (tid & 7) ^ ((lr >> 1) & 7);
     const uint4* side_a = p.c16 + static_cast<uint64_t>(c0) * p.slots;
     const uint4* side_b = p.x16 + row0 * p.slots;
     const uint32_t a_last = p.k - 1 - c0;
     const uint32_t b_last = static_cast<uint32_t>(p.rows - 1 - row0 < kTile ? p.rows - 1 - row0 : kTile);
-    auto offset = [&](uint32_t r, uint32_t last) __attribute__((always_inline)) { return (r < last ? r : last) * p.slots + ls; };
+    auto offset = [&](uint32_t r, uint32_t last) __attribute__((always_inline)) {
+        return ((r < last ? r : last) * p.slots + ls) * 16;
+    };
     const uint32_t oa0 = offset(lr, a_last), oa1 = offset(lr + 64, a_last), oa2 = offset(lr + 128, a_last),
                    oa3 = offset(lr + 192, a_last);
     const uint32_t ob0 = offset(lr, b_last), ob1 = offset(lr + 64, b_last), ob2 = offset(lr + 128, b_last),
                    ob3 = offset(lr + 192, b_last);
-    const uint32_t put = lr * kSlots + (ls ^ ((lr >> 1) & 7));  // + 64 i rows
+    const uint32_t lds_wave = __builtin_amdgcn_readfirstlane(lds_offset(lds) + wave * 8 * kSlots * 16);
     const uint32_t open_groups = p.state->open_groups;
     if (tid < kTile) {
         const float sq = c0 + tid < p.k ? p.cnorm[c0 + tid] : 3.0e38F;
         cn[tid] = sq <= __uint_as_float(p.state->far_from) ? sq : 3.0e38F;
     }
 
-    uint4 ga0, ga1, ga2, ga3, gb0, gb1, gb2, gb3;  // (separate variables: an array went to scratch memory)
     auto fetch = [&](uint32_t st) __attribute__((always_inline)) {
         const uint4* a = side_a + st * kSlots;
         const uint4* b = side_b + st * kSlots;
-        ga0 = a[oa0];
-        ga1 = a[oa1];
-        ga2 = a[oa2];
-        ga3 = a[oa3];
-        gb0 = b[ob0];
-        gb1 = b[ob1];
-        gb2 = b[ob2];
-        gb3 = b[ob3];
+        const uint32_t to = lds_wave + (st & 1) * 2 * kSide * 16;
+        constexpr uint32_t kStep = 64 * kSlots * 16;
+        load_to_lds(a, oa0, to);
+        load_to_lds(a, oa1, to + kStep);
+        load_to_lds(a, oa2, to + 2 * kStep);
+        load_to_lds(a, oa3, to + 3 * kStep);
+        load_to_lds(b, ob0, to + 4 * kStep);
+        load_to_lds(b, ob1, to + 5 * kStep);
+        load_to_lds(b, ob2, to + 6 * kStep);
+        load_to_lds(b, ob3, to + 7 * kStep);
     };
-    auto park = [&](uint4* buf) __attribute__((always_inline)) {
-        buf[put] = ga0;
-        buf[put + 64 * kSlots] = ga1;
-        buf[put + 128 * kSlots] = ga2;
-        buf[put + 192 * kSlots] = ga3;
-        buf[kSide + put] = gb0;
-        buf[kSide + put + 64 * kSlots] = gb1;
-        buf[kSide + put + 128 * kSlots] = gb2;
-        buf[kSide + put + 192 * kSlots] = gb3;
+    // One line of the stage after that per thread, into the XCD's L2: a word of it goes to a corner of LDS that nobody reads.
+    const uint32_t side = wave >> 2;  // the first four waves: centroids
+    const uint32_t tr = tid & (kTile - 1);
+    const uint32_t touch_off = (tr < (side == 0 ? a_last : b_last) ? tr : (side == 0 ? a_last : b_last)) * p.slots * 16;
+    const uint32_t touch_to = __builtin_amdgcn_readfirstlane(lds_offset(cn + kTile) + wave * 256);
+    const uint32_t side_u = __builtin_amdgcn_readfirstlane(side);
+    auto touch = [&](uint32_t st) __attribute__((always_inline)) {
+        touch_line((side_u == 0 ? side_a : side_b) + st * kSlots, touch_off, touch_to);
+    };
+    // What this wave asked for but for its last load (the line) has landed, and its reads of LDS are done; then the others'.
+    auto landed = [&](auto touched) __attribute__((always_inline)) {
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_s_waitcnt(touched ? 0x0071 : 0x0070);  // vmcnt 1 or 0, lgkmcnt 0
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
     };
     const uint32_t swap = (l32 >> 1) & 7;
     const uint32_t a_row = (wm * 128 + l32) * kSlots;
@@ -507,37 +542,55 @@ kmeans_h16_kernel(KmeansH16Args p) {
         }
     };
 
-    fetch(0);
     if (given_up(open_groups, p.probed)) {
         return;
     }
-    park(lds);
-    __syncthreads();
-    for (uint32_t st = 0; st + 1 < stages; ++st) {
+    using Yes = std::true_type;
+    using No = std::false_type;
+    fetch(0);
+    touch(stages > 1 ? 1 : 0);
+    landed(Yes{});
+    operands(lds, 0, 0);
+    // (The barriers to the scheduler keep every step's reads a step ahead of its products, where it would read them late to
+    // save registers.)
+    auto stage = [&](uint32_t st, auto fetches, auto touches) __attribute__((always_inline)) {
         const uint4* cur = lds + (st & 1) * 2 * kSide;
-        fetch(st + 1);
-        operands(cur, 0, 0);
+        if constexpr (fetches) {
+            fetch(st + 1);  // the last readers of its buffer passed the barrier that ended stage st - 1
+        }
+        if constexpr (touches) {
+            touch(st + 2);
+        }
         operands(cur, 1, 1);
+        __builtin_amdgcn_sched_barrier(0);
         multiply(0);
+        __builtin_amdgcn_sched_barrier(0);
         operands(cur, 2, 0);
+        __builtin_amdgcn_sched_barrier(0);
         multiply(1);
+        __builtin_amdgcn_sched_barrier(0);
         operands(cur, 3, 1);
+        __builtin_amdgcn_sched_barrier(0);
         multiply(0);
-        park(lds + ((st + 1) & 1) * 2 * kSide);  // its last readers passed the barrier that ended stage st - 1
+        __builtin_amdgcn_sched_barrier(0);
+        // The last step is multiplied behind the barrier, beside the reads of the next stage's first operands.
+        if constexpr (fetches) {
+            landed(touches);
+            operands(lds + ((st + 1) & 1) * 2 * kSide, 0, 0);
+        }
+        __builtin_amdgcn_sched_barrier(0);
         multiply(1);
-        __syncthreads();
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    uint32_t st = 0;
+    for (; st + 2 < stages; ++st) {
+        stage(st, Yes{}, Yes{});
     }
-    {
-        const uint4* cur = lds + ((stages - 1) & 1) * 2 * kSide;
-        operands(cur, 0, 0);
-        operands(cur, 1, 1);
-        multiply(0);
-        operands(cur, 2, 0);
-        multiply(1);
-        operands(cur, 3, 1);
-        multiply(0);
-        multiply(1);
+    if (st + 1 < stages) {
+        stage(st, Yes{}, No{});
+        ++st;
     }
+    stage(st, No{}, No{});
 
     // acc[i][j][e] = <C, X> (scaled) of centroid c0 + wm 128 + 32 i + 8 (e / 4) + 4 half + e % 4 and row wn 64 + 32 j + l32:
     // the 64 of a lane are one group of the table, 16 i + e the place in it.
@@ -560,7 +613,8 @@ kmeans_h16_kernel(KmeansH16Args p) {
                     const float v = __uint_as_float((__float_as_uint(d) & ~63U) | (16U * i + 4U * e4 + e));
                     third = __builtin_amdgcn_fmed3f(second, third, v);
                     second = __builtin_amdgcn_fmed3f(least, second, v);
-                    least = fminf(least, v);
+                    // (fminf would make v canonical first, one instruction in six here)
+                    asm("v_min_f32 %0, %1, %2" : "=v"(least) : "v"(least), "v"(v));
                 }
             }
             __builtin_amdgcn_sched_barrier(0);  // keeps the reads of cn from piling up in registers
@@ -819,7 +873,8 @@ kmeans_h16_rescore_kernel(KmeansRescoreArgs p) {
 int
 launch_kmeans_h16(const float* x, uint64_t n, uint32_t dim, const float* cent, uint32_t k, const float* cnorm_raw,
                   float* xnorm, int iteration, unsigned long long* best, const KmeansH16Buffers& b, hipStream_t st) {
-    constexpr size_t lds_bytes = 4 * static_cast<size_t>(kTile) * kSlots * sizeof(uint4) + kTile * sizeof(float);
+    constexpr size_t lds_bytes = 4 * static_cast<size_t>(kTile) * kSlots * sizeof(uint4) + kTile * sizeof(float) +
+                                 kThreads * sizeof(uint32_t);
     static std::once_flag lds_once;
     static hipError_t lds_rc = hipSuccess;
     std::call_once(lds_once, []() {
