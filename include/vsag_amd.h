@@ -420,7 +420,9 @@ VSAG_AMD_API int vsag_amd_ivf_scan_topk_ex(const vsag_amd_store_t* lists, const 
                               void* workspace_dev, size_t workspace_bytes, void* stream);
 
 /* Number of codes in the lists a batch probes, summed over all (query, probe) pairs: the approximate-phase
- * distance_evaluations of SearchStatistics (src/query_context.h:215-246).  total_dev: 8 bytes of device memory. */
+ * distance_evaluations of SearchStatistics (src/query_context.h:215-246).  total_dev: 8 bytes of device memory, or, with
+ * at most VSAG_AMD_PROBED_CODES_STORED pairs, of any memory that the device can write (pinned host memory). */
+#define VSAG_AMD_PROBED_CODES_STORED 16384u
 VSAG_AMD_API int vsag_amd_ivf_probed_codes(const vsag_amd_store_t* lists, const int32_t* buckets_dev, uint64_t nq,
                               uint32_t nprobe, uint64_t* total_dev, void* stream);
 

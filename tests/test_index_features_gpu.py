@@ -10,8 +10,10 @@ import threading
 import numpy as np
 import pytest
 
+import oracle as orc
+from gpu_helpers import Store, dev
 from test_index_api_gpu import RECALL_THRESHOLD, ground_truth, make, recall, vectors
-from vsag_amd import pyvsag
+from vsag_amd import capi, pyvsag
 
 pytestmark = pytest.mark.gpu
 
@@ -406,3 +408,38 @@ def test_concurrent_searches_equal_serial(lib, name, params, search):
     one_i, one_d = idx.knn_search(q[5], k, search, statistics=False)
     assert np.array_equal(one_i, want_ids[5]) and np.array_equal(one_d, want_d[5])
     idx.close()
+
+
+@pytest.mark.parametrize("name", ["brute_force", "ivf"])
+@pytest.mark.parametrize("quant", ["fp32", "sq8", "sq8_uniform"])
+@pytest.mark.parametrize("dim,k", [(640, 10), (33, 4)])
+def test_small_calls_without_copies(lib, name, quant, dim, k):
+    """Queries up to 128 KB and up to 512 results lie in pinned memory; on both sides of either line a batch gives what
+    its queries give one by one."""
+    n = 3000
+    x, q = vectors(n, dim), vectors(600, dim, seed=9)
+    extra = {"buckets_count": 16} if name == "ivf" else {}
+    index = make(name, dim, "l2", base_quantization_type=quant, **extra)
+    index.build(x, np.arange(n, dtype=np.int64) + 5, n, dim)
+    params = json.dumps({"ivf": {"scan_buckets_count": 5}}) if name == "ivf" else "{}"
+    one = [index.knn_search(q[i], k, params) for i in range(130)]
+    limit = 512 // k
+    for nq in (2, limit, limit + 1, min(130, 131072 // (4 * dim)), min(130, 131072 // (4 * dim) + 1)):
+        ids, dists = index.knn_search_batch(q[:nq], k, params)
+        for i in range(nq):
+            assert np.array_equal(dists[i], one[i][1]) and np.array_equal(ids[i], one[i][0])
+
+
+@pytest.mark.parametrize("nq,nprobe", [(1, 1), (256, 64), (257, 64), (16384, 1), (16385, 1)])
+def test_probed_codes_on_both_sides_of_one_workgroup(lib, nq, nprobe):
+    L = lib.load_library()
+    nlist, d, n = 70, 8, 900
+    rng = np.random.default_rng(nq + nprobe)
+    labels = rng.integers(0, nlist, n).astype(np.int32)
+    store = Store(capi.KIND_FP32, orc.L2, d)
+    store.set_lists(rng.random((n, d), dtype=np.float32).view(np.uint8), labels, nlist)
+    buckets = rng.integers(-1, nlist, (nq, nprobe)).astype(np.int32)
+    total = capi.DeviceBuffer(8)
+    capi.check(L.vsag_amd_ivf_probed_codes(store.handle, dev(buckets).ptr, nq, nprobe, total.ptr, None))
+    sizes = np.append(np.bincount(labels, minlength=nlist), 0)
+    assert int(total.to_numpy(np.uint64, (1,))[0]) == int(sizes[buckets].sum())

@@ -975,7 +975,33 @@ vsag_amd_ivf_scan_topk_ex(const vsag_amd_store_t* s, const float* queries_dev, u
 }
 
 namespace vsag_amd {
-// Codes in the lists the queries probe, summed over all (query, probe) pairs.
+// Codes in the lists the queries probe, summed over all (query, probe) pairs.  Few pairs: one workgroup that stores the sum.
+__global__ void __launch_bounds__(1024)
+probed_codes_few_kernel(const int32_t* buckets, uint32_t npairs, uint32_t nlist, const uint32_t* list_sizes,
+                        unsigned long long* total) {
+    __shared__ unsigned long long part[16];
+    unsigned long long mine = 0;
+#pragma unroll 4
+    for (uint32_t i = threadIdx.x; i < npairs; i += 1024) {
+        const int32_t b = buckets[i];
+        mine += b >= 0 && static_cast<uint32_t>(b) < nlist ? list_sizes[b] : 0;
+    }
+    for (int off = 32; off > 0; off >>= 1) {
+        mine += __shfl_xor(mine, off);
+    }
+    if ((threadIdx.x & 63) == 0) {
+        part[threadIdx.x >> 6] = mine;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        unsigned long long sum = 0;
+        for (uint32_t w = 0; w < 16; ++w) {
+            sum += part[w];
+        }
+        *total = sum;
+    }
+}
+
 __global__ void __launch_bounds__(256)
 probed_codes_kernel(const int32_t* buckets, uint64_t npairs, uint32_t nlist, const uint32_t* list_sizes,
                     unsigned long long* total) {
@@ -1003,6 +1029,13 @@ vsag_amd_ivf_probed_codes(const vsag_amd_store_t* s, const int32_t* buckets_dev,
     VA_CHECK_ARG(s != nullptr && s->nlist > 0, "not a posting-list store");
     VA_CHECK_ARG(buckets_dev && total_dev, "null pointer");
     hipStream_t st = static_cast<hipStream_t>(stream);
+    if (nq <= VSAG_AMD_PROBED_CODES_STORED && nq * nprobe <= VSAG_AMD_PROBED_CODES_STORED) {
+        hipLaunchKernelGGL(probed_codes_few_kernel, dim3(1), dim3(1024), 0, st, buckets_dev,
+                           static_cast<uint32_t>(nq * nprobe), s->nlist, s->list_sizes_dev,
+                           reinterpret_cast<unsigned long long*>(total_dev));
+        VA_HIP(hipGetLastError());
+        return 0;
+    }
     hipLaunchKernelGGL(fill_jobs_kernel, dim3(1), dim3(256), 0, st,
                        FillJob{{reinterpret_cast<uint32_t*>(total_dev), nullptr, nullptr, nullptr, nullptr}, {0, 0, 0, 0, 0},
                                {2, 0, 0, 0, 0}});

@@ -165,8 +165,13 @@ struct DevBuf {
 // without waiting, a download queues the transfer into it and hands the bytes over at finish(), which is the one
 // point where a search waits for the device.  (A copy from or to pageable memory waits on its own, and the caller's
 // arrays cannot be pinned after the fact.)  Transfers too large for the area go the plain, waiting way.
+//
+// Few bytes are not copied at all: the device reads the queries of a small call from pinned memory where they lie, and
+// writes few results there.  A queued copy costs a small search more than its bytes (one query against 1M sq8 codes: 66 us
+// with three copies, 59 without; one query on an ivf index 122 and 103, its statistic no longer waited for).
 struct SearchContext {
     void* stream = nullptr;
+    const float* rows = nullptr;  // the queries, for the device (set_queries)
     DevBuf queries, buckets, bucket_d, cand_ids, cand_d, out_ids, out_d, workspace, deny, scalar;
     SearchContext() {
         dev(vsag_amd_stream_create(&stream));
@@ -180,6 +185,79 @@ struct SearchContext {
             vsag_amd_stream_destroy(stream);
         }
         vsag_amd_host_free(stage_);
+        vsag_amd_host_free(query_stage_);
+    }
+    // The queries of a call, in `rows` until the next one.  `once`: the device reads every row a few times at most (the kinds
+    // that turn a query into a table row in one launch), so that memory of the host serves where they are few.
+    void
+    set_queries(const float* src, size_t n, bool once) {
+        if (!once || n > kDirectQueries) {
+            upload(queries, src, n);
+            rows = queries.as<float>();
+            return;
+        }
+        if (query_stage_ == nullptr) {
+            dev(vsag_amd_host_malloc(&query_stage_, kDirectQueries));
+        }
+        std::memcpy(query_stage_, src, n);
+        in_flight_ = true;
+        rows = static_cast<const float*>(query_stage_);
+    }
+    // Where the device puts ids and distances of `count` results: pinned memory if they are few (valid until finish()), else
+    // the two buffers.
+    struct Results {
+        uint32_t* ids;
+        float* dists;
+        bool direct;
+    };
+    Results
+    results(DevBuf& ids, DevBuf& dists, size_t count) {
+        if (count <= kDirectResults) {
+            const size_t half = (count * 4 + 63) / 64 * 64;
+            auto* p = static_cast<uint8_t*>(staged(2 * half));
+            in_flight_ = true;
+            return {reinterpret_cast<uint32_t*>(p), reinterpret_cast<float*>(p + half), true};
+        }
+        ids.reserve(count * 4);
+        dists.reserve(count * 4);
+        return {ids.as<uint32_t>(), dists.as<float>(), false};
+    }
+    // Where the device puts a number that the next finish() hands over to *dst: pinned memory, or the buffer that the
+    // caller downloads.
+    uint64_t*
+    scalar_result(uint64_t* dst, bool direct) {
+        if (!direct) {
+            scalar.reserve(8);
+            return scalar.as<uint64_t>();
+        }
+        void* p = staged(8);
+        in_flight_ = true;
+        pending_.push_back({dst, p, 8});
+        return static_cast<uint64_t*>(p);
+    }
+    // Hands the results over and waits.
+    void
+    take_results(const Results& r, size_t count, std::vector<uint32_t>& ids, std::vector<float>& dists) {
+        ids.resize(count);
+        dists.resize(count);
+        if (r.direct) {
+            pending_.push_back({ids.data(), r.ids, count * 4});
+            pending_.push_back({dists.data(), r.dists, count * 4});
+        } else {
+            download_later(ids.data(), r.ids, count * 4);
+            download_later(dists.data(), r.dists, count * 4);
+        }
+        finish();
+    }
+    // A search that ended early (an exception) may leave work on the stream that still reads or writes this context's memory.
+    void
+    settle() noexcept {
+        if (in_flight_ || !pending_.empty()) {
+            vsag_amd_stream_synchronize(stream);
+            pending_.clear();
+            stage_used_ = 0;
+            in_flight_ = false;
+        }
     }
     void
     upload(DevBuf& buf, const void* src, size_t n) {
@@ -190,6 +268,7 @@ struct SearchContext {
             return;
         }
         std::memcpy(s, src, n);
+        in_flight_ = true;
         dev(vsag_amd_memcpy_h2d_async(buf.p, s, n, stream));
     }
     // The bytes are in `dst` after the next finish().
@@ -217,6 +296,7 @@ struct SearchContext {
         }
         pending_.clear();
         stage_used_ = 0;
+        in_flight_ = false;
     }
 
 private:
@@ -226,6 +306,8 @@ private:
         size_t bytes;
     };
     static constexpr size_t kStageLimit = 8u << 20;  // larger transfers are not staged
+    static constexpr size_t kDirectQueries = 128u << 10;  // bytes
+    static constexpr size_t kDirectResults = 512;  // (some batches read the distances of an early pass back: not many of them)
     // Room for n bytes in the pinned area (null: too large).  A full area is emptied by finish() first.
     void*
     staged(size_t n) {
@@ -251,7 +333,9 @@ private:
         return s;
     }
     uint8_t* stage_ = nullptr;
+    void* query_stage_ = nullptr;  // kDirectQueries bytes of pinned memory
     size_t stage_cap_ = 0, stage_used_ = 0;
+    bool in_flight_ = false;  // something was queued since the last finish()
     std::vector<Pending> pending_;
 };
 
@@ -264,6 +348,7 @@ public:
         Lease(Lease&&) = default;
         ~Lease() {
             if (ctx_ != nullptr) {
+                ctx_->settle();
                 std::lock_guard<std::mutex> lock(pool_->mutex_);
                 pool_->free_.push_back(std::move(ctx_));
             }
@@ -551,6 +636,12 @@ struct Quantizer {
     int
     rabitq_bits() const {
         return VSAG_AMD_RABITQ_BITS(rabitq_query_bits, rabitq_base_bits);
+    }
+    // Whether the device turns queries into rows of its table in a launch or two, instead of reading them over and over.
+    bool
+    queries_read_once() const {
+        return kind == VSAG_AMD_KIND_FP32 || kind == VSAG_AMD_KIND_SQ8 || kind == VSAG_AMD_KIND_SQ4 ||
+               kind == VSAG_AMD_KIND_SQ8_UNIFORM || kind == VSAG_AMD_KIND_SQ4_UNIFORM;
     }
     uint64_t
     code_size() const {
@@ -2042,7 +2133,7 @@ protected:
             return search_rows_one_by_one(query, k, parameters, spec);
         }
         auto ctx = pool_.acquire();
-        ctx->upload(ctx->queries, query->GetFloat32Vectors(), static_cast<size_t>(nq) * q_.dim * 4);
+        ctx->set_queries(query->GetFloat32Vectors(), static_cast<size_t>(nq) * q_.dim * 4, q_.queries_read_once());
         DenyMask mask;
         mask.init(*ctx, labels_, spec.valid, looped, 1);
         const vsag_amd_search_options_t opt = mask.options(*ctx, spec, 0.0F);
@@ -2186,16 +2277,13 @@ private:
     void
     scan(SearchContext& ctx, int64_t nq, uint32_t kk, const vsag_amd_search_options_t& opt, std::vector<uint32_t>& ids,
          std::vector<float>& dists) const {
-        ctx.out_ids.reserve(static_cast<size_t>(nq) * kk * 4);
-        ctx.out_d.reserve(static_cast<size_t>(nq) * kk * 4);
+        const size_t count = static_cast<size_t>(nq) * kk;
+        const SearchContext::Results out = ctx.results(ctx.out_ids, ctx.out_d, count);
         size_t wsb = vsag_amd_flat_scan_workspace_bytes(store_.s, nq, kk);
         ctx.workspace.reserve(wsb);
-        dev(vsag_amd_flat_scan_topk_ex(store_.s, ctx.queries.as<float>(), nq, kk, &opt, ctx.out_ids.as<uint32_t>(),
-                                       ctx.out_d.as<float>(), ctx.workspace.p, wsb, ctx.stream));
-        ids.resize(static_cast<size_t>(nq) * kk);
-        dists.resize(ids.size());
-        ctx.download_later(ids.data(), ctx.out_ids.p, ids.size() * 4);
-        ctx.download(dists.data(), ctx.out_d.p, dists.size() * 4);
+        dev(vsag_amd_flat_scan_topk_ex(store_.s, ctx.rows, nq, kk, &opt, out.ids, out.dists, ctx.workspace.p, wsb,
+                                       ctx.stream));
+        ctx.take_results(out, count, ids, dists);
     }
 
     std::vector<int64_t>
@@ -2429,7 +2517,9 @@ protected:
 
         auto lease = pool_.acquire();
         SearchContext& ctx = *lease;
-        ctx.upload(ctx.queries, query->GetFloat32Vectors(), static_cast<size_t>(nq) * q_.dim * 4);
+        // (the reorder step and the residuals' terms read a query once per candidate or list)
+        ctx.set_queries(query->GetFloat32Vectors(), static_cast<size_t>(nq) * q_.dim * 4,
+                        q_.queries_read_once() && !reorder && !use_residual_);
         SearchStats stats;
         stats.base_kind = q_.kind;
         stats.precise_kind = pq_.kind;
@@ -2454,7 +2544,7 @@ protected:
             ctx.bucket_d.reserve(static_cast<size_t>(nq) * nprobe * 4);
             const size_t wsb = vsag_amd_ivf_route_workspace_bytes(centroid_store_.s, nq, nprobe);
             ctx.workspace.reserve(wsb);
-            dev(vsag_amd_ivf_route(centroid_store_.s, ctx.queries.as<float>(), nq, nprobe, ctx.buckets.as<int32_t>(),
+            dev(vsag_amd_ivf_route(centroid_store_.s, ctx.rows, nq, nprobe, ctx.buckets.as<int32_t>(),
                                    ctx.bucket_d.as<float>(), ctx.workspace.p, wsb, ctx.stream));
             stats.routing = static_cast<uint64_t>(nq) * nlist_;
         }
@@ -2470,7 +2560,8 @@ protected:
             }
             return pack_results(ids, dists, nq, nprobe, identity, stats.dump());
         }
-        const uint64_t probed = probed_codes(ctx, nq, nprobe);
+        uint64_t probed = 0;  // (in it once the first results are)
+        probed_codes(ctx, nq, nprobe, &probed);
         DenyMask mask;
         mask.init(ctx, labels_, spec.valid, looped, bpd_);
         // FlatBucketSearcher compares against radius + THRESHOLD_ERROR (flat_bucket_searcher.cpp:121,
@@ -2481,22 +2572,26 @@ protected:
             // 2. scan the probed lists; 3. exact rerank, best min(k, candidates) kept (flatten_reorder.cpp:77)
             const auto kc = static_cast<uint32_t>(kcand * bpd_);
             const int64_t kout = reorder ? std::min<int64_t>(k, kcand) : kcand;
-            scan_lists(ctx, nq, nprobe, kc, opt);
-            stats.approximate = probed;
             std::vector<uint32_t> ids;
             std::vector<float> dists;
             if (bpd_ == 1 && reorder && pq_.kind == VSAG_AMD_KIND_FP32) {
                 // the whole batch stays on the device
-                ctx.out_ids.reserve(static_cast<size_t>(nq) * kout * 4);
-                ctx.out_d.reserve(static_cast<size_t>(nq) * kout * 4);
-                dev(vsag_amd_rerank_fp32(raw_.as<float>(), labels_.size(), q_.dim, q_.metric, ctx.queries.as<float>(), nq,
-                                         ctx.cand_ids.as<uint32_t>(), kc, static_cast<uint32_t>(kout),
-                                         ctx.out_ids.as<uint32_t>(), ctx.out_d.as<float>(), ctx.stream));
-                fetch(ctx, ctx.out_ids, ctx.out_d, static_cast<size_t>(nq) * kout, ids, dists);
+                scan_lists(ctx, nq, nprobe, kc, opt, cand_buffers(ctx, nq, kc));
+                const size_t count = static_cast<size_t>(nq) * kout;
+                const SearchContext::Results out = ctx.results(ctx.out_ids, ctx.out_d, count);
+                dev(vsag_amd_rerank_fp32(raw_.as<float>(), labels_.size(), q_.dim, q_.metric, ctx.rows, nq,
+                                         ctx.cand_ids.as<uint32_t>(), kc, static_cast<uint32_t>(kout), out.ids,
+                                         out.dists, ctx.stream));
+                ctx.take_results(out, count, ids, dists);
+                stats.approximate = probed;
                 stats.rerank = static_cast<uint64_t>(nq) * kc;  // at most: lists may hold fewer candidates
                 return pack_results(ids, dists, nq, kout, labels_, stats.dump());
             }
-            fetch(ctx, ctx.cand_ids, ctx.cand_d, static_cast<size_t>(nq) * kc, ids, dists);
+            const size_t count = static_cast<size_t>(nq) * kc;
+            const SearchContext::Results out = ctx.results(ctx.cand_ids, ctx.cand_d, count);
+            scan_lists(ctx, nq, nprobe, kc, opt, out);
+            ctx.take_results(out, count, ids, dists);
+            stats.approximate = probed;
             if (bpd_ > 1) {
                 merge_postings(ids, dists, nq, kc, static_cast<uint32_t>(kcand));
             }
@@ -2526,11 +2621,11 @@ protected:
         while (remaining > 0) {
             const auto kc = static_cast<uint32_t>(
                 std::min<int64_t>({remaining * bpd_, kMaxDeviceK, n * static_cast<int64_t>(bpd_)}));
-            scan_lists(ctx, 1, nprobe, kc, opt);
-            stats.approximate += probed;
+            scan_lists(ctx, 1, nprobe, kc, opt, cand_buffers(ctx, 1, kc));
             std::vector<uint32_t> ids;
             std::vector<float> dists;
             fetch(ctx, ctx.cand_ids, ctx.cand_d, kc, ids, dists);
+            stats.approximate += probed;
             uint32_t got = 0;
             while (got < kc && ids[got] != VSAG_AMD_INVALID_ID) {
                 // ascending: the first posting of a vector carries its smallest distance (ivf.cpp:1799-1812)
@@ -3048,28 +3143,31 @@ private:
         ctx.download(dists.data(), d_dev.p, count * 4);
     }
 
-    // Codes in the lists of ctx.buckets, over all (query, list) pairs.
-    uint64_t
-    probed_codes(SearchContext& ctx, int64_t nq, uint32_t nprobe) const {
-        ctx.scalar.reserve(8);
-        dev(vsag_amd_ivf_probed_codes(lists_.s, ctx.buckets.as<int32_t>(), nq, nprobe, ctx.scalar.as<uint64_t>(),
-                                      ctx.stream));
-        uint64_t total = 0;
-        ctx.download(&total, ctx.scalar.p, 8);
-        return total;
+    // Codes in the lists of ctx.buckets, over all (query, list) pairs: in *total after the next finish().
+    void
+    probed_codes(SearchContext& ctx, int64_t nq, uint32_t nprobe, uint64_t* total) const {
+        uint64_t* to = ctx.scalar_result(total, static_cast<uint64_t>(nq) * nprobe <= VSAG_AMD_PROBED_CODES_STORED);
+        dev(vsag_amd_ivf_probed_codes(lists_.s, ctx.buckets.as<int32_t>(), nq, nprobe, to, ctx.stream));
+        if (to == ctx.scalar.as<uint64_t>()) {
+            ctx.download_later(total, to, 8);
+        }
     }
 
-    // Scan of the lists in ctx.buckets for the uploaded queries: kc (distance, posting id) per query, ascending, in
-    // ctx.cand_ids / ctx.cand_d.
-    void
-    scan_lists(SearchContext& ctx, int64_t nq, uint32_t nprobe, uint32_t kc, const vsag_amd_search_options_t& opt) const {
+    static SearchContext::Results
+    cand_buffers(SearchContext& ctx, int64_t nq, uint32_t kc) {
         ctx.cand_ids.reserve(static_cast<size_t>(nq) * kc * 4);
         ctx.cand_d.reserve(static_cast<size_t>(nq) * kc * 4);
+        return {ctx.cand_ids.as<uint32_t>(), ctx.cand_d.as<float>(), false};
+    }
+
+    // Scan of the lists in ctx.buckets for the call's queries: kc (distance, posting id) per query, ascending, to `out`.
+    void
+    scan_lists(SearchContext& ctx, int64_t nq, uint32_t nprobe, uint32_t kc, const vsag_amd_search_options_t& opt,
+               const SearchContext::Results& out) const {
         const size_t wsb = vsag_amd_ivf_scan_workspace_bytes(lists_.s, nq, nprobe, kc);
         ctx.workspace.reserve(wsb);
-        dev(vsag_amd_ivf_scan_topk_ex(lists_.s, ctx.queries.as<float>(), nq, ctx.buckets.as<int32_t>(), nprobe, kc, &opt,
-                                      ctx.cand_ids.as<uint32_t>(), ctx.cand_d.as<float>(), ctx.workspace.p, wsb,
-                                      ctx.stream));
+        dev(vsag_amd_ivf_scan_topk_ex(lists_.s, ctx.rows, nq, ctx.buckets.as<int32_t>(), nprobe, kc, &opt, out.ids,
+                                      out.dists, ctx.workspace.p, wsb, ctx.stream));
     }
 
     // Posting ids to vectors (ivf.cpp:1799-1826): per query the smallest distance of every vector, ascending, the best
@@ -3112,7 +3210,7 @@ private:
         if (pq_.kind == VSAG_AMD_KIND_FP32) {
             ctx.out_ids.reserve(static_cast<size_t>(nq) * keep * 4);
             ctx.out_d.reserve(static_cast<size_t>(nq) * keep * 4);
-            dev(vsag_amd_rerank_fp32(raw_.as<float>(), labels_.size(), q_.dim, q_.metric, ctx.queries.as<float>(), nq,
+            dev(vsag_amd_rerank_fp32(raw_.as<float>(), labels_.size(), q_.dim, q_.metric, ctx.rows, nq,
                                      ctx.cand_ids.as<uint32_t>(), kcand, keep, ctx.out_ids.as<uint32_t>(),
                                      ctx.out_d.as<float>(), ctx.stream));
             fetch(ctx, ctx.out_ids, ctx.out_d, static_cast<size_t>(nq) * keep, ids, dists);
@@ -3121,7 +3219,7 @@ private:
         ctx.out_d.reserve(static_cast<size_t>(nq) * kcand * 4);
         const size_t wsb = vsag_amd_store_distances_workspace_bytes(precise_.s, nq);
         ctx.workspace.reserve(wsb);
-        dev(vsag_amd_store_distances(precise_.s, ctx.queries.as<float>(), nq, ctx.cand_ids.as<uint32_t>(), kcand,
+        dev(vsag_amd_store_distances(precise_.s, ctx.rows, nq, ctx.cand_ids.as<uint32_t>(), kcand,
                                      ctx.out_d.as<float>(), ctx.workspace.p, wsb, ctx.stream));
         std::vector<float> exact(static_cast<size_t>(nq) * kcand);
         ctx.download(exact.data(), ctx.out_d.p, exact.size() * 4);
