@@ -816,3 +816,24 @@ def test_settings_of_one_store_leave_the_others_alone(lib):
     assert L.vsag_amd_store_set_scan_tuning(a.handle, 3, 0) == capi.INVALID_ARGUMENT
     a.destroy()
     b.destroy()
+
+
+@pytest.mark.parametrize("kind,metric,d", [("fp32", orc.L2, 127), ("fp32", orc.COSINE, 129), ("fp32", orc.IP, 261),
+                                           ("sq8", orc.L2, 513), ("sq8", orc.IP, 1030), ("sq4", orc.L2, 1030),
+                                           ("sq8_uniform", orc.L2, 513), ("sq4_uniform", orc.IP, 1030)])
+@pytest.mark.parametrize("k", [1, 31, 33, 128])
+def test_rescoring_at_the_edges_of_its_pieces(lib, modes, kind, metric, d, k):
+    """Candidates on both sides of 32 and 64, rows a granule short of and beyond the 32 or 64 that are in LDS at a time; rows
+    that are copies of each other, so that more candidates than k are equal to the last bit."""
+    rng = np.random.default_rng(d + k)
+    n, nq = 2100, 17
+    x, means = gaussian_mixture(rng, n, d, 12, 0.05)
+    x[100:260] = x[99]
+    q, _ = gaussian_mixture(rng, nq, d, 12, 0.05, means=means)
+    q[0] = x[99]
+    st = _store_of(kind, metric, x, rng)
+    plain, fast, tile = modes(st, q, k, 1)
+    if kind != "sq8" and kind != "sq4":
+        assert tile in (64, 128), "the bf16 pass did not run"
+    assert same(plain, fast)
+    st.destroy()

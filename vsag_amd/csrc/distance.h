@@ -75,6 +75,11 @@ acc_reset(Acc<KIND, T>& a) {
 template <int T>
 struct QueryRows {
     cu32_p row[T];
+
+    __device__ inline cfloat_p
+    scale(const ScanArgs& a) const {
+        return as_const(a.scale);
+    }
 };
 
 template <int T>
@@ -88,10 +93,11 @@ query_rows(const ScanArgs& a, const uint32_t (&qidx)[T]) {
     return r;
 }
 
-// One granule (16 bytes of this lane's code, granule index j) against the T queries.
-template <int KIND, int METRIC, int T>
+// One granule (16 bytes of this lane's code, granule index j) against the T queries: Q is QueryRows<T>, or what stands in for
+// it with the same words elsewhere (rescore_valued_kernel).
+template <int KIND, int METRIC, int T, typename Q>
 __device__ __forceinline__ void
-accumulate_granule(const ScanArgs& a, const QueryRows<T>& q, uint32_t j, uint4 c, Acc<KIND, T>& acc) {
+accumulate_granule(const ScanArgs& a, const Q& q, uint32_t j, uint4 c, Acc<KIND, T>& acc) {
     const uint32_t w[4] = {c.x, c.y, c.z, c.w};
     if constexpr (KIND == VSAG_AMD_KIND_FP32) {
 #pragma unroll
@@ -110,7 +116,7 @@ accumulate_granule(const ScanArgs& a, const QueryRows<T>& q, uint32_t j, uint4 c
         }
     } else if constexpr (KIND == VSAG_AMD_KIND_SQ8) {
         // qtab row: L2 -> q[d] - lb[d];  IP -> q[d] * scale[d], qmeta[0] = sum q[d] * lb[d].
-        cfloat_p sc = as_const(a.scale);
+        const auto sc = q.scale(a);
 #pragma unroll
         for (int e = 0; e < 16; ++e) {
             float cf = static_cast<float>((w[e >> 2] >> (8 * (e & 3))) & 0xffU);
@@ -130,7 +136,7 @@ accumulate_granule(const ScanArgs& a, const QueryRows<T>& q, uint32_t j, uint4 c
         }
     } else if constexpr (KIND == VSAG_AMD_KIND_SQ4) {
         // Byte b of a code holds dim 2b in its low nibble and dim 2b+1 in its high nibble.
-        cfloat_p sc = as_const(a.scale);
+        const auto sc = q.scale(a);
 #pragma unroll
         for (int m = 0; m < 4; ++m) {
             uint32_t lo = w[m] & 0x0F0F0F0FU;

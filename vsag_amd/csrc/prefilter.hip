@@ -438,8 +438,8 @@ struct RescoreArgs {
     uint32_t sub_lists, sub_cap, gather;
     const uint4* rows;  // the codes a row per code (store.h), or null: read the tiles
     uint32_t row_granules;  // granules of a row: G, or G + 1 with the code's metadata words behind the code
-    // VALUED: records of the approximate distance's ordered bits above the slot, cap a query (their counts 32 words apart),
-    // and per query twice what the approximation can be off by.
+    // rescore_valued_kernel: records of the approximate distance's ordered bits above the slot, cap a query (their counts 32
+    // words apart), and per query twice what the approximation can be off by.
     const uint64_t* valued;
     const float* slack;
 };
@@ -448,14 +448,114 @@ struct RescoreArgs {
 // kernel lives on memory latency), but never less than one private list.
 constexpr uint32_t kRescoreGather = 1024;
 
+// The streaming kernel will scan every tile behind the prefix for this query: the `nlev` lists of it so far must not
+// contribute the same codes a second time.
+__device__ inline void
+rescore_leaves_query(const RescoreArgs& r, uint32_t q, uint32_t nlev, uint32_t lane) {
+    for (uint32_t i = lane; i < nlev; i += kWave) {
+        r.partial_cnt[static_cast<uint64_t>(q) * r.nslots + r.first_slot + i] = 0;
+    }
+    if (lane == 0) {
+        r.gate[q] = 1;
+    }
+}
+
+constexpr uint32_t kRankedKeys = 256;
+
+// The k best keys of a query, by one wave: a selector in LDS and the query's bound in memory.
+struct RescoreKeys {
+    uint64_t* keys;
+    uint32_t S, k, pend, cnt, lane;
+    uint32_t* bound;
+    uint64_t tau;
+    bool flushed;  // keys in front of the pending ones
+
+    __device__ inline void
+    init(uint64_t* lds, const RescoreArgs& r, uint32_t q, uint32_t l) {
+        keys = lds;
+        S = r.S;
+        k = r.k;
+        pend = selector_base(S, k);  // where the selector's pending keys start
+        cnt = 0;
+        flushed = false;
+        lane = l;
+        bound = r.bound + q;
+        selector_init(keys, S, lane);
+        const uint32_t bs = __builtin_amdgcn_readfirstlane(__atomic_load_n(bound, __ATOMIC_RELAXED));
+        // Candidates arrive in no particular order, so ties are decided on whole (distance, id) keys.
+        tau = (static_cast<uint64_t>(bs) << 32) | 0xFFFFFFFFULL;
+    }
+    __device__ inline void
+    add(uint64_t key, bool real) {
+        const bool pass = real && key <= tau;
+        const uint64_t mask = __ballot(pass);
+        if (mask == 0) {
+            return;
+        }
+        const uint32_t np = __popcll(mask);
+        if (pend + cnt + np > S) {
+            const uint64_t th = selector_flush(keys, S, k, cnt, lane);
+            cnt = 0;
+            flushed = true;
+            const uint32_t b = lower_shared(bound, static_cast<uint32_t>(th >> 32), lane);
+            const uint64_t shared_tau = (static_cast<uint64_t>(b) << 32) | 0xFFFFFFFFULL;
+            tau = th < shared_tau ? th : shared_tau;
+        }
+        if (pass) {
+            keys[pend + cnt + mask_rank(mask)] = key;
+        }
+        cnt += np;
+    }
+    __device__ inline void
+    store(const RescoreArgs& r, uint64_t list) {
+        wave_lds_fence();
+        uint32_t bs = __builtin_amdgcn_readfirstlane(__atomic_load_n(bound, __ATOMIC_RELAXED));
+        uint32_t kept = pend + cnt;
+        uint32_t admitted = selector_count_admitted(keys, kept, bs, lane);
+        if (admitted > k && !flushed && cnt <= kRankedKeys) {
+            const uint64_t* all = keys + pend;
+            // Keys that came once: each goes where the number of smaller ones says (28 steps of a sorting network over 128
+            // keys took 5.5 us, the counting takes one).
+            for (uint32_t i = lane; i < cnt; i += kWave) {
+                const uint64_t mine = all[i];
+                uint32_t rank = 0;
+                const uint4* pairs = reinterpret_cast<const uint4*>(all);
+#pragma unroll 8
+                for (uint32_t j = 0; j < cnt / 2; ++j) {
+                    const uint4 v = pairs[j];
+                    const uint64_t x = (static_cast<uint64_t>(v.y) << 32) | v.x, y = (static_cast<uint64_t>(v.w) << 32) | v.z;
+                    rank += (x < mine ? 1U : 0U) + (y < mine ? 1U : 0U);
+                }
+                rank += (cnt & 1U) != 0 && all[cnt - 1] < mine ? 1U : 0U;
+                if (rank < k && mine != kInfKey) {
+                    r.partial[list * k + rank] = mine;
+                    if (rank + 1 == k) {
+                        atomicMin(bound, static_cast<uint32_t>(mine >> 32));
+                    }
+                }
+            }
+            if (lane == 0) {
+                r.partial_cnt[list] = k;
+            }
+            return;
+        }
+        if (admitted > k) {
+            const uint64_t th = selector_flush(keys, S, k, cnt, lane);
+            bs = lower_shared(bound, static_cast<uint32_t>(th >> 32), lane);
+            kept = k;
+            admitted = selector_count_admitted(keys, kept, bs, lane);
+        }
+        if (lane == 0) {
+            r.partial_cnt[list] = admitted;
+        }
+        if (admitted != 0) {
+            selector_copy_admitted(keys, kept, bs, r.partial + list * k, lane);
+        }
+    }
+};
+
 // One wave per query: exact distances of its candidates by the streaming kernel's arithmetic, best k kept.
-//
-// VALUED: a candidate comes with its approximate distance v.  At least k of them have v at or below a_k, and v is off by
-// at most slack / 2 from the streaming distance less the query's constant, so whoever has v above a_k + slack stands
-// behind k others: of the hundreds of candidates that the bound of the level before let through, the few that are left
-// are rescored.  (fp32 rows are gathered a memory line per granule: 300 queries x 160 candidates x 768 dimensions took
-// 312 us.)
-template <int KIND, int METRIC, bool VALUED>
+template <int KIND, int METRIC>
 __global__ void __launch_bounds__(64)
 rescore_kernel(ScanArgs a, RescoreArgs r) {
     extern __shared__ uint64_t keys[];
@@ -463,7 +563,7 @@ rescore_kernel(ScanArgs a, RescoreArgs r) {
     const uint32_t q = blockIdx.x;
     const uint64_t list = static_cast<uint64_t>(q) * r.nslots + r.out_slot;
     bool overflow = false;
-    const uint32_t* counts = r.cand_cnt + static_cast<uint64_t>(q) * (VALUED ? 32 : r.sub_lists != 0 ? r.sub_lists : 1);
+    const uint32_t* counts = r.cand_cnt + static_cast<uint64_t>(q) * (r.sub_lists != 0 ? r.sub_lists : 1);
     if (r.sub_lists == 0) {
         overflow = as_const(counts)[0] > r.cap;
     } else {
@@ -473,25 +573,11 @@ rescore_kernel(ScanArgs a, RescoreArgs r) {
         }
     }
     if (overflow || as_const(r.gate)[q] != 0) {
-        // The streaming kernel will scan every tile behind the prefix for this query: the lists of the levels so
-        // far must not contribute the same codes a second time.
-        // (VALUED: all of the query's lists, which nothing has cleared so far.)
-        const uint32_t nlev = VALUED ? r.nslots : r.out_slot - r.first_slot + 1;
-        for (uint32_t i = lane; i < nlev; i += kWave) {
-            r.partial_cnt[static_cast<uint64_t>(q) * r.nslots + r.first_slot + i] = 0;
-        }
-        if (lane == 0) {
-            r.gate[q] = 1;
-        }
+        rescore_leaves_query(r, q, r.out_slot - r.first_slot + 1, lane);
         return;
     }
-    const uint32_t S = r.S, k = r.k;
-    const uint32_t pend = selector_base(S, k);  // where the selector's pending keys start
-    selector_init(keys, S, lane);
-    uint32_t cnt = 0;
-    uint32_t bs = __builtin_amdgcn_readfirstlane(__atomic_load_n(&r.bound[q], __ATOMIC_RELAXED));
-    // Candidates arrive in no particular order, so ties are decided on whole (distance, id) keys.
-    uint64_t tau = (static_cast<uint64_t>(bs) << 32) | 0xFFFFFFFFULL;
+    RescoreKeys best;
+    best.init(keys, r, q, lane);
     const uint32_t qidx[1] = {q};
     const QueryRows<1> qrows = query_rows<1>(a, qidx);
     auto rescore = [&](const uint32_t* mine, uint32_t total) __attribute__((always_inline)) {
@@ -506,9 +592,7 @@ rescore_kernel(ScanArgs a, RescoreArgs r) {
             // A few granules are fetched before the first is used: a candidate's loads wait for memory together.
             // (sq8 l2 holds scale and query of every dimension in flight in scalar registers: two granules' worth; an sq4
             // granule is 32 dimensions.)
-            // VALUED: a wave or two of candidates per query, so latency is all there is: as many as registers allow.
-            constexpr uint32_t kAhead = VALUED && KIND == VSAG_AMD_KIND_FP32 ? 16
-                                       : KIND == VSAG_AMD_KIND_SQ4 ? (METRIC == VSAG_AMD_METRIC_L2 ? 1 : 2)
+            constexpr uint32_t kAhead = KIND == VSAG_AMD_KIND_SQ4 ? (METRIC == VSAG_AMD_METRIC_L2 ? 1 : 2)
                                        : (KIND == VSAG_AMD_KIND_SQ8 && METRIC == VSAG_AMD_METRIC_L2 ? 2 : 4);
             accumulate_code<KIND, METRIC, kAhead>(a, qrows, row != nullptr ? row : a.tiles + tile * a.G * kWave + ln,
                                                   row != nullptr ? 1 : kWave, acc);
@@ -523,67 +607,10 @@ rescore_kernel(ScanArgs a, RescoreArgs r) {
             } else {
                 finish_distances<KIND, METRIC, 1>(a, qidx, slot, acc, d);
             }
-            const uint64_t key = make_key(d[0], slot);
-            bool pass = have && slot < r.n && key <= tau;
-            uint64_t mask = __ballot(pass);
-            if (mask != 0) {
-                uint32_t np = __popcll(mask);
-                if (pend + cnt + np > S) {
-                    uint64_t th = selector_flush(keys, S, k, cnt, lane);
-                    cnt = 0;
-                    uint32_t b = lower_shared(&r.bound[q], static_cast<uint32_t>(th >> 32), lane);
-                    uint64_t shared_tau = (static_cast<uint64_t>(b) << 32) | 0xFFFFFFFFULL;
-                    tau = th < shared_tau ? th : shared_tau;
-                }
-                if (pass) {
-                    keys[pend + cnt + mask_rank(mask)] = key;
-                }
-                cnt += np;
-            }
+            best.add(make_key(d[0], slot), have && slot < r.n);
         }
     };
-    if constexpr (VALUED) {
-        uint32_t* pick = reinterpret_cast<uint32_t*>(keys + S);  // 128 slots waiting, then 256 bins
-        const uint64_t* valued = r.valued + static_cast<uint64_t>(q) * r.cap;
-        const uint32_t total = as_const(counts)[0];
-        float limit = __builtin_inff();
-        if (total > k) {
-            const float kth = kth_value_or_above(
-                [&](uint32_t i) { return ordered_to_float(static_cast<uint32_t>(valued[i] >> 32)); }, total, k, pick + 128, lane);
-            const float slack = r.slack[q];
-            if (slack < 3.0e38F && kth > -3.0e38F) {
-                limit = kth + slack;
-                limit += fabsf(limit) * 2.4e-7F;  // not below the sum
-            }
-        }
-        uint32_t waiting = 0;
-        for (uint32_t base = 0; base < total; base += kWave) {
-            const uint64_t key = base + lane < total ? valued[base + lane] : kInfKey;
-            const bool take = base + lane < total && !(ordered_to_float(static_cast<uint32_t>(key >> 32)) > limit);
-            const uint64_t mask = __ballot(take);
-            if (take) {
-                pick[waiting + mask_rank(mask)] = static_cast<uint32_t>(key);
-            }
-            waiting += static_cast<uint32_t>(__popcll(mask));
-            wave_lds_fence();
-            if (waiting >= kWave || base + kWave >= total) {
-                // (a round of at most 64, what is left over moves to the front)
-                const uint32_t now = waiting < kWave ? waiting : kWave;
-                rescore(pick, now);
-                const uint32_t left = waiting - now;
-                const uint32_t moved = lane < left ? pick[kWave + lane] : 0U;
-                wave_lds_fence();
-                if (lane < left) {
-                    pick[lane] = moved;
-                }
-                waiting = left;
-                wave_lds_fence();
-            }
-        }
-        if (waiting != 0) {
-            rescore(pick, waiting);
-        }
-    } else if (r.sub_lists == 0) {
+    if (r.sub_lists == 0) {
         rescore(r.cand + static_cast<uint64_t>(q) * r.cap, as_const(counts)[0]);
     } else {
         // Gather the private lists of the query behind the selector -- a lane per list, offsets by a wave scan -- and
@@ -594,7 +621,7 @@ rescore_kernel(ScanArgs a, RescoreArgs r) {
         uint32_t piece = r.gather / r.sub_cap;
         piece = piece > kWave ? kWave : (piece == 0 ? 1 : piece);
         uint32_t fill = 0;
-        auto gather = [&](uint32_t g, uint32_t c) {
+        auto gather = [&](uint32_t g, uint32_t c) __attribute__((always_inline)) {
             // c = this lane's share (0: none); returns after the lanes' entries are in flat[fill ...].
             uint32_t incl = c;
             for (int off = 1; off < 64; off <<= 1) {
@@ -631,7 +658,7 @@ rescore_kernel(ScanArgs a, RescoreArgs r) {
         };
         // The counts of four rounds are asked for together: a query with thousands of (mostly empty) private lists
         // would otherwise wait for memory once per 64 of them.
-        auto round = [&](uint32_t g, uint32_t c) {
+        auto round = [&](uint32_t g, uint32_t c) __attribute__((always_inline)) {
             uint32_t total = c;
             for (int off = 32; off > 0; off >>= 1) {
                 total += __shfl_xor(total, off);
@@ -662,21 +689,295 @@ rescore_kernel(ScanArgs a, RescoreArgs r) {
         wave_lds_fence();
         rescore(flat, fill);
     }
-    wave_lds_fence();
-    bs = __builtin_amdgcn_readfirstlane(__atomic_load_n(&r.bound[q], __ATOMIC_RELAXED));
-    uint32_t kept = pend + cnt;
-    uint32_t admitted = selector_count_admitted(keys, kept, bs, lane);
-    if (admitted > k) {
-        uint64_t th = selector_flush(keys, S, k, cnt, lane);
-        bs = lower_shared(&r.bound[q], static_cast<uint32_t>(th >> 32), lane);
-        kept = k;
-        admitted = selector_count_admitted(keys, kept, bs, lane);
+    best.store(r, list);
+}
+
+// The same for records that carry an approximate distance v (a flat scan on the bf16 matrix cores), a workgroup per query.
+// At least k of the records have v at or below a_k, and v is off by at most slack / 2 from the streaming distance less the
+// query's constant, so whoever has v above a_k + slack stands behind k others: of the hundreds of records, the k and a handful
+// that are left are rescored.
+//
+// A wave or less of candidates, so memory's latency is all there is.  The four waves bring the records into LDS at once (the
+// first of them before the count is known), then the candidates' rows and the query, a piece of up to 32 KB on its way while
+// one is worked on; the first wave works, a lane per candidate, the streaming kernel's chain of sums from LDS.  (A wave per
+// query whose lanes read their own rows, 16 granules ahead, and the query through the scalar cache, which missed every line of
+// it: 100k x 768 fp32 cosine, 32 queries 47.5 us, now 36.4; 100k x 128 fp32, 1000 queries 17.5 and 18.1; 500k x 100 sq8, k 100, 200
+// queries 25.4 and 23.5.  With the rows through LDS but the query still through the scalar cache 52.7, 25.4 and 26.4.  Of a
+// query of the first 7000 of 60 000 cycles go to the k-th smallest, 15 000 to the sums, the rest to waits for memory.)
+constexpr uint32_t kValuedStage = 64 * 33;  // granules in LDS: of 64 rows 32, or of 32 rows 64, and one apart (32 x 65)
+constexpr uint32_t kValuedThreads = 256;
+constexpr uint32_t kValuedEach = 8;      // records of a thread
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+constexpr uint32_t kValuedWords = 1024;  // words of the query in LDS: the most that a piece takes
+
+// Words of a query's row per granule of a code.
+template <int KIND>
+constexpr uint32_t kGranuleWords = KIND == VSAG_AMD_KIND_SQ8 ? 16 : KIND == VSAG_AMD_KIND_SQ4 ? 32
+                                   : KIND == VSAG_AMD_KIND_SQ4_UNIFORM ? 8 : 4;
+
+// The words of a few granules, and the scales of their dimensions, in registers.
+template <uint32_t WORDS, bool SCALED>
+struct LocalQueryRow {
+    uint32_t row[1][WORDS];
+    float scales[SCALED ? WORDS : 1];
+
+    __device__ inline const float*
+    scale(const ScanArgs&) const {
+        return scales;
     }
-    if (lane == 0) {
-        r.partial_cnt[list] = admitted;
+};
+
+template <int KIND, int METRIC>
+__global__ void __launch_bounds__(kValuedThreads)
+rescore_valued_kernel(ScanArgs a, RescoreArgs r) {
+    extern __shared__ uint4 valued_lds[];  // [kValuedStage] granules, [S] keys, [cap] slots
+    constexpr bool kScaled = (KIND == VSAG_AMD_KIND_SQ8 || KIND == VSAG_AMD_KIND_SQ4) && METRIC == VSAG_AMD_METRIC_L2;
+    __shared__ __align__(16) uint32_t query[kValuedWords];
+    __shared__ __align__(16) float scales[kScaled ? kValuedWords : 4];
+    __shared__ __align__(16) uint32_t hist[256];
+    __shared__ float ends[2][4];
+    __shared__ uint32_t lefts[4], picked;
+    uint4* stage = valued_lds;
+    uint64_t* keys = reinterpret_cast<uint64_t*>(stage + kValuedStage);
+    uint32_t* pick = reinterpret_cast<uint32_t*>(keys + r.S);
+    const uint32_t tid = threadIdx.x, lane = tid & 63U;
+    if (tid == 0) {
+        picked = 0;
     }
-    if (admitted != 0) {
-        selector_copy_admitted(keys, kept, bs, r.partial + list * k, lane);
+    __syncthreads();
+    const bool first_wave = tid < kWave;
+    const uint32_t q = blockIdx.x;
+    const uint64_t* valued = r.valued + static_cast<uint64_t>(q) * r.cap;
+    // Records tid, tid + 256, ... of the query, in registers.
+    uint64_t record[kValuedEach];
+    auto read = [&](uint32_t u) __attribute__((always_inline)) {
+        const uint32_t i = tid + u * kValuedThreads;
+        record[u] = valued[i < r.cap ? i : r.cap - 1];
+    };
+    read(0);
+    read(1);
+    const float slack = r.slack[q];
+    const uint32_t total = as_const(r.cand_cnt)[static_cast<uint64_t>(q) * 32];
+    if (total > r.cap || as_const(r.gate)[q] != 0) {
+        if (first_wave) {
+            rescore_leaves_query(r, q, r.nslots, lane);  // (all of the query's lists, which nothing has cleared so far)
+        }
+        return;
+    }
+    if (total > 2 * kValuedThreads) {
+#pragma unroll
+        for (uint32_t u = 2; u < kValuedEach; ++u) {
+            read(u);
+        }
+    }
+    RescoreKeys best;
+    if (first_wave) {
+        best.init(keys, r, q, lane);
+    }
+    const float inf = __builtin_inff();
+    // The value of record u, or a NaN where there is none; those that count for the k-th smallest (kth_value_or_above, here by
+    // a whole workgroup on registers).
+    auto value = [&](uint32_t u) __attribute__((always_inline)) {
+        return tid + u * kValuedThreads < total ? ordered_to_float(static_cast<uint32_t>(record[u] >> 32)) : __builtin_nanf("");
+    };
+    auto counts = [](float v) __attribute__((always_inline)) { return v > -3.0e38F && v < 3.0e38F; };
+    float limit = inf;
+    if (total > r.k) {
+        float vmin = inf, vmax = -inf;
+        uint32_t left = 0;
+#pragma unroll
+        for (uint32_t u = 0; u < kValuedEach; ++u) {
+            const float v = value(u);
+            if (counts(v)) {
+                vmin = fminf(vmin, v);
+                vmax = fmaxf(vmax, v);
+                ++left;
+            }
+        }
+        for (int off = 32; off > 0; off >>= 1) {
+            vmin = fminf(vmin, __shfl_xor(vmin, off));
+            vmax = fmaxf(vmax, __shfl_xor(vmax, off));
+            left += __shfl_xor(left, off);
+        }
+        hist[tid] = 0;
+        if (lane == 0) {
+            ends[0][tid >> 6] = vmin;
+            ends[1][tid >> 6] = vmax;
+            lefts[tid >> 6] = left;
+        }
+        __syncthreads();
+        vmin = fminf(fminf(ends[0][0], ends[0][1]), fminf(ends[0][2], ends[0][3]));
+        vmax = fmaxf(fmaxf(ends[1][0], ends[1][1]), fmaxf(ends[1][2], ends[1][3]));
+        left = lefts[0] + lefts[1] + lefts[2] + lefts[3];
+        float kth = left < r.k ? inf : vmax;
+        const float width = (vmax - vmin) * (1.0F / 256.0F);
+        if (left >= r.k && width > 1.0e-30F && width < 1.0e30F) {
+            const float inv_width = 1.0F / width;
+#pragma unroll
+            for (uint32_t u = 0; u < kValuedEach; ++u) {
+                const float v = value(u);
+                if (counts(v)) {
+                    const float f = (v - vmin) * inv_width;
+                    atomicAdd(&hist[f < 255.0F ? static_cast<uint32_t>(f) : 255U], 1U);
+                }
+            }
+            __syncthreads();
+            // (every wave for itself: the first bin at which the running count reaches k, and two more)
+            const uint4 h = *reinterpret_cast<const uint4*>(hist + 4 * lane);
+            const uint32_t mine = h.x + h.y + h.z + h.w;
+            uint32_t incl = mine;
+            for (int off = 1; off < 64; off <<= 1) {
+                const uint32_t o = __shfl_up(incl, off);
+                incl += lane >= static_cast<uint32_t>(off) ? o : 0U;
+            }
+            const uint32_t c1 = incl - mine + h.x, c2 = c1 + h.y, c3 = c2 + h.z;
+            uint32_t bin = 4 * lane + (c1 >= r.k ? 0 : c2 >= r.k ? 1 : c3 >= r.k ? 2 : 3);
+            bin = __shfl(bin, static_cast<int>(__builtin_ctzll(__ballot(incl >= r.k))));
+            kth = fminf(vmin + static_cast<float>(bin + 3) * width, vmax);
+        }
+        if (slack < 3.0e38F && kth > -3.0e38F) {
+            limit = kth + slack;
+            limit += fabsf(limit) * 2.4e-7F;  // not below the sum
+        }
+    }
+#pragma unroll
+    for (uint32_t u = 0; u < kValuedEach; ++u) {
+        if (u * kValuedThreads < total) {
+            const bool take = tid + u * kValuedThreads < total && !(value(u) > limit);
+            const uint64_t mask = __ballot(take);
+            uint32_t at = 0;
+            if (lane == 0 && mask != 0) {
+                at = atomicAdd(&picked, static_cast<uint32_t>(__popcll(mask)));
+            }
+            at = __builtin_amdgcn_readfirstlane(at);
+            if (take) {
+                pick[at + mask_rank(mask)] = static_cast<uint32_t>(record[u]);
+            }
+        }
+    }
+    __syncthreads();
+    const uint32_t candidates = picked;
+    const uint32_t qidx[1] = {q};
+    const uint32_t* qrow = a.qtab + static_cast<size_t>(q) * a.qstride;
+    constexpr uint32_t kPerGranule = kGranuleWords<KIND>;
+    for (uint32_t base = 0; base < candidates; base += kWave) {
+        const uint32_t now = candidates - base < kWave ? candidates - base : kWave;
+        // A piece of every row at a time: eight threads bring a row's, of 64 granules, or, with more than 32 rows, of two rows'
+        // 32 each.  Rows lie an odd number of granules apart: the lanes' reads fall on all banks.
+        const bool both = now > kValuedThreads / 8;
+        const uint32_t most = both ? 32 : 64;
+        const uint32_t piece = most < kValuedWords / kPerGranule ? most : kValuedWords / kPerGranule;
+        const uint32_t pitch = piece + 1;
+        constexpr uint32_t kLoads = 8;
+        const uint32_t g0 = tid & 7U, row_a = tid >> 3, row_b = row_a + 32;
+        const uint32_t step = r.rows != nullptr ? 1 : kWave;
+        auto code_of = [&](uint32_t c) __attribute__((always_inline)) {
+            const uint32_t slot = pick[base + (c < now ? c : now - 1)];
+            return r.rows != nullptr ? r.rows + static_cast<uint64_t>(slot) * r.row_granules
+                                     : a.tiles + static_cast<uint64_t>(slot >> 6) * a.G * kWave + (slot & 63U);
+        };
+        const uint4* code_a = code_of(row_a);
+        const uint4* code_b = code_of(both ? row_b : row_a);
+        u32x4 v[kLoads], vq, vs;
+        // Load u is granule g0 + 8 u of row_a, or, with both, granule g0 + 8 (u % 4) of row_a and then of row_b.
+        const uint32_t per = both ? 4 : 8;  // granules of a row
+        auto fetch = [&](uint32_t j0) __attribute__((always_inline)) {
+#pragma unroll
+            for (uint32_t u = 0; u < kLoads; ++u) {
+                const uint32_t j = j0 + g0 + 8 * (u & (per - 1));
+                v[u] = *reinterpret_cast<const u32x4*>((u < per ? code_a : code_b) + static_cast<size_t>(j < a.G ? j : a.G - 1) * step);
+            }
+            // (rows of the query table are whole granules' worth of words, on 16 bytes)
+            const uint32_t here = (a.G - j0 < piece ? a.G - j0 : piece) * kPerGranule;
+            if (4 * tid < here) {
+                vq = *reinterpret_cast<const u32x4*>(qrow + j0 * kPerGranule + 4 * tid);
+                if constexpr (kScaled) {
+                    vs = *reinterpret_cast<const u32x4*>(a.scale + j0 * kPerGranule + 4 * tid);
+                }
+            }
+        };
+        auto park = [&](uint32_t j0) __attribute__((always_inline)) {
+#pragma unroll
+            for (uint32_t u = 0; u < kLoads; ++u) {
+                const uint32_t g = g0 + 8 * (u & (per - 1)), c = u < per ? row_a : row_b;
+                if (g < piece) {
+                    *reinterpret_cast<u32x4*>(stage + c * pitch + g) = v[u];
+                }
+            }
+            const uint32_t here = (a.G - j0 < piece ? a.G - j0 : piece) * kPerGranule;
+            if (4 * tid < here) {
+                *reinterpret_cast<u32x4*>(query + 4 * tid) = vq;
+                if constexpr (kScaled) {
+                    *reinterpret_cast<u32x4*>(scales + 4 * tid) = vs;
+                }
+            }
+        };
+        Acc<KIND, 1> acc;
+        acc_reset(acc);
+        fetch(0);
+        for (uint32_t j0 = 0; j0 < a.G; j0 += piece) {
+            park(j0);
+            __syncthreads();
+            if (j0 + piece < a.G) {
+                fetch(j0 + piece);
+            }
+            if (first_wave) {
+                const uint4* code = stage + (lane < now ? lane : now - 1) * pitch;
+                const uint32_t here = a.G - j0 < piece ? a.G - j0 : piece;
+                // 32 words of the query at a time, read while those before are worked on.
+                constexpr uint32_t kAhead = 32 / kPerGranule;
+                LocalQueryRow<32, kScaled> row[2];
+                uint4 c[2][kAhead];
+                auto look = [&](uint32_t j, int b) __attribute__((always_inline)) {
+#pragma unroll
+                    for (uint32_t u = 0; u < kAhead; ++u) {
+                        c[b][u] = code[j + u < here ? j + u : here - 1];
+                    }
+#pragma unroll
+                    for (uint32_t w = 0; w < 32; w += 4) {  // (behind the last granule: what an earlier piece left)
+                        const uint4 f = *reinterpret_cast<const uint4*>(query + ((j * kPerGranule + w) & (kValuedWords - 1)));
+                        row[b].row[0][w] = f.x, row[b].row[0][w + 1] = f.y, row[b].row[0][w + 2] = f.z, row[b].row[0][w + 3] = f.w;
+                        if constexpr (kScaled) {
+                            const float4 e = *reinterpret_cast<const float4*>(scales + ((j * kPerGranule + w) & (kValuedWords - 1)));
+                            row[b].scales[w] = e.x, row[b].scales[w + 1] = e.y, row[b].scales[w + 2] = e.z, row[b].scales[w + 3] = e.w;
+                        }
+                    }
+                };
+                auto work = [&](uint32_t j, int b) __attribute__((always_inline)) {
+#pragma unroll
+                    for (uint32_t u = 0; u < kAhead; ++u) {
+                        if (j + u < here) {
+                            accumulate_granule<KIND, METRIC, 1>(a, row[b], u, c[b][u], acc);
+                        }
+                    }
+                };
+                look(0, 0);
+                for (uint32_t j = 0; j < here; j += 2 * kAhead) {
+                    look(j + kAhead, 1);
+                    work(j, 0);
+                    look(j + 2 * kAhead, 0);
+                    work(j + kAhead, 1);
+                }
+            }
+            __syncthreads();
+        }
+        if (first_wave) {
+            const uint32_t slot = pick[base + (lane < now ? lane : now - 1)];
+            float d[1];
+            if (r.row_granules > a.G) {
+                // (the metadata words of the code sit behind it in its row, see rescore_kernel)
+                ScanArgs b = a;
+                b.meta = reinterpret_cast<const uint32_t*>(r.rows + static_cast<uint64_t>(slot) * r.row_granules + a.G);
+                b.meta_stride = 1;
+                finish_distances<KIND, METRIC, 1>(b, qidx, 0, acc, d);
+            } else {
+                finish_distances<KIND, METRIC, 1>(a, qidx, slot, acc, d);
+            }
+            best.add(make_key(d[0], slot), lane < now && slot < r.n);
+        }
+    }
+    if (first_wave) {
+        best.store(r, static_cast<uint64_t>(q) * r.nslots + r.out_slot);
     }
 }
 
@@ -1325,13 +1626,23 @@ launch_code_terms(vsag_amd_store* s, uint64_t first, uint64_t count, hipStream_t
     return 0;
 }
 
-template <int KIND, bool VALUED = false>
+template <int KIND>
 static void
 launch_rescore_m(int metric, dim3 grid, size_t lds, hipStream_t st, const ScanArgs& a, const RescoreArgs& r) {
     if (metric == VSAG_AMD_METRIC_L2) {
-        hipLaunchKernelGGL((rescore_kernel<KIND, VSAG_AMD_METRIC_L2, VALUED>), grid, dim3(kWave), lds, st, a, r);
+        hipLaunchKernelGGL((rescore_kernel<KIND, VSAG_AMD_METRIC_L2>), grid, dim3(kWave), lds, st, a, r);
     } else {
-        hipLaunchKernelGGL((rescore_kernel<KIND, VSAG_AMD_METRIC_IP, VALUED>), grid, dim3(kWave), lds, st, a, r);
+        hipLaunchKernelGGL((rescore_kernel<KIND, VSAG_AMD_METRIC_IP>), grid, dim3(kWave), lds, st, a, r);
+    }
+}
+
+template <int KIND>
+static void
+launch_rescore_valued_m(int metric, dim3 grid, size_t lds, hipStream_t st, const ScanArgs& a, const RescoreArgs& r) {
+    if (metric == VSAG_AMD_METRIC_L2) {
+        hipLaunchKernelGGL((rescore_valued_kernel<KIND, VSAG_AMD_METRIC_L2>), grid, dim3(kValuedThreads), lds, st, a, r);
+    } else {
+        hipLaunchKernelGGL((rescore_valued_kernel<KIND, VSAG_AMD_METRIC_IP>), grid, dim3(kValuedThreads), lds, st, a, r);
     }
 }
 
@@ -1408,17 +1719,18 @@ launch_rescore_valued(const vsag_amd_store* s, const ScanArgs& a, uint64_t nq, u
     r.rows = s->rows;
     r.row_granules = s->row_granules;
     const dim3 grid(static_cast<uint32_t>(nq));
-    const size_t lds = S * 8 + (128 + 256) * 4;
+    VA_CHECK_ARG(cap <= kValuedEach * kValuedThreads, "%u records a query are too many", cap);
+    const size_t lds = kValuedStage * sizeof(uint4) + S * sizeof(uint64_t) + cap * sizeof(uint32_t);
     if (s->kind == VSAG_AMD_KIND_SQ8_UNIFORM) {
-        launch_rescore_m<VSAG_AMD_KIND_SQ8_UNIFORM, true>(s->metric, grid, lds, st, a, r);
+        launch_rescore_valued_m<VSAG_AMD_KIND_SQ8_UNIFORM>(s->metric, grid, lds, st, a, r);
     } else if (s->kind == VSAG_AMD_KIND_SQ4_UNIFORM) {
-        launch_rescore_m<VSAG_AMD_KIND_SQ4_UNIFORM, true>(s->metric, grid, lds, st, a, r);
+        launch_rescore_valued_m<VSAG_AMD_KIND_SQ4_UNIFORM>(s->metric, grid, lds, st, a, r);
     } else if (s->kind == VSAG_AMD_KIND_SQ8) {
-        launch_rescore_m<VSAG_AMD_KIND_SQ8, true>(s->metric, grid, lds, st, a, r);
+        launch_rescore_valued_m<VSAG_AMD_KIND_SQ8>(s->metric, grid, lds, st, a, r);
     } else if (s->kind == VSAG_AMD_KIND_SQ4) {
-        launch_rescore_m<VSAG_AMD_KIND_SQ4, true>(s->metric, grid, lds, st, a, r);
+        launch_rescore_valued_m<VSAG_AMD_KIND_SQ4>(s->metric, grid, lds, st, a, r);
     } else {
-        launch_rescore_m<VSAG_AMD_KIND_FP32, true>(s->metric, grid, lds, st, a, r);
+        launch_rescore_valued_m<VSAG_AMD_KIND_FP32>(s->metric, grid, lds, st, a, r);
     }
     VA_HIP(hipGetLastError());
     return 0;
