@@ -455,3 +455,34 @@ def test_residual_rabitq_lists_match_oracle(lib, metric, mname, qbits):
     for b in (cdev, rdev, cendev, out, cb, lb_dev):
         b.free()
     st.destroy()
+
+
+@pytest.mark.parametrize("kind,metric,d,kcand", [("sq8", orc.IP, 100, 80), ("sq8", orc.IP, 256, 256), ("sq8", orc.COSINE, 33, 41),
+                                                 ("sq8", orc.IP, 257, 80), ("fp32", orc.L2, 40, 100), ("sq8", orc.IP, 100, 20)])
+def test_middling_batches_with_more_kept_than_items(lib, kind, metric, d, kcand):
+    """16 000 pairs of lists that are cut into chunks, with and without the nearest list ahead of the others and with and without
+    seeds: the ids and distance bits of a few queries at a time.  Lists of no code, of one and of many, columns that name no
+    list, the nearest among them."""
+    rng = np.random.default_rng(d + kcand)
+    n, nlist, nq, nprobe = 40000, 100, 800, 20
+    x, means = gaussian_mixture(rng, n, d, 100, 0.05)
+    q, _ = gaussian_mixture(rng, nq, d, 100, 0.05, means=means)
+    labels = rng.integers(2, nlist, n).astype(np.int32)
+    labels[labels == 3] = 4
+    labels[0], labels[1:900] = 3, 5
+    if kind == "fp32":
+        st, codes = Store(capi.KIND_FP32, metric, d), x.view(np.uint8).reshape(n, -1)
+    else:
+        lb, diff = orc.sq_train(x, 8, metric)
+        st, codes = Store(capi.KIND_SQ8, metric, d, lb=lb, diff=diff), orc.sq_encode(x, 8, lb, diff, metric)
+    st.set_lists(codes, labels, nlist)
+    buckets = np.argsort(rng.random((nq, nlist)), 1)[:, :nprobe].astype(np.int32)
+    buckets[::9, 0] = -1
+    buckets[::7, 3] = -1
+    buckets[::5, 0] = 0
+    buckets[1::11, 0] = 3
+    ids, ds = st.ivf_scan(q, buckets, kcand)
+    for i in range(0, nq, 50):
+        rids, rds = st.ivf_scan(q[i:i + 3], buckets[i:i + 3], kcand)
+        assert np.array_equal(ds[i:i + 3].view(np.uint32), rds.view(np.uint32)) and np.array_equal(ids[i:i + 3], rids)
+    st.destroy()

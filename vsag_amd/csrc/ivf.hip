@@ -30,7 +30,8 @@ struct ScanPlanIvf {
     uint64_t npairs;
     uint32_t tiles_per_item;  // 0xFFFFFFFF: a work item walks its whole list
     uint32_t chunks_max;      // partial lists per (query, list) pair
-    bool chunked;             // one launch over all probe columns, seeded cold start
+    bool chunked;             // lists cut into chunks, and seeds for a cold start
+    bool nearest_first;       // chunked: the nearest list of every query ahead of the others, as the whole-list plan does
     bool seeded;
     bool mfma;                // probe columns behind the first go through the int8 matrix cores (ivf_i8.hip)
     bool planes;              // ... with sq8 codes: two int8 planes per query, records rescored (prefilter_i8.hip)
@@ -308,20 +309,26 @@ scatter_pairs_kernel(const int32_t* buckets, uint64_t nq, uint32_t nprobe, uint3
     }
 }
 
-// The three regrouping steps above for a small batch (all probe columns) in one workgroup.  A chain of latencies bounds it:
+// The three regrouping steps above for a small batch (probe columns [p0, p1); ALL: they are all) in one workgroup.  A chain of latencies bounds it:
 // a bucket is loaded, its counter raised, its place written.  With the counters in LDS (LDS: lists up to kRegroupLists;
 // more lists count in memory) and kRegroupInFlight buckets of a thread loaded together, 24 000 pairs of 512 lists take 17 us
 // (one bucket at a time, counters in memory: 81; the call 651 -> 589), 32 pairs of 1024 lists 5 (the call 127 -> 122).
 constexpr uint32_t kRegroupInFlight = 8;
 
-template <bool LDS>
+template <bool LDS, bool ALL>
 __global__ void __launch_bounds__(1024)
-regroup_small_kernel(const int32_t* buckets, uint64_t nq, uint32_t nprobe, const uint32_t* list_tile, uint32_t nlist,
-                     uint32_t T, uint32_t tiles_per_item, uint32_t chunks_max, uint32_t* counts, uint32_t* cursor,
+regroup_small_kernel(const int32_t* buckets, uint64_t nq, uint32_t nprobe, uint32_t p0, uint32_t p1,
+                     const uint32_t* list_tile, uint32_t nlist, uint32_t T, uint32_t tiles_per_item, uint32_t chunks_max, uint32_t* counts, uint32_t* cursor,
                      uint32_t* pair_off, uint32_t* item_off, uint32_t* sorted_pair) {
     __shared__ uint32_t wave_sums[2][16];
     __shared__ uint32_t place[LDS ? kRegroupLists : 1];  // of a list: its pairs, then the place of its next one
-    const uint64_t npairs = nq * nprobe;
+    const uint32_t cols = p1 - p0;
+    const uint64_t npairs = nq * cols;
+    // (a pair of all columns, from its place among these; both fit 32 bits)
+    auto pair_of = [&](uint64_t i) {
+        const uint32_t at = static_cast<uint32_t>(i);
+        return ALL ? at : at / cols * nprobe + p0 + at % cols;
+    };
     for (uint32_t i = threadIdx.x; i < nlist; i += blockDim.x) {
         if (LDS) {
             place[i] = 0;
@@ -337,12 +344,12 @@ regroup_small_kernel(const int32_t* buckets, uint64_t nq, uint32_t nprobe, const
 #pragma unroll
             for (uint32_t u = 0; u < kRegroupInFlight; ++u) {
                 const uint64_t i = i0 + static_cast<uint64_t>(u) * blockDim.x;
-                b[u] = i < npairs ? buckets[i] : -1;
+                b[u] = i < npairs ? buckets[pair_of(i)] : -1;
             }
 #pragma unroll
             for (uint32_t u = 0; u < kRegroupInFlight; ++u) {
                 if (b[u] >= 0 && static_cast<uint32_t>(b[u]) < nlist) {
-                    visit(static_cast<uint32_t>(b[u]), static_cast<uint32_t>(i0 + static_cast<uint64_t>(u) * blockDim.x));
+                    visit(static_cast<uint32_t>(b[u]), pair_of(i0 + static_cast<uint64_t>(u) * blockDim.x));
                 }
             }
         }
@@ -630,6 +637,8 @@ plan_ivf(const vsag_amd_store* s, uint64_t nq, uint32_t nprobe, uint32_t kcand, 
     p->chunked = groups < 8192 && s->max_list_tiles > 2;
     p->tiles_per_item = 0xFFFFFFFFU;
     p->chunks_max = 1;
+    bool four_pays = false;
+    uint64_t items = nprobe;  // of a query, in lists of average length
     if (p->chunked) {
         const uint64_t avg_tiles = std::max<uint64_t>(1, s->nlist ? s->ntiles / s->nlist : 1);
         const bool four = fine && t == 4 && groups >= 3900 && kcand <= 256 &&
@@ -641,8 +650,20 @@ plan_ivf(const vsag_amd_store* s, uint64_t nq, uint32_t nprobe, uint32_t kcand, 
         }
         p->tiles_per_item = static_cast<uint32_t>(std::min<uint64_t>(tpi, 0x7FFFFFFFU));
         p->chunks_max = static_cast<uint32_t>(cap);
+        four_pays = four;
+        items = nprobe * std::min<uint64_t>(cap, div_up(avg_tiles, tpi));
     }
-    p->seeded = p->chunked && kcand <= 256;
+    // Seeds give a bound once every one of kcand slots holds a minimum; with fewer items than that a query looks at its row of
+    // them in vain, a wait for memory per tile (fp32 l2 200k x 200, 512 lists, k 100, 1000 queries x 24: 706 -> 667 us).
+    const bool fills = kcand <= items;
+    p->seeded = p->chunked && kcand <= 256 && fills;
+    // Then the nearest list of every query goes ahead, a list to a wave, where its bound spares the others more selecting than
+    // its own scan costs: sq8 codes of up to 256 dimensions (cheap to scan) and lists of at most six times as many codes as are
+    // kept (sq8 ip 200k x 200, 512 lists, 80 kept, 1000 queries x 24: 569 -> 490 us; 500k x 128, 800 lists, 200 kept, 3000 x 8:
+    // 825 -> 729.  Not with ten times as many, 1M x 96, 1000 lists, 100 kept, 900 x 20: 407 -> 428; nor of 960 dimensions, 300k,
+    // 1000 lists, 200 kept, 1500 x 12: 1516 -> 1701; nor fp32 codes, the first above with k 100: 667 -> 736).
+    p->nearest_first = p->chunked && four_pays && !fills && s->kind == VSAG_AMD_KIND_SQ8 && s->dpad <= 256 &&
+                       s->ntiles * kWave <= 6ull * kcand * s->nlist;
     // Large batches on sq4_uniform (and sq8_uniform / l2) lists: the streaming kernel scans the nearest list of every query, the int8
     // matrix cores the other columns, into two private lists per (query, list) pair.
     p->mfma = !p->chunked && nprobe > 1 && scan_contraction_mode(s) >= 0 && ivf_i8_supports(s) &&
@@ -828,7 +849,7 @@ vsag_amd_ivf_scan_topk_ex(const vsag_amd_store_t* s, const float* queries_dev, u
     size_t lds = static_cast<size_t>(waves) * p.T * p.S * 8;
     // Whole lists: two passes, the nearest list of every query first (it seeds the per-query bound), then the
     // rest.  Chunked lists: all probe columns at once.
-    uint32_t cols[3] = {0, p.chunked ? nprobe : 1, nprobe};
+    uint32_t cols[3] = {0, p.chunked && !p.nearest_first ? nprobe : 1, nprobe};
     // A pre-filter or a radius goes the streaming way (the matrix-core pass knows neither).
     const bool mfma = p.mfma && (options == nullptr || (options->deny_bits_dev == nullptr && options->use_radius == 0));
     // The pairs of columns [c0, c1) grouped by list (pair_off, sorted_pair) and the work items of every list (item_off).
@@ -859,7 +880,7 @@ vsag_amd_ivf_scan_topk_ex(const vsag_amd_store_t* s, const float* queries_dev, u
             continue;
         }
         uint64_t pairs = nq * (p1 - p0);
-        if (pass == 1) {
+        if (pass == 1 && !p.chunked) {
             fill(FillJob{{b.counts, b.cursor, mfma ? b.gate : nullptr, nullptr, nullptr}, {0U, 0U, 0U, 0U, 0U},
                          {nlists1, nlists1, mfma ? nq + 3 : 0, 0, 0}});
         }
@@ -946,23 +967,30 @@ vsag_amd_ivf_scan_topk_ex(const vsag_amd_store_t* s, const float* queries_dev, u
         // That pass lives on its selectors (no bound to start from), not on the list bytes: two queries per wave
         // instead of four mean twice the waves to overlap the flushes of each other (10M x 128, 64 lists: 0.59 ->
         // 0.45 ms).
-        const int t_pass = cut_first ? std::min(p.T, 2) : p.T;
+        const bool nearest = p.nearest_first && pass == 0;
+        const int t_pass = nearest ? 1 : cut_first ? std::min(p.T, 2) : p.T;
+        if (nearest) {
+            first.tiles_per_item = 0x7FFFFFFFU;  // (a list at a time, by the kernel that knows chunks)
+            first.seed = nullptr;
+        }
         if (cut_first) {
             const uint32_t avg_tiles = std::max<uint32_t>(1, static_cast<uint32_t>(s->ntiles / s->nlist));
             first.tiles_per_item = std::max<uint32_t>(std::max<uint32_t>(16, avg_tiles + avg_tiles / 4),
                                                       static_cast<uint32_t>(div_up(s->max_list_tiles, p.chunks_max)));
         }
         if (p.chunked) {
-            hipLaunchKernelGGL(s->nlist <= kRegroupLists ? regroup_small_kernel<true> : regroup_small_kernel<false>, dim3(1),
-                               dim3(1024), 0, st, buckets_dev, nq, nprobe, s->list_tile_dev, s->nlist,
-                               static_cast<uint32_t>(p.T), p.tiles_per_item, p.chunks_max, b.counts, b.cursor, b.pair_off,
+            const bool in_lds = s->nlist <= kRegroupLists, all = p0 == 0 && p1 == nprobe;
+            auto kernel = in_lds ? (all ? regroup_small_kernel<true, true> : regroup_small_kernel<true, false>)
+                                 : (all ? regroup_small_kernel<false, true> : regroup_small_kernel<false, false>);
+            hipLaunchKernelGGL(kernel, dim3(1), dim3(1024), 0, st, buckets_dev, nq, nprobe, p0, p1, s->list_tile_dev, s->nlist,
+                               static_cast<uint32_t>(t_pass), first.tiles_per_item, p.chunks_max, b.counts, b.cursor, b.pair_off,
                                b.item_off, b.sorted_pair);
         } else {
             regroup(p0, p1, pairs, static_cast<uint32_t>(t_pass), first.tiles_per_item, p.chunks_max);
         }
         // At most one partly filled query group per probed list, each cut into at most chunks_max items.
         uint64_t max_items =
-            (div_up(pairs, t_pass) + std::min<uint64_t>(s->nlist, pairs)) * (p.chunked || cut_first ? p.chunks_max : 1);
+            (div_up(pairs, t_pass) + std::min<uint64_t>(s->nlist, pairs)) * ((p.chunked && !nearest) || cut_first ? p.chunks_max : 1);
         dim3 grid(static_cast<uint32_t>(div_up(max_items, waves)));
         VA_TRY(launch_ivf(s, t_pass, grid, dim3(waves * kWave), static_cast<size_t>(waves) * t_pass * p.S * 8, st, a, first));
     }

@@ -2561,7 +2561,7 @@ protected:
             return pack_results(ids, dists, nq, nprobe, identity, stats.dump());
         }
         uint64_t probed = 0;  // (in it once the first results are)
-        probed_codes(ctx, nq, nprobe, &probed);
+        const bool probed_later = probed_codes(ctx, nq, nprobe, &probed);
         DenyMask mask;
         mask.init(ctx, labels_, spec.valid, looped, bpd_);
         // FlatBucketSearcher compares against radius + THRESHOLD_ERROR (flat_bucket_searcher.cpp:121,
@@ -2582,6 +2582,9 @@ protected:
                 dev(vsag_amd_rerank_fp32(raw_.as<float>(), labels_.size(), q_.dim, q_.metric, ctx.rows, nq,
                                          ctx.cand_ids.as<uint32_t>(), kc, static_cast<uint32_t>(kout), out.ids,
                                          out.dists, ctx.stream));
+                if (probed_later) {
+                    ctx.download_later(&probed, ctx.scalar.p, 8);
+                }
                 ctx.take_results(out, count, ids, dists);
                 stats.approximate = probed;
                 stats.rerank = static_cast<uint64_t>(nq) * kc;  // at most: lists may hold fewer candidates
@@ -2590,6 +2593,9 @@ protected:
             const size_t count = static_cast<size_t>(nq) * kc;
             const SearchContext::Results out = ctx.results(ctx.cand_ids, ctx.cand_d, count);
             scan_lists(ctx, nq, nprobe, kc, opt, out);
+            if (probed_later) {
+                ctx.download_later(&probed, ctx.scalar.p, 8);
+            }
             ctx.take_results(out, count, ids, dists);
             stats.approximate = probed;
             if (bpd_ > 1) {
@@ -2624,6 +2630,9 @@ protected:
             scan_lists(ctx, 1, nprobe, kc, opt, cand_buffers(ctx, 1, kc));
             std::vector<uint32_t> ids;
             std::vector<float> dists;
+            if (probed_later) {
+                ctx.download_later(&probed, ctx.scalar.p, 8);
+            }
             fetch(ctx, ctx.cand_ids, ctx.cand_d, kc, ids, dists);
             stats.approximate += probed;
             uint32_t got = 0;
@@ -3143,14 +3152,13 @@ private:
         ctx.download(dists.data(), d_dev.p, count * 4);
     }
 
-    // Codes in the lists of ctx.buckets, over all (query, list) pairs: in *total after the next finish().
-    void
+    // Codes in the lists of ctx.buckets, over all (query, list) pairs: in *total after the next finish(), or, if true is
+    // returned, once the caller has downloaded ctx.scalar (behind its own work: a copy amid the kernels holds them up).
+    bool
     probed_codes(SearchContext& ctx, int64_t nq, uint32_t nprobe, uint64_t* total) const {
         uint64_t* to = ctx.scalar_result(total, static_cast<uint64_t>(nq) * nprobe <= VSAG_AMD_PROBED_CODES_STORED);
         dev(vsag_amd_ivf_probed_codes(lists_.s, ctx.buckets.as<int32_t>(), nq, nprobe, to, ctx.stream));
-        if (to == ctx.scalar.as<uint64_t>()) {
-            ctx.download_later(total, to, 8);
-        }
+        return to == ctx.scalar.as<uint64_t>();
     }
 
     static SearchContext::Results
