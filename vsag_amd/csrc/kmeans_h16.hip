@@ -28,9 +28,9 @@
 // 67.9; 480k x 960, k 256 2.42 / 3.51 / 2.68; of a single slab (65536 x 128, k 512) 0.12 / 0.18 / 0.18.  Where nothing is
 // open, asking costs 0.5 to 1 %.
 //
-// 1M x 960 rows, 4096 centroids (one assignment): 63.3 -> 11.4 ms.  Of that the contraction takes 7.4 (7.9e12 flop: 1070
+// 1M x 960 rows, 4096 centroids (one assignment): 63.3 -> 11.2 ms.  Of that the contraction takes 7.4 (7.9e12 flop: 1070
 // TFLOP/s, where matrix instructions on random operands in registers reach 1610 to 1690 and with their reads of LDS 1580,
-// all bound by power), the rounding of the rows 1.25 (5.8 GB at 4.6 TB/s) and the rescoring 2.8 (3.8 GB of rows, 0.8 GB of
+// all bound by power), the rounding of the rows 1.25 (5.8 GB at 4.6 TB/s) and the rescoring 2.4 (3.8 GB of rows, 0.8 GB of
 // table, one to three centroids a row).
 #include "kmeans_h16.h"
 
@@ -43,6 +43,7 @@ namespace vsag_amd {
 typedef _Float16 halfx8 __attribute__((ext_vector_type(8)));
 typedef _Float16 halfx4 __attribute__((ext_vector_type(4)));
 typedef float floatx16 __attribute__((ext_vector_type(16)));
+typedef float float4_v __attribute__((ext_vector_type(4)));
 
 constexpr uint32_t kTile = 256;        // centroids x rows of a workgroup's tile
 constexpr uint32_t kThreads = 512;
@@ -812,32 +813,40 @@ kmeans_h16_rescore_kernel(KmeansRescoreArgs p) {
             pair_c[tid] = c;
         }
         __syncthreads();
-        float4 gx[4], gc[4];
-        auto fetch = [&](uint32_t d) __attribute__((always_inline)) {
+        // Two pieces are on their way while one is summed (with one, 69 888 x 960 rows took 200 us, a wait of 2 us per piece;
+        // 168 now).
+        const float *xrow[4], *crow[4];
+        bool used[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const uint32_t pr = (tid >> 3) + 32 * i;
+            const uint32_t c = pair_c[pr];
+            used[i] = c != 0xFFFFFFFFU;
+            xrow[i] = p.x + (block_row + pair_row[pr]) * p.dim;
+            crow[i] = p.cent + static_cast<uint64_t>(used[i] ? c : 0) * p.dim;
+        }
+        float4_v gx[2][4], gc[2][4];
+        auto fetch = [&](uint32_t d, int b) __attribute__((always_inline)) {
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
-                const uint32_t pr = (tid >> 3) + 32 * i;
-                const uint32_t c = pair_c[pr];
-                const bool in = c != 0xFFFFFFFFU && d < p.dim;
-                gx[i] = in ? load4(p.x + (block_row + pair_row[pr]) * p.dim, d, p.dim, p.wide != 0)
-                           : make_float4(0.0F, 0.0F, 0.0F, 0.0F);
-                gc[i] = in ? load4(p.cent + static_cast<uint64_t>(c) * p.dim, d, p.dim, p.wide != 0)
-                           : make_float4(0.0F, 0.0F, 0.0F, 0.0F);
+                gx[b][i] = gc[b][i] = float4_v{0.0F, 0.0F, 0.0F, 0.0F};
+                if (used[i] && d < p.dim) {
+                    const float4 vx = load4(xrow[i], d, p.dim, p.wide != 0), vc = load4(crow[i], d, p.dim, p.wide != 0);
+                    gx[b][i] = float4_v{vx.x, vx.y, vx.z, vx.w};
+                    gc[b][i] = float4_v{vc.x, vc.y, vc.z, vc.w};
+                }
             }
         };
         float acc = 0.0F;
-        fetch(quad);
-        for (uint32_t piece = 0; piece < pieces; ++piece) {
+        auto sum = [&](uint32_t piece, int b) __attribute__((always_inline)) {
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 const uint32_t pr = (tid >> 3) + 32 * i;
-                *reinterpret_cast<float4*>(&seg_x[pr][quad]) = gx[i];
-                *reinterpret_cast<float4*>(&seg_c[pr][quad]) = gc[i];
+                *reinterpret_cast<float4_v*>(&seg_x[pr][quad]) = gx[b][i];
+                *reinterpret_cast<float4_v*>(&seg_c[pr][quad]) = gc[b][i];
             }
             __syncthreads();
-            if (piece + 1 < pieces) {
-                fetch((piece + 1) * kPiece + quad);
-            }
+            fetch((piece + 2) * kPiece + quad, b);  // (nothing past the dimension)
             if (tid < kPairs) {
 #pragma unroll
                 for (uint32_t d = 0; d < kPiece; d += 8) {
@@ -855,6 +864,14 @@ kmeans_h16_rescore_kernel(KmeansRescoreArgs p) {
                 }
             }
             __syncthreads();
+        };
+        fetch(quad, 0);
+        fetch(kPiece + quad, 1);
+        for (uint32_t piece = 0; piece < pieces; piece += 2) {
+            sum(piece, 0);
+            if (piece + 1 < pieces) {
+                sum(piece + 1, 1);
+            }
         }
         if (base + tid < total && tid < kPairs) {
             const uint32_t c = pair_c[tid];
