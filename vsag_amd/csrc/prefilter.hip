@@ -692,20 +692,107 @@ rescore_kernel(ScanArgs a, RescoreArgs r) {
     best.store(r, list);
 }
 
-// The same for records that carry an approximate distance v (a flat scan on the bf16 matrix cores), a workgroup per query.
-// At least k of the records have v at or below a_k, and v is off by at most slack / 2 from the streaming distance less the
-// query's constant, so whoever has v above a_k + slack stands behind k others: of the hundreds of records, the k and a handful
-// that are left are rescored.
+// The same for records that carry an approximate distance v (a flat scan on the bf16 matrix cores).  At least k of the records
+// have v at or below a_k, and v is off by at most slack / 2 from the streaming distance less the query's constant, so whoever
+// has v above a_k + slack stands behind k others: of the hundreds of records, the k and a handful that are left are rescored.
+//
+// Two forms.  With many queries, a wave per query, whose lanes read their candidates' rows up to 16 granules ahead: small
+// workgroups, of which many share a compute unit.  With few (kValuedFewQueries), a workgroup per query, below.  Calls with
+// either, us: 2000 queries against 100k x 128 fp32 248 / 254, 10000 1012 / 1097, 9693 against 115k x 768 sq4_uniform 2300 / 2414;
+// 32 against 100k x 768 fp32 185 / 170.
+template <int KIND, int METRIC>
+__global__ void __launch_bounds__(64)
+rescore_valued_wave_kernel(ScanArgs a, RescoreArgs r) {
+    extern __shared__ uint64_t keys[];  // [S] keys, then 128 slots waiting and 256 bins
+    const uint32_t lane = threadIdx.x;
+    const uint32_t q = blockIdx.x;
+    const uint32_t total = as_const(r.cand_cnt)[static_cast<uint64_t>(q) * 32];
+    if (total > r.cap || as_const(r.gate)[q] != 0) {
+        rescore_leaves_query(r, q, r.nslots, lane);  // (all of the query's lists, which nothing has cleared so far)
+        return;
+    }
+    RescoreKeys best;
+    best.init(keys, r, q, lane);
+    const uint32_t qidx[1] = {q};
+    const QueryRows<1> qrows = query_rows<1>(a, qidx);
+    auto rescore = [&](const uint32_t* mine, uint32_t now) __attribute__((always_inline)) {
+        const bool have = lane < now;
+        const uint32_t slot = have ? mine[lane] : 0U;
+        Acc<KIND, 1> acc;
+        acc_reset(acc);
+        const uint4* row = r.rows != nullptr ? r.rows + static_cast<uint64_t>(slot) * r.row_granules : nullptr;
+        // A wave or two of candidates per query, so latency is all there is: as many granules ahead as registers allow.
+        constexpr uint32_t kAhead = KIND == VSAG_AMD_KIND_FP32 ? 16
+                                   : KIND == VSAG_AMD_KIND_SQ4 ? (METRIC == VSAG_AMD_METRIC_L2 ? 1 : 2)
+                                   : (KIND == VSAG_AMD_KIND_SQ8 && METRIC == VSAG_AMD_METRIC_L2 ? 2 : 4);
+        accumulate_code<KIND, METRIC, kAhead>(
+            a, qrows, row != nullptr ? row : a.tiles + static_cast<uint64_t>(slot >> 6) * a.G * kWave + (slot & 63U),
+            row != nullptr ? 1 : kWave, acc);
+        float d[1];
+        if (r.row_granules > a.G) {
+            ScanArgs b = a;  // (see rescore_kernel)
+            b.meta = reinterpret_cast<const uint32_t*>(row + a.G);
+            b.meta_stride = 1;
+            finish_distances<KIND, METRIC, 1>(b, qidx, 0, acc, d);
+        } else {
+            finish_distances<KIND, METRIC, 1>(a, qidx, slot, acc, d);
+        }
+        best.add(make_key(d[0], slot), have && slot < r.n);
+    };
+    uint32_t* pick = reinterpret_cast<uint32_t*>(keys + r.S);
+    const uint64_t* valued = r.valued + static_cast<uint64_t>(q) * r.cap;
+    float limit = __builtin_inff();
+    if (total > r.k) {
+        const float kth = kth_value_or_above(
+            [&](uint32_t i) { return ordered_to_float(static_cast<uint32_t>(valued[i] >> 32)); }, total, r.k, pick + 128, lane);
+        const float slack = r.slack[q];
+        if (slack < 3.0e38F && kth > -3.0e38F) {
+            limit = kth + slack;
+            limit += fabsf(limit) * 2.4e-7F;  // not below the sum
+        }
+    }
+    uint32_t waiting = 0;
+    for (uint32_t base = 0; base < total; base += kWave) {
+        const uint64_t key = base + lane < total ? valued[base + lane] : kInfKey;
+        const bool take = base + lane < total && !(ordered_to_float(static_cast<uint32_t>(key >> 32)) > limit);
+        const uint64_t mask = __ballot(take);
+        if (take) {
+            pick[waiting + mask_rank(mask)] = static_cast<uint32_t>(key);
+        }
+        waiting += static_cast<uint32_t>(__popcll(mask));
+        wave_lds_fence();
+        if (waiting >= kWave || base + kWave >= total) {
+            // (a round of at most 64, what is left over moves to the front)
+            const uint32_t now = waiting < kWave ? waiting : kWave;
+            rescore(pick, now);
+            const uint32_t left = waiting - now;
+            const uint32_t moved = lane < left ? pick[kWave + lane] : 0U;
+            wave_lds_fence();
+            if (lane < left) {
+                pick[lane] = moved;
+            }
+            waiting = left;
+            wave_lds_fence();
+        }
+    }
+    if (waiting != 0) {
+        rescore(pick, waiting);
+    }
+    best.store(r, static_cast<uint64_t>(q) * r.nslots + r.out_slot);
+}
+
+// The form for few queries.
 //
 // A wave or less of candidates, so memory's latency is all there is.  The four waves bring the records into LDS at once (the
 // first of them before the count is known), then the candidates' rows and the query, a piece of up to 32 KB on its way while
 // one is worked on; the first wave works, a lane per candidate, the streaming kernel's chain of sums from LDS.  (A wave per
 // query whose lanes read their own rows, 16 granules ahead, and the query through the scalar cache, which missed every line of
-// it: 100k x 768 fp32 cosine, 32 queries 47.5 us, now 36.4; 100k x 128 fp32, 1000 queries 17.5 and 18.1; 500k x 100 sq8, k 100, 200
-// queries 25.4 and 23.5.  With the rows through LDS but the query still through the scalar cache 52.7, 25.4 and 26.4.  Of a
+// it: 100k x 768 fp32 cosine, 32 queries 47.5 us, here 36.4; 500k x 100 sq8, k 100, 200
+// queries 25.4 and 23.5.  With the rows through LDS but the query still through the scalar cache 52.7 and 26.4.  Of a
 // query of the first 7000 of 60 000 cycles go to the k-th smallest, 15 000 to the sums, the rest to waits for memory.)
 constexpr uint32_t kValuedStage = 64 * 33;  // granules in LDS: of 64 rows 32, or of 32 rows 64, and one apart (32 x 65)
 constexpr uint32_t kValuedThreads = 256;
+constexpr uint64_t kValuedFewQueries = 512;  // (1000 queries against 100k x 128 fp32: 18.1 us, and 17.5 with a wave each)
 constexpr uint32_t kValuedEach = 8;      // records of a thread
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 constexpr uint32_t kValuedWords = 1024;  // words of the query in LDS: the most that a piece takes
@@ -1638,11 +1725,22 @@ launch_rescore_m(int metric, dim3 grid, size_t lds, hipStream_t st, const ScanAr
 
 template <int KIND>
 static void
-launch_rescore_valued_m(int metric, dim3 grid, size_t lds, hipStream_t st, const ScanArgs& a, const RescoreArgs& r) {
+launch_rescore_valued_m(int metric, uint64_t nq, hipStream_t st, const ScanArgs& a, const RescoreArgs& r) {
+    const dim3 grid(static_cast<uint32_t>(nq));
+    const bool few = nq <= kValuedFewQueries;
+    const size_t lds = few ? kValuedStage * sizeof(uint4) + r.S * sizeof(uint64_t) + r.cap * sizeof(uint32_t)
+                           : r.S * sizeof(uint64_t) + (128 + 256) * sizeof(uint32_t);
+    auto launch = [&](auto kernel, uint32_t threads) { hipLaunchKernelGGL(kernel, grid, dim3(threads), lds, st, a, r); };
     if (metric == VSAG_AMD_METRIC_L2) {
-        hipLaunchKernelGGL((rescore_valued_kernel<KIND, VSAG_AMD_METRIC_L2>), grid, dim3(kValuedThreads), lds, st, a, r);
+        if (few) {
+            launch(rescore_valued_kernel<KIND, VSAG_AMD_METRIC_L2>, kValuedThreads);
+        } else {
+            launch(rescore_valued_wave_kernel<KIND, VSAG_AMD_METRIC_L2>, kWave);
+        }
+    } else if (few) {
+        launch(rescore_valued_kernel<KIND, VSAG_AMD_METRIC_IP>, kValuedThreads);
     } else {
-        hipLaunchKernelGGL((rescore_valued_kernel<KIND, VSAG_AMD_METRIC_IP>), grid, dim3(kValuedThreads), lds, st, a, r);
+        launch(rescore_valued_wave_kernel<KIND, VSAG_AMD_METRIC_IP>, kWave);
     }
 }
 
@@ -1718,19 +1816,17 @@ launch_rescore_valued(const vsag_amd_store* s, const ScanArgs& a, uint64_t nq, u
     r.gate = gate;
     r.rows = s->rows;
     r.row_granules = s->row_granules;
-    const dim3 grid(static_cast<uint32_t>(nq));
     VA_CHECK_ARG(cap <= kValuedEach * kValuedThreads, "%u records a query are too many", cap);
-    const size_t lds = kValuedStage * sizeof(uint4) + S * sizeof(uint64_t) + cap * sizeof(uint32_t);
     if (s->kind == VSAG_AMD_KIND_SQ8_UNIFORM) {
-        launch_rescore_valued_m<VSAG_AMD_KIND_SQ8_UNIFORM>(s->metric, grid, lds, st, a, r);
+        launch_rescore_valued_m<VSAG_AMD_KIND_SQ8_UNIFORM>(s->metric, nq, st, a, r);
     } else if (s->kind == VSAG_AMD_KIND_SQ4_UNIFORM) {
-        launch_rescore_valued_m<VSAG_AMD_KIND_SQ4_UNIFORM>(s->metric, grid, lds, st, a, r);
+        launch_rescore_valued_m<VSAG_AMD_KIND_SQ4_UNIFORM>(s->metric, nq, st, a, r);
     } else if (s->kind == VSAG_AMD_KIND_SQ8) {
-        launch_rescore_valued_m<VSAG_AMD_KIND_SQ8>(s->metric, grid, lds, st, a, r);
+        launch_rescore_valued_m<VSAG_AMD_KIND_SQ8>(s->metric, nq, st, a, r);
     } else if (s->kind == VSAG_AMD_KIND_SQ4) {
-        launch_rescore_valued_m<VSAG_AMD_KIND_SQ4>(s->metric, grid, lds, st, a, r);
+        launch_rescore_valued_m<VSAG_AMD_KIND_SQ4>(s->metric, nq, st, a, r);
     } else {
-        launch_rescore_valued_m<VSAG_AMD_KIND_FP32>(s->metric, grid, lds, st, a, r);
+        launch_rescore_valued_m<VSAG_AMD_KIND_FP32>(s->metric, nq, st, a, r);
     }
     VA_HIP(hipGetLastError());
     return 0;
