@@ -101,7 +101,7 @@ int launch_ivf_i8(const vsag_amd_store* s, const ScanArgs& a, uint64_t nq, uint3
                   int32_t* tq, uint64_t* partial, uint32_t* partial_cnt, uint32_t* gate, const int32_t* buckets,
                   uint32_t* gpairs, uint32_t gpairs_cap, hipStream_t st);
 int prepare_queries(const vsag_amd_store* s, const float* queries, uint64_t nq, uint64_t nq_pad, const QueryLayout& ql,
-                    uint32_t* qtab, float* qmeta, uint8_t* qcodes, hipStream_t st);
+                    uint32_t* qtab, float* qmeta, uint8_t* qcodes, const FillJob* job, hipStream_t st);
 ScanArgs make_scan_args(const vsag_amd_store* s, const QueryLayout& ql, const uint32_t* qtab, const float* qmeta);
 void timing_begin(hipStream_t st);
 void timing_end(hipStream_t st);
@@ -112,23 +112,6 @@ int launch_merge_partials(const uint64_t* partial, const uint32_t* partial_cnt, 
                           hipStream_t st);
 
 // Up to five word arrays set in one launch.
-struct FillJob {
-    uint32_t* p[5];
-    uint32_t v[5];
-    uint64_t n[5];
-};
-
-__global__ void
-fill_jobs_kernel(FillJob j) {
-    uint64_t i = static_cast<uint64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-#pragma unroll
-    for (int a = 0; a < 5; ++a) {
-        if (i < j.n[a]) {
-            j.p[a][i] = j.v[a];
-        }
-    }
-}
-
 // Pairs of probe columns [p0, p1): how many queries probe each list.
 __global__ void
 count_pairs_kernel(const int32_t* buckets, uint64_t nq, uint32_t nprobe, uint32_t p0, uint32_t p1, uint32_t nlist,
@@ -801,23 +784,15 @@ vsag_amd_ivf_scan_topk_ex(const vsag_amd_store_t* s, const float* queries_dev, u
     }
     VA_CHECK_ARG(c.ok(), "workspace too small: need %zu bytes, got %zu", c.used, workspace_bytes);
 
-    // Row nq of the query tables is the all-zero row that idle slots of a query tile point at.
-    VA_TRY(prepare_queries(s, queries_dev, nq, nq + 1, p.ql, b.qtab, b.qmeta, b.qcodes, st));
-    ScanArgs a = make_scan_args(s, p.ql, b.qtab, b.qmeta);
     const uint64_t nlists1 = static_cast<uint64_t>(s->nlist) + 1;
     const uint64_t nslots_all = p.npairs * p.chunks_max;
     const uint64_t nseed = p.seeded ? nq * kcand : 0;
-    auto fill = [&](const FillJob& job) {
-        uint64_t most = 0;
-        for (uint64_t n : job.n) {
-            most = std::max(most, n);
-        }
-        hipLaunchKernelGGL(fill_jobs_kernel, dim3(blocks_for(most)), dim3(256), 0, st, job);
-    };
-    fill(FillJob{{b.bound, b.partial_cnt, b.counts, b.cursor, b.seed},
-                 {initial_bound(options), 0U, 0U, 0U, 0xFFFFFFFFU},
-                 {nq, nslots_all, p.chunked ? 0 : nlists1, p.chunked ? 0 : nlists1, nseed}});
-
+    const FillJob start{{b.bound, b.partial_cnt, b.counts, b.cursor, b.seed},
+                        {initial_bound(options), 0U, 0U, 0U, 0xFFFFFFFFU},
+                        {nq, nslots_all, p.chunked ? 0 : nlists1, p.chunked ? 0 : nlists1, nseed}};
+    // Row nq of the query tables is the all-zero row that idle slots of a query tile point at.
+    VA_TRY(prepare_queries(s, queries_dev, nq, nq + 1, p.ql, b.qtab, b.qmeta, b.qcodes, &start, st));
+    ScanArgs a = make_scan_args(s, p.ql, b.qtab, b.qmeta);
     IvfArgs v{};
     v.ids = s->ids_dev;
     v.list_tile = s->list_tile_dev;
@@ -881,8 +856,8 @@ vsag_amd_ivf_scan_topk_ex(const vsag_amd_store_t* s, const float* queries_dev, u
         }
         uint64_t pairs = nq * (p1 - p0);
         if (pass == 1 && !p.chunked) {
-            fill(FillJob{{b.counts, b.cursor, mfma ? b.gate : nullptr, nullptr, nullptr}, {0U, 0U, 0U, 0U, 0U},
-                         {nlists1, nlists1, mfma ? nq + 3 : 0, 0, 0}});
+            VA_TRY(launch_fill(FillJob{{b.counts, b.cursor, mfma ? b.gate : nullptr, nullptr, nullptr}, {0U, 0U, 0U, 0U, 0U},
+                                       {nlists1, nlists1, mfma ? nq + 3 : 0, 0, 0}}, st));
         }
         if (pass == 1 && mfma) {
             // Pairs grouped by list once; workgroups of 256 pairs for the matrix cores, then -- for the queries whose
@@ -1064,9 +1039,7 @@ vsag_amd_ivf_probed_codes(const vsag_amd_store_t* s, const int32_t* buckets_dev,
         VA_HIP(hipGetLastError());
         return 0;
     }
-    hipLaunchKernelGGL(fill_jobs_kernel, dim3(1), dim3(256), 0, st,
-                       FillJob{{reinterpret_cast<uint32_t*>(total_dev), nullptr, nullptr, nullptr, nullptr}, {0, 0, 0, 0, 0},
-                               {2, 0, 0, 0, 0}});
+    VA_TRY(launch_fill(FillJob{{reinterpret_cast<uint32_t*>(total_dev)}, {0}, {2}}, st));
     hipLaunchKernelGGL(probed_codes_kernel, dim3(blocks_for(nq * nprobe)), dim3(256), 0, st, buckets_dev, nq * nprobe,
                        s->nlist, s->list_sizes_dev, reinterpret_cast<unsigned long long*>(total_dev));
     VA_HIP(hipGetLastError());

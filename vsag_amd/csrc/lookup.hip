@@ -9,7 +9,7 @@ namespace vsag_amd {
 
 uint64_t rabitq_query_code_size(uint32_t dim, int metric, int query_bits);
 int prepare_queries(const vsag_amd_store* s, const float* queries, uint64_t nq, uint64_t nq_pad, const QueryLayout& ql,
-                    uint32_t* qtab, float* qmeta, uint8_t* qcodes, hipStream_t st);
+                    uint32_t* qtab, float* qmeta, uint8_t* qcodes, const FillJob* job, hipStream_t st);
 ScanArgs make_scan_args(const vsag_amd_store* s, const QueryLayout& ql, const uint32_t* qtab, const float* qmeta);
 
 struct LookupArgs {
@@ -304,7 +304,7 @@ vsag_amd_store_distances(const vsag_amd_store_t* s, const float* queries_dev, ui
     carve_lookup(c, s, nq, &b);
     VA_CHECK_ARG(c.ok(), "workspace too small: need %zu bytes, got %zu", c.used, workspace_bytes);
     const QueryLayout ql = query_layout(s);
-    VA_TRY(prepare_queries(s, queries_dev, nq, nq, ql, b.qtab, b.qmeta, b.qcodes, st));
+    VA_TRY(prepare_queries(s, queries_dev, nq, nq, ql, b.qtab, b.qmeta, b.qcodes, nullptr, st));
     ScanArgs a = make_scan_args(s, ql, b.qtab, b.qmeta);
     LookupArgs p{};
     p.ids = ids_dev;

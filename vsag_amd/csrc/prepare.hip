@@ -9,9 +9,39 @@ namespace vsag_amd {
 // ------------------------------------------------------------------ query preparation
 // One workgroup (256 threads) per query row; rows >= nq are written as zeros so that a partly filled
 // query tile computes harmless values.
+// It also sets the words that the scan behind it starts from (a launch of their own was 2 to 4 us of a call of one query:
+// on an ivf index of 300k x 128 fp32 98 -> 95 us).
+__device__ inline void
+fill_words(const FillJob& j) {
+    const uint64_t threads = static_cast<uint64_t>(gridDim.x) * blockDim.x;
+#pragma unroll
+    for (int a = 0; a < 5; ++a) {
+        for (uint64_t i = static_cast<uint64_t>(blockIdx.x) * blockDim.x + threadIdx.x; i < j.n[a]; i += threads) {
+            j.p[a][i] = j.v[a];
+        }
+    }
+}
+
 __global__ void __launch_bounds__(256)
-prepare_float_queries(FloatQueryArgs p) {
+prepare_float_queries(FloatQueryArgs p, FillJob j) {
+    fill_words(j);
     prepare_float_row(p, blockIdx.x);
+}
+
+__global__ void __launch_bounds__(256)
+fill_jobs_kernel(FillJob j) {
+    fill_words(j);
+}
+
+int
+launch_fill(const FillJob& job, hipStream_t st) {
+    uint64_t most = 1;
+    for (uint64_t n : job.n) {
+        most = n > most ? n : most;
+    }
+    hipLaunchKernelGGL(fill_jobs_kernel, dim3(static_cast<uint32_t>(div_up(most, 256))), dim3(256), 0, st, job);
+    VA_HIP(hipGetLastError());
+    return 0;
 }
 
 // Uniform kinds: the query has been encoded with the base encoder (ProcessQueryImpl = EncodeOneImpl,
@@ -255,10 +285,13 @@ prepare_rabitq_f32_queries(const uint8_t* qcodes, uint64_t nq, uint32_t qcode_si
 
 // Runs ProcessQueryImpl of the store's quantizer for nq raw queries and fills the scan tables.  `qcodes` is
 // query_staging_bytes(s, nq) of device memory (the encoded queries, then the encoders' scratch): nothing is
-// allocated here.
+// allocated here.  `job` (or null): words to set, by the same launch where there is one launch.
 int
 prepare_queries(const vsag_amd_store* s, const float* queries, uint64_t nq, uint64_t nq_pad, const QueryLayout& ql,
-                uint32_t* qtab, float* qmeta, uint8_t* qcodes, hipStream_t st) {
+                uint32_t* qtab, float* qmeta, uint8_t* qcodes, const FillJob* job, hipStream_t st) {
+    if (job != nullptr && s->kind != VSAG_AMD_KIND_FP32 && s->kind != VSAG_AMD_KIND_SQ8 && s->kind != VSAG_AMD_KIND_SQ4) {
+        VA_TRY(launch_fill(*job, st));
+    }
     dim3 grid(static_cast<uint32_t>(nq_pad));
     float* scratch = query_scratch_bytes(s, nq) == 0 ? nullptr :
                      reinterpret_cast<float*>(qcodes + round_up(query_code_bytes(s, nq), 256));
@@ -266,7 +299,8 @@ prepare_queries(const vsag_amd_store* s, const float* queries, uint64_t nq, uint
         case VSAG_AMD_KIND_FP32:
         case VSAG_AMD_KIND_SQ8:
         case VSAG_AMD_KIND_SQ4:
-            hipLaunchKernelGGL(prepare_float_queries, grid, dim3(256), 0, st, float_query_args(s, queries, nq, ql, qtab, qmeta));
+            hipLaunchKernelGGL(prepare_float_queries, grid, dim3(256), 0, st, float_query_args(s, queries, nq, ql, qtab, qmeta),
+                               job != nullptr ? *job : FillJob{});
             break;
         case VSAG_AMD_KIND_SQ4_UNIFORM:
         case VSAG_AMD_KIND_SQ8_UNIFORM: {

@@ -16,7 +16,7 @@ namespace vsag_amd {
 void timing_begin(hipStream_t st);
 void timing_end(hipStream_t st);
 int prepare_queries(const vsag_amd_store* s, const float* queries, uint64_t nq, uint64_t nq_pad, const QueryLayout& ql,
-                    uint32_t* qtab, float* qmeta, uint8_t* qcodes, hipStream_t st);
+                    uint32_t* qtab, float* qmeta, uint8_t* qcodes, const FillJob* job, hipStream_t st);
 ScanArgs make_scan_args(const vsag_amd_store* s, const QueryLayout& ql, const uint32_t* qtab, const float* qmeta);
 uint64_t rabitq_query_code_size(uint32_t dim, int metric, int query_bits);
 
@@ -46,18 +46,6 @@ tighten_bound_kernel(const float* dists, uint32_t k, uint64_t nq, uint32_t* boun
                 bound[q] = o;
             }
         }
-    }
-}
-
-// Per query: no bound yet, no seeds yet.
-__global__ void
-reset_queries_kernel(uint32_t* bound, uint32_t bound0, uint64_t nq, uint32_t* seed, uint64_t nseed) {
-    uint64_t i = static_cast<uint64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (i < nq) {
-        bound[i] = bound0;
-    }
-    if (i < nseed) {
-        seed[i] = 0xFFFFFFFFU;
     }
 }
 
@@ -1302,12 +1290,18 @@ flat_scan_call(const vsag_amd_store_t* s, const float* queries_dev, uint64_t nq,
     const bool contraction = cp.contraction && !ranged;
     const ScanPlan& p = cp.all;
 
+    const uint64_t nseed = b.seed != nullptr ? nq * k : 0;
     FloatQueryArgs raw{};
     if (contraction && cp.b16 && !cp.one &&
         (s->kind == VSAG_AMD_KIND_FP32 || s->kind == VSAG_AMD_KIND_SQ8 || s->kind == VSAG_AMD_KIND_SQ4)) {
         raw = float_query_args(s, queries_dev, nq, p.ql, b.qtab, b.qmeta);  // (that route's first launch prepares them)
     } else {
-        VA_TRY(prepare_queries(s, queries_dev, nq, p.nq_pad, p.ql, b.qtab, b.qmeta, b.qcodes, st));
+        // Per query: no bound yet, no seeds yet (the table and the one-query route start from neither, the bf16 route's first
+        // launch sets them).
+        const bool starts = !(cp.table && plain) && !(cp.one && s->ntiles == cp.one_tiles) &&
+                            !(contraction && cp.b16 && s->ntiles != 0);
+        const FillJob start{{b.bound, b.seed}, {initial_bound(options), 0xFFFFFFFFU}, {nq, nseed}};
+        VA_TRY(prepare_queries(s, queries_dev, nq, p.nq_pad, p.ql, b.qtab, b.qmeta, b.qcodes, starts ? &start : nullptr, st));
     }
     if (cp.table && plain) {
         const ScanArgs ta = make_scan_args(s, p.ql, b.qtab, b.qmeta);
@@ -1343,10 +1337,8 @@ flat_scan_call(const vsag_amd_store_t* s, const float* queries_dev, uint64_t nq,
         tl_last_bytes = s->ntiles * s->G * kWave * kGranule;
         return 0;
     }
-    const uint64_t nseed = b.seed != nullptr ? nq * k : 0;
-    if (!contraction || !cp.b16 || s->ntiles == 0) {  // (that route's first launch does it)
-        hipLaunchKernelGGL(reset_queries_kernel, dim3(static_cast<uint32_t>(div_up(nq > nseed ? nq : nseed, 256))), dim3(256),
-                           0, st, b.bound, initial_bound(options), nq, b.seed, nseed);
+    if (raw.q != nullptr && s->ntiles == 0) {  // (that route's first launch does it, but does not run)
+        VA_TRY(launch_fill(FillJob{{b.bound, b.seed}, {initial_bound(options), 0xFFFFFFFFU}, {nq, nseed}}, st));
     }
     ScanArgs a = make_scan_args(s, p.ql, b.qtab, b.qmeta);
     uint32_t nslots = 0;

@@ -131,6 +131,14 @@ struct QueryLayout {
 };
 
 QueryLayout query_layout(const vsag_amd_store* s);
+
+// Up to five arrays of words that a launch sets before others use them: n[a] words at p[a] become v[a].
+struct FillJob {
+    uint32_t* p[5];
+    uint32_t v[5];
+    uint64_t n[5];
+};
+int launch_fill(const FillJob& job, hipStream_t st);
 // Device bytes prepare_queries needs behind its `qcodes` pointer for nq queries: the encoded queries of the kinds
 // that encode them, then whatever their encoders use as scratch.
 size_t query_staging_bytes(const vsag_amd_store* s, uint64_t nq);
