@@ -837,3 +837,20 @@ def test_rescoring_at_the_edges_of_its_pieces(lib, modes, kind, metric, d, k):
         assert tile in (64, 128), "the bf16 pass did not run"
     assert same(plain, fast)
     st.destroy()
+
+
+@pytest.mark.parametrize("kind,metric", [("fp32", orc.L2), ("fp32", orc.IP), ("sq8_uniform", orc.L2), ("sq4_uniform", orc.IP)])
+def test_either_form_of_rescoring(lib, modes, kind, metric):
+    """512 queries have a workgroup each, 513 a wave."""
+    rng = np.random.default_rng(11)
+    n, d, k = 3000, 200, 33
+    x, means = gaussian_mixture(rng, n, d, 15, 0.05)
+    x[500:620] = x[499]
+    q, _ = gaussian_mixture(rng, 513, d, 15, 0.05, means=means)
+    q[7] = x[499]
+    st = _store_of(kind, metric, x, rng)
+    for nq in (512, 513):
+        plain, fast, tile = modes(st, q[:nq], k, 1)
+        assert tile in (64, 128), "the bf16 pass did not run"
+        assert same(plain, fast)
+    st.destroy()
