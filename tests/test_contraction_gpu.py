@@ -17,11 +17,11 @@ pytestmark = pytest.mark.gpu
 def modes(lib):
     L = capi.load_library()
 
-    def both(store, q, k, mode=1):
+    def both(store, q, k, mode=1, deny=None):
         capi.check(L.vsag_amd_set_scan_contraction(-1))
-        plain = store.flat_scan(q, k)
+        plain = store.flat_scan(q, k, deny)
         capi.check(L.vsag_amd_set_scan_contraction(mode))
-        fast = store.flat_scan(q, k)
+        fast = store.flat_scan(q, k, deny)
         tile = capi.C.c_int()
         L.vsag_amd_last_scan_info(capi.C.byref(tile), None, None)
         capi.check(L.vsag_amd_set_scan_contraction(0))
@@ -853,4 +853,23 @@ def test_either_form_of_rescoring(lib, modes, kind, metric):
         plain, fast, tile = modes(st, q[:nq], k, 1)
         assert tile in (64, 128), "the bf16 pass did not run"
         assert same(plain, fast)
+    st.destroy()
+
+
+@pytest.mark.parametrize("kind,metric,d", [("fp32", orc.L2, 100), ("fp32", orc.IP, 37), ("sq8", orc.L2, 100),
+                                           ("sq4", orc.IP, 132), ("sq8_uniform", orc.L2, 200), ("sq4_uniform", orc.IP, 200)])
+@pytest.mark.parametrize("nq", [33, 513])
+def test_many_neighbours_behind_the_bf16_pass(lib, modes, kind, metric, d, nq):
+    """Beyond 128 neighbours a query has room for more records than a workgroup of the rescoring holds in registers; mode 1 asks
+    for the bf16 pass all the same (of sq8 and sq4 stores under a mask)."""
+    rng = np.random.default_rng(d + nq)
+    n = 9000
+    x, means = gaussian_mixture(rng, n, d, 12, 0.05)
+    q, _ = gaussian_mixture(rng, nq, d, 12, 0.05, means=means)
+    st = _store_of(kind, metric, x, rng)
+    deny = rng.random(n) < 0.1 if kind in ("sq8", "sq4") else None
+    for k in (129, 256, 1024):
+        plain, fast, tile = modes(st, q, k, 1, deny)
+        assert tile in (64, 128), "the bf16 pass did not run"
+        assert same(plain, fast), k
     st.destroy()

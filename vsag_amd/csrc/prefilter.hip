@@ -697,7 +697,8 @@ rescore_kernel(ScanArgs a, RescoreArgs r) {
 // has v above a_k + slack stands behind k others: of the hundreds of records, the k and a handful that are left are rescored.
 //
 // Two forms.  With many queries, a wave per query, whose lanes read their candidates' rows up to 16 granules ahead: small
-// workgroups, of which many share a compute unit.  With few (kValuedFewQueries), a workgroup per query, below.  Calls with
+// workgroups, of which many share a compute unit.  With few (kValuedFewQueries), a workgroup per query, below, which holds the
+// records of a query in registers: where a query has room for more than those (k beyond 128), a wave too.  Calls with
 // either, us: 2000 queries against 100k x 128 fp32 248 / 254, 10000 1012 / 1097, 9693 against 115k x 768 sq4_uniform 2300 / 2414;
 // 32 against 100k x 768 fp32 185 / 170.
 template <int KIND, int METRIC>
@@ -1727,7 +1728,7 @@ template <int KIND>
 static void
 launch_rescore_valued_m(int metric, uint64_t nq, hipStream_t st, const ScanArgs& a, const RescoreArgs& r) {
     const dim3 grid(static_cast<uint32_t>(nq));
-    const bool few = nq <= kValuedFewQueries;
+    const bool few = nq <= kValuedFewQueries && r.cap <= kValuedEach * kValuedThreads;
     const size_t lds = few ? kValuedStage * sizeof(uint4) + r.S * sizeof(uint64_t) + r.cap * sizeof(uint32_t)
                            : r.S * sizeof(uint64_t) + (128 + 256) * sizeof(uint32_t);
     auto launch = [&](auto kernel, uint32_t threads) { hipLaunchKernelGGL(kernel, grid, dim3(threads), lds, st, a, r); };
@@ -1816,7 +1817,6 @@ launch_rescore_valued(const vsag_amd_store* s, const ScanArgs& a, uint64_t nq, u
     r.gate = gate;
     r.rows = s->rows;
     r.row_granules = s->row_granules;
-    VA_CHECK_ARG(cap <= kValuedEach * kValuedThreads, "%u records a query are too many", cap);
     if (s->kind == VSAG_AMD_KIND_SQ8_UNIFORM) {
         launch_rescore_valued_m<VSAG_AMD_KIND_SQ8_UNIFORM>(s->metric, nq, st, a, r);
     } else if (s->kind == VSAG_AMD_KIND_SQ4_UNIFORM) {
