@@ -873,3 +873,20 @@ def test_many_neighbours_behind_the_bf16_pass(lib, modes, kind, metric, d, nq):
         assert tile in (64, 128), "the bf16 pass did not run"
         assert same(plain, fast), k
     st.destroy()
+
+
+@pytest.mark.parametrize("kind,metric,d,mode,tiles", [("fp32", orc.L2, 100, 1, (64, 128)), ("fp32", orc.IP, 60, 2, (128,)),
+                                                      ("sq8", orc.L2, 100, 1, (256,)), ("sq4_uniform", orc.IP, 64, 1, (256,))])
+def test_odd_numbers_of_neighbours(lib, modes, kind, metric, d, mode, tiles):
+    """The keys that the rescoring ranks stand behind the k kept ones, with an odd k on 8 bytes only (up to 32 and from 129 to 160
+    neighbours): each route that ranks them, with a wave per query."""
+    rng = np.random.default_rng(d)
+    n, nq = 6000, 513
+    x, means = gaussian_mixture(rng, n, d, 60, 0.05)
+    q, _ = gaussian_mixture(rng, nq, d, 60, 0.05, means=means)
+    st = _store_of(kind, metric, x, rng)
+    for k in (1, 2, 5, 21, 31, 32, 33, 129, 131, 160):
+        plain, fast, tile = modes(st, q, k, mode)
+        assert tile in tiles, "the matrix cores did not run"
+        assert same(plain, fast), k
+    st.destroy()

@@ -515,18 +515,14 @@ struct RescoreKeys {
         if (admitted > k && !flushed && cnt <= kRankedKeys) {
             const uint64_t* all = keys + pend;
             // Keys that came once: each goes where the number of smaller ones says (28 steps of a sorting network over 128
-            // keys took 5.5 us, the counting takes one).
+            // keys took 5.5 us, the counting takes one).  Read as 64-bit keys: with an odd k the first of them lies on 8 bytes.
             for (uint32_t i = lane; i < cnt; i += kWave) {
                 const uint64_t mine = all[i];
                 uint32_t rank = 0;
-                const uint4* pairs = reinterpret_cast<const uint4*>(all);
-#pragma unroll 8
-                for (uint32_t j = 0; j < cnt / 2; ++j) {
-                    const uint4 v = pairs[j];
-                    const uint64_t x = (static_cast<uint64_t>(v.y) << 32) | v.x, y = (static_cast<uint64_t>(v.w) << 32) | v.z;
-                    rank += (x < mine ? 1U : 0U) + (y < mine ? 1U : 0U);
+#pragma unroll 16
+                for (uint32_t j = 0; j < cnt; ++j) {
+                    rank += all[j] < mine ? 1U : 0U;
                 }
-                rank += (cnt & 1U) != 0 && all[cnt - 1] < mine ? 1U : 0U;
                 if (rank < k && mine != kInfKey) {
                     r.partial[list * k + rank] = mine;
                     if (rank + 1 == k) {
