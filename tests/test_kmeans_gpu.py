@@ -231,6 +231,8 @@ def _routed_data(kind, n, d, k):
                                         ("outliers", 62001, 260, 256), ("plain", 20011, 100, 2049), ("plain", 20011, 132, 1601),
                                         ("plain", 62001, 196, 400), ("exact", 20011, 132, 1601), ("crowd", 20011, 101, 2049),
                                         ("crowd", 70001, 192, 320), ("holes", 20011, 101, 2049), ("holes", 70001, 192, 320),
+                                        # one, two and three stages of 64 dimensions
+                                        ("plain", 81921, 33, 1601), ("plain", 65537, 65, 1024), ("plain", 65537, 129, 512),
                                         # more rows than are rounded at a time (65536)
                                         ("holes", 70001, 1000, 260), ("outliers", 70001, 1000, 260),
                                         # the rows behind a slab of open ones are not pre-selected

@@ -549,8 +549,12 @@ kmeans_h16_kernel(KmeansH16Args p) {
     using Yes = std::true_type;
     using No = std::false_type;
     fetch(0);
-    touch(stages > 1 ? 1 : 0);
-    landed(Yes{});
+    if (stages > 1) {
+        touch(1);
+        landed(Yes{});
+    } else {
+        landed(No{});  // (a wave must not end with a write to LDS on its way)
+    }
     operands(lds, 0, 0);
     // (The barriers to the scheduler keep every step's reads a step ahead of its products, where it would read them late to
     // save registers.)
