@@ -824,7 +824,8 @@ def test_settings_of_one_store_leave_the_others_alone(lib):
 @pytest.mark.parametrize("k", [1, 31, 33, 128])
 def test_rescoring_at_the_edges_of_its_pieces(lib, modes, kind, metric, d, k):
     """Candidates on both sides of 32 and 64, rows a granule short of and beyond the 32 or 64 that are in LDS at a time; rows
-    that are copies of each other, so that more candidates than k are equal to the last bit."""
+    that are copies of each other, so that more candidates than k are equal to the last bit.  (Mode 1 sends sq8 and sq4 stores
+    through this pass under a mask.)"""
     rng = np.random.default_rng(d + k)
     n, nq = 2100, 17
     x, means = gaussian_mixture(rng, n, d, 12, 0.05)
@@ -832,9 +833,12 @@ def test_rescoring_at_the_edges_of_its_pieces(lib, modes, kind, metric, d, k):
     q, _ = gaussian_mixture(rng, nq, d, 12, 0.05, means=means)
     q[0] = x[99]
     st = _store_of(kind, metric, x, rng)
-    plain, fast, tile = modes(st, q, k, 1)
-    if kind != "sq8" and kind != "sq4":
-        assert tile in (64, 128), "the bf16 pass did not run"
+    if kind in ("sq8", "sq4"):
+        plain, fast, _ = modes(st, q, k, 1)
+        assert same(plain, fast)
+    deny = rng.random(n) < 0.03 if kind in ("sq8", "sq4") else None
+    plain, fast, tile = modes(st, q, k, 1, deny)
+    assert tile in (64, 128), "the bf16 pass did not run"
     assert same(plain, fast)
     st.destroy()
 
