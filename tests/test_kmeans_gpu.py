@@ -419,8 +419,11 @@ def test_run_with_the_fp16_preselection_keeps_its_rows(lib, n, d, k, iters):
 
 
 @pytest.mark.parametrize("n,k,kind", [(1, 1, "even"), (63, 2, "even"), (1023, 3, "even"), (1024, 64, "even"), (1025, 65, "even"),
-                                      (5000, 98, "skewed"), (5000, 98, "runs"), (40000, 4097, "even"), (40000, 16384, "even"),
-                                      (40000, 16385, "even"), (70000, 1000, "one")])
+                                      (5000, 98, "skewed"), (5000, 98, "runs"), (40000, 4097, "even"),
+                                      # the most labels of the counting sort (five units of 8256 rows, their table fits in 2 n
+                                      # words), a table too large, and more labels: the general sort
+                                      (41280, 16384, "even"), (41280, 16384, "skewed"), (40000, 16384, "even"),
+                                      (40000, 16385, "even"), (41280, 16385, "even"), (70000, 1000, "one")])
 def test_update_groups_the_rows_of_every_label(lib, n, k, kind):
     """Rows grouped by label around the edges of the counting sort's units and label bits: every mean is the sequential fp32 sum
     of the rows in row order, bit for bit, which holds only if the grouping is stable and complete."""
