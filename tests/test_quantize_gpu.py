@@ -1,6 +1,7 @@
 """Parity of quantizer training / encoding on the device against the CPU checker: codes are compared bit
 for bit, trained bounds exactly (they are order statistics of the same deterministic sample)."""
 import ctypes as C
+import math
 
 import numpy as np
 import pytest
@@ -404,6 +405,34 @@ def test_sq_encode_at_the_levels_edges(lib, bits, metric, n, d):
     xb, lbb, dfb, out = dev(x), dev(lb), dev(diff), capi.DeviceBuffer(n * code_size)
     capi.check(L.vsag_amd_sq_encode(xb.ptr, n, d, bits, metric, lbb.ptr, dfb.ptr, out.ptr, None))
     assert np.array_equal(out.to_numpy(np.uint8, (n, code_size)), orc.sq_encode(x, bits, lb, diff, metric))
+
+
+@pytest.mark.parametrize("bits", [8, 4])
+@pytest.mark.parametrize("metric", [orc.L2, orc.COSINE])
+@pytest.mark.parametrize("d,shift", [(100, 0), (100, 4), (130, 0), (260, 8), (1020, 0), (257, 0), (4, 0)])
+def test_sq_encode_on_both_sides_of_four_runs_a_thread(lib, bits, metric, d, shift):
+    """As many rows as four runs a thread begin with (a workgroup's threads are a multiple of the words after which dimensions
+    repeat) and one less; dimensions that are a multiple of four and not, bounds that lie on 16 bytes and not."""
+    if bits == 4 and d % 2 != 0:
+        pytest.skip("rows of no whole number of bytes have a kernel of their own")
+    L = lib.load_library()
+    kdims = 32 // bits
+    period = d // math.gcd(d, kdims)
+    threads = period if period > 256 else 256 // period * period if period > 1 else 256
+    words = 4 * threads * (3072 if metric == orc.COSINE else 1536)
+    rows = -(-(words * kdims - kdims + 1) // d)
+    rng = np.random.default_rng(d + bits)
+    lb, diff = rng.normal(0, 0.2, d).astype(np.float32), rng.uniform(0.5, 2, d).astype(np.float32)
+    x = rng.random((rows + 3, d), dtype=np.float32)
+    want = orc.sq_encode(x, bits, lb, diff, metric)
+    pad = np.zeros(shift // 4, np.float32)
+    lbb, dfb = dev(np.concatenate([pad, lb])), dev(np.concatenate([pad, diff]))
+    for n in (rows + 3, rows, rows - 1):
+        size = want[:n].nbytes
+        xb, out = dev(x[:n]), dev(np.full(size + 8, 0x5A, np.uint8))
+        capi.check(L.vsag_amd_sq_encode(xb.ptr, n, d, bits, metric, lbb.ptr + shift, dfb.ptr + shift, out.ptr, None))
+        got = out.to_numpy(np.uint8, (size + 8,))
+        assert np.array_equal(got[:size].reshape(want[:n].shape), want[:n]) and (got[size:] == 0x5A).all(), n
 
 
 @pytest.mark.parametrize("n", [32768, 32769, 65536, 65537, 100352, 100353])

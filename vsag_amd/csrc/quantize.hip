@@ -4,6 +4,7 @@
 // that arithmetic is order-dependent (running fp32 sums are kept in element order, products and sums are
 // not fused: this translation unit is compiled with -ffp-contract=off).
 #include <cfloat>
+#include <type_traits>
 
 #include "common.h"
 #include "topk.h"
@@ -157,9 +158,15 @@ sq_level_by_inverse(float v, float lb, float diff, float inv, float levels) {
 // stores at any dimension.  A workgroup of `blockDim` threads takes RUNS x blockDim consecutive runs; with RUNS > 1 blockDim
 // runs are whole rows, so a thread meets the same dimensions in each of its runs and keeps their bounds in registers, with
 // RUNS loads on their way.  What bounds it is memory: 1M x 128 rows to sq8 466 us with a thread per byte, 138 us with a run
-// per thread and a division per value, 132 us without the division, and 108 us with short workgroups of four runs a
-// thread that pass the caches by (2048 long-lived ones, loads and stores as they come: 132; the reading alone 72).
-template <int BITS, bool NORM, int RUNS>
+// per thread and a division per value, 132 us without the division, and 102 us with short workgroups of four runs a
+// thread that pass the caches by (2048 long-lived ones, loads and stores as they come: 132; the reading alone 72).  Past the
+// caches go neither the two loads of a run of sq4, which share their lines (161 -> 148 us), nor rows whose norms were taken just
+// before (20 000 x 960 to sq8 under cosine: 60 -> 52 us with the norms).
+//
+// VEC: the dimension is a multiple of four, so bounds (then on 16 bytes) come four a load and a norm serves four values.  In
+// single words they were more loads than the rows: 1M x 128 to sq4 148 us and 101 so (134 with a run per thread), 427k x 300 under
+// cosine 302 and 237 with the norms (261).
+template <int BITS, bool NORM, bool VEC, int RUNS>
 __global__ void __launch_bounds__(1024)
 sq_encode_kernel(const float* x, uint64_t total, uint32_t dim, const float* lb, const float* diff, const float* norms,
                  uint8_t* codes) {
@@ -177,11 +184,16 @@ sq_encode_kernel(const float* x, uint64_t total, uint32_t dim, const float* lb, 
         const uint64_t at = run + r * blockDim.x;
 #pragma unroll
         for (uint32_t e = 0; e < kDims; e += 4) {
-            float4_v a = {0.0F, 0.0F, 0.0F, 0.0F};
             if (at < whole) {
-                a = __builtin_nontemporal_load(reinterpret_cast<const float4_v*>(x + at * kDims + e));
+                const float4_v* from = reinterpret_cast<const float4_v*>(x + at * kDims + e);
+                const float4_v a = BITS == 8 && !NORM && RUNS > 1 ? __builtin_nontemporal_load(from) : *from;
+                v[r][e] = a.x, v[r][e + 1] = a.y, v[r][e + 2] = a.z, v[r][e + 3] = a.w;
+            } else {
+#pragma unroll
+                for (uint32_t u = e; u < e + 4; ++u) {
+                    v[r][u] = at * kDims + u < total ? x[at * kDims + u] : 0.0F;
+                }
             }
-            v[r][e] = a.x, v[r][e + 1] = a.y, v[r][e + 2] = a.z, v[r][e + 3] = a.w;
         }
     }
     // Row and dimension of the first value, from those of the workgroup (wave-uniform).
@@ -193,18 +205,38 @@ sq_encode_kernel(const float* x, uint64_t total, uint32_t dim, const float* lb, 
     uint32_t row_off[kDims];
     {
         uint32_t d = off % dim, r = 0;
+        constexpr uint32_t kStep = VEC ? 4 : 1;
 #pragma unroll
-        for (uint32_t e = 0; e < kDims; ++e) {
-            lo[e] = lb[d];
-            df[e] = diff[d];
-            inv[e] = sq_inverse(df[e]);
+        for (uint32_t e = 0; e < kDims; e += kStep) {
+            if constexpr (VEC) {
+                const float4_v l4 = *reinterpret_cast<const float4_v*>(lb + d), f4 = *reinterpret_cast<const float4_v*>(diff + d);
+                lo[e] = l4.x, lo[e + 1] = l4.y, lo[e + 2] = l4.z, lo[e + 3] = l4.w;
+                df[e] = f4.x, df[e + 1] = f4.y, df[e + 2] = f4.z, df[e + 3] = f4.w;
+            } else {
+                lo[e] = lb[d];
+                df[e] = diff[d];
+            }
             row_off[e] = r;
-            ++d;
+            d += kStep;
             r += d == dim ? 1 : 0;
             d = d == dim ? 0 : d;
         }
+#pragma unroll
+        for (uint32_t e = 0; e < kDims; ++e) {
+            inv[e] = sq_inverse(df[e]);
+        }
     }
     const float levels = static_cast<float>((1 << BITS) - 1);
+    float nrm[RUNS][kDims / 4];
+    if constexpr (NORM && VEC) {
+#pragma unroll
+        for (uint32_t r = 0; r < RUNS; ++r) {
+#pragma unroll
+            for (uint32_t e = 0; e < kDims; e += 4) {
+                nrm[r][e / 4] = (run + r * blockDim.x) * kDims + e < total ? norms[row + r * step_rows + row_off[e]] : 1.0F;
+            }
+        }
+    }
 #pragma unroll
     for (uint32_t r = 0; r < RUNS; ++r) {
         const uint64_t at = run + r * blockDim.x;
@@ -212,14 +244,30 @@ sq_encode_kernel(const float* x, uint64_t total, uint32_t dim, const float* lb, 
             break;
         }
         const uint32_t values = at < whole ? kDims : static_cast<uint32_t>(total - at * kDims);
+        float each[kDims];
+        if constexpr (NORM && !VEC) {
+            if (at < whole) {
+#pragma unroll
+                for (uint32_t e = 0; e < kDims; ++e) {
+                    each[e] = norms[row + r * step_rows + row_off[e]];
+                }
+            } else {
+#pragma unroll
+                for (uint32_t e = 0; e < kDims; ++e) {
+                    each[e] = e < values ? norms[row + r * step_rows + row_off[e]] : 1.0F;
+                }
+            }
+        }
         uint32_t word = 0;
 #pragma unroll
         for (uint32_t e = 0; e < kDims; ++e) {
-            float value = at < whole || e >= values ? v[r][e] : x[at * kDims + e];
+            float value = v[r][e];
             if constexpr (NORM) {
-                value /= e < values ? norms[row + r * step_rows + row_off[e]] : 1.0F;
+                value /= VEC ? nrm[r][e / 4] : each[e];
             }
-            word |= sq_level_by_inverse(value, lo[e], df[e], inv[e], levels) << (e * BITS);
+            // (a reciprocal is a division too: with one value to a dimension there is nothing to save)
+            const uint32_t level = RUNS > 1 ? sq_level_by_inverse(value, lo[e], df[e], inv[e], levels) : sq_level(value, lo[e], df[e], levels);
+            word |= level << (e * BITS);
         }
         if (at < whole) {
             __builtin_nontemporal_store(word, reinterpret_cast<uint32_t*>(codes) + at);
@@ -232,16 +280,18 @@ sq_encode_kernel(const float* x, uint64_t total, uint32_t dim, const float* lb, 
 }
 
 // The workgroup of the kernel above: threads, runs per thread.  After `period` runs the dimensions repeat; workgroups are
-// multiples of it with four runs where that makes at most 1024 threads, and one run otherwise (odd dimensions beyond 1024).
+// multiples of it with four runs where that makes at most 1024 threads and six workgroups a compute unit (twelve under
+// cosine, whose divisions make the threads longer), and one run otherwise: odd dimensions beyond 1024, and few rows, which four
+// runs leave on a fourth of the chip (20 000 x 128 sq8 6.0 us, 5.0 with one; 99 000 x 128 sq4 under cosine 30.9 and 28.4).
 static void
-sq_encode_shape(uint32_t dim, uint32_t kdims, uint32_t* threads, uint32_t* runs) {
+sq_encode_shape(uint32_t dim, uint32_t kdims, uint64_t words, bool norm, uint32_t* threads, uint32_t* runs) {
     uint32_t g = kdims;
     while (dim % g != 0) {
         g /= 2;
     }
     const uint32_t period = dim / g;
-    *runs = period <= 1024 ? 4 : 1;
     *threads = period > 1024 || period == 1 ? 256 : period > 256 ? period : 256 / period * period;
+    *runs = period <= 1024 && words >= 4ull * *threads * (norm ? 3072 : 1536) ? 4 : 1;
 }
 
 // The same with one thread per code byte: sq4 codes of an odd dimension (the last byte of a row holds one value), and
@@ -1879,19 +1929,27 @@ vsag_amd_sq_encode(const float* x_dev, uint64_t n, uint32_t dim, int bits, int m
                            n, dim, bits, lower_bound_dev, diff_dev, norms, code_size, codes_dev);
     } else {
         uint32_t block = 0, runs = 0;
-        sq_encode_shape(dim, 32U / bits, &block, &runs);
+        sq_encode_shape(dim, 32U / bits, threads, norms != nullptr, &block, &runs);
         auto launch = [&](auto kernel) {
             hipLaunchKernelGGL(kernel, dim3(static_cast<uint32_t>(div_up(threads, static_cast<uint64_t>(block) * runs))),
                                dim3(block), 0, st, x_dev, total, dim, lower_bound_dev, diff_dev, norms, codes_dev);
         };
-        if (bits == 8 && runs == 4) {
-            launch(norms != nullptr ? sq_encode_kernel<8, true, 4> : sq_encode_kernel<8, false, 4>);
-        } else if (bits == 8) {
-            launch(norms != nullptr ? sq_encode_kernel<8, true, 1> : sq_encode_kernel<8, false, 1>);
-        } else if (runs == 4) {
-            launch(norms != nullptr ? sq_encode_kernel<4, true, 4> : sq_encode_kernel<4, false, 4>);
+        const bool vec = (dim & 3U) == 0 && ((reinterpret_cast<uintptr_t>(lower_bound_dev) |
+                                              reinterpret_cast<uintptr_t>(diff_dev)) & 15U) == 0;
+        auto pick = [&](auto bits_c, auto runs_c) {
+            constexpr int kBits = decltype(bits_c)::value, kRuns = decltype(runs_c)::value;
+            if (norms != nullptr) {
+                launch(vec ? sq_encode_kernel<kBits, true, true, kRuns> : sq_encode_kernel<kBits, true, false, kRuns>);
+            } else {
+                launch(vec ? sq_encode_kernel<kBits, false, true, kRuns> : sq_encode_kernel<kBits, false, false, kRuns>);
+            }
+        };
+        if (bits == 8) {
+            runs == 4 ? pick(std::integral_constant<int, 8>{}, std::integral_constant<int, 4>{})
+                      : pick(std::integral_constant<int, 8>{}, std::integral_constant<int, 1>{});
         } else {
-            launch(norms != nullptr ? sq_encode_kernel<4, true, 1> : sq_encode_kernel<4, false, 1>);
+            runs == 4 ? pick(std::integral_constant<int, 4>{}, std::integral_constant<int, 4>{})
+                      : pick(std::integral_constant<int, 4>{}, std::integral_constant<int, 1>{});
         }
     }
     VA_HIP(hipGetLastError());
