@@ -435,6 +435,11 @@ def test_sq_encode_on_both_sides_of_four_runs_a_thread(lib, bits, metric, d, shi
         assert np.array_equal(got[:size].reshape(want[:n].shape), want[:n]) and (got[size:] == 0x5A).all(), n
 
 
+@pytest.mark.parametrize("n", [1024, 8192, 8193, 16384, 16385, 49152, 49153, 81920, 81921])
+def test_sq_train_at_the_ends_of_the_finer_register_tiers(lib, n):
+    test_sq_train_at_the_ends_of_the_register_tiers(lib, n)
+
+
 @pytest.mark.parametrize("n", [32768, 32769, 65536, 65537, 100352, 100353])
 def test_sq_train_at_the_ends_of_the_register_tiers(lib, n):
     rng = np.random.default_rng(n)

@@ -1528,10 +1528,16 @@ struct ColumnValues {
     __device__ inline void
     load() {
         if constexpr (REGS > 0) {
+            const uint32_t end = static_cast<uint32_t>(count);
 #pragma unroll
-            for (uint32_t u = 0; u < REGS; ++u) {
-                const uint32_t i = threadIdx.x + u * kBoundThreads;
-                v[u] = vals[i < static_cast<uint32_t>(count) ? i : static_cast<uint32_t>(count) - 1];
+            for (uint32_t u0 = 0; u0 < REGS; u0 += 16) {
+                if (u0 == 0 || u0 * kBoundThreads < end) {  // (the same for all threads)
+#pragma unroll
+                    for (uint32_t u = u0; u < u0 + 16 && u < REGS; ++u) {
+                        const uint32_t i = threadIdx.x + u * kBoundThreads;
+                        v[u] = vals[i < end ? i : end - 1];
+                    }
+                }
             }
         }
     }
@@ -1673,9 +1679,11 @@ kth_key_in(const float* vals, uint64_t count, uint32_t base, uint32_t last, uint
 // serves, and bins of the float's bits put nearly all values of a column into a few of them, where the atomics of a wave
 // wait for each other --; that one histogram places both order statistics in bins of a few hundred values, which are ranked
 // in LDS: three passes over the column, whose values stay in registers where 1024 threads hold them (up to REGS each: 98
-// for the default sample of 100 000) -- a workgroup per column leaves every second compute unit idle at 128 dimensions, and
-// the other half waited for the same 400 KB three times.  100 000 x 128: 980 us with eight reads by 256 threads, 50 us with
-// three reads by 1024, 37 us now.
+// for the default sample of 100 000, of which six spill) -- a workgroup per column leaves every second compute unit idle at
+// 128 dimensions, and the other half waited for the same 400 KB three times.  100 000 x 128: 980 us with eight reads by 256
+// threads, 50 us with three reads by 1024, 37 us now.  REGS that a sample leaves unused cost as much as used ones, so there is a
+// form for every few thousand rows (training on 33 000 x 960 with 64 of them for 33: 175 us, three reads 166, with 48 165; 3000 x
+// 960 with 32 for 3: 132, three reads 123, with 8 120).
 // A column with values beyond any such range (NaN, infinities) takes bins of the ordered bits.
 template <uint32_t REGS>
 __global__ void __launch_bounds__(kBoundThreads)
@@ -1861,7 +1869,9 @@ sq_train_common(const float* x, uint64_t n, uint32_t dim, int bits, int metric, 
     hipLaunchKernelGGL(sq_sample_kernel, dim3(static_cast<uint32_t>(div_up(p.sample_count, 4 * kWave))), dim3(256), 0, st,
                        x, n, dim, p.step, p.sample_count, norms, sample_t);
     const uint64_t each = div_up(p.sample_count, kBoundThreads);
-    auto bounds = each <= 32 ? sq_bounds_kernel<32> : each <= 64 ? sq_bounds_kernel<64> : each <= 98 ? sq_bounds_kernel<98> : sq_bounds_kernel<0>;
+    auto bounds = each <= 8 ? sq_bounds_kernel<8> : each <= 16 ? sq_bounds_kernel<16> : each <= 32 ? sq_bounds_kernel<32>
+                  : each <= 48 ? sq_bounds_kernel<48> : each <= 64 ? sq_bounds_kernel<64>
+                  : each <= 80 ? sq_bounds_kernel<80> : each <= 98 ? sq_bounds_kernel<98> : sq_bounds_kernel<0>;
     hipLaunchKernelGGL(bounds, dim3(dim), dim3(kBoundThreads), 0, st, sample_t, p.sample_count, p.ignore_count, lb, diff,
                        upper, lower);
     if (uniform_out != nullptr) {
