@@ -23,7 +23,12 @@ fill_words(const FillJob& j) {
 }
 
 __global__ void __launch_bounds__(256)
-prepare_float_queries(FloatQueryArgs p, FillJob j) {
+prepare_float_queries(FloatQueryArgs p) {
+    prepare_float_row(p, blockIdx.x);
+}
+
+__global__ void __launch_bounds__(256)
+prepare_float_queries_filling(FloatQueryArgs p, FillJob j) {
     fill_words(j);
     prepare_float_row(p, blockIdx.x);
 }
@@ -299,8 +304,13 @@ prepare_queries(const vsag_amd_store* s, const float* queries, uint64_t nq, uint
         case VSAG_AMD_KIND_FP32:
         case VSAG_AMD_KIND_SQ8:
         case VSAG_AMD_KIND_SQ4:
-            hipLaunchKernelGGL(prepare_float_queries, grid, dim3(256), 0, st, float_query_args(s, queries, nq, ql, qtab, qmeta),
-                               job != nullptr ? *job : FillJob{});
+            if (job != nullptr) {
+                hipLaunchKernelGGL(prepare_float_queries_filling, grid, dim3(256), 0, st,
+                                   float_query_args(s, queries, nq, ql, qtab, qmeta), *job);
+            } else {
+                hipLaunchKernelGGL(prepare_float_queries, grid, dim3(256), 0, st,
+                                   float_query_args(s, queries, nq, ql, qtab, qmeta));
+            }
             break;
         case VSAG_AMD_KIND_SQ4_UNIFORM:
         case VSAG_AMD_KIND_SQ8_UNIFORM: {
