@@ -57,6 +57,23 @@ def test_one_query_sq8_equals_streaming_and_checker(lib, metric, n, d, k):
     st.destroy()
 
 
+@pytest.mark.parametrize("n", [65536, 131073, 196609, 300000])
+def test_one_query_around_the_selections_steps(lib, n):
+    """64 to 293 runs, a number of neighbours on both sides of every eight: rounds of the selection that are left out and not,
+    candidates that fill a step and not."""
+    lib = lib.load_library()
+    rng = np.random.default_rng(n)
+    st, _, _, _ = _sq8_store(rng, n, 16, orc.L2)
+    for k in (1, 7, 8, 9, 16, 17, 24, 25, 31, 32):
+        q = rng.standard_normal((1, 16)).astype(np.float32)
+        ids, ds = st.flat_scan(q, k)
+        tile, passes, _ = _route(lib)
+        sids, sds = _streaming(lib, st, q, k)
+        assert (tile, passes) == (1, 1)
+        assert np.array_equal(ids, sids) and np.array_equal(ds.view(np.uint32), sds.view(np.uint32)), k
+    st.destroy()
+
+
 def test_one_query_every_kind_equals_streaming(lib):
     lib = lib.load_library()
     rng = np.random.default_rng(5)

@@ -165,7 +165,8 @@ one_query_select_kernel(OneSelectArgs o) {
     const uint32_t k = o.k;
     // The k smallest minima.  Ranking all of them against each other is runs^2 comparisons on one compute unit; so
     // first, round by round, every group of 64 keys (a wave's worth) keeps its own k smallest -- the k smallest of all
-    // are among them -- until 64 are left, or a round would leave more than half of the last few.
+    // are among them -- until at most 128 are left, which are ranked in less than a round takes (by 0.3 us), or a round would
+    // leave more than half of the last few.
     uint32_t n = (o.runs + 63U) / 64U * 64U;
     for (uint32_t i = tid; i < n; i += blockDim.x) {
         keys[i] = i < o.runs ? o.mins[i] : kInfKey;
@@ -175,7 +176,7 @@ one_query_select_kernel(OneSelectArgs o) {
     }
     uint64_t* src = keys;
     uint64_t* dst = sv;
-    while (n > 64) {
+    while (n > 128) {
         const uint32_t groups = n / 64;
         const uint32_t kept = (groups * k + 63U) / 64U * 64U;
         if (n <= 256 && 2 * kept > n) {
@@ -226,23 +227,23 @@ one_query_select_kernel(OneSelectArgs o) {
     }
     __syncthreads();
     const uint32_t run_codes = o.run_tiles * kWave;
-    // What the bound admits out of the runs whose minimum it admits.  Sixteen runs at a time, a thread one code of each:
-    // the loads are issued together, before any of them is looked at.
+    // What the bound admits out of the runs whose minimum it admits.  Eight runs at a time, a thread one code of each: the eight
+    // loads are issued together, before any of them is looked at.  (Sixteen at a time: 100k x 128 sq8, k 1 18.3 -> 20.6 us a call,
+    // 1M x 128, k 20 40.4 -> 42.6, k 10 and k 16 37.5 and 37.8 either way.)
     const uint64_t nslots = o.ntiles * kWave;
-    constexpr uint32_t kTogether = 16;
-    for (uint32_t c0 = 0; c0 < ncand; c0 += kTogether) {
+    for (uint32_t c0 = 0; c0 < ncand; c0 += 8) {
         for (uint32_t off = tid; off < run_codes; off += blockDim.x) {
-            uint32_t od[kTogether];
-            uint64_t at[kTogether];
+            uint32_t od[8];
+            uint64_t at[8];
 #pragma unroll
-            for (uint32_t u = 0; u < kTogether; ++u) {
+            for (uint32_t u = 0; u < 8; ++u) {
                 const uint64_t key = c0 + u < ncand ? keys[c0 + u] : kInfKey;
                 const bool admitted = key != kInfKey && key <= bound;
                 at[u] = static_cast<uint64_t>(static_cast<uint32_t>(key) / run_codes) * run_codes + off;
                 od[u] = admitted && at[u] < nslots ? o.dist[at[u]] : 0xFFFFFFFFU;
             }
 #pragma unroll
-            for (uint32_t u = 0; u < kTogether; ++u) {
+            for (uint32_t u = 0; u < 8; ++u) {
                 const uint64_t kk = (static_cast<uint64_t>(od[u]) << 32) | static_cast<uint32_t>(at[u]);
                 if (od[u] != 0xFFFFFFFFU && kk <= bound) {
                     const uint32_t pos = atomicAdd(&nsv, 1U);
