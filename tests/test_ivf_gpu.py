@@ -486,3 +486,33 @@ def test_middling_batches_with_more_kept_than_items(lib, kind, metric, d, kcand)
         rids, rds = st.ivf_scan(q[i:i + 3], buckets[i:i + 3], kcand)
         assert np.array_equal(ds[i:i + 3].view(np.uint32), rds.view(np.uint32)) and np.array_equal(ids[i:i + 3], rids)
     st.destroy()
+
+
+@pytest.mark.parametrize("metric,d,kcand,nq,nprobe,long", [(orc.IP, 100, 80, 1000, 20, 0), (orc.IP, 256, 256, 1200, 14, 3000),
+                                                           (orc.COSINE, 33, 100, 1000, 20, 900), (orc.IP, 64, 90, 5300, 4, 6000)])
+@pytest.mark.parametrize("masked", [False, True])
+def test_the_nearest_list_goes_ahead(lib, metric, d, kcand, nq, nprobe, long, masked):
+    """16 000 to 22 000 pairs, lists of about seven tiles, more kept than a query has items: the nearest list of every query is scanned
+    before the others, longer ones in pieces (a list of `long` codes among them).  The ids and distance bits of a few queries
+    at a time."""
+    rng = np.random.default_rng(d + kcand)
+    n, nlist = 40000, 100
+    x, means = gaussian_mixture(rng, n, d, 100, 0.05)
+    q, _ = gaussian_mixture(rng, nq, d, 100, 0.05, means=means)
+    labels = rng.integers(1, nlist, n).astype(np.int32)
+    labels[:long] = 5
+    lb, diff = orc.sq_train(x, 8, metric)
+    st = Store(capi.KIND_SQ8, metric, d, lb=lb, diff=diff)
+    st.set_lists(orc.sq_encode(x, 8, lb, diff, metric), labels, nlist)
+    buckets = np.argsort(rng.random((nq, nlist)), 1)[:, :nprobe].astype(np.int32)
+    buckets[::13, 0] = 0     # an empty list
+    buckets[::9, 0] = -1
+    others = buckets[::3, 1:]
+    others[others == 5] = -1
+    buckets[::3, 0] = 5
+    deny = rng.random(n) < 0.3 if masked else None
+    ids, ds = st.ivf_scan(q, buckets, kcand, deny)
+    for i in list(range(0, nq, 100)) + [nq - 3]:
+        rids, rds = st.ivf_scan(q[i:i + 3], buckets[i:i + 3], kcand, deny)
+        assert np.array_equal(ds[i:i + 3].view(np.uint32), rds.view(np.uint32)) and np.array_equal(ids[i:i + 3], rids)
+    st.destroy()

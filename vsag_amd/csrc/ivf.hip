@@ -111,7 +111,6 @@ int launch_merge_partials(const uint64_t* partial, const uint32_t* partial_cnt, 
                           uint32_t stride, uint32_t k, uint32_t S, uint64_t nq, uint32_t* ids, float* dists,
                           hipStream_t st);
 
-// Up to five word arrays set in one launch.
 // Pairs of probe columns [p0, p1): how many queries probe each list.
 __global__ void
 count_pairs_kernel(const int32_t* buckets, uint64_t nq, uint32_t nprobe, uint32_t p0, uint32_t p1, uint32_t nlist,
@@ -640,12 +639,16 @@ plan_ivf(const vsag_amd_store* s, uint64_t nq, uint32_t nprobe, uint32_t kcand, 
     // them in vain, a wait for memory per tile (fp32 l2 200k x 200, 512 lists, k 100, 1000 queries x 24: 706 -> 667 us).
     const bool fills = kcand <= items;
     p->seeded = p->chunked && kcand <= 256 && fills;
-    // Then the nearest list of every query goes ahead, a list to a wave, where its bound spares the others more selecting than
-    // its own scan costs: sq8 codes of up to 256 dimensions (cheap to scan) and lists of at most six times as many codes as are
-    // kept (sq8 ip 200k x 200, 512 lists, 80 kept, 1000 queries x 24: 569 -> 490 us; 500k x 128, 800 lists, 200 kept, 3000 x 8:
-    // 825 -> 729.  Not with ten times as many, 1M x 96, 1000 lists, 100 kept, 900 x 20: 407 -> 428; nor of 960 dimensions, 300k,
-    // 1000 lists, 200 kept, 1500 x 12: 1516 -> 1701; nor fp32 codes, the first above with k 100: 667 -> 736).
+    // Then the nearest list of every query goes ahead where its bound spares the others more selecting than its own scan costs: sq8
+    // codes of up to 256 dimensions (cheap to scan), lists of four tiles or more but at most six times as many codes as are kept,
+    // and 6000 (query, tile) pairs in that pass, which fewer leave as a chain of latencies on a chip that is not full.  173 points
+    // of both sides, time without it over time with it: above the lines 0.95 to 1.37, 1.12 at the mean (sq8 ip 200k x 200, 512
+    // lists, 80 kept, 1000 queries x 24: 560 -> 475 us; 55k x 100, 128 lists, 200 kept, 3136 x 8: 1088 -> 794; the worst, 658k x
+    // 256, 2174 lists, 80 kept, 1165 x 17: 445 -> 469), below them 0.82 to 1.33, 1.01 at the mean and every third below 0.985.
+    // Nor with ten times as many codes as are kept, 1M x 96, 1000 lists, 100 kept, 900 x 20: 407 -> 428; nor of 960 dimensions,
+    // 300k, 1000 lists, 200 kept, 1500 x 12: 1516 -> 1701; nor fp32 codes, 200k x 200, k 100: 667 -> 736.
     p->nearest_first = p->chunked && four_pays && !fills && s->kind == VSAG_AMD_KIND_SQ8 && s->dpad <= 256 &&
+                       s->ntiles >= 4ull * s->nlist && nq * s->ntiles >= 6000ull * s->nlist &&
                        s->ntiles * kWave <= 6ull * kcand * s->nlist;
     // Large batches on sq4_uniform (and sq8_uniform / l2) lists: the streaming kernel scans the nearest list of every query, the int8
     // matrix cores the other columns, into two private lists per (query, list) pair.
@@ -823,7 +826,7 @@ vsag_amd_ivf_scan_topk_ex(const vsag_amd_store_t* s, const float* queries_dev, u
     }
     size_t lds = static_cast<size_t>(waves) * p.T * p.S * 8;
     // Whole lists: two passes, the nearest list of every query first (it seeds the per-query bound), then the
-    // rest.  Chunked lists: all probe columns at once.
+    // rest.  Chunked lists: all probe columns at once, or the nearest lists first (nearest_first).
     uint32_t cols[3] = {0, p.chunked && !p.nearest_first ? nprobe : 1, nprobe};
     // A pre-filter or a radius goes the streaming way (the matrix-core pass knows neither).
     const bool mfma = p.mfma && (options == nullptr || (options->deny_bits_dev == nullptr && options->use_radius == 0));
@@ -945,7 +948,10 @@ vsag_amd_ivf_scan_topk_ex(const vsag_amd_store_t* s, const float* queries_dev, u
         const bool nearest = p.nearest_first && pass == 0;
         const int t_pass = nearest ? 1 : cut_first ? std::min(p.T, 2) : p.T;
         if (nearest) {
-            first.tiles_per_item = 0x7FFFFFFFU;  // (a list at a time, by the kernel that knows chunks)
+            // An average list is one item, which gives the best bound; a list walked whole whatever its length was the chain that
+            // the launch ended with (98k x 32, 413 lists of 237 codes and one of 20 000: 597 -> 775 us with the pass, cut 563).
+            const uint32_t avg_tiles = static_cast<uint32_t>(s->ntiles / s->nlist);
+            first.tiles_per_item = std::max<uint32_t>(8, avg_tiles + avg_tiles / 4);
             first.seed = nullptr;
         }
         if (cut_first) {
@@ -964,8 +970,10 @@ vsag_amd_ivf_scan_topk_ex(const vsag_amd_store_t* s, const float* queries_dev, u
             regroup(p0, p1, pairs, static_cast<uint32_t>(t_pass), first.tiles_per_item, p.chunks_max);
         }
         // At most one partly filled query group per probed list, each cut into at most chunks_max items.
+        const uint64_t most = nearest ? std::min<uint64_t>(p.chunks_max, div_up(s->max_list_tiles, first.tiles_per_item))
+                                      : p.chunked || cut_first ? p.chunks_max : 1;
         uint64_t max_items =
-            (div_up(pairs, t_pass) + std::min<uint64_t>(s->nlist, pairs)) * ((p.chunked && !nearest) || cut_first ? p.chunks_max : 1);
+            (div_up(pairs, t_pass) + std::min<uint64_t>(s->nlist, pairs)) * most;
         dim3 grid(static_cast<uint32_t>(div_up(max_items, waves)));
         VA_TRY(launch_ivf(s, t_pass, grid, dim3(waves * kWave), static_cast<size_t>(waves) * t_pass * p.S * 8, st, a, first));
     }
