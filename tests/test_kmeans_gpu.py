@@ -54,6 +54,24 @@ def test_assign_matches_bruteforce_and_oracle(lib, n, d, k):
     assert abs(loss - oloss) <= 1e-4 * abs(oloss) + 1e-6
 
 
+@pytest.mark.parametrize("d,k", [(4, 1), (20, 100), (36, 128), (12, 129), (60, 384)])
+def test_assign_on_both_sides_of_two_workgroups_a_compute_unit(lib, d, k):
+    """As many workgroups as the chip holds at once and one row of tiles more: labels and distances of a few thousand rows at a
+    time, bit for bit."""
+    rng = np.random.default_rng(d + k)
+    tiles = -(-k // 128)
+    cus = 256
+    n = 2 * cus // tiles * 256
+    x = rng.standard_normal((n + 1, d)).astype(np.float32)
+    cent = rng.standard_normal((k, d)).astype(np.float32)
+    for rows in (n, n + 1):
+        labels, dist, _ = gpu_assign(x[:rows], cent)
+        for a in list(range(0, rows, 40000)) + [rows - 1]:
+            part, pdist, _ = gpu_assign(x[a:min(a + 3000, rows)], cent)
+            assert np.array_equal(labels[a:a + 3000], part)
+            assert np.array_equal(dist[a:a + 3000].view(np.uint32), pdist.view(np.uint32))
+
+
 def test_first_minimum_wins_ties(lib):
     # duplicated centroids: std::min_element keeps the first of equal minima
     rng = np.random.default_rng(3)

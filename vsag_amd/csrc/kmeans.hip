@@ -556,10 +556,12 @@ assign_tile(const float* __restrict__ X, uint64_t n, const float* __restrict__ C
     }
 }
 
-// (Tiles of 128 centroids: two workgroups to a compute unit, 128 registers a lane, so that one's start and end lie beside the
-// other's contraction: 904 914 x 416 rows, 98 centroids 919 -> 874 us.)
-template <int MI, bool STORE = false>
-__global__ void __launch_bounds__(kTileThreads, MI == 2 ? 4 : 1)
+// PAIR: two workgroups to a compute unit, so that one's start and end lie beside the other's contraction.  That leaves a lane 128
+// registers, of which tiles of 128 centroids spill 21, so it is for calls with more workgroups than the chip holds at once:
+// 1M x 128 rows, 100 centroids 940 -> 918 us an iteration, 1M x 960 3582 -> 3536, 150k x 24, 380 centroids 142 -> 136; with 79 to
+// 391 workgroups it was slower, 20k x 128, 64 centroids 70.2 -> 72.8, 100k x 128, 128 centroids 120.4 -> 121.8.
+template <int MI, bool STORE = false, bool PAIR = false>
+__global__ void __launch_bounds__(kTileThreads, PAIR ? 4 : 1)
 kmeans_assign_tile_kernel(const float* __restrict__ X, uint64_t n, const float* __restrict__ C, uint32_t k, uint32_t dim,
                           const float* __restrict__ ynorm, unsigned long long* __restrict__ best, TilePlan plan) {
     assign_tile<MI, STORE, false>(X, n, C, k, dim, ynorm, best, plan, blockIdx.x);
@@ -1131,6 +1133,7 @@ assign_launch(const float* x, uint64_t n, uint32_t dim, const float* cent, uint3
                 }
             };
             allow(reinterpret_cast<const void*>(kmeans_assign_tile_kernel<2>), 2);
+            allow(reinterpret_cast<const void*>(kmeans_assign_tile_kernel<2, false, true>), 2);
             allow(reinterpret_cast<const void*>(kmeans_assign_tile_kernel<4>), 4);
             allow(reinterpret_cast<const void*>(kmeans_assign_open_kernel<2>), 2);
             allow(reinterpret_cast<const void*>(kmeans_assign_open_kernel<4>), 4);
@@ -1167,8 +1170,10 @@ assign_launch(const float* x, uint64_t n, uint32_t dim, const float* cent, uint3
                 hipLaunchKernelGGL(kmeans_assign_tile_kernel<4>, grid, dim3(kTileThreads), tile_lds_bytes(4), st,
                                    x + r0 * dim, rows, cent, k, dim, b.ynorm, b.best + r0, plan);
             } else {
-                hipLaunchKernelGGL(kmeans_assign_tile_kernel<2>, grid, dim3(kTileThreads), tile_lds_bytes(2), st,
-                                   x + r0 * dim, rows, cent, k, dim, b.ynorm, b.best + r0, plan);
+                const bool pair = static_cast<uint64_t>(plan.rtiles) * plan.ctiles > 2ull * device_cu_count();
+                hipLaunchKernelGGL((pair ? kmeans_assign_tile_kernel<2, false, true> : kmeans_assign_tile_kernel<2>), grid,
+                                   dim3(kTileThreads), tile_lds_bytes(2), st, x + r0 * dim, rows, cent, k, dim, b.ynorm,
+                                   b.best + r0, plan);
             }
         }
     } else {
