@@ -291,10 +291,10 @@ scatter_pairs_kernel(const int32_t* buckets, uint64_t nq, uint32_t nprobe, uint3
     }
 }
 
-// The three regrouping steps above for a small batch (probe columns [p0, p1); ALL: they are all) in one workgroup.  A chain of latencies bounds it:
-// a bucket is loaded, its counter raised, its place written.  With the counters in LDS (LDS: lists up to kRegroupLists;
-// more lists count in memory) and kRegroupInFlight buckets of a thread loaded together, 24 000 pairs of 512 lists take 17 us
-// (one bucket at a time, counters in memory: 81; the call 651 -> 589), 32 pairs of 1024 lists 5 (the call 127 -> 122).
+// The three regrouping steps above for a small batch (probe columns [p0, p1); ALL: they are all) in one workgroup.  A chain of
+// latencies bounds it: a bucket is loaded, its counter raised, its place written.  With the counters in LDS (LDS: lists up to
+// kRegroupLists; more lists count in memory) and kRegroupInFlight buckets of a thread loaded together, 24 000 pairs of 512 lists
+// take 17 us (one bucket at a time, counters in memory: 81; the call 651 -> 589), 32 pairs of 1024 lists 5 (the call 127 -> 122).
 constexpr uint32_t kRegroupInFlight = 8;
 
 template <bool LDS, bool ALL>

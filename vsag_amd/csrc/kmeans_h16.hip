@@ -28,10 +28,10 @@
 // 67.9; 480k x 960, k 256 2.42 / 3.51 / 2.68; of a single slab (65536 x 128, k 512) 0.12 / 0.18 / 0.18.  Where nothing is
 // open, asking costs 0.5 to 1 %.
 //
-// 1M x 960 rows, 4096 centroids (one assignment): 63.3 -> 11.2 ms.  Of that the contraction takes 7.4 (7.9e12 flop: 1070
-// TFLOP/s, where matrix instructions on random operands in registers reach 1610 to 1690 and with their reads of LDS 1580,
-// all bound by power), the rounding of the rows 1.25 (5.8 GB at 4.6 TB/s) and the rescoring 2.4 (3.8 GB of rows, 0.8 GB of
-// table, one to three centroids a row).
+// 1M x 960 rows, 4096 centroids (one assignment): 63.3 -> 11.2 ms.  Of that the contraction takes 7.4 to 7.8 (7.9e12 flop: 1010
+// to 1070 TFLOP/s, from card to card, where matrix instructions on random operands in registers reach 1730 and with their reads
+// of LDS 1610, bound by power: 2330 and 2240 on zeros), the rounding of the rows 1.25 (5.8 GB at 4.6 TB/s) and the rescoring 2.4
+// (3.8 GB of rows, 0.8 GB of table, one to three centroids a row).
 #include "kmeans_h16.h"
 
 #include <algorithm>
@@ -385,7 +385,8 @@ lds_offset(const void* p) {
 
 // Lane l's 16 bytes (touch_line: 4, for the sake of their line) at base + bytes go to LDS at to + 16 l (4 l); `to` is the same
 // in all lanes.  In assembly because the compiler would wait for all such loads before any read of LDS; who reads what they
-// bring waits for vmcnt and a barrier itself.
+// bring waits for vmcnt and a barrier itself.  (m0 is reserved: the compiler keeps nothing in it from one instruction to the
+// next, sets it itself where it needs it, and takes it in no list of clobbers.)
 __device__ inline void
 load_to_lds(const void* base, uint32_t bytes, uint32_t to) {
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" : : "s"(to), "v"(bytes), "s"(base) : "memory");

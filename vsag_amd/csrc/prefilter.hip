@@ -388,7 +388,7 @@ prefilter_tau_kernel(const float* qtab, uint32_t qstride, uint32_t kdim, const f
 
 // One candidate per lane against one query: the granules of its code, AHEAD fetched before the first is used.  Whole groups
 // go without a condition on any granule: each condition was a branch, behind which the query's scalars were waited for alone
-// (rescore_kernel, 100k x 768 fp32 cosine, 32 queries: 60 -> 42 us, the call 222 -> 211; 100k x 128 fp32, 1000 queries: 19.4
+// (rescore_valued_wave_kernel, 100k x 768 fp32 cosine, 32 queries: 60 -> 42 us, the call 222 -> 211; 100k x 128 fp32, 1000 queries: 19.4
 // -> 17.9 us).
 template <int KIND, int METRIC, uint32_t AHEAD>
 __device__ __forceinline__ void
@@ -789,7 +789,10 @@ rescore_valued_wave_kernel(ScanArgs a, RescoreArgs r) {
 // query of the first 7000 of 60 000 cycles go to the k-th smallest, 15 000 to the sums, the rest to waits for memory.)
 constexpr uint32_t kValuedStage = 64 * 33;  // granules in LDS: of 64 rows 32, or of 32 rows 64, and one apart (32 x 65)
 constexpr uint32_t kValuedThreads = 256;
-constexpr uint64_t kValuedFewQueries = 512;  // (1000 queries against 100k x 128 fp32: 18.1 us, and 17.5 with a wave each)
+// Calls with a workgroup / a wave each, us: fp32 100k x 128, k 10, 400 queries 106 / 112, 512 114 / 118, 640 133 / 132, 1000 174 /
+// 174; sq4 300k x 256 under a mask, k 20, 512 223 / 229, 640 266 / 265, 1000 393 / 391; sq8_uniform 200k x 384, 512 185 / 189, 640
+// 204 / 203, 1000 287 / 282; fp32 100k x 768 512 451 / 458, 640 500 / 509, 1000 741 / 749.
+constexpr uint64_t kValuedFewQueries = 512;
 constexpr uint32_t kValuedEach = 8;      // records of a thread
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 constexpr uint32_t kValuedWords = 1024;  // words of the query in LDS: the most that a piece takes
